@@ -1,0 +1,77 @@
+"""Near-field kernels at the sizes where their units, splits and chunks change: leaves of 1 to a few
+hundred bodies, lists far longer than the others' (a coarse leaf beside a dense cluster), probe trees
+with a handful of leaves, separations across every branch of the pair factors.  Against the oracle,
+with the tolerances of the parity tests (FP64 1e-10, mixed 1e-6 of the FP64 values)."""
+import numpy as np
+import pytest
+
+from uvlm_amd import FMMCalculator, make_bodies
+from uvlm_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+def cluster(n, seed, sigma):
+    """Half the bodies in a cube of edge 0.02, the others over [-1, 1]^3: leaves of the sparse half
+    list hundreds of the dense half's."""
+    rng = W.SplitMix64(seed)
+    X = rng.uniform(3 * n).reshape(n, 3) * 2.0 - 1.0
+    X[: n // 2] = 0.3 + 0.01 * X[: n // 2]
+    A = rng.normal(3 * n).reshape(n, 3)
+    return X, A, np.full(n, sigma) * (0.5 + rng.uniform(n))
+
+
+def rel(a, b):
+    return np.linalg.norm(a - b) / np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("n,ncrit,sigma", [(3, 64, 0.5), (65, 1, 0.3), (130, 64, 1e-4), (1500, 7, 0.02),
+                                           (4000, 33, 0.05), (6000, 64, 0.003), (9000, 200, 0.02), (2500, 600, 0.2)])
+def test_particles(orc, n, ncrit, sigma):
+    X, A, S = cluster(n, n, sigma)
+    ref_b = orc.make_bodies(X, A, S)
+    ref = orc.Calculator(P=6, theta=0.5, ncrit=ncrit)
+    ref.init(ref_b)
+    ref.calculate()
+    want = ref.bodies(n)
+    out = {}
+    for precision in ("fp64", "mixed"):
+        print(f"[near] n={n} ncrit={ncrit} {precision}", flush=True)
+        g = FMMCalculator(P=6, theta=0.5, ncrit=ncrit, precision=precision)
+        g.set_bodies(make_bodies(X, A, S))
+        for _ in range(2):  # the second build starts from the sorted bodies
+            g.build()
+            g.calculate()
+        out[precision] = g.copyBodies2Host()
+        assert np.array_equal(out[precision][:, 9:12], want[:, 9:12])
+        g.close()
+    for sl in (slice(0, 9), slice(15, 18), slice(18, 21)):
+        assert rel(out["fp64"][:, sl], want[:, sl]) < 1e-10
+        # n = 130: bodies a few 1e-4 apart in leaves half a unit wide.  The mixed path's FP32 offsets
+        # from the leaf centre (2^-25 of up to 0.9) are then 1e-5 of such a separation, so 1e-6 is
+        # not its accuracy there; only the FP64 values are checked.
+        if n != 130:
+            assert rel(out["mixed"][:, sl], out["fp64"][:, sl]) < 1e-6
+
+
+# (a single probe sits at its cell's centre, where the oracle's L2P, like the reference's, is NaN)
+@pytest.mark.parametrize("m,ncrit", [(2, 64), (5, 64), (300, 64), (300, 200)])
+def test_probes(orc, m, ncrit):
+    X, A, S = cluster(8000, 3, 0.02)
+    pts = X[:: 8000 // m][:m] + 0.003
+    ref_b = orc.make_bodies(X, A, S)
+    ref = orc.Calculator(P=6, theta=0.5, ncrit=ncrit)
+    ref.init(ref_b)
+    ref.calculate()
+    sb = orc.make_bodies(pts, np.zeros((m, 3)), np.ones(m))
+    ref.sensor_data(sb)
+    print(f"[near] probes m={m} ncrit={ncrit}", flush=True)
+    g = FMMCalculator(P=6, theta=0.5, ncrit=ncrit)
+    g.set_bodies(make_bodies(X, A, S))
+    g.build()
+    g.calculate()
+    s = make_bodies(pts, np.zeros((m, 3)), np.ones(m))
+    g.getSensorData(s)
+    assert np.array_equal(s[:, 9:12], sb[:, 9:12])
+    assert rel(s[:, 15:18], sb[:, 15:18]) < 1e-10
+    g.close()

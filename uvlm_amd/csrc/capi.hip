@@ -188,8 +188,7 @@ void do_build(uvlm_handle h, bool defer_outputs = false)
   h->gap = h->near_c > 0.0 ? h->near_c * max_value(s, h->sc, h->F(F_SIG), h->N) : 0.0;
   traverse(s, h->sc, h->tree, h->tree, h->prm.theta, h->lists, h->gap);
   UVLM_HIP(hipEventRecord(h->ev[EV_LISTS], s));
-  count_interactions(s, h->sc, h->tree, h->tree, h->lists, &h->lists.n_interactions);
-  UVLM_HIP(hipStreamSynchronize(s));
+  near_units(s, h->sc, h->tree, h->tree, h->prm.ncrit, h->lists);  // ends with a synchronisation
   h->tm.tree_ms        = ev_ms(h, EV_B0, EV_TREE);
   h->tm.lists_ms       = ev_ms(h, EV_TREE, EV_LISTS);
   h->tm.n_bodies       = h->N;
@@ -222,8 +221,8 @@ void do_eval(uvlm_handle h, bool sync)
   UVLM_HIP(hipEventRecord(h->ev[EV_UP], s));
   m2l(s, P, t, t, h->lists, h->sched, M, L);
   UVLM_HIP(hipEventRecord(h->ev[EV_M2L], s));
-  p2p(s, t, t, h->lists, h->st.as<double>(), h->cap, h->st.as<double>(), h->cap, h->st.as<double>(), h->cap,
-      h->prm.precision, 0, h->prm.ncrit);
+  p2p(s, h->sc, t, t, h->lists, h->st.as<double>(), h->cap, h->st.as<double>(), h->cap, h->st.as<double>(), h->cap,
+      h->prm.precision, 0);
   UVLM_HIP(hipEventRecord(h->ev[EV_P2P], s));
   for (int l = 1; l < t.nlevels; l++) l2l_level(s, P, t, l, L, h->sched);
   l2p_stretch(s, P, t, L, h->st.as<double>(), h->cap, h->prm.stretching, h->prm.formulation, 0);
@@ -326,13 +325,14 @@ void sensor_pass(uvlm_handle h, int64_t m, bool with_j = false)
   gather_fields(s, h->sst.as<double>(), h->sst2.as<double>(), sc, sc, N_FIELDS, h->sperm.as<int32_t>(), m);
   swap_buf(h->sst, h->sst2);
   traverse(s, h->sc, h->stree, h->tree, h->prm.theta, h->slists, h->gap);
+  near_units(s, h->sc, h->stree, h->tree, h->prm.ncrit, h->slists);
   const int P = h->prm.P;
   h->Ls.reserve(sizeof(double2) * h->NT * h->stree.C);
   double2 *Ls = h->Ls.as<double2>();
   reset_sensor_rates(s, h->sst.as<double>(), sc, m);
   m2l(s, P, h->stree, h->tree, h->slists, h->sched, h->M.as<double2>(), Ls, &h->sc);
-  p2p(s, h->stree, h->tree, h->slists, h->sst.as<double>(), sc, h->st.as<double>(), h->cap, h->sst.as<double>(), sc,
-      h->prm.precision, with_j ? 0 : 1, h->prm.ncrit, &h->sc);
+  p2p(s, h->sc, h->stree, h->tree, h->slists, h->sst.as<double>(), sc, h->st.as<double>(), h->cap, h->sst.as<double>(),
+      sc, h->prm.precision, with_j ? 0 : 1);
   for (int l = 1; l < h->stree.nlevels; l++) l2l_level(s, P, h->stree, l, Ls, h->sched);
   l2p_stretch(s, P, h->stree, Ls, h->sst.as<double>(), sc, h->prm.stretching, h->prm.formulation, 1);
 }
@@ -423,6 +423,7 @@ void probe_adjoint_core(uvlm_handle h, int64_t m)
   // the forward probe lists, transposed: targets = particle cells, sources = probe cells
   traverse(s, h->sc, h->stree, h->tree, h->prm.theta, h->slists, h->gap);
   transpose_lists(s, h->sc, h->stree, h->tree, h->slists, h->alists);
+  near_units(s, h->sc, h->tree, h->stree, h->prm.ncrit, h->alists);
   // probe multipoles (root included: a probe cell is a source here)
   h->Ms.reserve(sizeof(double2) * NT * h->stree.C);
   double2 *Ms = h->Ms.as<double2>();
@@ -440,7 +441,7 @@ void probe_adjoint_core(uvlm_handle h, int64_t m)
   m2l(s, P, h->tree, h->stree, h->alists, h->sched, Ms, La);
   zero_doubles(s, (double *)La, 2 * NT);  // the particle root multipole is never formed forward
   for (int l = 1; l < h->tree.nlevels; l++) l2l_level(s, P, h->tree, l, La, h->sched);
-  p2p(s, h->tree, h->stree, h->alists, a, cap, h->sst.as<double>(), sc, a, cap, h->prm.precision, 2, h->prm.ncrit);
+  p2p(s, h->sc, h->tree, h->stree, h->alists, a, cap, h->sst.as<double>(), sc, a, cap, h->prm.precision, 2);
   l2p_stretch(s, P, h->tree, La, a, cap, UVLM_TRANSPOSED, UVLM_CVPM, 0);
   h->evaluated = false;  // L now holds adjoint locals
 }

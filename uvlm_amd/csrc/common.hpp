@@ -106,6 +106,11 @@ struct Tree {
 struct Lists {
   int64_t np2p = 0, nm2l = 0, n_interactions = 0;
   DevBuf  p2p_off, p2p_src, m2l_off, m2l_src;  // int32
+  // near-field units of the P2P list (near_units): runs of entries of one target leaf each, rows of
+  // partial sums and leaves cut into several units
+  int64_t n_units = 0, n_rows = 0, n_multi = 0;
+  bool    wide = false;  // 256 lanes per unit's workgroup, else 64
+  DevBuf  units, multi;  // int4
 };
 
 // Scratch shared by tree builds and traversals.
@@ -115,8 +120,8 @@ struct Scratch {
   DevBuf rec_cx, rec_cy, rec_cz;
   DevBuf partial, counters, perm;
   DevBuf front0, front1, out_p2p, out_m2l;
-  DevBuf p2p_seg, p2p_part;  // P2P list segments and their partial sums (few-target case)
-  DevBuf m2l_seg, m2l_part;  // the same for M2L
+  DevBuf unit_work, unit_cnt, p2p_part;  // near-field units: work per leaf, totals, partial sums
+  DevBuf m2l_seg, m2l_part;  // M2L list segments and their partial sums (few-target case)
   int64_t rec_cap = 0;
 };
 
@@ -135,7 +140,6 @@ void gather_i32(hipStream_t s, const int32_t *src, int32_t *dst, const int32_t *
 // Lists of (sources as targets): CSR by the cells of `in_sources`, entries = cells of `in_targets`.
 void transpose_lists(hipStream_t s, Scratch &sc, const Tree &in_targets, const Tree &in_sources, const Lists &in,
                      Lists &out);
-void count_interactions(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &st, const Lists &l, int64_t *out);
 
 // far.hip
 struct M2LSchedule {
@@ -179,9 +183,9 @@ void l2p_stretch(hipStream_t s, int P, const Tree &t, const double2 *L, double *
 
 // near.hip
 // max_leaf: an upper bound of the target leaves' body counts (ncrit for a built tree)
-void p2p(hipStream_t s, const Tree &tt, const Tree &stree, const Lists &l, const double *tgt, int64_t tcap,
-         const double *src, int64_t scap, double *out, int64_t ocap, int precision, int sensor_mode,
-         int64_t max_leaf, Scratch *sc = nullptr);
+void near_units(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &st, int64_t max_leaf, Lists &l);
+void p2p(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &stree, const Lists &l, const double *tgt, int64_t tcap,
+         const double *src, int64_t scap, double *out, int64_t ocap, int precision, int sensor_mode);
 
 void gauss_near(hipStream_t s, const Tree &tt, const Tree &stree, const Lists &l, const double *tgt, int64_t tcap,
                 const double *srcst, int64_t scap, double *out, int64_t ocap, int mode, int field, double prefix);

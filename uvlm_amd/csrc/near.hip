@@ -7,15 +7,14 @@
 //   u -= f1 (dX x a_j),   J[a][b] -= f2 (dX x a_j)_a dX_b + f1 eps_{abk} a_j,k.
 // Only the source core size sigma_j enters (multipoleKernels.hpp:243).
 //
-// Layout: one workgroup of BLK lanes per target leaf (64, or 256 when leaves may hold more than
-// 64 bodies).  Lanes = (target t) x (source split s): a pass takes ntp of the leaf's targets
-// (near_targets_per_pass) and S = BLK / ntp splits, each taking every S-th source, and the
-// partial sums are combined in a fixed order (cross-lane adds or LDS, no atomics).  The bodies
-// of all source leaves in the target's CSR list are streamed through LDS in full chunks of BLK
-// across leaf boundaries (prefix sums of the leaf sizes in LDS, binary search per slot), so
-// small leaves do not pay a barrier per leaf.
+// Layout: one workgroup of BLK lanes (64 or 256) per unit of a target leaf's list (near_units).  Lanes = (target t) x (source split s): a pass takes ntp
+// of the leaf's targets (near_targets_per_pass) and S = BLK / ntp splits, each taking every S-th
+// source, and the partial sums are combined in a fixed order (LDS, no atomics).  The bodies of all
+// source leaves in the unit's list entries are streamed through LDS in full chunks across leaf
+// boundaries (prefix sums of the leaf sizes in LDS, binary search per slot), so small leaves do
+// not pay a barrier per leaf.
 //
-// FP64 path: the reference formula (erf, exp, sqrt in double).
+// FP64 path: G = g/s^3 and its derivative in double (pair_kernel.hpp), two sources per step.
 // Mixed path: FP32 arithmetic on coordinates relative to the target leaf centre (the source
 // offsets are formed in FP64 while staging), two sources per step over zero-padded chunks (one
 // trip count for all lanes), per-chunk FP32 partial sums added into FP64 per-target
@@ -33,6 +32,7 @@ namespace {
 
 constexpr int WG = 64;
 
+// Staged sources of the direct sum.
 struct SrcF64 {
   double x, y, z, ax, ay, az, invS2, halfInvS2;
 };
@@ -42,31 +42,33 @@ struct SrcF64 {
 // into J once per chunk (fold_antisym) instead of six multiply-adds per pair.  c is
 // perpendicular to dX, so c (x) dX is traceless and its zz entry (acc[11]) is formed from the
 // xx and yy sums in fold_antisym.
-__device__ __forceinline__ void accumulate_pair(float *acc, float dx, float dy, float dz, float ax, float ay, float az,
-                                                float f1, float f2, bool withJ)
+__device__ __forceinline__ float  fma_(float a, float b, float c) { return fmaf(a, b, c); }
+__device__ __forceinline__ double fma_(double a, double b, double c) { return fma(a, b, c); }
+template <class T>
+__device__ __forceinline__ void accumulate_pair(T *acc, T dx, T dy, T dz, T ax, T ay, T az, T f1, T f2, bool withJ)
 {
-  const float cx = dy * az - dz * ay, cy = dz * ax - dx * az, cz = dx * ay - dy * ax;
-  acc[0] = fmaf(f1, cx, acc[0]);
-  acc[1] = fmaf(f1, cy, acc[1]);
-  acc[2] = fmaf(f1, cz, acc[2]);
+  const T cx = dy * az - dz * ay, cy = dz * ax - dx * az, cz = dx * ay - dy * ax;
+  acc[0] = fma_(f1, cx, acc[0]);
+  acc[1] = fma_(f1, cy, acc[1]);
+  acc[2] = fma_(f1, cz, acc[2]);
   if (withJ) {
-    const float k0 = f2 * cx, k1 = f2 * cy, k2 = f2 * cz;
-    acc[3]  = fmaf(k0, dx, acc[3]);
-    acc[4]  = fmaf(k0, dy, acc[4]);
-    acc[5]  = fmaf(k0, dz, acc[5]);
-    acc[6]  = fmaf(k1, dx, acc[6]);
-    acc[7]  = fmaf(k1, dy, acc[7]);
-    acc[8]  = fmaf(k1, dz, acc[8]);
-    acc[9]  = fmaf(k2, dx, acc[9]);
-    acc[10] = fmaf(k2, dy, acc[10]);
-    acc[12] = fmaf(f1, ax, acc[12]);
-    acc[13] = fmaf(f1, ay, acc[13]);
-    acc[14] = fmaf(f1, az, acc[14]);
+    const T k0 = f2 * cx, k1 = f2 * cy, k2 = f2 * cz;
+    acc[3]  = fma_(k0, dx, acc[3]);
+    acc[4]  = fma_(k0, dy, acc[4]);
+    acc[5]  = fma_(k0, dz, acc[5]);
+    acc[6]  = fma_(k1, dx, acc[6]);
+    acc[7]  = fma_(k1, dy, acc[7]);
+    acc[8]  = fma_(k1, dz, acc[8]);
+    acc[9]  = fma_(k2, dx, acc[9]);
+    acc[10] = fma_(k2, dy, acc[10]);
+    acc[12] = fma_(f1, ax, acc[12]);
+    acc[13] = fma_(f1, ay, acc[13]);
+    acc[14] = fma_(f1, az, acc[14]);
   }
 }
 // J[2][2] = -(J[0][0] + J[1][1]) and J[a][b] += eps_{abk} F_k with F = acc[12..14] (row-major J
 // in acc[3..11]).
-__device__ __forceinline__ void fold_antisym(float *acc)
+template <class T> __device__ __forceinline__ void fold_antisym(T *acc)
 {
   acc[11] = -(acc[3] + acc[7]);
   acc[4] += acc[14];
@@ -80,70 +82,82 @@ __device__ __forceinline__ void fold_antisym(float *acc)
 // TSIG: the core size comes from the TARGET body instead of the source.  That is the
 // transposed near-field kernel used by the adjoint (a particle's own sigma, with the
 // particle now on the target side).
-// SPLIT: workgroup b takes the list entries [seg[3b+1], seg[3b+2]) of target leaf seg[3b] and
-// writes its un-negated sums to part + b * 12 * maxnt (field-major, maxnt entries per field);
-// k_p2p_reduce adds the segments of each target in order.
-template <bool MIXED, bool WITH_J, bool TSIG, int BLK, bool SPLIT = false>
-__global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(MIXED ? 5 : 1))) void k_p2p(const int32_t *__restrict__ leaves, int64_t nleaf,
-                                            const int32_t *__restrict__ tbody, const int32_t *__restrict__ tnbody,
-                                            const double *__restrict__ tcx, const double *__restrict__ tcy,
-                                            const double *__restrict__ tcz, const int32_t *__restrict__ off,
-                                            const int32_t *__restrict__ src, const int32_t *__restrict__ sbody,
-                                            const int32_t *__restrict__ snbody, const double *__restrict__ tst,
-                                            int64_t tcap, const double *__restrict__ sst, int64_t scap,
-                                            double *__restrict__ out, int64_t ocap,
-                                            const int32_t *__restrict__ seg = nullptr, double *__restrict__ part = nullptr,
-                                            int maxnt = 0)
+//
+// One workgroup per unit (near_units): the list entries [q0, q1) of target leaf w.  A leaf whose
+// list is one unit is stored directly; a leaf cut into several units leaves each unit's sums
+// (12 rows of nt doubles) at part + 12 * row, and k_p2p_reduce adds them in unit order, so the
+// result does not depend on which unit runs when.
+//
+// Chunks: 64 lanes stage 128 sources at a time (two per lane, both searches and all loads in
+// flight together) and 256 lanes 256.
+//
+// Bound by VALU issue: 47 lane-instructions a pair in FP32, 82 in FP64 while x < X64 (62 of them
+// multiply-adds).  Units and chunks against one workgroup per leaf, and in FP64 the polynomial pair
+// factors against erf, exp, sqrt and divisions: 1M two rings FP64 10.2 -> 4.4 ms (1.54e9 pairs), 8k
+// ring FP64 1.34 -> 0.075 ms, 60k cube mixed 2.65 -> 1.18 ms; 4M two rings
+// mixed 10.0 -> 9.6 ms.
+template <bool MIXED, bool WITH_J, bool TSIG, int BLK>
+__global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(MIXED ? 5 : 3))) void k_p2p(
+    const int4 *__restrict__ units, const int32_t *__restrict__ leaves, const int32_t *__restrict__ tbody,
+    const int32_t *__restrict__ tnbody, const double *__restrict__ tcx, const double *__restrict__ tcy,
+    const double *__restrict__ tcz, const int32_t *__restrict__ src, const int32_t *__restrict__ sbody,
+    const int32_t *__restrict__ snbody, const double *__restrict__ tst, int64_t tcap, const double *__restrict__ sst,
+    int64_t scap, double *__restrict__ out, int64_t ocap, double *__restrict__ part)
 {
-  // One LDS buffer holds the staged sources during the pair loops and the split partial sums
-  // after them: mixed sources take two float4 per entry for 2 BLK entries (BLK staged, the rest
-  // zero padding), FP64 sources one SrcF64 per entry, the partials 12 doubles per lane.
-  constexpr int SMEM = BLK == 64 ? 64 * BLK : 96 * BLK;
+  // One LDS buffer holds the staged sources during the pair loops (two float4 or two double4 an
+  // entry) and the partial sums of the splits after them (12 doubles per lane).  CH entries are
+  // staged; up to ENT are read, those past the chunk are padding (2 S <= CH, see near_splits: at
+  // most 2 S ceil(CH / 2 S) <= 3/2 CH entries).
+  constexpr int CH = BLK == 64 ? 128 : 256, ENT = CH + CH / 2, PER = CH / BLK, ESZ = MIXED ? 32 : 64;
+  constexpr int SMEM = ENT * ESZ > 96 * BLK ? ENT * ESZ : 96 * BLK;
   __shared__ __align__(16) unsigned char smem[SMEM];
-  __shared__ int pref[SEG + 1], lb[SEG], ln[SEG];
-  float4 *s32 = reinterpret_cast<float4 *>(smem);
-  SrcF64 *s64 = reinterpret_cast<SrcF64 *>(smem);
+  __shared__ int pref[SEG + 1], lb[SEG];
+  using T  = typename std::conditional<MIXED, float, double>::type;
+  using T4 = typename std::conditional<MIXED, float4, double4>::type;
+  T4     *sv  = reinterpret_cast<T4 *>(smem);
   double *red = reinterpret_cast<double *>(smem);
-  const int64_t w = SPLIT ? seg[3 * blockIdx.x] : blockIdx.x;
-  if (w >= nleaf) return;
-  const int t = leaves[w], tb = tbody[t], nt = tnbody[t];
-  const int lane = threadIdx.x;
-  // lanes = (target ti) x (source split si): ntp targets per pass (near_targets_per_pass), S = BLK /
-  // ntp splits; the BLK - ntp * S lanes left over take no sources
-  const int    ntp = near_targets_per_pass<BLK>(nt), S = BLK / ntp, ti = lane % ntp, si = lane / ntp;
+  const int4 un = units[blockIdx.x];
+  const int  t = leaves[un.x], tb = tbody[t], nt = tnbody[t], q0 = un.y, q1 = un.z, prow = un.w;
+  const int  lane = threadIdx.x;
+  // lanes = (target ti) x (source split si): ntp targets per pass (near_targets_per_pass); the
+  // BLK - ntp * S lanes left over take the first split's sources and are dropped
+  const int    ntp = near_targets_per_pass<BLK>(nt), S = near_splits<BLK>(ntp), ti = lane % ntp, si = lane / ntp;
   const bool   lane_on = si < S;
-  const double cxt = tcx[t], cyt = tcy[t], czt = tcz[t];
-  const int    q0 = SPLIT ? seg[3 * blockIdx.x + 1] : off[t], q1 = SPLIT ? seg[3 * blockIdx.x + 2] : off[t + 1];
+  // offsets from the target leaf's centre (mixed: formed in FP64, then rounded to FP32); FP64 keeps
+  // the absolute coordinates
+  const double cxt = MIXED ? tcx[t] : 0.0, cyt = MIXED ? tcy[t] : 0.0, czt = MIXED ? tcz[t] : 0.0;
   for (int c0 = 0; c0 < nt; c0 += ntp) {
-    const int  i     = c0 + ti;
-    const bool valid = lane_on && i < nt;
+    const int     i     = c0 + ti;
+    const bool    valid = lane_on && i < nt;
     const int64_t bi = tb + (valid ? i : 0);
-    const double  xi = tst[(F_X + 0) * tcap + bi], yi = tst[(F_X + 1) * tcap + bi], zi = tst[(F_X + 2) * tcap + bi];
-    const float   rxi = (float)(xi - cxt), ryi = (float)(yi - cyt), rzi = (float)(zi - czt);
-    const int     jfirst = lane_on ? si : BLK;  // lanes without a split skip the FP64 pair loop
+    const T rxi = (T)(tst[(F_X + 0) * tcap + bi] - cxt), ryi = (T)(tst[(F_X + 1) * tcap + bi] - cyt),
+            rzi = (T)(tst[(F_X + 2) * tcap + bi] - czt);
     // target-sigma constants (TSIG only)
-    const double  tsg = TSIG ? tst[F_SIG * tcap + bi] : 1.0;
-    const double  tqq = 0.5 / (tsg * tsg), tsq = sqrt(tqq);
-    const float   t_q = (float)tqq, t_c1 = (float)(tqq * tsq * INV_4PI), t_c2 = (float)(2.0 * tqq * tqq * tsq * INV_4PI);
-    const double  t_is2 = 1.0 / (tsg * tsg), t_half = 0.5 * t_is2;
-    double        acc[12];
-    for (int k = 0; k < 12; k++) acc[k] = 0.0;
+    const double tsg = TSIG ? tst[F_SIG * tcap + bi] : 1.0;
+    const double tqq = 0.5 / (tsg * tsg), tc1 = tqq * sqrt(tqq) * INV_4PI;
+    const T      t_q = (T)tqq, t_c1 = (T)tc1, t_c2 = (T)(2.0 * tqq * tc1);
+    double       acc[MIXED ? 12 : 15];
+    for (int k = 0; k < (MIXED ? 12 : 15); k++) acc[k] = 0.0;
     for (int g0 = q0; g0 < q1; g0 += SEG) {
       const int nseg = min(SEG, q1 - g0);
       __syncthreads();
       for (int k = lane; k < nseg; k += BLK) {
         const int sl = src[g0 + k];
         lb[k]        = sbody[sl];
-        ln[k]        = snbody[sl];
+        pref[k]      = snbody[sl];
       }
       __syncthreads();
-      if (lane < 64) lds_prefix(pref, ln, nseg);
+      if (lane < 64) lds_prefix(pref, pref, nseg);
       __syncthreads();
       const int total = pref[nseg];
-      for (int j0 = 0; j0 < total; j0 += BLK) {
-        const int cnt = min(BLK, total - j0);
-        if (lane < cnt) {
-          const int g  = j0 + lane;
+      for (int j0 = 0; j0 < total; j0 += CH) {
+        const int cnt = min(CH, total - j0);
+        const int T2  = 2 * ((cnt + 2 * S - 1) / (2 * S));  // entries per lane: si, si + S, ...
+        double    x[PER], y[PER], z[PER], sg[PER], ax[PER], ay[PER], az[PER];
+#pragma unroll
+        for (int p = 0; p < PER; p++) {
+          // entries past the chunk load its last one again and are stored as padding
+          const int g  = j0 + min(lane + p * BLK, cnt - 1);
           int       lo = 0, hi = nseg - 1;  // last q with pref[q] <= g
           while (lo < hi) {
             const int mid = (lo + hi + 1) >> 1;
@@ -151,38 +165,38 @@ __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(MIXED ? 5 :
             else hi = mid - 1;
           }
           const int64_t bj = lb[lo] + (g - pref[lo]);
-          const double  x = sst[(F_X + 0) * scap + bj], y = sst[(F_X + 1) * scap + bj], z = sst[(F_X + 2) * scap + bj];
-          const double  sg = sst[F_SIG * scap + bj];
-          const double  ax = sst[(F_A + 0) * scap + bj], ay = sst[(F_A + 1) * scap + bj], az = sst[(F_A + 2) * scap + bj];
-          if (MIXED) {
+          x[p] = sst[(F_X + 0) * scap + bj], y[p] = sst[(F_X + 1) * scap + bj], z[p] = sst[(F_X + 2) * scap + bj];
+          sg[p] = sst[F_SIG * scap + bj];
+          ax[p] = sst[(F_A + 0) * scap + bj], ay[p] = sst[(F_A + 1) * scap + bj], az[p] = sst[(F_A + 2) * scap + bj];
+        }
+        // Entries of no strength past the chunk: every lane runs the same trip count.  Their offset
+        // and q put x = |r - (1024, 0, 0)|^2 / 2^20 near 1 for any target within a few hundred units
+        // of the leaf centre, so they stay on the pair loop's common path (a pad at x = 0 would take
+        // its coincident-pair test); TSIG takes q from the target, where a pad at the centre gives
+        // x = |r|^2 q of the same order as the real pairs.
+        T4 padA, padB;
+        padA.x = (T)(TSIG ? 0.0 : 1024.0) + (T)(MIXED ? 0.0 : tcx[t]), padA.y = (T)(MIXED ? 0.0 : tcy[t]);
+        padA.z = (T)(MIXED ? 0.0 : tcz[t]), padA.w = (T)0x1p-20;
+        padB.x = padB.y = padB.z = padB.w = (T)0.0;
+#pragma unroll
+        for (int p = 0; p < PER; p++) {
+          const int e = lane + p * BLK;
+          if (e < cnt) {
             // (offset, q) and (alpha c1, 2 q) with q = 1 / (2 sigma^2), c1 = q^{3/2} / (4 pi): then
             // f1 = G(x) and f2 = 2 q G'(x) for the scaled strength.  TSIG keeps alpha as is.
-            const double qq = 0.5 / (sg * sg), c1 = TSIG ? 1.0 : qq * sqrt(qq) * INV_4PI;
-            s32[2 * lane + 0] = make_float4((float)(x - cxt), (float)(y - cyt), (float)(z - czt), (float)qq);
-            s32[2 * lane + 1] = make_float4((float)(ax * c1), (float)(ay * c1), (float)(az * c1), (float)(2.0 * qq));
-          } else {
-            const double is2 = 1.0 / (sg * sg);
-            s64[lane]        = SrcF64{x, y, z, ax, ay, az, is2, 0.5 * is2};
+            const double qq = 0.5 / (sg[p] * sg[p]), c1 = TSIG ? 1.0 : qq * sqrt(qq) * INV_4PI;
+            T4           A, B;
+            A.x = (T)(x[p] - cxt), A.y = (T)(y[p] - cyt), A.z = (T)(z[p] - czt), A.w = (T)qq;
+            B.x = (T)(ax[p] * c1), B.y = (T)(ay[p] * c1), B.z = (T)(az[p] * c1), B.w = (T)(2.0 * qq);
+            sv[2 * e] = A, sv[2 * e + 1] = B;
           }
         }
-        if (MIXED) {
-          // entries of no strength past the chunk: every lane runs the same trip count.  Their
-          // offset and q put x = |r - (1024, 0, 0)|^2 / 2^20 near 1 for any target within a few
-          // hundred units of the leaf centre, so they stay on the pair loop's common path (a pad
-          // at x = 0 would take its coincident-pair test); TSIG takes q from the target, where
-          // a pad at the centre gives x = |r|^2 q of the same order as the real pairs.
-          const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-          const float4 pad  = TSIG ? zero : make_float4(1024.f, 0.f, 0.f, 0x1p-20f);
-          if (lane >= cnt) s32[2 * lane] = pad, s32[2 * lane + 1] = zero;
-          s32[2 * (BLK + lane)] = pad, s32[2 * (BLK + lane) + 1] = zero;
-        }
+        for (int e = cnt + lane; e < T2 * S; e += BLK) sv[2 * e] = padA, sv[2 * e + 1] = padB;
         __syncthreads();
-        if (MIXED) {
-          // lane (ti, si) takes entries si, si + S, ... two per step; T2 * S <= 2 BLK entries
-          // are read (S <= BLK), those from cnt on are the zero padding
-          float        fa[15];
-          const int    T2 = 2 * ((cnt + 2 * S - 1) / (2 * S));
-          const float4 *ps = s32 + 2 * (lane_on ? si : 0);
+        const T4 *ps = sv + 2 * (lane_on ? si : 0);
+        if constexpr (MIXED) {
+          // lane (ti, si) takes entries si, si + S, ... two per step.
+          float fa[15];
           // FP32 partial sums cover at most FLUSH entries per lane before they go into the FP64 sums
           constexpr int FLUSH = 64;
           for (int k0 = 0; k0 < T2; k0 += FLUSH) {
@@ -221,73 +235,36 @@ __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(MIXED ? 5 :
             for (int k = 0; k < (WITH_J ? 12 : 3); k++) acc[k] += (double)fa[k];
           }
         } else {
-          for (int j = jfirst; j < cnt; j += S) {
-            const SrcF64 &sj = s64[j];
-            const double  dx = xi - sj.x, dy = yi - sj.y, dz = zi - sj.z;
-            const double  R2 = dx * dx + dy * dy + dz * dz;
-            if (R2 == 0.0) continue;
-            const double RS     = R2 * (TSIG ? t_half : sj.halfInvS2);
-            const double sqrtRS = sqrt(RS);
-            const double erfS   = erf(sqrtRS);
-            const double expm   = exp(-RS);
-            const double invR   = 1.0 / sqrt(R2);
-            const double t2     = 2.0 * INV_SQRTPI * sqrtRS * expm;
-            const double o4pr3  = 0.25 * INV_PI / R2 * invR;
-            const double g      = erfS - t2;
-            const double f1     = g * o4pr3;
-            const double cx = dy * sj.az - dz * sj.ay, cy = dz * sj.ax - dx * sj.az, cz = dx * sj.ay - dy * sj.ax;
-            acc[0] += f1 * cx;
-            acc[1] += f1 * cy;
-            acc[2] += f1 * cz;
-            if (WITH_J) {
-              const double f2 = (t2 * (TSIG ? t_is2 : sj.invS2) - 3.0 * g / R2) * o4pr3;
-              const double k0 = f2 * cx, k1 = f2 * cy, k2 = f2 * cz;
-              acc[3] += k0 * dx;
-              acc[4] += k0 * dy + f1 * sj.az;
-              acc[5] += k0 * dz - f1 * sj.ay;
-              acc[6] += k1 * dx - f1 * sj.az;
-              acc[7] += k1 * dy;
-              acc[8] += k1 * dz + f1 * sj.ax;
-              acc[9] += k2 * dx + f1 * sj.ay;
-              acc[10] += k2 * dy - f1 * sj.ax;
-              acc[11] += k2 * dz;
-            }
+          for (int k = 0; k < T2; k += 2, ps += 4 * S) {
+            const double4 A0 = ps[0], B0 = ps[1], A1 = ps[2 * S], B1 = ps[2 * S + 1];
+            const double  dx0 = rxi - A0.x, dy0 = ryi - A0.y, dz0 = rzi - A0.z;
+            const double  dx1 = rxi - A1.x, dy1 = ryi - A1.y, dz1 = rzi - A1.z;
+            const double  r20 = dx0 * dx0 + dy0 * dy0 + dz0 * dz0, r21 = dx1 * dx1 + dy1 * dy1 + dz1 * dz1;
+            double        G0, Gp0, G1, Gp1;
+            g64_pair2(r20, r21, TSIG ? t_q : A0.w, TSIG ? t_q : A1.w, G0, Gp0, G1, Gp1);
+            const double f10 = TSIG ? G0 * t_c1 : G0;
+            const double f11 = TSIG ? G1 * t_c1 : G1;
+            accumulate_pair(acc, dx0, dy0, dz0, B0.x, B0.y, B0.z, f10, Gp0 * (TSIG ? t_c2 : B0.w), WITH_J);
+            accumulate_pair(acc, dx1, dy1, dz1, B1.x, B1.y, B1.z, f11, Gp1 * (TSIG ? t_c2 : B1.w), WITH_J);
           }
         }
         __syncthreads();
       }
     }
-    // combine the S source splits (threads ti + q*ntp) in split order
-    if constexpr (BLK == 64) {
-      if (S > 1)
-        for (int k = 0; k < (WITH_J ? 12 : 3); k++) {
-          double v = acc[k];
-          for (int q = 1; q < S; q++) v += __shfl(acc[k], ti + q * ntp, 64);
-          acc[k] = v;
-        }
-    } else if (S > 1) {
-      __syncthreads();
-      for (int k = 0; k < 12; k++) red[k * BLK + lane] = acc[k];
-      __syncthreads();
-      // not unrolled: unrolled, the compiler kept twelve loop-invariant LDS addresses from the
-      // kernel start and spilled them to scratch (an extra 3 GB of HBM traffic per 4M launch)
-      if (si == 0)
-#pragma unroll 1
-        for (int k = 0; k < (WITH_J ? 12 : 3); k++) {
-          double v = 0.0;
-          for (int q = 0; q < S; q++) v += red[k * BLK + ti + q * ntp];
-          acc[k] = v;
-        }
-    }
-    if (si == 0 && valid) {
-      if (SPLIT) {
-        double *pb = part + (int64_t)blockIdx.x * 12 * maxnt;
-        for (int k = 0; k < (WITH_J ? 12 : 3); k++) pb[k * maxnt + i] = acc[k];
-      } else {
-        for (int d = 0; d < 3; d++) out[(F_U + d) * ocap + bi] = -acc[d];
-        if (WITH_J)
-          for (int k = 0; k < 9; k++) out[(F_J + k) * ocap + bi] = -acc[3 + k];
-      }
+    if constexpr (!MIXED && WITH_J) fold_antisym(acc);
+    // Sum of the S splits (lanes t + q * ntp) in split order, through LDS: the lanes then take
+    // (field, target) pairs, consecutive targets in consecutive lanes.
+    constexpr int NK = WITH_J ? 12 : 3;
+    const int     np = min(ntp, nt - c0);
+    __syncthreads();
+    for (int k = 0; k < NK; k++) red[k * BLK + lane] = acc[k];
+    __syncthreads();
+    for (int o = lane; o < NK * np; o += BLK) {
+      const int k = o / np, tt = o - k * np;
+      double    v = red[k * BLK + tt];
+      for (int q = 1; q < S; q++) v += red[k * BLK + tt + q * ntp];
+      if (prow >= 0) part[((int64_t)prow * 12 + (int64_t)k * nt) + c0 + tt] = v;
+      else out[(k < 3 ? F_U + k : F_J + k - 3) * ocap + tb + c0 + tt] = -v;
     }
   }
 }
@@ -366,25 +343,125 @@ void direct(hipStream_t s, int64_t m, const double *xt, const double *at, const 
   UVLM_LAUNCH_CHECK();
 }
 
-// Sum of the SPLIT partials of each target leaf, segments in order, stored like k_p2p does.
-template <bool WITH_J>
-__global__ __launch_bounds__(WG) void k_p2p_reduce(const int32_t *__restrict__ leaves, int64_t nleaf,
-                                                   const int32_t *__restrict__ tbody,
-                                                   const int32_t *__restrict__ tnbody,
-                                                   const int32_t *__restrict__ segoff, const double *__restrict__ part,
-                                                   int maxnt, double *__restrict__ out, int64_t ocap)
+// Units of the near field: each target leaf's list in one or more runs of entries of about equal
+// work, so that a wave never walks a list far longer than the others' (a leaf next to much smaller
+// ones, a probe tree with few leaves) while the chip is idle.  A leaf's work is its lane steps: the
+// bodies of its list times its passes over its splits.  It is cut into ceil(work / limit) units,
+// limit = the larger of LANE_STEPS_MIN and 1/UNITS_AIM of all leaves' work: below LANE_STEPS_MIN the
+// staging and the prefix sums cost more than the pairs they serve (32 and 64 steps: 8k ring 72 and
+// 77 us; 128: 100 us).  More units shorten the last wave: 4M two rings (86k leaves) 10.0 ms with
+// 4096, 9.9 with 8192, 9.6 with 16384.
+constexpr int                LANE_STEPS_MIN = 64;
+constexpr unsigned long long UNITS_AIM      = 16384;
+enum { NU_INTER = 0, NU_WORK, NU_UNITS, NU_ROWS, NU_MULTI, NU_COUNT };
+
+__global__ void k_units_clear(unsigned long long *__restrict__ cnt)
 {
-  const int64_t w = blockIdx.x;
-  if (w >= nleaf) return;
-  const int t = leaves[w], tb = tbody[t], nt = tnbody[t];
-  for (int i = threadIdx.x; i < nt; i += WG) {
-    const int64_t bi = tb + i;
-    for (int k = 0; k < (WITH_J ? 12 : 3); k++) {
-      double v = 0.0;
-      for (int b = segoff[w]; b < segoff[w + 1]; b++) v += part[(int64_t)b * 12 * maxnt + k * maxnt + i];
-      if (k < 3) out[(F_U + k) * ocap + bi] = -v;
-      else out[(F_J + k - 3) * ocap + bi] = -v;
+  if (threadIdx.x < NU_COUNT) cnt[threadIdx.x] = 0;
+}
+
+// work[w] (lane steps) of each target leaf and the sums over all: interactions, work.  One
+// wavefront per leaf at a time, lanes over its list; at most UNITS_WORK_BLOCKS blocks keep the
+// same-address atomics few.
+constexpr int UNITS_WORK_BLOCKS = 512;
+template <int BLK>
+__global__ __launch_bounds__(256) void k_units_work(const int32_t *__restrict__ leaves, int64_t nleaf,
+                                                    const int32_t *__restrict__ tnbody,
+                                                    const int32_t *__restrict__ off, const int32_t *__restrict__ src,
+                                                    const int32_t *__restrict__ snbody, uint32_t *__restrict__ work,
+                                                    unsigned long long *__restrict__ cnt)
+{
+  __shared__ unsigned long long sum[2][4];
+  const int          lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  unsigned long long inter = 0, all = 0;
+  for (int64_t w = blockIdx.x * 4ll + wv; w < nleaf; w += gridDim.x * 4ll) {
+    const int t = leaves[w], nt = tnbody[t], q1 = off[t + 1];
+    unsigned  ns = 0;
+    for (int q = off[t] + lane; q < q1; q += 64) ns += (unsigned)snbody[src[q]];
+    for (int o = 32; o > 0; o >>= 1) ns += __shfl_xor(ns, o, 64);
+    const int ntp = near_targets_per_pass<BLK>(nt), S = near_splits<BLK>(ntp);
+    const unsigned long long steps = ((unsigned long long)ns * ((nt + ntp - 1) / ntp) + S - 1) / S;
+    const uint32_t           wk    = (uint32_t)min(steps, 0xffffffffull);
+    if (lane == 0) work[w] = wk;
+    inter += (unsigned long long)nt * ns;
+    all += wk;
+  }
+  if (lane == 0) sum[0][wv] = inter, sum[1][wv] = all;
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    unsigned long long v = 0;
+    for (int k = 0; k < 4; k++) v += sum[threadIdx.x][k];
+    if (v) atomicAdd(&cnt[threadIdx.x], v);
+  }
+}
+
+// Units (w, first entry, end, row of the partial sums or -1) and the leaves cut into several
+// (w, first row, units).  Ranges are reserved once per block.
+__global__ __launch_bounds__(256) void k_units_fill(const int32_t *__restrict__ leaves, int64_t nleaf,
+                                                    const int32_t *__restrict__ tnbody,
+                                                    const int32_t *__restrict__ off,
+                                                    const uint32_t *__restrict__ work,
+                                                    unsigned long long *__restrict__ cnt, int4 *__restrict__ units,
+                                                    int4 *__restrict__ multi)
+{
+  __shared__ unsigned long long tot[4][3], base[3];
+  const int64_t            w    = blockIdx.x * 256ll + threadIdx.x;
+  const int                lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const unsigned long long lim = max((unsigned long long)LANE_STEPS_MIN, cnt[NU_WORK] / UNITS_AIM);
+  int                      nu = 0, q0 = 0, len = 0, nt = 0;
+  if (w < nleaf) {
+    const int t = leaves[w];
+    nt = tnbody[t], q0 = off[t], len = off[t + 1] - q0;
+    nu = (int)min((unsigned long long)max(len, 1), (work[w] + lim - 1) / lim);
+    nu = max(nu, 1);
+  }
+  // exclusive prefix sums over the block of units, rows and cut leaves
+  unsigned long long v[3] = {(unsigned long long)nu, nu > 1 ? (unsigned long long)nu * nt : 0, nu > 1 ? 1ull : 0}, ex[3];
+  for (int c = 0; c < 3; c++) {
+    unsigned long long x = v[c];
+    for (int o = 1; o < 64; o <<= 1) {
+      const unsigned long long u = __shfl_up(x, o, 64);
+      if (lane >= o) x += u;
     }
+    if (lane == 63) tot[wv][c] = x;
+    ex[c] = x - v[c];
+  }
+  __syncthreads();
+  if (threadIdx.x < 3) {
+    unsigned long long sum = 0;
+    for (int k = 0; k < 4; k++) sum += tot[k][threadIdx.x];
+    base[threadIdx.x] = sum ? atomicAdd(&cnt[NU_UNITS + threadIdx.x], sum) : 0;
+  }
+  __syncthreads();
+  for (int c = 0; c < 3; c++) {
+    ex[c] += base[c];
+    for (int k = 0; k < wv; k++) ex[c] += tot[k][c];
+  }
+  if (w >= nleaf) return;
+  for (int j = 0; j < nu; j++) {
+    const int a = q0 + (int)((int64_t)len * j / nu), b = q0 + (int)((int64_t)len * (j + 1) / nu);
+    units[ex[0] + j] = make_int4((int)w, a, b, nu > 1 ? (int)(ex[1] + (unsigned long long)j * nt) : -1);
+  }
+  if (nu > 1) multi[ex[2]] = make_int4((int)w, (int)ex[1], nu, 0);
+}
+
+// Sums of the leaves cut into several units, units in order, stored as k_p2p stores a single one.
+template <bool WITH_J>
+__global__ __launch_bounds__(256) void k_p2p_reduce(const int4 *__restrict__ multi, const int32_t *__restrict__ leaves,
+                                                    const int32_t *__restrict__ tbody,
+                                                    const int32_t *__restrict__ tnbody,
+                                                    const double *__restrict__ part, double *__restrict__ out,
+                                                    int64_t ocap)
+{
+  const int4    m = multi[blockIdx.x];
+  const int     t = leaves[m.x], tb = tbody[t], nt = tnbody[t];
+  const double *p = part + (int64_t)m.y * 12;
+  for (int o = threadIdx.x; o < (WITH_J ? 12 : 3) * nt; o += 256) {
+    const int k = o / nt;
+    double    v = 0.0;
+#pragma unroll 4
+    for (int u = 0; u < m.z; u++) v += p[(int64_t)u * 12 * nt + o];
+    out[(k < 3 ? F_U + k : F_J + k - 3) * ocap + tb + (o - k * nt)] = -v;
   }
 }
 
@@ -470,89 +547,64 @@ __global__ __launch_bounds__(WG) void k_gauss(const int32_t *__restrict__ leaves
   }
 }
 
-// Below this many target leaves (probe trees), long lists are cut into segments of E list
-// entries that run as separate workgroups, so the GPU stays full.
-constexpr int64_t SPLIT_TARGETS = 4096, SPLIT_SEGMENTS = 8192;
+// Lanes per near-field workgroup.  With 64 lanes a leaf of 33..64 targets leaves up to half of them
+// idle (one split), with 256 a twentieth, and four waves share a staged chunk: 1M cube (leaves of
+// about 32 bodies, mixed) P2P 5.58 -> 4.03 ms, 60k cube with c = 6 1.39 -> 1.18, 8k ring (FP64) 0.110
+// -> 0.075 ms.  64 lanes stay for the lists of a few entries that an adjoint of few probes leaves most
+// leaves with (1M blobs, 4096 probes, 1.6 entries a leaf: 2.96 against 3.08 ms for the whole pass),
+// where 256 lanes have nothing to share.
+constexpr int64_t WIDE_ENTRIES = 8;  // list entries per target leaf from which 256 lanes are used
 
-void p2p(hipStream_t s, const Tree &tt, const Tree &stree, const Lists &l, const double *tgt, int64_t tcap,
-         const double *srcst, int64_t scap, double *out, int64_t ocap, int precision, int sensor_mode,
-         int64_t max_leaf, Scratch *sc)
+// Units of the P2P list `l` of target tree tt against source tree st (see k_units_work), and the
+// number of near-field interactions.  One read-back of the totals.
+void near_units(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &st, int64_t max_leaf, Lists &l)
+{
+  l.n_units = l.n_rows = l.n_multi = l.n_interactions = 0;
+  if (tt.nleaf == 0) return;
+  sc.unit_work.reserve(4 * tt.nleaf);
+  sc.unit_cnt.reserve(8 * NU_COUNT);
+  unsigned long long *cnt = sc.unit_cnt.as<unsigned long long>();
+  // at most UNITS_AIM units beyond one per leaf: sum ceil(work / limit) <= nleaf + work / limit
+  l.units.reserve(sizeof(int4) * (tt.nleaf + UNITS_AIM));
+  l.multi.reserve(sizeof(int4) * std::min<int64_t>(tt.nleaf, UNITS_AIM));
+  const int32_t *lv = tt.leaves.as<int32_t>(), *tn = tt.nbody.as<int32_t>(), *sn = st.nbody.as<int32_t>();
+  const int32_t *off = l.p2p_off.as<int32_t>(), *src = l.p2p_src.as<int32_t>();
+  const int      gw = (int)std::min<int64_t>(UNITS_WORK_BLOCKS, (tt.nleaf + 3) / 4);
+  l.wide = max_leaf > 64 || l.np2p >= WIDE_ENTRIES * tt.nleaf;
+  k_units_clear<<<1, 64, 0, s>>>(cnt);
+  if (l.wide) k_units_work<256><<<gw, 256, 0, s>>>(lv, tt.nleaf, tn, off, src, sn, sc.unit_work.as<uint32_t>(), cnt);
+  else k_units_work<64><<<gw, 256, 0, s>>>(lv, tt.nleaf, tn, off, src, sn, sc.unit_work.as<uint32_t>(), cnt);
+  k_units_fill<<<(int)((tt.nleaf + 255) / 256), 256, 0, s>>>(lv, tt.nleaf, tn, off, sc.unit_work.as<uint32_t>(), cnt,
+                                                             l.units.as<int4>(), l.multi.as<int4>());
+  UVLM_LAUNCH_CHECK();
+  unsigned long long h[NU_COUNT];
+  UVLM_HIP(hipMemcpyAsync(h, cnt, sizeof(h), hipMemcpyDeviceToHost, s));
+  UVLM_HIP(hipStreamSynchronize(s));
+  l.n_interactions = (int64_t)h[NU_INTER];
+  l.n_units        = (int64_t)h[NU_UNITS];
+  l.n_rows         = (int64_t)h[NU_ROWS];
+  l.n_multi        = (int64_t)h[NU_MULTI];
+  if (l.n_rows >= (int64_t(1) << 31)) throw Error(UVLM_ERR_INTERNAL, "near-field partial rows");
+}
+
+// sensor_mode: 0 particles (u and J), 1 probes (u only), 2 adjoint (u and J, target sigma).
+void p2p(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &stree, const Lists &l, const double *tgt, int64_t tcap,
+         const double *srcst, int64_t scap, double *out, int64_t ocap, int precision, int sensor_mode)
 {
   if (tt.nleaf == 0) return;
-  const int nb = (int)tt.nleaf;
-  if (sc && tt.nleaf < SPLIT_TARGETS && l.np2p >= 4 * tt.nleaf) {
-    // segment table on the host: the target tree is small
-    const int64_t        E = std::max<int64_t>(2, (l.np2p + SPLIT_SEGMENTS - 1) / SPLIT_SEGMENTS);
-    std::vector<int32_t> lv(tt.nleaf), off(tt.C + 1);
-    UVLM_HIP(hipMemcpyAsync(lv.data(), tt.leaves.p, 4 * lv.size(), hipMemcpyDeviceToHost, s));
-    UVLM_HIP(hipMemcpyAsync(off.data(), l.p2p_off.p, 4 * off.size(), hipMemcpyDeviceToHost, s));
-    UVLM_HIP(hipStreamSynchronize(s));
-    std::vector<int32_t> seg, segoff(tt.nleaf + 1, 0);
-    for (int64_t w = 0; w < tt.nleaf; w++) {
-      const int32_t q0 = off[lv[w]], q1 = off[lv[w] + 1];
-      int32_t       e0 = q0;
-      do {
-        const int32_t e1 = (int32_t)std::min<int64_t>(q1, e0 + E);
-        seg.push_back((int32_t)w);
-        seg.push_back(e0);
-        seg.push_back(e1);
-        e0 = e1;
-      } while (e0 < q1);
-      segoff[w + 1] = (int32_t)(seg.size() / 3);
-    }
-    const int64_t nsg = segoff[tt.nleaf];
-    sc->p2p_seg.reserve(4 * (seg.size() + segoff.size()));
-    int32_t *dseg = sc->p2p_seg.as<int32_t>(), *dsegoff = dseg + seg.size();
-    UVLM_HIP(hipMemcpyAsync(dseg, seg.data(), 4 * seg.size(), hipMemcpyHostToDevice, s));
-    UVLM_HIP(hipMemcpyAsync(dsegoff, segoff.data(), 4 * segoff.size(), hipMemcpyHostToDevice, s));
-    UVLM_HIP(hipStreamSynchronize(s));
-    const int maxnt = (int)max_leaf;
-    sc->p2p_part.reserve(sizeof(double) * nsg * 12 * maxnt);
-    double    *part = sc->p2p_part.as<double>();
-    const bool mixed = precision == UVLM_MIXED, wj = sensor_mode != 1, ts = sensor_mode == 2;
-#define UVLM_P2P_SPLIT(MX, WJ, TS)                                                                                \
-  k_p2p<MX, WJ, TS, 64, true><<<(int)nsg, WG, 0, s>>>(                                                             \
-      tt.leaves.as<int32_t>(), tt.nleaf, tt.body.as<int32_t>(), tt.nbody.as<int32_t>(), tt.cx.as<double>(),        \
-      tt.cy.as<double>(), tt.cz.as<double>(), l.p2p_off.as<int32_t>(), l.p2p_src.as<int32_t>(),                   \
-      stree.body.as<int32_t>(), stree.nbody.as<int32_t>(), tgt, tcap, srcst, scap, out, ocap, dseg, part, maxnt)
-    if (ts) {
-      if (mixed) UVLM_P2P_SPLIT(true, true, true);
-      else UVLM_P2P_SPLIT(false, true, true);
-    } else if (wj) {
-      if (mixed) UVLM_P2P_SPLIT(true, true, false);
-      else UVLM_P2P_SPLIT(false, true, false);
-    } else {
-      if (mixed) UVLM_P2P_SPLIT(true, false, false);
-      else UVLM_P2P_SPLIT(false, false, false);
-    }
-#undef UVLM_P2P_SPLIT
-    UVLM_LAUNCH_CHECK();
-    if (wj)
-      k_p2p_reduce<true><<<nb, WG, 0, s>>>(tt.leaves.as<int32_t>(), tt.nleaf, tt.body.as<int32_t>(),
-                                           tt.nbody.as<int32_t>(), dsegoff, part, maxnt, out, ocap);
-    else
-      k_p2p_reduce<false><<<nb, WG, 0, s>>>(tt.leaves.as<int32_t>(), tt.nleaf, tt.body.as<int32_t>(),
-                                            tt.nbody.as<int32_t>(), dsegoff, part, maxnt, out, ocap);
-    UVLM_LAUNCH_CHECK();
-    return;
-  }
-#define UVLM_P2P(MX, WJ, TS)                                                                                      \
-  if (big)                                                                                                         \
-    k_p2p<MX, WJ, TS, 256><<<nb, 256, 0, s>>>(tt.leaves.as<int32_t>(), tt.nleaf, tt.body.as<int32_t>(),           \
-                                              tt.nbody.as<int32_t>(), tt.cx.as<double>(), tt.cy.as<double>(),       \
-                                              tt.cz.as<double>(), l.p2p_off.as<int32_t>(), l.p2p_src.as<int32_t>(), \
-                                              stree.body.as<int32_t>(), stree.nbody.as<int32_t>(), tgt, tcap, srcst,\
-                                              scap, out, ocap);                                                    \
-  else                                                                                                             \
-  k_p2p<MX, WJ, TS, 64><<<nb, WG, 0, s>>>(tt.leaves.as<int32_t>(), tt.nleaf, tt.body.as<int32_t>(), tt.nbody.as<int32_t>(), \
-                                  tt.cx.as<double>(), tt.cy.as<double>(), tt.cz.as<double>(),                     \
-                                  l.p2p_off.as<int32_t>(), l.p2p_src.as<int32_t>(), stree.body.as<int32_t>(),      \
-                                  stree.nbody.as<int32_t>(), tgt, tcap, srcst, scap, out, ocap)
-  // sensor_mode: 0 particles (u and J), 1 probes (u only), 2 adjoint (u and J, target sigma).
-  // Leaves of more than 64 bodies get 256-thread workgroups, so all their targets share one
-  // pass over the sources.
+  if (l.n_units < tt.nleaf) throw Error(UVLM_ERR_INTERNAL, "P2P without its units");
+  sc.p2p_part.reserve(sizeof(double) * 12 * l.n_rows);
+  double    *part  = sc.p2p_part.as<double>();
   const bool mixed = precision == UVLM_MIXED;
-  const bool big   = max_leaf > 64;
+  auto       launch = [&](auto kern, int blk) {
+    kern<<<(int)l.n_units, blk, 0, s>>>(l.units.as<int4>(), tt.leaves.as<int32_t>(), tt.body.as<int32_t>(),
+                                        tt.nbody.as<int32_t>(), tt.cx.as<double>(), tt.cy.as<double>(),
+                                        tt.cz.as<double>(), l.p2p_src.as<int32_t>(), stree.body.as<int32_t>(),
+                                        stree.nbody.as<int32_t>(), tgt, tcap, srcst, scap, out, ocap, part);
+  };
+#define UVLM_P2P(MX, WJ, TS)                      \
+  if (l.wide) launch(k_p2p<MX, WJ, TS, 256>, 256);   \
+  else launch(k_p2p<MX, WJ, TS, 64>, 64)
   if (sensor_mode == 2) {
     if (mixed) UVLM_P2P(true, true, true);
     else UVLM_P2P(false, true, true);
@@ -562,6 +614,15 @@ void p2p(hipStream_t s, const Tree &tt, const Tree &stree, const Lists &l, const
   else UVLM_P2P(false, false, false);
 #undef UVLM_P2P
   UVLM_LAUNCH_CHECK();
+  if (l.n_multi > 0) {
+    auto reduce = [&](auto kern) {
+      kern<<<(int)l.n_multi, 256, 0, s>>>(l.multi.as<int4>(), tt.leaves.as<int32_t>(), tt.body.as<int32_t>(),
+                                          tt.nbody.as<int32_t>(), part, out, ocap);
+    };
+    if (sensor_mode != 1) reduce(k_p2p_reduce<true>);
+    else reduce(k_p2p_reduce<false>);
+    UVLM_LAUNCH_CHECK();
+  }
 }
 
 // PSE (mode 0, adds prefix * sum to dadt) or Gaussian vorticity (mode 1, subtracts the sum

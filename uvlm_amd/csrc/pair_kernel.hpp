@@ -119,6 +119,146 @@ __device__ __forceinline__ void g_far(float xq, float &G, float &Gp)
   Gp             = w2 * fmaf(1.1283791670955126f, e, -1.5f * G);
 }
 
+// ---- FP64 pair factors --------------------------------------------------------------------
+// The FP64 near field used the reference formula with the library's erf, exp, sqrt and three
+// divisions: about 250 instructions a pair (11.0 ms for 1.54e9 pairs of the 1M two rings).
+// Here G and G' (and G'' for the adjoint) come from polynomials too:
+//  * x < X64 = 3: degree-16 interpolants of G and G' (17 for G'') at the Chebyshev nodes of
+//    [0, 3] in t = x - 3/2: relative error 3.5e-18, 8.4e-18 and 5.7e-19 in exact arithmetic and
+//    1.7e-16, 2.2e-16, 2.2e-16 by fused Horner.  Unlike erf - t2 there is no cancellation at
+//    small x (the formula loses a factor 1/x on f1 and 1/x^2 on f2).  3 rather than 2 (degree 14)
+//    costs 4 multiply-adds a pair and keeps more waves off the far form; 4 needs degree 18.
+//  * x >= 3: g = 1 - e^{-x} (erfcx(s) + (2/sqrt(pi)) s) as in FP32, with rsq refined by one cubic
+//    step, a degree-11 e^r on |r| <= ln 2 / 2 and erfcx as a degree-11 minimax polynomial in
+//    w = 1/s whose error weighted by e^{-x} is 1.2e-17.  From x = FAR64 = 44 on, e^{-x} no longer
+//    shows in G or G' and a wave all of whose lanes are there skips it.
+constexpr double X64 = 3.0, FAR64 = 44.0;
+constexpr unsigned X64_HI = 0x40080000u;  // high word of X64: x < X64 where the high word is below
+constexpr int NG64 = 17, NGPP64 = 18, NFAR64 = 12, NEXP64 = 12;
+constexpr double FAR64_WC = 0.3640529707392538, FAR64_WMIN = 0.15075567228888181;
+constexpr double TWO_SQRTPI = 1.1283791670955126;
+__constant__ double c_g64[17] = {
+    3.31157308998109245e-01, -1.63307026156660179e-01, 5.21640470431589676e-02, -1.25969894488822884e-02,
+    2.45398030160123067e-03, -4.00833197494527367e-04, 5.63652498002339511e-05, -6.95726516926421291e-06,
+    7.65109382981209354e-07, -7.58599198635941649e-08, 6.84690821463335333e-09, -5.67087542187630871e-10,
+    4.33916973335413845e-11, -3.08354343847775088e-12, 2.04760655365041072e-13, -1.31590474790122235e-14,
+    7.69092086651117093e-16};
+__constant__ double c_gp64[17] = {
+    -1.63307026156660207e-01, 1.04328094086317935e-01, -3.77909683466464003e-02, 9.81592120640503718e-03,
+    -2.00416598747744749e-03, 3.38191498800797814e-04, -4.87008561660276932e-05, 6.12087506526053526e-06,
+    -6.82739314636161485e-07, 6.84690804739502330e-08, -6.23792611506433268e-09, 5.20701422245581422e-10,
+    -4.01069139650919117e-11, 2.86631274157453670e-12, -1.91274669263023203e-13, 1.23481991649719220e-14,
+    -7.24413669201184165e-16};
+__constant__ double c_gpp64[18] = {
+    1.04328094086317935e-01, -7.55819366932928005e-02, 2.94477636192146709e-02, -8.01666394990975875e-03,
+    1.69095749400854705e-03, -2.92205136996453215e-04, 4.28461254389931391e-05, -5.46191451601966715e-06,
+    6.16221758233975666e-07, -6.23792631318532978e-08, 5.72768074901313056e-09, -4.81280969224836532e-10,
+    3.72818068782074733e-11, -2.67896141427953826e-12, 1.79437434662867233e-13, -1.12666500869749876e-14,
+    6.85754757690162003e-16, -3.81177028769169991e-17};
+__constant__ double c_far64[12] = {
+    1.93861300091875771e-01, 4.78080369979300202e-01, -1.85163134573934129e-01, -3.15745193379613209e-02,
+    1.40862568085704715e-01, -1.32543619759139197e-01, 2.74017194880180233e-02, 1.19121362382883136e-01,
+    -2.26096713052116927e-01, 2.21406339543712638e-01, -1.10008955300923306e-01, 8.88054390278034469e-03};
+__constant__ double c_exp64[12] = {
+    1.00000000000000000e+00, 1.00000000000000000e+00, 5.00000000000001887e-01, 1.66666666666666796e-01,
+    4.16666666664879531e-02, 8.33333333331958900e-03, 1.38888889523528631e-03, 1.98412698900764028e-04,
+    2.48014854415613131e-05, 2.75572408872298695e-06, 2.76326547225277896e-07, 2.51100492048186583e-08};
+
+// G and G' of both pairs at t = x - 3/2 (x < X64): four independent Horner chains.
+__device__ __forceinline__ void g64_near(double t0, double t1, double &G0, double &Gp0, double &G1, double &Gp1)
+{
+  double g0 = c_g64[NG64 - 1], g1 = g0, p0 = c_gp64[NG64 - 1], p1 = p0;
+#pragma unroll
+  for (int k = NG64 - 2; k >= 0; k--) {
+    g0 = fma(g0, t0, c_g64[k]);
+    g1 = fma(g1, t1, c_g64[k]);
+    p0 = fma(p0, t0, c_gp64[k]);
+    p1 = fma(p1, t1, c_gp64[k]);
+  }
+  G0 = g0, Gp0 = p0, G1 = g1, Gp1 = p1;
+}
+
+// 1/sqrt(x) from the hardware estimate and one cubic step (x > 0 and finite).
+__device__ __forceinline__ double rsqrt64(double x)
+{
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
+// The far form's coefficients, read through a pointer the compiler cannot see through: it would
+// otherwise keep all 24 doubles in scalar registers across the pair loop beside the 34 of the near
+// polynomials, and spill both to vector lanes (one readlane an instruction).
+using ConstF64 = const double __attribute__((address_space(4))) *;  // scalar loads
+__device__ __forceinline__ ConstF64 here(const double *q)
+{
+  ConstF64 p = (ConstF64)q;
+  asm volatile("" : "+s"(p));
+  return p;
+}
+
+// a b + c with c in scalar registers (left to the compiler, a coefficient used once is copied to
+// vector registers first: two moves a multiply-add).
+__device__ __forceinline__ double fma_sc(double a, double b, double c)
+{
+  double d;
+  asm("v_fma_f64 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "s"(c));
+  return d;
+}
+
+// e^{-x} for x >= 0 (0 from x = 745 on).
+__device__ __forceinline__ double exp64_neg(double x)
+{
+  const ConstF64 c = here(c_exp64);
+  const double xe = fmin(x, 800.0);
+  const double k  = rint(xe * -1.4426950408889634);
+  const double r  = fma(k, -2.3190468138462996e-17, fma(k, -0.6931471805599453, -xe))  /* ln 2 in two parts */;
+  double       p  = c[NEXP64 - 1];
+#pragma unroll
+  for (int i = NEXP64 - 2; i >= 0; i--) p = fma_sc(p, r, c[i]);
+  return __builtin_amdgcn_ldexp(p, (int)k);
+}
+
+// G, G' (and D2: G'') at x >= X64.
+template <bool D2>
+__device__ __forceinline__ void g64_far(double x, double &G, double &Gp, double &Gpp)
+{
+  const double w = rsqrt64(x), w2 = w * w;
+  double       g = 1.0, ce = 0.0;
+  if (x < FAR64) {
+    const double e = exp64_neg(x), t = fmax(w, FAR64_WMIN) - FAR64_WC;
+    const ConstF64 c = here(c_far64);
+    double         p = c[NFAR64 - 1];
+#pragma unroll
+    for (int k = NFAR64 - 2; k >= 0; k--) p = fma_sc(p, t, c[k]);
+    g  = fma(-e, fma(TWO_SQRTPI, x * w, p), 1.0);
+    ce = TWO_SQRTPI * e;
+  }
+  G  = g * w2 * w;
+  Gp = w2 * fma(-1.5, G, ce);
+  if (D2) Gpp = w2 * fma(-2.5, Gp, -ce);
+}
+
+// G and G' of two pairs at x = R^2 q.  A coincident pair (R^2 = 0) is skipped
+// (multipoleKernels.hpp:242): only the f1 alpha terms survive a zero separation, so G = 0 is enough.
+// The common path is taken where both x lie in (0, X64), one unsigned test of each high word (x
+// below 2^-1022 counts as 0 there and is looked at again).
+__device__ __forceinline__ void g64_pair2(double r20, double r21, double q0, double q1, double &G0, double &Gp0,
+                                          double &G1, double &Gp1)
+{
+  const double   x0 = r20 * q0, x1 = r21 * q1;
+  const unsigned h0 = (unsigned)__double2hiint(x0), h1 = (unsigned)__double2hiint(x1);
+  G0 = G1 = Gp0 = Gp1 = 0.0;
+  if (min(h0, h1) < X64_HI) g64_near(x0 - 0.5 * X64, x1 - 0.5 * X64, G0, Gp0, G1, Gp1);
+  if (max(h0 - 1u, h1 - 1u) >= X64_HI - 1u) {
+    double d2;
+    if (h0 >= X64_HI) g64_far<false>(x0, G0, Gp0, d2);
+    if (h1 >= X64_HI) g64_far<false>(x1, G1, Gp1, d2);
+    if (r20 == 0.0) G0 = 0.0;
+    if (r21 == 0.0) G1 = 0.0;
+  }
+}
+
 // Targets per pass of a near-field workgroup of BLK lanes over a leaf of nt targets: lanes are
 // (target, source split) with S = BLK / ntp splits, and the leaf takes ceil(nt / ntp) passes over
 // its source list.  With BLK = 256 a pass costs about 1/S of the list per lane plus the staging
@@ -139,6 +279,10 @@ __device__ __forceinline__ int near_targets_per_pass(int nt)
   }
   return best;
 }
+
+// Source splits of a pass of ntp targets; 2 S entries must fit in half a staged chunk (BLK <= 64
+// stages 2 BLK entries, BLK = 256 stages 256).
+template <int BLK> __device__ __forceinline__ int near_splits(int ntp) { return min(BLK / ntp, BLK <= 64 ? 64 : 128); }
 
 constexpr int SEG = 256;  // source leaves whose prefix sums sit in LDS at once
 

@@ -544,31 +544,6 @@ __global__ void k_transpose_keys(int64_t C, int64_t n, const int32_t *__restrict
   keys[q] = ((uint64_t)(uint32_t)src[q] << tbits) | (uint64_t)(uint32_t)lo;
 }
 
-// Sum over the P2P list's sorted keys (target << sbits | source) of nbody[target] * nbody[source]:
-// lanes stride over the list entries (a lane per target cell walked its list serially: 98 us at
-// 4M), and a grid of at most COUNT_BLOCKS blocks keeps the same-address atomics few.
-constexpr int COUNT_BLOCKS = 512;
-__global__ void k_count_inter(int64_t n, const uint64_t *__restrict__ keys, int sbits,
-                              const int32_t *__restrict__ tn, const int32_t *__restrict__ sn,
-                              unsigned long long *__restrict__ out)
-{
-  unsigned long long acc = 0;
-  for (int64_t q = blockIdx.x * (int64_t)BLK + threadIdx.x; q < n; q += (int64_t)gridDim.x * BLK) {
-    const uint64_t k = keys[q];
-    acc += (unsigned long long)tn[k >> sbits] * (unsigned long long)sn[k & ((uint64_t(1) << sbits) - 1)];
-  }
-  for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o, 64);
-  // one atomic per block (the wavefronts' sums meet in LDS)
-  __shared__ unsigned long long wsum[BLK / 64];
-  if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = acc;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    unsigned long long tot = 0;
-    for (int w = 0; w < BLK / 64; w++) tot += wsum[w];
-    if (tot) atomicAdd(out, tot);
-  }
-}
-
 void h2d(hipStream_t s, void *d, const void *h, size_t bytes)
 {
   UVLM_HIP(hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, s));
@@ -877,14 +852,6 @@ void traverse(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &st, double
     src.reserve(4 * std::max<int64_t>(n, 1));
     sc.keys1.reserve(8 * std::max<int64_t>(n, 1));
     if (n > 0) sort_keys_u64(s, sc, raw.as<uint64_t>(), sc.keys1.as<uint64_t>(), n, eb);
-    if (which == 0) {  // interactions of the P2P list, read by count_interactions
-      unsigned long long *d = (unsigned long long *)sc.counters.p + 7;  // slots 0..5: the traversal's
-      UVLM_HIP(hipMemsetAsync(d, 0, 8, s));
-      if (n > 0)
-        k_count_inter<<<std::min(nblocks(n), COUNT_BLOCKS), BLK, 0, s>>>(n, sc.keys1.as<uint64_t>(), sbits,
-                                                                         tt.nbody.as<int32_t>(),
-                                                                         st.nbody.as<int32_t>(), d);
-    }
     k_csr<<<nblocks(C + 1), BLK, 0, s>>>(C, sc.keys1.as<uint64_t>(), n, sbits, off.as<int32_t>());
     k_low_bits<<<nblocks(n), BLK, 0, s>>>(n, sc.keys1.as<uint64_t>(), sbits, src.as<int32_t>());
     UVLM_LAUNCH_CHECK();
@@ -919,16 +886,6 @@ void transpose_lists(hipStream_t s, Scratch &sc, const Tree &in_targets, const T
     k_low_bits<<<nblocks(n), BLK, 0, s>>>(n, sc.keys1.as<uint64_t>(), tbits, src.as<int32_t>());
     UVLM_LAUNCH_CHECK();
   }
-}
-
-void count_interactions(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &st, const Lists &l, int64_t *out)
-{
-  // summed by traverse() from the sorted P2P keys of these trees' lists
-  (void)tt, (void)st, (void)l;
-  const unsigned long long *d = (const unsigned long long *)sc.counters.p + 7;
-  unsigned long long h = 0;
-  to_host(s, &h, d);
-  *out = (int64_t)h;
 }
 
 }  // namespace uvlm
