@@ -75,3 +75,23 @@ def test_probes(orc, m, ncrit):
     assert np.array_equal(s[:, 9:12], sb[:, 9:12])
     assert rel(s[:, 15:18], sb[:, 15:18]) < 1e-10
     g.close()
+
+
+@pytest.mark.parametrize("m,n", [(1, 1), (1, 1025), (3, 700), (511, 1), (513, 2049), (1100, 1024), (16384, 333)])
+def test_direct(orc, m, n):
+    X, A, S = cluster(max(n, 2), 5, 0.05)
+    X, A, S = X[:n], A[:n], S[:n]
+    rng = W.SplitMix64(m)
+    xt = 1.5 * (rng.uniform(3 * m).reshape(m, 3) * 2.0 - 1.0)
+    xt[: min(m, n) // 2] = X[: min(m, n) // 2]  # coincident with sources: skipped pairs
+    at = rng.normal(3 * m).reshape(m, 3)
+    print(f"[near] direct m={m} n={n}", flush=True)
+    g = FMMCalculator(P=4, theta=0.5, ncrit=64)
+    g.set_arrays(X, A, S)
+    u, J, D = g.direct(xt, at)
+    u2, _, _ = g.direct(xt, want_J=False)
+    wu, wJ = orc.direct(xt, X, A, S)
+    wD = np.einsum("iab,ib->ia", wJ.reshape(m, 3, 3), at)
+    assert rel(u, wu) < 1e-12 and rel(u2, wu) < 1e-12
+    assert rel(J, wJ.reshape(m, 9)) < 1e-11 and rel(D, wD) < 1e-11
+    g.close()

@@ -1983,10 +1983,9 @@ int uvlm_direct(uvlm_handle h, int64_t m, const double *xt, const double *at, do
   return guarded([&] {
     check_direct_args(h, m, xt, at, u, dadt);
     set_device(h);
-    DevBuf        buf;
     const int64_t nin = 3 * m + (at ? 3 * m : 0), nout = 3 * m + (J ? 9 * m : 0) + (dadt ? 3 * m : 0);
-    buf.reserve(sizeof(double) * (nin + nout));
-    direct_staged(h, m, xt, at, u, J, dadt, buf.as<double>());
+    h->staging.reserve(sizeof(double) * (nin + nout));
+    direct_staged(h, m, xt, at, u, J, dadt, h->staging.as<double>());
   });
 }
 

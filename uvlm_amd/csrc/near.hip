@@ -32,11 +32,6 @@ namespace {
 
 constexpr int WG = 64;
 
-// Staged sources of the direct sum.
-struct SrcF64 {
-  double x, y, z, ax, ay, az, invS2, halfInvS2;
-};
-
 // acc[0..2] += f1 c, acc[3..10] += f2 c (x) dX with c = dX x a, and acc[12..14] += f1 a: the
 // f1 eps_{abk} a_k part of J is antisymmetric, so its sum is kept as one vector and folded
 // into J once per chunk (fold_antisym) instead of six multiply-adds per pair.  c is
@@ -269,68 +264,98 @@ __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(MIXED ? 5 :
   }
 }
 
-// O(M*N) direct sum, FP64, reference formula; one thread per target, sources tiled
-// through LDS.  Output: u (m,3), J (m,9) and, when target strengths are given, the
+// O(m n) direct sum, FP64.  Output: u (m,3), J (m,9) and, when target strengths are given, the
 // classic stretching J.alpha_t (the quantity exafmm::direct produces, traverse.hpp:88-98).
-__global__ __launch_bounds__(256) void k_direct(int64_t m, const double *__restrict__ xt,
-                                                const double *__restrict__ at, const double *__restrict__ sst,
-                                                int64_t scap, int64_t n, double *__restrict__ u,
-                                                double *__restrict__ J, double *__restrict__ dadt)
+//
+// A workgroup of 1024 lanes takes NT targets against all sources: lanes = (target) x (1024 / NT
+// source splits), sources staged 1024 at a time, the next chunk's loads in flight during the pair
+// loop, the splits added in order through LDS.  NT is the largest power of two that still gives
+// DIRECT_BLOCKS workgroups: a target per lane and no splits left 4096 targets on 16 of 256 CUs
+// (109.7 ms against 200k sources).  Fewer targets per workgroup stage each source more often: at
+// NT = 16 the staging is 1 of 17 lane-steps.  No workspace: uvlm_direct_noalloc runs it too.
+constexpr int DIRECT_LANES = 1024, DIRECT_BLOCKS = 256;
+template <bool WITH_J>
+__global__ __launch_bounds__(DIRECT_LANES) void k_direct(int NT, int64_t m, const double *__restrict__ xt,
+                                                         const double *__restrict__ at,
+                                                         const double *__restrict__ sst, int64_t scap, int64_t n,
+                                                         double *__restrict__ u, double *__restrict__ J,
+                                                         double *__restrict__ dadt)
 {
-  __shared__ SrcF64 sh[256];
-  const int64_t i  = blockIdx.x * (int64_t)256 + threadIdx.x;
-  const bool    ok = i < m;
-  const double  xi = ok ? xt[3 * i] : 0.0, yi = ok ? xt[3 * i + 1] : 0.0, zi = ok ? xt[3 * i + 2] : 0.0;
-  double        acc[12];
-  for (int k = 0; k < 12; k++) acc[k] = 0.0;
-  for (int64_t j0 = 0; j0 < n; j0 += 256) {
-    const int64_t j = j0 + threadIdx.x;
-    if (j < n) {
-      const double sg  = sst[F_SIG * scap + j];
-      const double is2 = 1.0 / (sg * sg);
-      sh[threadIdx.x]  = SrcF64{sst[(F_X + 0) * scap + j], sst[(F_X + 1) * scap + j], sst[(F_X + 2) * scap + j],
-                                sst[(F_A + 0) * scap + j], sst[(F_A + 1) * scap + j], sst[(F_A + 2) * scap + j], is2,
-                                0.5 * is2};
+  __shared__ __align__(32) unsigned char smem[64 * DIRECT_LANES];
+  // (x, q), (alpha, c1), q and c1 as in k_p2p; alpha unscaled, so a separation along it still gives 0
+  double4      *sv  = reinterpret_cast<double4 *>(smem);
+  double       *red = reinterpret_cast<double *>(smem);   // half of the 12 sums at a time
+  const int     tid = threadIdx.x, ti = tid & (NT - 1), si = tid / NT, S = DIRECT_LANES / NT;
+  const int64_t i0 = blockIdx.x * (int64_t)NT, i = min(i0 + ti, m - 1);
+  const double  xi = xt[3 * i], yi = xt[3 * i + 1], zi = xt[3 * i + 2];
+  double        acc[15];
+  for (int k = 0; k < 15; k++) acc[k] = 0.0;
+  double v[7];
+  auto   load = [&](int64_t j) {
+    j = min(j, n - 1);
+    for (int d = 0; d < 3; d++) v[d] = sst[(F_X + d) * scap + j], v[3 + d] = sst[(F_A + d) * scap + j];
+    v[6] = sst[F_SIG * scap + j];
+  };
+  load(tid);
+  for (int64_t j0 = 0; j0 < n; j0 += DIRECT_LANES) {
+    const int cnt = (int)min<int64_t>(DIRECT_LANES, n - j0);
+    const int T2  = 2 * ((cnt + 2 * S - 1) / (2 * S));  // entries per lane; T2 * S <= DIRECT_LANES as NT is even
+    double4   A, B;
+    if (tid < cnt) {
+      const double qq = 0.5 / (v[6] * v[6]);
+      A.x = v[0], A.y = v[1], A.z = v[2], A.w = qq;
+      B.x = v[3], B.y = v[4], B.z = v[5], B.w = qq * sqrt(qq) * INV_4PI;
+    } else {  // no strength, x near 1 for targets within some hundred units (see k_p2p)
+      A.x = v[0] + 1024.0, A.y = v[1], A.z = v[2], A.w = 0x1p-20;
+      B.x = B.y = B.z = B.w = 0.0;
     }
+    sv[2 * tid] = A, sv[2 * tid + 1] = B;
     __syncthreads();
-    const int cnt = (int)min<int64_t>(256, n - j0);
-    for (int q = 0; q < cnt; q++) {
-      const SrcF64 &sj = sh[q];
-      const double  dx = xi - sj.x, dy = yi - sj.y, dz = zi - sj.z;
-      const double  R2 = dx * dx + dy * dy + dz * dz;
-      if (R2 == 0.0) continue;
-      const double RS     = R2 * sj.halfInvS2;
-      const double sqrtRS = sqrt(RS);
-      const double t2     = 2.0 * INV_SQRTPI * sqrtRS * exp(-RS);
-      const double invR   = 1.0 / sqrt(R2);
-      const double o4pr3  = 0.25 * INV_PI / R2 * invR;
-      const double g      = erf(sqrtRS) - t2;
-      const double f1     = g * o4pr3;
-      const double f2     = (t2 * sj.invS2 - 3.0 * g / R2) * o4pr3;
-      const double cx = dy * sj.az - dz * sj.ay, cy = dz * sj.ax - dx * sj.az, cz = dx * sj.ay - dy * sj.ax;
-      acc[0] += f1 * cx;
-      acc[1] += f1 * cy;
-      acc[2] += f1 * cz;
-      const double k0 = f2 * cx, k1 = f2 * cy, k2 = f2 * cz;
-      acc[3] += k0 * dx;
-      acc[4] += k0 * dy + f1 * sj.az;
-      acc[5] += k0 * dz - f1 * sj.ay;
-      acc[6] += k1 * dx - f1 * sj.az;
-      acc[7] += k1 * dy;
-      acc[8] += k1 * dz + f1 * sj.ax;
-      acc[9] += k2 * dx + f1 * sj.ay;
-      acc[10] += k2 * dy - f1 * sj.ax;
-      acc[11] += k2 * dz;
+    if (j0 + DIRECT_LANES < n) load(j0 + DIRECT_LANES + tid);
+    const double4 *ps = sv + 2 * si;
+    for (int k = 0; k < T2; k += 2, ps += 4 * S) {
+      const double4 A0 = ps[0], B0 = ps[1], A1 = ps[2 * S], B1 = ps[2 * S + 1];
+      const double  dx0 = xi - A0.x, dy0 = yi - A0.y, dz0 = zi - A0.z;
+      const double  dx1 = xi - A1.x, dy1 = yi - A1.y, dz1 = zi - A1.z;
+      const double  r20 = dx0 * dx0 + dy0 * dy0 + dz0 * dz0, r21 = dx1 * dx1 + dy1 * dy1 + dz1 * dz1;
+      double        G0, Gp0, G1, Gp1;
+      g64_pair2(r20, r21, A0.w, A1.w, G0, Gp0, G1, Gp1);
+      accumulate_pair(acc, dx0, dy0, dz0, B0.x, B0.y, B0.z, G0 * B0.w, 2.0 * Gp0 * (A0.w * B0.w), WITH_J);
+      accumulate_pair(acc, dx1, dy1, dz1, B1.x, B1.y, B1.z, G1 * B1.w, 2.0 * Gp1 * (A1.w * B1.w), WITH_J);
     }
     __syncthreads();
   }
-  if (!ok) return;
-  for (int d = 0; d < 3; d++) u[3 * i + d] = -acc[d];
-  if (J)
-    for (int k = 0; k < 9; k++) J[9 * i + k] = -acc[3 + k];
-  if (dadt && at)
-    for (int a = 0; a < 3; a++)
-      dadt[3 * i + a] = -(acc[3 + 3 * a] * at[3 * i] + acc[4 + 3 * a] * at[3 * i + 1] + acc[5 + 3 * a] * at[3 * i + 2]);
+  if (WITH_J) fold_antisym(acc);
+  // the splits of each (field, target), six fields at a time; lanes (field, target)
+  for (int h = 0; h < (WITH_J ? 2 : 1); h++) {
+    for (int k = 0; k < 6; k++) red[k * DIRECT_LANES + tid] = acc[h ? 6 + k : k];
+    __syncthreads();
+    for (int o = tid; o < (WITH_J ? 6 : 3) * NT; o += DIRECT_LANES) {
+      const int k = o / NT, t = o & (NT - 1);
+      double    w = 0.0;
+      for (int q = 0; q < S; q++) w += red[k * DIRECT_LANES + q * NT + t];
+      const int f = 6 * h + k;
+      if (i0 + t < m) {
+        if (f < 3) u[3 * (i0 + t) + f] = -w;
+        else if (J) J[9 * (i0 + t) + f - 3] = -w;
+      }
+      // kept for the stretching: this lane's sum goes back where it came from, split 0
+      red[k * DIRECT_LANES + t] = w;
+    }
+    __syncthreads();
+    if (WITH_J && dadt && at && tid < NT && i0 + tid < m) {
+      const double *a = at + 3 * (i0 + tid);
+      if (h == 0) acc[0] = red[3 * DIRECT_LANES + tid] * a[0] + red[4 * DIRECT_LANES + tid] * a[1] + red[5 * DIRECT_LANES + tid] * a[2];
+      else {
+        double *o = dadt + 3 * (i0 + tid);
+        o[0] = -acc[0];
+        for (int r = 0; r < 2; r++)
+          o[1 + r] = -(red[3 * r * DIRECT_LANES + tid] * a[0] + red[(3 * r + 1) * DIRECT_LANES + tid] * a[1] +
+                       red[(3 * r + 2) * DIRECT_LANES + tid] * a[2]);
+      }
+    }
+    __syncthreads();
+  }
 }
 
 }  // namespace
@@ -339,7 +364,11 @@ void direct(hipStream_t s, int64_t m, const double *xt, const double *at, const 
             double *u, double *J, double *dadt)
 {
   if (m <= 0) return;
-  k_direct<<<(int)((m + 255) / 256), 256, 0, s>>>(m, xt, at, sst, scap, n, u, J, dadt);
+  int NT = 64;
+  while (NT > 2 && (m + NT - 1) / NT < DIRECT_BLOCKS) NT /= 2;
+  const int nb = (int)((m + NT - 1) / NT);
+  if (J || dadt) k_direct<true><<<nb, DIRECT_LANES, 0, s>>>(NT, m, xt, at, sst, scap, n, u, J, dadt);
+  else k_direct<false><<<nb, DIRECT_LANES, 0, s>>>(NT, m, xt, at, sst, scap, n, u, J, dadt);
   UVLM_LAUNCH_CHECK();
 }
 
