@@ -95,3 +95,36 @@ def test_direct(orc, m, n):
     assert rel(u, wu) < 1e-12 and rel(u2, wu) < 1e-12
     assert rel(J, wJ.reshape(m, 9)) < 1e-11 and rel(D, wD) < 1e-11
     g.close()
+
+
+@pytest.mark.parametrize("n,ncrit", [(3, 64), (65, 1), (1500, 7), (4000, 33), (9000, 200)])
+def test_gaussian_sums(orc, n, ncrit):
+    """PSE rates and probe vorticity over the same lists; two coincident bodies among them (that
+    pair is skipped by PSE and counted by the vorticity)."""
+    X, A, S = cluster(n, n + 1, 0.05)
+    if ncrit > 1:
+        X[-1] = X[0]
+    ref_b = orc.make_bodies(X, A, S)
+    ref = orc.Calculator(P=4, theta=0.5, ncrit=ncrit)
+    ref.init(ref_b)
+    ref.calculate()
+    ref.set_viscosity("pse", 0.3)
+    ref.viscosity(0.01)
+    want = ref.bodies(n)
+    m = min(n, 37)
+    sb = orc.make_bodies(X[:m] + 0.002, np.zeros((m, 3)), np.ones(m))
+    ref.vorticity(sb)
+    print(f"[near] gauss n={n} ncrit={ncrit}", flush=True)
+    g = FMMCalculator(P=4, theta=0.5, ncrit=ncrit)
+    g.set_bodies(make_bodies(X, A, S))
+    g.build()
+    g.calculate()
+    g.set_viscosity("pse", 0.3)
+    g.viscosity(0.01)
+    out = g.copyBodies2Host()
+    assert rel(out[:, 18:21], want[:, 18:21]) < 1e-10
+    s = make_bodies(X[:m] + 0.002, np.zeros((m, 3)), np.ones(m))
+    g.vorticity(s)
+    assert np.array_equal(s[:, 9:12], sb[:, 9:12])
+    assert rel(s[:, 21:24], sb[:, 21:24]) < 1e-10
+    g.close()

@@ -242,7 +242,7 @@ void do_eval(uvlm_handle h, bool sync)
 void apply_viscosity(uvlm_handle h, double dt)
 {
   if (h->viscous == UVLM_PSE)
-    gauss_near(h->s, h->tree, h->tree, h->lists, h->st.as<double>(), h->cap, h->st.as<double>(), h->cap,
+    gauss_near(h->s, h->sc, h->tree, h->tree, h->lists, h->st.as<double>(), h->cap, h->st.as<double>(), h->cap,
                h->st.as<double>(), h->cap, 0, 0, h->nu / std::sqrt(2.0) * INV_PI * INV_SQRTPI);
   else if (h->viscous == UVLM_CSM)
     csm(h->s, h->st.as<double>(), h->cap, h->N, h->nu, dt);
@@ -293,8 +293,9 @@ void probe_vorticity(uvlm_handle h, int64_t m)
 {
   Region region("Calculation of Vorticity");  // fmmCalculator.hpp:735
   traverse(h->s, h->sc, h->stree, h->tree, h->prm.theta, h->slists, h->gap);
+  near_units(h->s, h->sc, h->stree, h->tree, h->prm.ncrit, h->slists);
   zero_fields(h->s, h->sst.as<double>(), h->scap, m, F_UOLD, 3);
-  gauss_near(h->s, h->stree, h->tree, h->slists, h->sst.as<double>(), h->scap, h->st.as<double>(), h->cap,
+  gauss_near(h->s, h->sc, h->stree, h->tree, h->slists, h->sst.as<double>(), h->scap, h->st.as<double>(), h->cap,
              h->sst.as<double>(), h->scap, 1, F_UOLD, 0.0);
 }
 
@@ -1294,6 +1295,7 @@ int uvlm_rbf_aos(uvlm_handle h, void *points, int64_t m, int64_t stride, int64_t
     // tree over the kept points and its self lists (createSensorTree(sensorOnly), 164-201)
     upload_probes(h, keep.data(), k, 296);
     traverse(s, h->sc, h->stree, h->stree, h->prm.theta, h->slists, h->gap);
+    near_units(s, h->sc, h->stree, h->stree, h->prm.ncrit, h->slists);
     double       *st = h->sst.as<double>();
     const int64_t sc = h->scap;
     h->sc.partial.reserve(sizeof(double) * 3 * 512);
@@ -1301,7 +1303,7 @@ int uvlm_rbf_aos(uvlm_handle h, void *points, int64_t m, int64_t stride, int64_t
     auto single = [&] {  // calculateVorticitySingleTree (788-795): velocity = -A alpha
       zero_fields(s, st, sc, k, F_U, 3);
       zero_fields(s, st, sc, k, F_DADT, 3);
-      gauss_near(s, h->stree, h->stree, h->slists, st, sc, st, sc, st, sc, 1, F_U, 0.0);
+      gauss_near(s, h->sc, h->stree, h->stree, h->slists, st, sc, st, sc, st, sc, 1, F_U, 0.0);
     };
     const double tol = 1e-10, eps = 2.220446049250313e-16;
     rbf_vec(s, st, sc, k, 0, nullptr);  // initAlphaValues

@@ -187,7 +187,7 @@ void near_units(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &st, int6
 void p2p(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &stree, const Lists &l, const double *tgt, int64_t tcap,
          const double *src, int64_t scap, double *out, int64_t ocap, int precision, int sensor_mode);
 
-void gauss_near(hipStream_t s, const Tree &tt, const Tree &stree, const Lists &l, const double *tgt, int64_t tcap,
+void gauss_near(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &stree, const Lists &l, const double *tgt, int64_t tcap,
                 const double *srcst, int64_t scap, double *out, int64_t ocap, int mode, int field, double prefix);
 void direct(hipStream_t s, int64_t m, const double *xt, const double *at, const double *sst, int64_t scap, int64_t n,
             double *u, double *J, double *dadt);

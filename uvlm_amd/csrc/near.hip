@@ -152,14 +152,7 @@ __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(MIXED ? 5 :
 #pragma unroll
         for (int p = 0; p < PER; p++) {
           // entries past the chunk load its last one again and are stored as padding
-          const int g  = j0 + min(lane + p * BLK, cnt - 1);
-          int       lo = 0, hi = nseg - 1;  // last q with pref[q] <= g
-          while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (pref[mid] <= g) lo = mid;
-            else hi = mid - 1;
-          }
-          const int64_t bj = lb[lo] + (g - pref[lo]);
+          const int64_t bj = list_body(pref, lb, nseg, j0 + min(lane + p * BLK, cnt - 1));
           x[p] = sst[(F_X + 0) * scap + bj], y[p] = sst[(F_X + 1) * scap + bj], z[p] = sst[(F_X + 2) * scap + bj];
           sg[p] = sst[F_SIG * scap + bj];
           ax[p] = sst[(F_A + 0) * scap + bj], ay[p] = sst[(F_A + 1) * scap + bj], az[p] = sst[(F_A + 2) * scap + bj];
@@ -495,84 +488,144 @@ __global__ __launch_bounds__(256) void k_p2p_reduce(const int4 *__restrict__ mul
 }
 
 // Gaussian near-field sums over the P2P lists, FP64 (the viscous and vorticity kernels of
-// multipoleKernels.hpp:343-450).  One 64-lane workgroup per target leaf, lane <-> target;
-// the source bodies of each list entry pass through LDS; sums in list order (deterministic).
+// multipoleKernels.hpp:343-450).
 //  GAUSS_PSE : dadt_i += prefix * sum_j (vol_i a_j - vol_j a_i) e^{-R^2 / (2 s_ij^2)} / s_ij^5,
 //              s_ij^2 = sigma_i^2 + sigma_j^2, vol = 4/3 pi sigma^3, pairs with R^2 = 0 skipped
 //  GAUSS_VORT: out[field + d]_i -= sum_j a_j,d e^{-R^2 / (2 sigma_j^2)} / ((2 pi)^{3/2} sigma_j^3)
+// Units, chunks, lanes and the sum of the splits are k_p2p's; sums in a fixed order.  Bound by VALU
+// issue: about 55 lane-instructions a pair (PSE: the exponential 18, the reciprocal root of s_ij^2
+// 7).  One lane per target with library exp, sqrt and two divisions took 2.6 ms for the 100k two
+// rings (136e6 pairs, up to 100 bodies a leaf).
 enum { GAUSS_PSE = 0, GAUSS_VORT = 1 };
-template <int MODE>
-__global__ __launch_bounds__(WG) void k_gauss(const int32_t *__restrict__ leaves, int64_t nleaf,
-                                              const int32_t *__restrict__ tbody, const int32_t *__restrict__ tnbody,
-                                              const int32_t *__restrict__ off, const int32_t *__restrict__ src,
-                                              const int32_t *__restrict__ sbody, const int32_t *__restrict__ snbody,
-                                              const double *__restrict__ tst, int64_t tcap,
-                                              const double *__restrict__ sst, int64_t scap, double *__restrict__ out,
-                                              int64_t ocap, int field, double prefix)
+template <int MODE, int BLK>
+__global__ __launch_bounds__(BLK) void k_gauss(const int4 *__restrict__ units, const int32_t *__restrict__ leaves,
+                                               const int32_t *__restrict__ tbody, const int32_t *__restrict__ tnbody,
+                                               const int32_t *__restrict__ src, const int32_t *__restrict__ sbody,
+                                               const int32_t *__restrict__ snbody, const double *__restrict__ tst,
+                                               int64_t tcap, const double *__restrict__ sst, int64_t scap,
+                                               double *__restrict__ out, int64_t ocap, int field, double prefix,
+                                               double *__restrict__ part)
 {
-  __shared__ double sx[WG], sy[WG], sz[WG], ss[WG], sa0[WG], sa1[WG], sa2[WG];
-  const int64_t w = blockIdx.x;
-  if (w >= nleaf) return;
-  const int t = leaves[w], tb = tbody[t], nt = tnbody[t], lane = threadIdx.x;
-  const int q0 = off[t], q1 = off[t + 1];
-  for (int c0 = 0; c0 < nt; c0 += WG) {
-    const int     i     = c0 + lane;
-    const bool    valid = i < nt;
-    const int64_t bi    = tb + (valid ? i : 0);
+  constexpr int CH = BLK == 64 ? 128 : 256, ENT = CH + CH / 2, PER = CH / BLK;
+  __shared__ __align__(32) unsigned char smem[ENT * 64];
+  __shared__ int pref[SEG + 1], lb[SEG];
+  double4 *sv  = reinterpret_cast<double4 *>(smem);  // (x, sigma^2 or q), (alpha, vol) or (alpha c, 0)
+  double  *red = reinterpret_cast<double *>(smem);
+  const int4 un = units[blockIdx.x];
+  const int  t = leaves[un.x], tb = tbody[t], nt = tnbody[t], q0 = un.y, q1 = un.z, prow = un.w;
+  const int  lane = threadIdx.x;
+  const int  ntp = near_targets_per_pass<BLK>(nt), S = near_splits<BLK>(ntp), ti = lane % ntp, si = lane / ntp;
+  const bool lane_on = si < S;
+  for (int c0 = 0; c0 < nt; c0 += ntp) {
+    const int     i  = c0 + ti;
+    const int64_t bi = tb + (lane_on && i < nt ? i : 0);
     const double  xi = tst[(F_X + 0) * tcap + bi], yi = tst[(F_X + 1) * tcap + bi], zi = tst[(F_X + 2) * tcap + bi];
-    double        sgi = 0.0, voli = 0.0, ai[3] = {0.0, 0.0, 0.0};
+    double        s2i = 0.0, voli = 0.0, ai[3] = {0.0, 0.0, 0.0};
     if (MODE == GAUSS_PSE) {
-      sgi  = tst[F_SIG * tcap + bi];
-      voli = 4. / 3. * M_PI * sgi * sgi * sgi;
+      const double sg = tst[F_SIG * tcap + bi];
+      s2i  = sg * sg;
+      voli = 4. / 3. * M_PI * sg * sg * sg;
       for (int d = 0; d < 3; d++) ai[d] = tst[(F_A + d) * tcap + bi];
     }
     double acc[3] = {0.0, 0.0, 0.0};
-    for (int q = q0; q < q1; q++) {
-      const int sl = src[q], b0 = sbody[sl], nb = snbody[sl];
-      for (int j0 = 0; j0 < nb; j0 += WG) {
-        const int cnt = min(WG, nb - j0);
-        __syncthreads();
-        if (lane < cnt) {
-          const int64_t bj = b0 + j0 + lane;
-          sx[lane]         = sst[(F_X + 0) * scap + bj];
-          sy[lane]         = sst[(F_X + 1) * scap + bj];
-          sz[lane]         = sst[(F_X + 2) * scap + bj];
-          ss[lane]         = sst[F_SIG * scap + bj];
-          sa0[lane]        = sst[(F_A + 0) * scap + bj];
-          sa1[lane]        = sst[(F_A + 1) * scap + bj];
-          sa2[lane]        = sst[(F_A + 2) * scap + bj];
+    auto   pair = [&](const double4 &A, const double4 &B) {
+      const double dx = xi - A.x, dy = yi - A.y, dz = zi - A.z, R2 = dx * dx + dy * dy + dz * dz;
+      if (MODE == GAUSS_PSE) {
+        const double r = rsqrt64(s2i + A.w), o2 = r * r;
+        const double e = R2 == 0.0 ? 0.0 : exp64_neg(0.5 * R2 * o2, c_exp64) * (o2 * o2 * r);
+        acc[0] = fma(voli * B.x - B.w * ai[0], e, acc[0]);
+        acc[1] = fma(voli * B.y - B.w * ai[1], e, acc[1]);
+        acc[2] = fma(voli * B.z - B.w * ai[2], e, acc[2]);
+      } else {
+        const double e = exp64_neg(R2 * A.w, c_exp64);
+        acc[0] = fma(B.x, e, acc[0]);
+        acc[1] = fma(B.y, e, acc[1]);
+        acc[2] = fma(B.z, e, acc[2]);
+      }
+    };
+    for (int g0 = q0; g0 < q1; g0 += SEG) {
+      const int nseg = min(SEG, q1 - g0);
+      __syncthreads();
+      for (int k = lane; k < nseg; k += BLK) {
+        const int sl = src[g0 + k];
+        lb[k]        = sbody[sl];
+        pref[k]      = snbody[sl];
+      }
+      __syncthreads();
+      if (lane < 64) lds_prefix(pref, pref, nseg);
+      __syncthreads();
+      const int total = pref[nseg];
+      for (int j0 = 0; j0 < total; j0 += CH) {
+        const int cnt = min(CH, total - j0);
+        const int T2  = 2 * ((cnt + 2 * S - 1) / (2 * S));
+        double    v[PER][7];
+#pragma unroll
+        for (int p = 0; p < PER; p++) {
+          const int64_t bj = list_body(pref, lb, nseg, j0 + min(lane + p * BLK, cnt - 1));
+          for (int d = 0; d < 3; d++) v[p][d] = sst[(F_X + d) * scap + bj], v[p][3 + d] = sst[(F_A + d) * scap + bj];
+          v[p][6] = sst[F_SIG * scap + bj];
         }
-        __syncthreads();
-        if (!valid) continue;
-        for (int j = 0; j < cnt; j++) {
-          const double dx = xi - sx[j], dy = yi - sy[j], dz = zi - sz[j];
-          const double R2 = dx * dx + dy * dy + dz * dz;
-          const double sj = ss[j];
-          if (MODE == GAUSS_PSE) {
-            if (R2 == 0.0) continue;
-            const double o2   = 1.0 / (sgi * sgi + sj * sj);
-            const double s5   = o2 * o2 * sqrt(o2);
-            const double volj = 4. / 3. * M_PI * sj * sj * sj;
-            const double e    = exp(-0.5 * R2 * o2) * s5;
-            acc[0] += (voli * sa0[j] - volj * ai[0]) * e;
-            acc[1] += (voli * sa1[j] - volj * ai[1]) * e;
-            acc[2] += (voli * sa2[j] - volj * ai[2]) * e;
-          } else {
-            const double S2 = 2.0 * sj * sj;
-            const double z  = exp(-R2 / S2) * (INV_PI * INV_SQRTPI * 0.70710678118654752440) / S2 / sj;
-            acc[0] += sa0[j] * z;
-            acc[1] += sa1[j] * z;
-            acc[2] += sa2[j] * z;
+#pragma unroll
+        for (int p = 0; p < PER; p++) {
+          const int e = lane + p * BLK;
+          if (e < cnt) {
+            const double sg = v[p][6], S2 = 2.0 * sg * sg;
+            const double c  = MODE == GAUSS_PSE ? 1.0 : (INV_PI * INV_SQRTPI * 0.70710678118654752440) / S2 / sg;
+            double4      A, B;
+            A.x = v[p][0], A.y = v[p][1], A.z = v[p][2], A.w = MODE == GAUSS_PSE ? sg * sg : 1.0 / S2;
+            B.x = v[p][3] * c, B.y = v[p][4] * c, B.z = v[p][5] * c;
+            B.w = MODE == GAUSS_PSE ? 4. / 3. * M_PI * sg * sg * sg : 0.0;
+            sv[2 * e] = A, sv[2 * e + 1] = B;
           }
         }
+        // entries of no strength and no volume past the chunk
+        double4 pad;
+        pad.x = pad.y = pad.z = pad.w = 1.0;
+        double4 none;
+        none.x = none.y = none.z = none.w = 0.0;
+        for (int e = cnt + lane; e < T2 * S; e += BLK) sv[2 * e] = pad, sv[2 * e + 1] = none;
+        __syncthreads();
+        const double4 *ps = sv + 2 * (lane_on ? si : 0);
+        for (int k = 0; k < T2; k += 2, ps += 4 * S) {
+          pair(ps[0], ps[1]);
+          pair(ps[2 * S], ps[2 * S + 1]);
+        }
+        __syncthreads();
       }
     }
-    if (valid) {
-      if (MODE == GAUSS_PSE)
-        for (int d = 0; d < 3; d++) out[(F_DADT + d) * ocap + bi] += acc[d] * prefix;
-      else
-        for (int d = 0; d < 3; d++) out[(field + d) * ocap + bi] -= acc[d];
+    const int np = min(ntp, nt - c0);
+    __syncthreads();
+    for (int d = 0; d < 3; d++) red[d * BLK + lane] = acc[d];
+    __syncthreads();
+    for (int o = lane; o < 3 * np; o += BLK) {
+      const int d = o / np, tt = o - d * np;
+      double    v = red[d * BLK + tt];
+      for (int q = 1; q < S; q++) v += red[d * BLK + tt + q * ntp];
+      if (prow >= 0) part[(int64_t)prow * 12 + (int64_t)d * nt + c0 + tt] = v;
+      else if (MODE == GAUSS_PSE) out[(F_DADT + d) * ocap + tb + c0 + tt] += v * prefix;
+      else out[(field + d) * ocap + tb + c0 + tt] -= v;
     }
+  }
+}
+
+template <int MODE>
+__global__ __launch_bounds__(256) void k_gauss_reduce(const int4 *__restrict__ multi,
+                                                      const int32_t *__restrict__ leaves,
+                                                      const int32_t *__restrict__ tbody,
+                                                      const int32_t *__restrict__ tnbody,
+                                                      const double *__restrict__ part, double *__restrict__ out,
+                                                      int64_t ocap, int field, double prefix)
+{
+  const int4    m = multi[blockIdx.x];
+  const int     t = leaves[m.x], tb = tbody[t], nt = tnbody[t];
+  const double *p = part + (int64_t)m.y * 12;
+  for (int o = threadIdx.x; o < 3 * nt; o += 256) {
+    const int d = o / nt;
+    double    v = 0.0;
+#pragma unroll 4
+    for (int u = 0; u < m.z; u++) v += p[(int64_t)u * 12 * nt + o];
+    if (MODE == GAUSS_PSE) out[(F_DADT + d) * ocap + tb + (o - d * nt)] += v * prefix;
+    else out[(field + d) * ocap + tb + (o - d * nt)] -= v;
   }
 }
 
@@ -655,22 +708,35 @@ void p2p(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &stree, const Li
 }
 
 // PSE (mode 0, adds prefix * sum to dadt) or Gaussian vorticity (mode 1, subtracts the sum
-// from fields field..field+2) of the source tree at the target tree's leaves, over the P2P lists.
-void gauss_near(hipStream_t s, const Tree &tt, const Tree &stree, const Lists &l, const double *tgt, int64_t tcap,
-                const double *srcst, int64_t scap, double *out, int64_t ocap, int mode, int field, double prefix)
+// from fields field..field+2) of the source tree at the target tree's leaves, over the P2P lists
+// and their units.
+void gauss_near(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &stree, const Lists &l, const double *tgt,
+                int64_t tcap, const double *srcst, int64_t scap, double *out, int64_t ocap, int mode, int field,
+                double prefix)
 {
   if (tt.nleaf == 0) return;
-  const int nb = (int)tt.nleaf;
-  if (mode == 0)
-    k_gauss<GAUSS_PSE><<<nb, WG, 0, s>>>(tt.leaves.as<int32_t>(), tt.nleaf, tt.body.as<int32_t>(),
-                                         tt.nbody.as<int32_t>(), l.p2p_off.as<int32_t>(), l.p2p_src.as<int32_t>(),
-                                         stree.body.as<int32_t>(), stree.nbody.as<int32_t>(), tgt, tcap, srcst, scap,
-                                         out, ocap, field, prefix);
-  else
-    k_gauss<GAUSS_VORT><<<nb, WG, 0, s>>>(tt.leaves.as<int32_t>(), tt.nleaf, tt.body.as<int32_t>(),
-                                          tt.nbody.as<int32_t>(), l.p2p_off.as<int32_t>(), l.p2p_src.as<int32_t>(),
-                                          stree.body.as<int32_t>(), stree.nbody.as<int32_t>(), tgt, tcap, srcst, scap,
-                                          out, ocap, field, prefix);
+  if (l.n_units < tt.nleaf) throw Error(UVLM_ERR_INTERNAL, "Gaussian near field without its units");
+  sc.p2p_part.reserve(sizeof(double) * 12 * l.n_rows);
+  double        *part = sc.p2p_part.as<double>();
+  const int32_t *lv = tt.leaves.as<int32_t>(), *tb = tt.body.as<int32_t>(), *tn = tt.nbody.as<int32_t>();
+  auto           launch = [&](auto kern, int blk) {
+    kern<<<(int)l.n_units, blk, 0, s>>>(l.units.as<int4>(), lv, tb, tn, l.p2p_src.as<int32_t>(),
+                                        stree.body.as<int32_t>(), stree.nbody.as<int32_t>(), tgt, tcap, srcst, scap,
+                                        out, ocap, field, prefix, part);
+  };
+  auto reduce = [&](auto kern) {
+    if (l.n_multi > 0)
+      kern<<<(int)l.n_multi, 256, 0, s>>>(l.multi.as<int4>(), lv, tb, tn, part, out, ocap, field, prefix);
+  };
+  if (mode == 0) {
+    if (l.wide) launch(k_gauss<GAUSS_PSE, 256>, 256);
+    else launch(k_gauss<GAUSS_PSE, 64>, 64);
+    reduce(k_gauss_reduce<GAUSS_PSE>);
+  } else {
+    if (l.wide) launch(k_gauss<GAUSS_VORT, 256>, 256);
+    else launch(k_gauss<GAUSS_VORT, 64>, 64);
+    reduce(k_gauss_reduce<GAUSS_VORT>);
+  }
   UVLM_LAUNCH_CHECK();
 }
 

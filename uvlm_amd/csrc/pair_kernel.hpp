@@ -206,10 +206,9 @@ __device__ __forceinline__ double fma_sc(double a, double b, double c)
   return d;
 }
 
-// e^{-x} for x >= 0 (0 from x = 745 on).
-__device__ __forceinline__ double exp64_neg(double x)
+// e^{-x} for x >= 0 (0 from x = 745 on).  c: c_exp64, or here(c_exp64) where the call is rare.
+template <class C> __device__ __forceinline__ double exp64_neg(double x, C c)
 {
-  const ConstF64 c = here(c_exp64);
   const double xe = fmin(x, 800.0);
   const double k  = rint(xe * -1.4426950408889634);
   const double r  = fma(k, -2.3190468138462996e-17, fma(k, -0.6931471805599453, -xe))  /* ln 2 in two parts */;
@@ -226,7 +225,7 @@ __device__ __forceinline__ void g64_far(double x, double &G, double &Gp, double 
   const double w = rsqrt64(x), w2 = w * w;
   double       g = 1.0, ce = 0.0;
   if (x < FAR64) {
-    const double e = exp64_neg(x), t = fmax(w, FAR64_WMIN) - FAR64_WC;
+    const double e = exp64_neg(x, here(c_exp64)), t = fmax(w, FAR64_WMIN) - FAR64_WC;
     const ConstF64 c = here(c_far64);
     double         p = c[NFAR64 - 1];
 #pragma unroll
@@ -308,6 +307,19 @@ __device__ __forceinline__ void lds_prefix(int *pref, const int *v, int n)
     run += loc[k];
   }
   if (lane == 63 && 256 <= n) pref[256] = run;
+}
+
+// Body g of the list entries whose leaf sizes have the prefix sums pref[0..n] and first bodies lb:
+// that of the last entry q with pref[q] <= g.
+__device__ __forceinline__ int64_t list_body(const int *pref, const int *lb, int n, int g)
+{
+  int lo = 0, hi = n - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (pref[mid] <= g) lo = mid;
+    else hi = mid - 1;
+  }
+  return lb[lo] + (g - pref[lo]);
 }
 
 }  // namespace
