@@ -46,46 +46,34 @@ template <class T> __device__ inline void cross(const T a[3], const T b[3], T o[
   o[2] = a[0] * b[1] - a[1] * b[0];
 }
 
-// W and dS/dr of one pair (see the header); returns false for R^2 = 0 (no interaction).
-__device__ inline bool pair_adj(const double r[3], const double al[3], double sg, const double ub[3],
-                                const double Jb[9], double W[3], double dS[3])
+// G, G', G'' at x = R^2 q (pair_kernel.hpp).
+__device__ __forceinline__ void pair_g(float r2, float q, float &G, float &Gp, float &Gpp)
 {
-  const double R2 = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
-  if (R2 == 0.0) return false;
-  const double is2 = 1.0 / (sg * sg);
-  const double RS = 0.5 * R2 * is2, s = sqrt(RS);
-  const double t2 = 2.0 * INV_SQRTPI * s * exp(-RS);
-  const double g  = erf(s) - t2;
-  const double q  = 0.25 * INV_PI / (R2 * sqrt(R2));
-  const double f1 = g * q;
-  const double f2 = (t2 * is2 - 3.0 * g / R2) * q;
-  const double f3 = (15.0 * g / (R2 * R2) - t2 * (5.0 + 2.0 * RS) * is2 / R2) * q;
-  const double e[3]  = {Jb[5] - Jb[7], Jb[6] - Jb[2], Jb[1] - Jb[3]};
-  const double Jr[3] = {Jb[0] * r[0] + Jb[1] * r[1] + Jb[2] * r[2], Jb[3] * r[0] + Jb[4] * r[1] + Jb[5] * r[2],
-                        Jb[6] * r[0] + Jb[7] * r[1] + Jb[8] * r[2]};
-  double uxr[3], Jrxr[3], rxa[3], axu[3], axJr[3];
-  cross(ub, r, uxr);
-  cross(Jr, r, Jrxr);
-  cross(r, al, rxa);
-  cross(al, ub, axu);
-  cross(al, Jr, axJr);
-  double c1 = 0.0, c3 = 0.0;
-  for (int d = 0; d < 3; d++) {
-    W[d] = f1 * (uxr[d] + e[d]) + f2 * Jrxr[d];
-    c1 += al[d] * (uxr[d] + e[d]);
-    c3 += al[d] * Jrxr[d];
-  }
-  for (int d = 0; d < 3; d++) {
-    const double JTrxa = Jb[d] * rxa[0] + Jb[3 + d] * rxa[1] + Jb[6 + d] * rxa[2];
-    dS[d]              = -((f2 * c1 + f3 * c3) * r[d] + f1 * axu[d] + f2 * (JTrxa + axJr[d]));
-  }
-  return true;
+  kernel_g<true>(r2 * q, G, Gp, Gpp);
 }
+__device__ __forceinline__ void pair_g(double r2, double q, double &G, double &Gp, double &Gpp)
+{
+  const double x = r2 * q;
+  if ((unsigned)__double2hiint(x) < X64_HI) {
+    const double t = x - 0.5 * X64;
+    double       g = c_g64[NG64 - 1], p = c_gp64[NG64 - 1], d = c_gpp64[NGPP64 - 1];
+#pragma unroll
+    for (int k = NG64 - 2; k >= 0; k--) {
+      g = fma(g, t, c_g64[k]);
+      p = fma(p, t, c_gp64[k]);
+    }
+#pragma unroll
+    for (int k = NGPP64 - 2; k >= 0; k--) d = fma(d, t, c_gpp64[k]);
+    G = g, Gp = p, Gpp = d;
+  } else g64_far<true>(x, G, Gp, Gpp);
+}
+__device__ __forceinline__ float  fma_(float a, float b, float c) { return fmaf(a, b, c); }
+__device__ __forceinline__ double fma_(double a, double b, double c) { return fma(a, b, c); }
 
-// Near-field adjoint, one 64-lane workgroup per leaf of the (single) tree.  Like the forward
-// P2P kernel, lanes = (own body) x (split s) so small leaves keep the wavefront busy, the
-// bodies of all listed leaves stream through LDS in full chunks across leaf boundaries, and
-// the splits are combined by cross-lane adds in a fixed order (deterministic, no atomics).
+// Near-field adjoint, one workgroup per near-field unit of the (single) tree's list.  Like the
+// forward P2P kernel, lanes = (own body) x (split s), the bodies of all listed leaves stream
+// through LDS in chunks across leaf boundaries, and the splits and a leaf's units are added in a
+// fixed order (deterministic, no atomics).
 //  SIDE 0 (forward P2P list, own = target i):            xbar_i += sum_j dS_ij/dr
 //  SIDE 1 (transposed list, own = source j): alphabar_j -= sum_i W_ij, xbar_j -= sum_i dS_ij/dr
 // Sums over the pairs are arranged so that what belongs to the own body is applied once per
@@ -94,235 +82,198 @@ __device__ inline bool pair_adj(const double r[3], const double al[3], double sg
 //          V = sum f2 (r x alpha_j), A = sum f2 alpha_j x (Jbar r), k = f2 c1 + f3 c3;
 //  SIDE 1: sum_i dS_ij = -[X + sum f2 Jbar_i^T (r x alpha) + alpha x sum (f1 ubar_i + f2 Jbar_i r)].
 // MIXED: FP32 pair arithmetic on coordinates relative to the own leaf centre (formed in FP64
-// while staging), f1, f2, f3 from G, G', G'' (pair_kernel.hpp), FP32 partial sums per chunk
-// added into FP64 accumulators.  Otherwise FP64 with erf and exp (pair_adj).
-template <bool MIXED, int SIDE>
-__global__ __launch_bounds__(WG) void k_p2p_adj(const int32_t *__restrict__ leaves, int64_t nleaf,
-                                                const int32_t *__restrict__ cbody, const int32_t *__restrict__ cnbody,
-                                                const double *__restrict__ ccx, const double *__restrict__ ccy,
-                                                const double *__restrict__ ccz, const int32_t *__restrict__ off,
-                                                const int32_t *__restrict__ src, const double *__restrict__ st,
-                                                double *__restrict__ aux, int64_t cap)
+// while staging), FP32 partial sums of at most FLUSH entries a lane added into FP64 accumulators.
+// Otherwise FP64 throughout.  Bound by VALU issue.  2.1e8 mixed pairs (260k blobs, P = 8,
+// ncrit 64), against one wavefront per leaf and chunks of 64: SIDE 0 1.19 -> 0.60 ms, SIDE 1 1.48 ->
+// 0.75 ms.
+template <bool MIXED, int SIDE, int BLK>
+__global__ __launch_bounds__(BLK) void k_p2p_adj(const int4 *__restrict__ units, const int32_t *__restrict__ leaves,
+                                                 const int32_t *__restrict__ cbody, const int32_t *__restrict__ cnbody,
+                                                 const double *__restrict__ ccx, const double *__restrict__ ccy,
+                                                 const double *__restrict__ ccz, const int32_t *__restrict__ src,
+                                                 const double *__restrict__ st, double *__restrict__ aux, int64_t cap,
+                                                 double *__restrict__ part)
 {
-  // staged per other body: MIXED SIDE 0: rel x, q | alpha, c1 | c2, c3; SIDE 1: rel x, ubar, e, Jbar
-  constexpr int NV = SIDE == 0 ? 3 : 5;   // float4 per slot (MIXED)
-  constexpr int ND = SIDE == 0 ? 7 : 15;  // doubles per slot (FP64): x, alpha, sigma | x, ubar, Jbar
-  __shared__ float4 s32[MIXED ? NV * WG : 1];
-  __shared__ double s64[MIXED ? 1 : ND * WG];
-  __shared__ int    pref[SEG + 1], lb[SEG], ln[SEG];
-  const int64_t w = blockIdx.x;
-  if (w >= nleaf) return;
-  const int c = leaves[w], tb = cbody[c], nt = cnbody[c], lane = threadIdx.x;
-  // lanes = (own body ti) x (split si), ntp = the leaf's size (at most WG), S = WG / ntp splits
-  const int    ntp = near_targets_per_pass<WG>(nt), S = WG / ntp, ti = lane % ntp, si = lane / ntp;
+  using T = typename std::conditional<MIXED, float, double>::type;
+  // staged per other body: SIDE 0: x, q, alpha, c1, c2, c3 (f_k = c_k G^(k-1));  SIDE 1: x, ubar, e, Jbar
+  constexpr int NV = SIDE == 0 ? 10 : 18, NK = SIDE == 0 ? 3 : 6, CH = BLK;
+  constexpr int SMEM = NV * CH * (int)sizeof(T) > NK * BLK * 8 ? NV * CH * (int)sizeof(T) : NK * BLK * 8;
+  __shared__ __align__(16) unsigned char smem[SMEM];
+  __shared__ int pref[SEG + 1], lb[SEG];
+  T      *sv  = reinterpret_cast<T *>(smem);       // [CH][NV]
+  double *red = reinterpret_cast<double *>(smem);  // [NK][BLK]
+  const int4 un = units[blockIdx.x];
+  const int  c = leaves[un.x], tb = cbody[c], nt = cnbody[c], q0 = un.y, q1 = un.z, prow = un.w, lane = threadIdx.x;
+  const int    ntp = near_targets_per_pass<BLK>(nt), S = near_splits<BLK>(ntp), ti = lane % ntp, si = lane / ntp;
   const bool   lane_on = si < S;
-  const double cxt = ccx[c], cyt = ccy[c], czt = ccz[c];
-  const int    q0 = off[c], q1 = off[c + 1];
+  const double cxt = MIXED ? ccx[c] : 0.0, cyt = MIXED ? ccy[c] : 0.0, czt = MIXED ? ccz[c] : 0.0;
   for (int c0 = 0; c0 < nt; c0 += ntp) {
-    const int     i     = c0 + ti;
-    const bool    valid = lane_on && i < nt;
-    const int     jfirst = lane_on ? si : WG;  // lanes without a split skip the pair loops
-    const int64_t bi    = tb + (valid ? i : 0);
-    const double  xo[3] = {st[(F_X + 0) * cap + bi], st[(F_X + 1) * cap + bi], st[(F_X + 2) * cap + bi]};
-    const float   ro[3] = {(float)(xo[0] - cxt), (float)(xo[1] - cyt), (float)(xo[2] - czt)};
+    const int     i      = c0 + ti;
+    const int     jfirst = lane_on ? si : CH;  // lanes without a split skip the pair loops
+    const int64_t bi     = tb + (lane_on && i < nt ? i : 0);
+    const T       ro[3]  = {(T)(st[(F_X + 0) * cap + bi] - cxt), (T)(st[(F_X + 1) * cap + bi] - cyt),
+                            (T)(st[(F_X + 2) * cap + bi] - czt)};
     // own quantities: SIDE 0 ubar, Jbar, e; SIDE 1 alpha, sigma and its kernel constants
-    double ubd[3] = {0, 0, 0}, Jbd[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, ald[3] = {0, 0, 0}, sgd = 1.0;
+    T      ub[3] = {0, 0, 0}, Jb[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, e[3] = {0, 0, 0}, al[3] = {0, 0, 0};
+    double sgd = 1.0;
     if (SIDE == 0) {
-      for (int d = 0; d < 3; d++) ubd[d] = aux[(A_UB + d) * cap + bi];
-      for (int k = 0; k < 9; k++) Jbd[k] = aux[(A_JB + k) * cap + bi];
+      for (int d = 0; d < 3; d++) ub[d] = (T)aux[(A_UB + d) * cap + bi];
+      for (int k = 0; k < 9; k++) Jb[k] = (T)aux[(A_JB + k) * cap + bi];
+      e[0] = Jb[5] - Jb[7], e[1] = Jb[6] - Jb[2], e[2] = Jb[1] - Jb[3];
     } else {
-      for (int d = 0; d < 3; d++) ald[d] = st[(F_A + d) * cap + bi];
+      for (int d = 0; d < 3; d++) al[d] = (T)st[(F_A + d) * cap + bi];
       sgd = st[F_SIG * cap + bi];
     }
-    const double oq = 0.5 / (sgd * sgd), osq = sqrt(oq);
-    const float  o_q = (float)oq, o_c1 = (float)(oq * osq * INV_4PI), o_c2 = (float)(2.0 * oq * oq * osq * INV_4PI),
-                o_c3 = (float)(4.0 * oq * oq * oq * osq * INV_4PI);
-    float ubf[3], Jbf[9], ef[3], alf[3];
-    for (int d = 0; d < 3; d++) {
-      ubf[d] = (float)ubd[d];
-      alf[d] = (float)ald[d];
-    }
-    for (int k = 0; k < 9; k++) Jbf[k] = (float)Jbd[k];
-    ef[0] = Jbf[5] - Jbf[7];
-    ef[1] = Jbf[6] - Jbf[2];
-    ef[2] = Jbf[1] - Jbf[3];
-    double ax[3] = {0, 0, 0}, aa[3] = {0, 0, 0};
+    const double oqd = 0.5 / (sgd * sgd), oc1 = oqd * sqrt(oqd) * INV_4PI;
+    const T      o_q = (T)oqd, o_c1 = (T)oc1, o_c2 = (T)(2.0 * oqd * oc1), o_c3 = (T)(4.0 * oqd * oqd * oc1);
+    double       ax[3] = {0, 0, 0}, aa[3] = {0, 0, 0};
     for (int g0 = q0; g0 < q1; g0 += SEG) {
       const int nseg = min(SEG, q1 - g0);
       __syncthreads();
-      for (int k = lane; k < nseg; k += WG) {
+      for (int k = lane; k < nseg; k += BLK) {
         const int sl = src[g0 + k];
         lb[k]        = cbody[sl];
-        ln[k]        = cnbody[sl];
+        pref[k]      = cnbody[sl];
       }
       __syncthreads();
-      lds_prefix(pref, ln, nseg);
+      if (lane < 64) lds_prefix(pref, pref, nseg);
       __syncthreads();
       const int total = pref[nseg];
-      for (int j0 = 0; j0 < total; j0 += WG) {
-        const int cnt = min(WG, total - j0);
+      for (int j0 = 0; j0 < total; j0 += CH) {
+        const int cnt = min(CH, total - j0);
         if (lane < cnt) {
-          const int g  = j0 + lane;
-          int       lo = 0, hi = nseg - 1;  // last q with pref[q] <= g
-          while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (pref[mid] <= g) lo = mid;
-            else hi = mid - 1;
-          }
-          const int64_t bj = lb[lo] + (g - pref[lo]);
-          const double  x = st[(F_X + 0) * cap + bj], y = st[(F_X + 1) * cap + bj], z = st[(F_X + 2) * cap + bj];
+          const int64_t bj = list_body(pref, lb, nseg, j0 + lane);
+          T            *v  = sv + NV * lane;
+          v[0] = (T)(st[(F_X + 0) * cap + bj] - cxt);
+          v[1] = (T)(st[(F_X + 1) * cap + bj] - cyt);
+          v[2] = (T)(st[(F_X + 2) * cap + bj] - czt);
           if (SIDE == 0) {
-            const double sg = st[F_SIG * cap + bj];
-            const double a0 = st[(F_A + 0) * cap + bj], a1 = st[(F_A + 1) * cap + bj], a2 = st[(F_A + 2) * cap + bj];
-            if (MIXED) {
-              const double qq = 0.5 / (sg * sg), sq = sqrt(qq);
-              s32[NV * lane + 0] = make_float4((float)(x - cxt), (float)(y - cyt), (float)(z - czt), (float)qq);
-              s32[NV * lane + 1] = make_float4((float)a0, (float)a1, (float)a2, (float)(qq * sq * INV_4PI));
-              s32[NV * lane + 2] = make_float4((float)(2.0 * qq * qq * sq * INV_4PI),
-                                               (float)(4.0 * qq * qq * qq * sq * INV_4PI), 0.f, 0.f);
-            } else {
-              const double v[7] = {x, y, z, a0, a1, a2, sg};
-              for (int f = 0; f < 7; f++) s64[f * WG + lane] = v[f];
-            }
+            const double sg = st[F_SIG * cap + bj], qq = 0.5 / (sg * sg);
+            v[3] = (T)qq;
+            for (int d = 0; d < 3; d++) v[4 + d] = (T)st[(F_A + d) * cap + bj];
+            const double c1 = qq * sqrt(qq) * INV_4PI;
+            v[7] = (T)c1, v[8] = (T)(2.0 * qq * c1), v[9] = (T)(4.0 * qq * qq * c1);
           } else {
-            double ub[3], Jb[9];
-            for (int d = 0; d < 3; d++) ub[d] = aux[(A_UB + d) * cap + bj];
-            for (int k = 0; k < 9; k++) Jb[k] = aux[(A_JB + k) * cap + bj];
-            if (MIXED) {
-              s32[NV * lane + 0] = make_float4((float)(x - cxt), (float)(y - cyt), (float)(z - czt), (float)ub[0]);
-              s32[NV * lane + 1] = make_float4((float)ub[1], (float)ub[2], (float)(Jb[5] - Jb[7]), (float)(Jb[6] - Jb[2]));
-              s32[NV * lane + 2] = make_float4((float)(Jb[1] - Jb[3]), (float)Jb[0], (float)Jb[1], (float)Jb[2]);
-              s32[NV * lane + 3] = make_float4((float)Jb[3], (float)Jb[4], (float)Jb[5], (float)Jb[6]);
-              s32[NV * lane + 4] = make_float4((float)Jb[7], (float)Jb[8], 0.f, 0.f);
-            } else {
-              s64[0 * WG + lane] = x;
-              s64[1 * WG + lane] = y;
-              s64[2 * WG + lane] = z;
-              for (int d = 0; d < 3; d++) s64[(3 + d) * WG + lane] = ub[d];
-              for (int k = 0; k < 9; k++) s64[(6 + k) * WG + lane] = Jb[k];
-            }
+            double Jd[9];
+            for (int d = 0; d < 3; d++) v[3 + d] = (T)aux[(A_UB + d) * cap + bj];
+            for (int k = 0; k < 9; k++) Jd[k] = aux[(A_JB + k) * cap + bj];
+            v[6] = (T)(Jd[5] - Jd[7]), v[7] = (T)(Jd[6] - Jd[2]), v[8] = (T)(Jd[1] - Jd[3]);
+            for (int k = 0; k < 9; k++) v[9 + k] = (T)Jd[k];
           }
         }
         __syncthreads();
-        if (MIXED) {
-          // SIDE 0: X, F1, V, A;  SIDE 1: X, JV, UQ, WA
-          float p0[3] = {0, 0, 0}, p1[3] = {0, 0, 0}, p2[3] = {0, 0, 0}, p3[3] = {0, 0, 0};
-          for (int j = jfirst; j < cnt; j += S) {
-            const float4 A0 = s32[NV * j], A1 = s32[NV * j + 1], A2 = s32[NV * j + 2];
-            float        r[3];
-            if (SIDE == 0) {
-              r[0] = ro[0] - A0.x;
-              r[1] = ro[1] - A0.y;
-              r[2] = ro[2] - A0.z;
-            } else {
-              r[0] = A0.x - ro[0];
-              r[1] = A0.y - ro[1];
-              r[2] = A0.z - ro[2];
-            }
-            const float r2 = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
-            float       G, Gp, Gpp;
-            kernel_g<true>(r2 * (SIDE == 0 ? A0.w : o_q), G, Gp, Gpp);
+        // SIDE 0: X, F1, V, A;  SIDE 1: X, JV, UQ, WA
+        constexpr int FLUSH = 64;
+        for (int k0 = jfirst; k0 < cnt; k0 += FLUSH * S) {
+          T p0[3] = {0, 0, 0}, p1[3] = {0, 0, 0}, p2[3] = {0, 0, 0}, p3[3] = {0, 0, 0};
+          const int kend = min(cnt, k0 + FLUSH * S);
+          for (int j = k0; j < kend; j += S) {
+            const T *v    = sv + NV * j;
+            const T  sgn1 = SIDE == 0 ? (T)1 : (T)-1;
+            const T  r[3] = {sgn1 * (ro[0] - v[0]), sgn1 * (ro[1] - v[1]), sgn1 * (ro[2] - v[2])};
+            const T  r2   = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
+            const T  q    = SIDE == 0 ? v[3] : o_q;
+            T        G, Gp, Gpp;
+            pair_g(r2, q, G, Gp, Gpp);
             // coincident pairs are skipped (multipoleKernels.hpp:242): every term but the f1 ones
             // carries r, so zeroing f1 is enough
-            const float f1 = r2 == 0.0f ? 0.0f : G * (SIDE == 0 ? A1.w : o_c1);
-            const float f2 = Gp * (SIDE == 0 ? A2.x : o_c2);
-            const float f3 = Gpp * (SIDE == 0 ? A2.y : o_c3);
+            const T f1 = r2 == (T)0 ? (T)0 : G * (SIDE == 0 ? v[7] : o_c1);
+            const T f2 = Gp * (SIDE == 0 ? v[8] : o_c2), f3 = Gpp * (SIDE == 0 ? v[9] : o_c3);
             if (SIDE == 0) {
-              const float al[3] = {A1.x, A1.y, A1.z};
-              float       v[3], Jr[3], aJ[3];
-              cross(r, al, v);
-              for (int d = 0; d < 3; d++) Jr[d] = Jbf[3 * d] * r[0] + Jbf[3 * d + 1] * r[1] + Jbf[3 * d + 2] * r[2];
-              cross(al, Jr, aJ);
-              const float c1 = ubf[0] * v[0] + ubf[1] * v[1] + ubf[2] * v[2] + al[0] * ef[0] + al[1] * ef[1] +
-                               al[2] * ef[2];
-              const float c3 = Jr[0] * v[0] + Jr[1] * v[1] + Jr[2] * v[2];
-              const float k  = f2 * c1 + f3 * c3;
+              const T aj[3] = {v[4], v[5], v[6]};
+              T       w[3], Jr[3], aJ[3];
+              cross(r, aj, w);
+              for (int d = 0; d < 3; d++) Jr[d] = Jb[3 * d] * r[0] + Jb[3 * d + 1] * r[1] + Jb[3 * d + 2] * r[2];
+              cross(aj, Jr, aJ);
+              const T cc1 = ub[0] * w[0] + ub[1] * w[1] + ub[2] * w[2] + aj[0] * e[0] + aj[1] * e[1] + aj[2] * e[2];
+              const T cc3 = Jr[0] * w[0] + Jr[1] * w[1] + Jr[2] * w[2];
+              const T k   = f2 * cc1 + f3 * cc3;
               for (int d = 0; d < 3; d++) {
-                p0[d] = fmaf(k, r[d], p0[d]);
-                p1[d] = fmaf(f1, al[d], p1[d]);
-                p2[d] = fmaf(f2, v[d], p2[d]);
-                p3[d] = fmaf(f2, aJ[d], p3[d]);
+                p0[d] = fma_(k, r[d], p0[d]);
+                p1[d] = fma_(f1, aj[d], p1[d]);
+                p2[d] = fma_(f2, w[d], p2[d]);
+                p3[d] = fma_(f2, aJ[d], p3[d]);
               }
             } else {
-              const float4 A3 = s32[NV * j + 3], A4 = s32[NV * j + 4];
-              const float  ub[3] = {A0.w, A1.x, A1.y}, e[3] = {A1.z, A1.w, A2.x};
-              const float  Jb[9] = {A2.y, A2.z, A2.w, A3.x, A3.y, A3.z, A3.w, A4.x, A4.y};
-              float        uxr[3], Jr[3], Jrxr[3], v[3];
-              cross(ub, r, uxr);
-              for (int d = 0; d < 3; d++) Jr[d] = Jb[3 * d] * r[0] + Jb[3 * d + 1] * r[1] + Jb[3 * d + 2] * r[2];
+              const T *bu = v + 3, *be = v + 6, *bJ = v + 9;
+              T        uxr[3], Jr[3], Jrxr[3], w[3];
+              cross(bu, r, uxr);
+              for (int d = 0; d < 3; d++) Jr[d] = bJ[3 * d] * r[0] + bJ[3 * d + 1] * r[1] + bJ[3 * d + 2] * r[2];
               cross(Jr, r, Jrxr);
-              cross(r, alf, v);
-              float c1 = 0.f, c3 = 0.f;
+              cross(r, al, w);
+              T cc1 = 0, cc3 = 0;
               for (int d = 0; d < 3; d++) {
-                c1 = fmaf(alf[d], uxr[d] + e[d], c1);
-                c3 = fmaf(alf[d], Jrxr[d], c3);
+                cc1 = fma_(al[d], uxr[d] + be[d], cc1);
+                cc3 = fma_(al[d], Jrxr[d], cc3);
               }
-              const float k = f2 * c1 + f3 * c3;
+              const T k = f2 * cc1 + f3 * cc3;
               for (int d = 0; d < 3; d++) {
-                const float JTv = Jb[d] * v[0] + Jb[3 + d] * v[1] + Jb[6 + d] * v[2];
-                p0[d]           = fmaf(k, r[d], p0[d]);
-                p1[d]           = fmaf(f2, JTv, p1[d]);
-                p2[d]           = fmaf(f1, ub[d], fmaf(f2, Jr[d], p2[d]));
-                p3[d]           = fmaf(f1, uxr[d] + e[d], fmaf(f2, Jrxr[d], p3[d]));
+                const T JTw = bJ[d] * w[0] + bJ[3 + d] * w[1] + bJ[6 + d] * w[2];
+                p0[d]       = fma_(k, r[d], p0[d]);
+                p1[d]       = fma_(f2, JTw, p1[d]);
+                p2[d]       = fma_(f1, bu[d], fma_(f2, Jr[d], p2[d]));
+                p3[d]       = fma_(f1, uxr[d] + be[d], fma_(f2, Jrxr[d], p3[d]));
               }
             }
           }
           if (SIDE == 0) {
             // sum dS = -[X + F1 x ubar + Jbar^T V + A]
-            float fxu[3];
-            cross(p1, ubf, fxu);
+            T fxu[3];
+            cross(p1, ub, fxu);
             for (int d = 0; d < 3; d++) {
-              const float JTV = Jbf[d] * p2[0] + Jbf[3 + d] * p2[1] + Jbf[6 + d] * p2[2];
+              const T JTV = Jb[d] * p2[0] + Jb[3 + d] * p2[1] + Jb[6 + d] * p2[2];
               ax[d] -= (double)(p0[d] + fxu[d] + JTV + p3[d]);
             }
           } else {
             // xbar_j -= sum dS = X + JV + alpha x UQ;  alphabar_j -= sum W
-            float axq[3];
-            cross(alf, p2, axq);
+            T axq[3];
+            cross(al, p2, axq);
             for (int d = 0; d < 3; d++) {
               ax[d] += (double)(p0[d] + p1[d] + axq[d]);
               aa[d] -= (double)p3[d];
-            }
-          }
-        } else {
-          for (int j = jfirst; j < cnt; j += S) {
-            double r[3], Wv[3], dS[3];
-            if (SIDE == 0) {
-              const double alj[3] = {s64[3 * WG + j], s64[4 * WG + j], s64[5 * WG + j]};
-              for (int d = 0; d < 3; d++) r[d] = xo[d] - s64[d * WG + j];
-              if (pair_adj(r, alj, s64[6 * WG + j], ubd, Jbd, Wv, dS))
-                for (int d = 0; d < 3; d++) ax[d] += dS[d];
-            } else {
-              const double ubi[3] = {s64[3 * WG + j], s64[4 * WG + j], s64[5 * WG + j]};
-              double       Jbi[9];
-              for (int k = 0; k < 9; k++) Jbi[k] = s64[(6 + k) * WG + j];
-              for (int d = 0; d < 3; d++) r[d] = s64[d * WG + j] - xo[d];
-              if (pair_adj(r, ald, sgd, ubi, Jbi, Wv, dS))
-                for (int d = 0; d < 3; d++) {
-                  ax[d] -= dS[d];
-                  aa[d] -= Wv[d];
-                }
             }
           }
         }
         __syncthreads();
       }
     }
-    // combine the splits (lanes ti + q * ntp) in split order
+    // the splits (lanes t + q * ntp) in split order; lanes then take (field, body)
+    const int np = min(ntp, nt - c0);
+    __syncthreads();
     for (int d = 0; d < 3; d++) {
-      double vx = ax[d], va = aa[d];
-      for (int q = 1; q < S; q++) {
-        vx += __shfl(ax[d], ti + q * ntp, 64);
-        if (SIDE == 1) va += __shfl(aa[d], ti + q * ntp, 64);
-      }
-      ax[d] = vx;
-      aa[d] = va;
+      red[d * BLK + lane] = ax[d];
+      if (SIDE == 1) red[(3 + d) * BLK + lane] = aa[d];
     }
-    if (si == 0 && valid) {
-      for (int d = 0; d < 3; d++) aux[(A_XB + d) * cap + bi] += ax[d];
-      if (SIDE == 1)
-        for (int d = 0; d < 3; d++) aux[(A_AB + d) * cap + bi] += aa[d];
+    __syncthreads();
+    for (int o = lane; o < NK * np; o += BLK) {
+      const int k = o / np, tt = o - k * np;
+      double    v = red[k * BLK + tt];
+      for (int q = 1; q < S; q++) v += red[k * BLK + tt + q * ntp];
+      if (prow >= 0) part[(int64_t)prow * 12 + (int64_t)k * nt + c0 + tt] = v;
+      else aux[(A_XB + k) * cap + tb + c0 + tt] += v;  // A_AB = A_XB + 3
     }
+  }
+}
+static_assert(A_AB == A_XB + 3, "xbar and alphabar fields are consecutive");
+
+// Sums of the leaves cut into several units, units in order.
+template <int SIDE>
+__global__ __launch_bounds__(256) void k_p2p_adj_reduce(const int4 *__restrict__ multi,
+                                                        const int32_t *__restrict__ leaves,
+                                                        const int32_t *__restrict__ cbody,
+                                                        const int32_t *__restrict__ cnbody,
+                                                        const double *__restrict__ part, double *__restrict__ aux,
+                                                        int64_t cap)
+{
+  const int4    m = multi[blockIdx.x];
+  const int     c = leaves[m.x], tb = cbody[c], nt = cnbody[c];
+  const double *p = part + (int64_t)m.y * 12;
+  for (int o = threadIdx.x; o < (SIDE == 0 ? 3 : 6) * nt; o += 256) {
+    const int k = o / nt;
+    double    v = 0.0;
+#pragma unroll 4
+    for (int u = 0; u < m.z; u++) v += p[(int64_t)u * 12 * nt + o];
+    aux[(A_XB + k) * cap + tb + (o - k * nt)] += v;
   }
 }
 
@@ -576,20 +527,35 @@ void sigma_bar(hipStream_t s, const Tree &stree, const Tree &ttree, const Lists 
   UVLM_LAUNCH_CHECK();
 }
 
-void p2p_adj(hipStream_t s, const Tree &t, const Lists &l, int side, int mixed, const double *st, double *aux,
-             int64_t cap)
+void p2p_adj(hipStream_t s, Scratch &sc, const Tree &t, const Lists &l, int side, int mixed, const double *st,
+             double *aux, int64_t cap)
 {
   if (t.nleaf == 0) return;
+  if (l.n_units < t.nleaf) throw Error(UVLM_ERR_INTERNAL, "near-field adjoint without its units");
+  sc.p2p_part.reserve(sizeof(double) * 12 * l.n_rows);
+  double        *part = sc.p2p_part.as<double>();
   const int32_t *lv = t.leaves.as<int32_t>(), *cb = t.body.as<int32_t>(), *cn = t.nbody.as<int32_t>();
-  const int32_t *off = l.p2p_off.as<int32_t>(), *src = l.p2p_src.as<int32_t>();
-  const double  *cx = t.cx.as<double>(), *cy = t.cy.as<double>(), *cz = t.cz.as<double>();
-  const int      nb = (int)t.nleaf;
+  auto           launch = [&](auto kern, int blk) {
+    kern<<<(int)l.n_units, blk, 0, s>>>(l.units.as<int4>(), lv, cb, cn, t.cx.as<double>(), t.cy.as<double>(),
+                                        t.cz.as<double>(), l.p2p_src.as<int32_t>(), st, aux, cap, part);
+  };
+#define UVLM_ADJ(MX, SD)                          \
+  if (l.wide) launch(k_p2p_adj<MX, SD, 256>, 256); \
+  else launch(k_p2p_adj<MX, SD, 64>, 64)
   if (mixed) {
-    if (side == 0) k_p2p_adj<true, 0><<<nb, WG, 0, s>>>(lv, t.nleaf, cb, cn, cx, cy, cz, off, src, st, aux, cap);
-    else k_p2p_adj<true, 1><<<nb, WG, 0, s>>>(lv, t.nleaf, cb, cn, cx, cy, cz, off, src, st, aux, cap);
+    if (side == 0) UVLM_ADJ(true, 0);
+    else UVLM_ADJ(true, 1);
   } else {
-    if (side == 0) k_p2p_adj<false, 0><<<nb, WG, 0, s>>>(lv, t.nleaf, cb, cn, cx, cy, cz, off, src, st, aux, cap);
-    else k_p2p_adj<false, 1><<<nb, WG, 0, s>>>(lv, t.nleaf, cb, cn, cx, cy, cz, off, src, st, aux, cap);
+    if (side == 0) UVLM_ADJ(false, 0);
+    else UVLM_ADJ(false, 1);
+  }
+#undef UVLM_ADJ
+  if (l.n_multi > 0) {
+    auto reduce = [&](auto kern) {
+      kern<<<(int)l.n_multi, 256, 0, s>>>(l.multi.as<int4>(), lv, cb, cn, part, aux, cap);
+    };
+    if (side == 0) reduce(k_p2p_adj_reduce<0>);
+    else reduce(k_p2p_adj_reduce<1>);
   }
   UVLM_LAUNCH_CHECK();
 }

@@ -199,8 +199,8 @@ void vjp_setup(hipStream_t s, int64_t N, const double *st, double *aux, int64_t 
 void vjp_finish(hipStream_t s, int64_t N, const double *ast, double *aux, int64_t cap);
 // side 0: forward P2P list (xbar of targets); side 1: transposed list (xbar, alphabar of sources)
 // mixed: FP32 pair arithmetic (FP64 accumulation), else FP64
-void p2p_adj(hipStream_t s, const Tree &t, const Lists &l, int side, int mixed, const double *st, double *aux,
-             int64_t cap);
+void p2p_adj(hipStream_t s, Scratch &sc, const Tree &t, const Lists &l, int side, int mixed, const double *st,
+             double *aux, int64_t cap);
 // sbar_j (device order of the sources) = d/dsigma_j of the near-pair sum of ubar_i . u_i +
 // Jbar_i : J_i (Jbar when with_jbar), over tl = the P2P list CSR by source cell (entries = target
 // cells); tcot holds ubar (3 fields) then Jbar (9 fields) with stride ccap, tx the targets' X.
