@@ -148,10 +148,9 @@ void iota(hipStream_t s, int32_t *p, int64_t n)
   UVLM_LAUNCH_CHECK();
 }
 
-// Fields of the state that an evaluation overwrites for every body (J, velocity, dadt, drdt)
-// and the rest, as [first, last) field ranges.
-constexpr int OUT_FIELDS[3][2]   = {{F_J, F_J + 9}, {F_U, F_DADT + 3}, {F_DSIG, F_DSIG + 1}};
-constexpr int STATE_FIELDS[3][2] = {{F_X, F_A + 3}, {F_UOLD, F_SIG + 1}, {F_SIGOLD, N_FIELDS}};
+// Fields of the state that an evaluation overwrites for every body (J, velocity, dadt, drdt), as
+// [first, last) field ranges.
+constexpr int OUT_FIELDS[3][2] = {{F_J, F_J + 9}, {F_U, F_DADT + 3}, {F_DSIG, F_DSIG + 1}};
 
 // Applies a deferred build permutation to the output fields (from the previous order in st2).
 void resolve_outputs(uvlm_handle h)
@@ -174,13 +173,15 @@ void do_build(uvlm_handle h, bool defer_outputs = false)
   UVLM_HIP(hipEventRecord(h->ev[EV_B0], s));
   resolve_outputs(h);
   build_tree(s, h->sc, h->F(F_X), h->F(F_X + 1), h->F(F_X + 2), h->N, h->prm.ncrit, h->tree, h->perm.as<int32_t>());
-  if (defer_outputs)
-    for (const auto &r : STATE_FIELDS)
-      gather_fields(s, h->st.as<double>() + (int64_t)r[0] * h->cap, h->st2.as<double>() + (int64_t)r[0] * h->cap,
-                    h->cap, h->cap, r[1] - r[0], h->perm.as<int32_t>(), h->N);
-  else
-    gather_fields(s, h->st.as<double>(), h->st2.as<double>(), h->cap, h->cap, N_FIELDS, h->perm.as<int32_t>(), h->N);
-  gather_i32(s, h->orig.as<int32_t>(), h->orig2.as<int32_t>(), h->perm.as<int32_t>(), h->N);
+  uint8_t fields[N_FIELDS];
+  int     nf = 0;
+  for (int f = 0; f < N_FIELDS; f++) {
+    bool output = false;
+    for (const auto &r : OUT_FIELDS) output = output || (f >= r[0] && f < r[1]);
+    if (!(defer_outputs && output)) fields[nf++] = (uint8_t)f;
+  }
+  gather_state(s, h->st.as<double>(), h->st2.as<double>(), h->cap, fields, nf, h->orig.as<int32_t>(),
+               h->orig2.as<int32_t>(), h->perm.as<int32_t>(), h->N);
   swap_buf(h->st, h->st2);
   swap_buf(h->orig, h->orig2);
   h->out_deferred = defer_outputs;

@@ -96,7 +96,7 @@ struct Tree {
   std::vector<int64_t> lvl_off;   // host: level l cells are lvl_cells[lvl_off[l] .. lvl_off[l+1])
   DevBuf nchild, nbody, child, body, level, parent;  // int32 [C]
   DevBuf cx, cy, cz, R;                              // double [C]
-  DevBuf lvl_cells;                                  // int32 [C], grouped by level, ascending index
+  DevBuf lvl_cells;                                  // int32 [C], grouped by level
   DevBuf leaves;                                     // int32 [nleaf]
   DevBuf X0R0;                                       // double[4]
   int32_t *i(DevBuf &b) { return b.as<int32_t>(); }
@@ -116,13 +116,11 @@ struct Lists {
 // Scratch shared by tree builds and traversals.
 struct Scratch {
   DevBuf keys0, keys1, idx0, idx1, sort_tmp, scan_tmp;
-  DevBuf rec_begin, rec_end, rec_parent, rec_rank, rec_nchild, rec_scan, rec_pfx, rec_pre, rec_gidx, rec_childoff;
-  DevBuf rec_cx, rec_cy, rec_cz;
+  DevBuf rec_begin, rec_end, rec_parent, rec_level, rec_mask, rec_scan;  // cells in pre-order
   DevBuf partial, counters, perm;
   DevBuf front0, front1, out_p2p, out_m2l;
   DevBuf unit_work, unit_cnt, p2p_part;  // near-field units: work per leaf, totals, partial sums
   DevBuf m2l_seg, m2l_part;  // M2L list segments and their partial sums (few-target case)
-  int64_t rec_cap = 0;
 };
 
 // ---------------------------------------------------------------------------------
@@ -136,7 +134,9 @@ void traverse(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &st, double
 double max_value(hipStream_t s, Scratch &sc, const double *x, int64_t n);
 void gather_fields(hipStream_t s, const double *src, double *dst, int64_t src_cap, int64_t dst_cap, int nfields,
                    const int32_t *perm, int64_t N);
-void gather_i32(hipStream_t s, const int32_t *src, int32_t *dst, const int32_t *perm, int64_t N);
+// the listed fields (fields of cap doubles) and the original indices, in one launch
+void gather_state(hipStream_t s, const double *src, double *dst, int64_t cap, const uint8_t *fields, int nfields,
+                  const int32_t *osrc, int32_t *odst, const int32_t *perm, int64_t N);
 // Lists of (sources as targets): CSR by the cells of `in_sources`, entries = cells of `in_targets`.
 void transpose_lists(hipStream_t s, Scratch &sc, const Tree &in_targets, const Tree &in_sources, const Lists &in,
                      Lists &out);

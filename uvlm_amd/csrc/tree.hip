@@ -12,14 +12,16 @@
 //   3. radix sort of (key, index): stable, so equal keys keep the input order.  Only the top
 //      digits the tree can use are sorted: the previous build's depth plus one level; a cell
 //      that must split below them flags the build, which then sorts all 21 digits again
-//   4. cells level by level: a cell splits iff NBODY > ncrit (tree.hpp:43); its children are
-//      the non-empty digit ranges, found by binary search in the sorted keys
+//   4. cells straight from the sorted keys, all levels at once (k_cells_count): a cell splits iff
+//      NBODY > ncrit (tree.hpp:43), so the cells that begin at body i are those of the levels
+//      from the first digit in which i differs from i - 1 (if the cell they share splits) down to
+//      the first level that i does not share with body i + ncrit.  One scan over the bodies
+//      numbers them in pre-order, the order by (BodyOffset, level)
 //   5. cell numbering of the reference: root 0, child groups appended in DFS pre-order of
 //      their parents (tree.hpp:81-96), i.e. ChildOffset(p) = 1 + sum of NCHILD over internal
-//      cells before p in pre-order; pre-order = order by (BodyOffset, level)
+//      cells before p in pre-order
 //   6. inside a leaf the bodies keep their input order (the reference stops sorting at the
-//      leaf), so a second, stable sort of the input indices by their leaf's first body fixes the
-//      final permutation.
+//      leaf): each leaf's input indices are ranked among themselves
 // Traversal (semantics of src/traverse.hpp:32-85): breadth-first over (target, source)
 // pairs with the reference's split rule and MAC; outputs are appended with one atomic per
 // wavefront and category, then sorted by (target, source).
@@ -133,191 +135,208 @@ __global__ void k_keys(const double *__restrict__ x, const double *__restrict__ 
   idx[i]  = (uint32_t)i;
 }
 
-// The root record (begin 0, end N, no parent, rank 0, centre X0) and the error flag, on the
-// device: no host round trip.
-__global__ void k_root_record(int32_t n, const double *__restrict__ X0R0, int32_t *rb, int32_t *re, int32_t *rp,
-                              int32_t *rr, double *cx, double *cy, double *cz, int32_t *err)
-{
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  rb[0] = 0;
-  re[0] = n;
-  rp[0] = -1;
-  rr[0] = 0;
-  cx[0] = X0R0[0];
-  cy[0] = X0R0[1];
-  cz[0] = X0R0[2];
-  *err  = 0;
-}
-
-// The three numbers the host needs after counting a level: last exclusive-scan entry, last
-// child count, error flag.
-__global__ void k_level_summary(const int32_t *__restrict__ scan_last, const int32_t *__restrict__ nchild_last,
-                                const int32_t *__restrict__ err, int32_t *__restrict__ out)
-{
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  out[0] = *scan_last;
-  out[1] = *nchild_last;
-  out[2] = *err;
-}
-
 __device__ __forceinline__ int digit_at(uint64_t key, int l) { return (int)((key >> (3 * (KEY_LEVELS - 1 - l))) & 7); }
 
-__device__ __forceinline__ void octant_bounds(const uint64_t *__restrict__ keys, int b, int e, int l, int bnd[9])
+// Leading octant digits two keys share, at most dlim (the digits that are sorted).
+__device__ __forceinline__ int common_digits(uint64_t a, uint64_t b, int dlim)
 {
-  bnd[0] = b;
-  bnd[8] = e;
-  for (int o = 1; o < 8; o++) {
-    int lo = bnd[o - 1], hi = e;
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      if (digit_at(keys[mid], l) < o) lo = mid + 1;
-      else hi = mid;
+  const uint64_t x = a ^ b;  // bit 63 of a key is clear
+  return min(dlim, x ? (__clzll((long long)x) - 1) / 3 : KEY_LEVELS);
+}
+
+// Totals of a build (32-bit): cells per level, leaves per level, error bits (0: deeper than the key holds;
+// 1: a split needs a digit below the sorted ones).
+enum { TOT_LEVEL = 0, TOT_LEAVES = 24, TOT_ERR = 47, TOT_COUNT = 48 };
+__global__ void k_zero_u32(int64_t n, uint32_t *__restrict__ p)
+{
+  const int64_t i = blockIdx.x * (int64_t)BLK + threadIdx.x;
+  if (i < n) p[i] = 0;
+}
+
+// info[i] = number of cells that begin at body i | level of the first << 8.  With s the digits i
+// shares with i - 1 (-1 for the first body) and D those it shares with i + ncrit (-1 past the end):
+// the cell of level s around i exists and splits, or nothing begins here; then the cells of levels
+// s + 1 .. max(s, D) + 1 do, and all but the last split.  Found with a few loads near i, where a
+// pass per level over the cells took a launch, a scan and a host read-back each, and 8 binary
+// searches one after another per cell (8k ring: tree 0.42 ms).
+constexpr int COUNT_BLOCKS = 1024;
+__global__ __launch_bounds__(BLK) void k_cells_count(int64_t N, int64_t ncrit, int dlim,
+                                                     const uint64_t *__restrict__ keys, uint32_t *__restrict__ info,
+                                                     uint32_t *__restrict__ tot)
+{
+  __shared__ uint32_t loc[TOT_COUNT];
+  if (threadIdx.x < TOT_COUNT) loc[threadIdx.x] = 0;
+  __syncthreads();
+  for (int64_t i = blockIdx.x * (int64_t)BLK + threadIdx.x; i < N; i += (int64_t)gridDim.x * BLK) {
+    const uint64_t ki = keys[i];
+    const int      s  = i > 0 ? common_digits(keys[i - 1], ki, dlim) : -1;
+    const int      D  = i + ncrit < N ? common_digits(ki, keys[i + ncrit], dlim) : -1;
+    if (D >= dlim) atomicOr(&loc[TOT_ERR], dlim < KEY_LEVELS ? 2u : 1u);
+    uint32_t out = 0;
+    if (s < dlim) {
+      bool split = s < 0;  // the cell of level s around i - 1 and i holds more than ncrit bodies
+      if (!split && i >= ncrit) split = common_digits(keys[i - ncrit], ki, dlim) >= s;
+      if (!split) {
+        int64_t lo = i >= ncrit ? i - ncrit + 1 : 0, hi = i - 1;  // its first body is here
+        while (lo < hi) {
+          const int64_t mid = (lo + hi) >> 1;
+          if (common_digits(keys[mid], ki, dlim) >= s) hi = mid;
+          else lo = mid + 1;
+        }
+        split = lo + ncrit < N && common_digits(keys[lo + ncrit], ki, dlim) >= s;
+      }
+      if (split) {
+        const int last = max(s, min(D, dlim - 1)) + 1;
+        out            = (uint32_t)(last - s) | (uint32_t)(s + 1) << 8;
+        for (int l = s + 1; l <= last; l++) atomicAdd(&loc[TOT_LEVEL + l], 1u);
+        atomicAdd(&loc[TOT_LEAVES + last], 1u);
+      }
     }
-    bnd[o] = lo;
+    info[i] = out;
+  }
+  __syncthreads();
+  if (threadIdx.x < TOT_COUNT && loc[threadIdx.x]) {
+    if (threadIdx.x == TOT_ERR) atomicOr(&tot[TOT_ERR], loc[TOT_ERR]);
+    else atomicAdd(&tot[threadIdx.x], loc[threadIdx.x]);
   }
 }
 
-// err bit 0: deeper than the key holds; bit 1: a split needs a digit below the dlim sorted ones.
-__global__ void k_count_children(int64_t off, int64_t cnt, int l, int64_t ncrit, int dlim, const int32_t *__restrict__ rb,
-                                 const int32_t *__restrict__ re, const uint64_t *__restrict__ keys,
-                                 int32_t *__restrict__ nchild, int32_t *__restrict__ err)
-{
-  const int64_t t = blockIdx.x * (int64_t)BLK + threadIdx.x;
-  if (t >= cnt) return;
-  const int64_t k = off + t;
-  const int     b = rb[k], e = re[k];
-  int           nc = 0;
-  if (e - b > ncrit) {
-    if (l >= KEY_LEVELS) {
-      atomicOr(err, 1);
-    } else if (l >= dlim) {
-      atomicOr(err, 2);
-    } else {
-      int bnd[9];
-      octant_bounds(keys, b, e, l, bnd);
-      for (int o = 0; o < 8; o++) nc += bnd[o + 1] > bnd[o];
-    }
-  }
-  nchild[k] = nc;
-}
-
-__global__ void k_write_children(int64_t off, int64_t cnt, int l, const int32_t *__restrict__ rb,
-                                 const int32_t *__restrict__ re, const uint64_t *__restrict__ keys,
-                                 const int32_t *__restrict__ nchild, const int32_t *__restrict__ scan,
-                                 int64_t child_base, const double *__restrict__ X0R0, int32_t *__restrict__ ob,
-                                 int32_t *__restrict__ oe, int32_t *__restrict__ opar, int32_t *__restrict__ orank,
-                                 double *__restrict__ cx, double *__restrict__ cy, double *__restrict__ cz)
-{
-  const int64_t t = blockIdx.x * (int64_t)BLK + threadIdx.x;
-  if (t >= cnt) return;
-  const int64_t k = off + t;
-  if (nchild[k] == 0) return;
-  int bnd[9];
-  octant_bounds(keys, rb[k], re[k], l, bnd);
-  const double r = X0R0[3] / (double)(1LL << (l + 1));
-  const double px = cx[k], py = cy[k], pz = cz[k];
-  int          c  = 0;
-  for (int o = 0; o < 8; o++) {
-    if (bnd[o + 1] == bnd[o]) continue;
-    const int64_t q = child_base + scan[t] + c;
-    ob[q]           = bnd[o];
-    oe[q]           = bnd[o + 1];
-    opar[q]         = (int32_t)k;
-    orank[q]        = c;
-    double x = px, y = py, z = pz;
-    x += r * (double)(((o & 1) >> 0) * 2 - 1);
-    y += r * (double)(((o & 2) >> 1) * 2 - 1);
-    z += r * (double)(((o & 4) >> 2) * 2 - 1);
-    cx[q] = x;
-    cy[q] = y;
-    cz[q] = z;
-    c++;
-  }
-}
-
-__global__ void k_flags(int64_t n, const int32_t *__restrict__ nchild, int32_t *__restrict__ flag)
-{
-  const int64_t k = blockIdx.x * (int64_t)BLK + threadIdx.x;
-  if (k < n) flag[k] = nchild[k] > 0;
-}
-
-struct LevelOffsets {
-  int32_t off[KEY_LEVELS + 3];
-  int     nlev;
+struct CellCount {
+  __device__ __host__ int32_t operator()(uint32_t info) const { return (int32_t)(info & 255); }
+};
+struct Popcount {
+  __device__ __host__ int32_t operator()(uint32_t m) const { return __builtin_popcount(m); }
 };
 
-// Pre-order rank of each internal record = #internal cells with (begin, level) before it.
-__global__ void k_preorder_rank(int64_t C, LevelOffsets lo, const int32_t *__restrict__ rb,
-                                const int32_t *__restrict__ nchild, const int32_t *__restrict__ pfx,
-                                int32_t *__restrict__ pre_nchild, int32_t *__restrict__ rank_out)
+// The cells that begin at body i, in pre-order: first body, end, parent, level | octant << 8;
+// and each cell's octant in its parent's mask of children.
+__global__ void k_cells_write(int64_t N, int64_t ncrit, int dlim, const uint64_t *__restrict__ keys,
+                              const uint32_t *__restrict__ info, const int32_t *__restrict__ scan,
+                              int32_t *__restrict__ rb, int32_t *__restrict__ re, int32_t *__restrict__ rpar,
+                              int32_t *__restrict__ rlvl, uint32_t *__restrict__ mask)
 {
-  const int64_t k = blockIdx.x * (int64_t)BLK + threadIdx.x;
-  if (k >= C || nchild[k] == 0) return;
-  int lk = 0;
-  while (lk + 1 < lo.nlev && lo.off[lk + 1] <= k) lk++;
-  const int b    = rb[k];
-  int       rank = 0;
-  for (int l = 0; l < lo.nlev; l++) {
-    int lo_ = lo.off[l], hi = lo.off[l + 1];
-    const int base = lo_;
-    // count records of level l with begin < b (l >= lk) or begin <= b (l < lk)
-    while (lo_ < hi) {
-      const int mid = (lo_ + hi) >> 1;
-      const bool before = (l < lk) ? (rb[mid] <= b) : (rb[mid] < b);
-      if (before) lo_ = mid + 1;
+  const int64_t i = blockIdx.x * (int64_t)BLK + threadIdx.x;
+  if (i >= N) return;
+  const int n = info[i] & 255, l0 = info[i] >> 8;
+  if (n == 0) return;
+  const uint64_t ki = keys[i];
+  const int      p0 = scan[i], last = l0 + n - 1;
+  int            par = -1;
+  if (i > 0) {  // the parent of the first cell begins at the first body that shares l0 - 1 digits
+    int64_t lo = 0, hi = i - 1;
+    while (lo < hi) {
+      const int64_t mid = (lo + hi) >> 1;
+      if (common_digits(keys[mid], ki, dlim) >= l0 - 1) hi = mid;
+      else lo = mid + 1;
+    }
+    par = scan[lo] + (l0 - 1 - (int)(info[lo] >> 8));
+  }
+  int64_t end = i + 1;
+  for (int l = last; l >= l0; l--) {
+    int64_t lo = end, hi = l == last ? min(N, i + ncrit) : N;  // first body that shares fewer than l digits
+    while (lo < hi) {
+      const int64_t mid = (lo + hi) >> 1;
+      if (common_digits(keys[mid], ki, dlim) >= l) lo = mid + 1;
       else hi = mid;
     }
-    rank += pfx[lo_] - pfx[base];
+    end          = lo;
+    const int p  = p0 + (l - l0), pp = l == l0 ? par : p - 1, o = l > 0 ? digit_at(ki, l - 1) : 0;
+    rb[p]   = (int32_t)i;
+    re[p]   = (int32_t)end;
+    rpar[p] = pp;
+    rlvl[p] = l | o << 8;
+    if (pp >= 0) atomicOr(&mask[pp], 1u << o);
   }
-  pre_nchild[rank] = nchild[k];
-  rank_out[k]      = rank;
 }
 
-__global__ void k_assign(int64_t C, const int32_t *__restrict__ par, const int32_t *__restrict__ rnk,
-                         const int32_t *__restrict__ pre_rank, const int32_t *__restrict__ pre_scan,
-                         int32_t *__restrict__ gidx)
+// First slots of each level's cells and leaves.
+struct LevelOffsets {
+  int32_t off[KEY_LEVELS + 3], leaf[KEY_LEVELS + 3];
+};
+
+// Reference index of the cell with pre-order number p: 1 + children of the internal cells before
+// its parent in pre-order + its siblings of lower octants.
+__device__ __forceinline__ int cell_index(int p, const int32_t *rpar, const int32_t *rlvl, const int32_t *scan,
+                                          const uint32_t *mask)
 {
-  const int64_t k = blockIdx.x * (int64_t)BLK + threadIdx.x;
-  if (k >= C) return;
-  if (k == 0) {
-    gidx[0] = 0;
-    return;
-  }
-  const int p = par[k];
-  gidx[k]     = 1 + pre_scan[pre_rank[p]] + rnk[k];
+  const int q = rpar[p];
+  return q < 0 ? 0 : 1 + scan[q] + __popc(mask[q] & ((1u << (rlvl[p] >> 8)) - 1u));
 }
 
-__global__ void k_scatter_cells(int64_t C, LevelOffsets lo, const int32_t *__restrict__ rb,
-                                const int32_t *__restrict__ re, const int32_t *__restrict__ nchild,
-                                const int32_t *__restrict__ par, const int32_t *__restrict__ pre_rank,
-                                const int32_t *__restrict__ pre_scan, const int32_t *__restrict__ gidx,
-                                const int32_t *__restrict__ pfx, const double *__restrict__ rcx,
-                                const double *__restrict__ rcy, const double *__restrict__ rcz,
-                                const double *__restrict__ X0R0, int32_t *__restrict__ c_nchild,
-                                int32_t *__restrict__ c_nbody, int32_t *__restrict__ c_child,
-                                int32_t *__restrict__ c_body, int32_t *__restrict__ c_level,
-                                int32_t *__restrict__ c_parent, double *__restrict__ cx, double *__restrict__ cy,
-                                double *__restrict__ cz, double *__restrict__ cR, int32_t *__restrict__ lvl_cells,
-                                int32_t *__restrict__ leaves)
+// The tree's arrays, from the cells in pre-order.  The centre is the recurrence of tree.hpp:86-92
+// along the cell's digits.  Cells and leaves are listed by level, coarse first (the large leaves with the
+// long lists start early), within a level in no fixed order (each block takes its range with one
+// atomic per level): what walks them treats every cell by itself.
+__global__ __launch_bounds__(BLK) void k_cells_out(
+    int64_t C, LevelOffsets lo, const uint64_t *__restrict__ keys,
+    const int32_t *__restrict__ rb, const int32_t *__restrict__ re, const int32_t *__restrict__ rpar,
+    const int32_t *__restrict__ rlvl, const uint32_t *__restrict__ mask, const int32_t *__restrict__ scan,
+    const double *__restrict__ X0R0, uint32_t *__restrict__ cursor, int32_t *__restrict__ c_nchild,
+    int32_t *__restrict__ c_nbody, int32_t *__restrict__ c_child, int32_t *__restrict__ c_body,
+    int32_t *__restrict__ c_level, int32_t *__restrict__ c_parent, double *__restrict__ cx, double *__restrict__ cy,
+    double *__restrict__ cz, double *__restrict__ cR, int32_t *__restrict__ lvl_cells, int32_t *__restrict__ leaves)
 {
-  const int64_t k = blockIdx.x * (int64_t)BLK + threadIdx.x;
-  if (k >= C) return;
-  int lk = 0;
-  while (lk + 1 < lo.nlev && lo.off[lk + 1] <= k) lk++;
-  const int g  = gidx[k];
-  const int nc = nchild[k];
-  c_nchild[g]  = nc;
-  c_nbody[g]   = re[k] - rb[k];
-  c_child[g]   = nc ? 1 + pre_scan[pre_rank[k]] : 0;
-  c_body[g]    = rb[k];
-  c_level[g]   = lk;
-  c_parent[g]  = k == 0 ? -1 : gidx[par[k]];
-  cx[g]        = rcx[k];
-  cy[g]        = rcy[k];
-  cz[g]        = rcz[k];
-  cR[g]        = X0R0[3] / (double)(1LL << lk);
-  lvl_cells[k] = g;
-  if (nc == 0) leaves[k - pfx[k]] = g;
+  constexpr int       NL = KEY_LEVELS + 1;
+  __shared__ uint32_t cnt[2 * NL], base[2 * NL];  // cells, then leaves
+  if (threadIdx.x < 2 * NL) cnt[threadIdx.x] = 0;
+  __syncthreads();
+  const int64_t p = blockIdx.x * (int64_t)BLK + threadIdx.x;
+  int           g = 0, l = 0;
+  uint32_t      r = 0, rl = 0;
+  bool          leaf = false;
+  if (p < C) {
+    l             = rlvl[p] & 255;
+    g             = cell_index((int)p, rpar, rlvl, scan, mask);
+    r             = atomicAdd(&cnt[l], 1u);
+    const int nc  = __popc(mask[p]), b = rb[p];
+    c_nchild[g]   = nc;
+    c_nbody[g]    = re[p] - b;
+    c_child[g]    = nc ? 1 + scan[p] : 0;
+    c_body[g]     = b;
+    c_level[g]    = l;
+    c_parent[g]   = p == 0 ? -1 : cell_index(rpar[p], rpar, rlvl, scan, mask);
+    const uint64_t key = keys[b];
+    double         x = X0R0[0], y = X0R0[1], z = X0R0[2];
+    const double   R0 = X0R0[3];
+    for (int d = 0; d < l; d++) {
+      const int    o = digit_at(key, d);
+      const double h = R0 / (double)(1LL << (d + 1));
+      x += h * (double)(((o & 1) >> 0) * 2 - 1);
+      y += h * (double)(((o & 2) >> 1) * 2 - 1);
+      z += h * (double)(((o & 4) >> 2) * 2 - 1);
+    }
+    cx[g] = x;
+    cy[g] = y;
+    cz[g] = z;
+    cR[g] = R0 / (double)(1LL << l);
+    leaf  = nc == 0;
+    if (leaf) rl = atomicAdd(&cnt[NL + l], 1u);
+  }
+  __syncthreads();
+  if (threadIdx.x < 2 * NL && cnt[threadIdx.x]) base[threadIdx.x] = atomicAdd(&cursor[threadIdx.x], cnt[threadIdx.x]);
+  __syncthreads();
+  if (p < C) lvl_cells[lo.off[l] + base[l] + r] = g;
+  if (leaf) leaves[lo.leaf[l] + base[NL + l] + rl] = g;
+}
+
+// Final order of each leaf's bodies: their input indices ascending.  One wavefront per leaf ranks
+// them against each other in LDS (ncrit <= RANK_MAX), in place of a radix sort of all N by leaf.
+constexpr int64_t RANK_MAX = 1024;
+__global__ __launch_bounds__(64) void k_leaf_rank(const int32_t *__restrict__ leaves, const int32_t *__restrict__ c_body,
+                                                  const int32_t *__restrict__ c_nbody,
+                                                  const uint32_t *__restrict__ idx, uint32_t *__restrict__ perm)
+{
+  extern __shared__ uint32_t v[];
+  const int g = leaves[blockIdx.x], b = c_body[g], n = c_nbody[g], lane = threadIdx.x;
+  for (int j = lane; j < n; j += 64) v[j] = idx[b + j];
+  __syncthreads();
+  for (int j = lane; j < n; j += 64) {
+    const uint32_t m = v[j];
+    int            r = 0;
+#pragma unroll 4
+    for (int k = 0; k < n; k++) r += v[k] < m;
+    perm[b + r] = m;
+  }
 }
 
 // lb[input index] = first body of its leaf (one wavefront per leaf; lanes stride over its bodies)
@@ -354,12 +373,29 @@ __global__ void k_gather_fields(const double *__restrict__ src, double *__restri
   for (int f = f0; f < f1; f++) dst[f * dcap + i] = v[f - f0];
 }
 
-__global__ void k_gather_i32(const int32_t *__restrict__ src, int32_t *__restrict__ dst,
-                             const int32_t *__restrict__ perm, int64_t N)
+// The listed state fields and the bodies' original indices (the last grid row) in one launch.
+struct FieldList {
+  uint8_t f[N_FIELDS + 1];
+  int     n;
+};
+__global__ void k_gather_state(const double *__restrict__ src, double *__restrict__ dst, int64_t cap,
+                               const int32_t *__restrict__ perm, int64_t N, FieldList fl,
+                               const int32_t *__restrict__ osrc, int32_t *__restrict__ odst)
 {
   const int64_t i = blockIdx.x * (int64_t)BLK + threadIdx.x;
-  if (i < N) dst[i] = src[perm[i]];
+  if (i >= N) return;
+  const int64_t j = perm[i];
+  const int     k = blockIdx.y * GATHER_FIELDS;
+  if (k >= fl.n) {
+    odst[i] = osrc[j];
+    return;
+  }
+  const int64_t f0 = fl.f[k], f1 = fl.f[min(k + 1, fl.n - 1)];  // an odd last field twice
+  const double  a = src[f0 * cap + j], b = src[f1 * cap + j];
+  dst[f0 * cap + i] = a;
+  dst[f1 * cap + i] = b;
 }
+static_assert(GATHER_FIELDS == 2, "k_gather_state takes two fields a row");
 
 // ------------------------------- traversal -------------------------------------
 struct TreeView {
@@ -564,12 +600,12 @@ void sort_keys_u64(hipStream_t s, Scratch &sc, uint64_t *in, uint64_t *out, int6
   UVLM_HIP(rocprim::radix_sort_keys(sc.sort_tmp.p, bytes, in, out, (size_t)n, 0, end_bit, s));
 }
 
-void excl_scan_i32(hipStream_t s, Scratch &sc, const int32_t *in, int32_t *out, int64_t n)
+template <class In, class T> void excl_scan(hipStream_t s, Scratch &sc, In in, T *out, int64_t n)
 {
   size_t bytes = 0;
-  UVLM_HIP(rocprim::exclusive_scan(nullptr, bytes, in, out, 0, (size_t)n, rocprim::plus<int32_t>(), s));
+  UVLM_HIP(rocprim::exclusive_scan(nullptr, bytes, in, out, T(0), (size_t)n, rocprim::plus<T>(), s));
   sc.scan_tmp.reserve(bytes);
-  UVLM_HIP(rocprim::exclusive_scan(sc.scan_tmp.p, bytes, in, out, 0, (size_t)n, rocprim::plus<int32_t>(), s));
+  UVLM_HIP(rocprim::exclusive_scan(sc.scan_tmp.p, bytes, in, out, T(0), (size_t)n, rocprim::plus<T>(), s));
 }
 
 int bits_for(int64_t v)
@@ -599,126 +635,84 @@ void build_tree(hipStream_t s, Scratch &sc, const double *x, const double *y, co
   sc.keys1.reserve(8 * N);
   sc.idx0.reserve(4 * N);
   sc.idx1.reserve(4 * N);
-  k_keys<<<nblocks(N), BLK, 0, s>>>(x, y, z, N, tree.X0R0.as<double>(), sc.keys0.as<uint64_t>(),
-                                     sc.idx0.as<uint32_t>());
-  UVLM_LAUNCH_CHECK();
   const uint64_t *keys = sc.keys1.as<uint64_t>();
   const uint32_t *idx  = sc.idx1.as<uint32_t>();
-  std::vector<int64_t> off;
-  int                  dlim = std::min(KEY_LEVELS, std::max(1, tree.sort_digits));
+  uint32_t       *info = sc.idx0.as<uint32_t>();  // free once sorted
+  int32_t        *scan = sc.keys0.as<int32_t>();
+  sc.counters.reserve(4 * TOT_COUNT);
+  uint32_t *tot  = sc.counters.as<uint32_t>();
+  int       dlim = std::min(KEY_LEVELS, std::max(1, tree.sort_digits));
+  uint32_t  h[TOT_COUNT];
   for (;;) {
-    // stable sort of (key, index) on the top dlim digits
-    {
-      size_t    bytes = 0;
-      const int b0    = 3 * (KEY_LEVELS - dlim);
-      UVLM_HIP(rocprim::radix_sort_pairs(nullptr, bytes, sc.keys0.as<uint64_t>(), sc.keys1.as<uint64_t>(),
-                                         sc.idx0.as<uint32_t>(), sc.idx1.as<uint32_t>(), (size_t)N, b0,
-                                         3 * KEY_LEVELS, s));
-      sc.sort_tmp.reserve(bytes);
-      UVLM_HIP(rocprim::radix_sort_pairs(sc.sort_tmp.p, bytes, sc.keys0.as<uint64_t>(), sc.keys1.as<uint64_t>(),
-                                         sc.idx0.as<uint32_t>(), sc.idx1.as<uint32_t>(), (size_t)N, b0,
-                                         3 * KEY_LEVELS, s));
-    }
-    // 4. records level by level
-    auto ensure_rec = [&](int64_t want, int64_t used) {
-      if (want <= sc.rec_cap) return;
-      int64_t cap = std::max<int64_t>(want, 2 * sc.rec_cap);
-      cap         = std::max<int64_t>(cap, 1024);
-      for (DevBuf *b : {&sc.rec_begin, &sc.rec_end, &sc.rec_parent, &sc.rec_rank, &sc.rec_nchild})
-        b->reserve(4 * cap, used > 0, s);
-      for (DevBuf *b : {&sc.rec_cx, &sc.rec_cy, &sc.rec_cz}) b->reserve(8 * cap, used > 0, s);
-      for (DevBuf *b : {&sc.rec_scan, &sc.rec_pfx, &sc.rec_pre, &sc.rec_gidx, &sc.rec_childoff})
-        b->reserve(4 * (cap + 1), used > 0, s);
-      sc.rec_cap = cap;
-    };
-    ensure_rec(std::max<int64_t>(1024, 8 * (N / std::max<int64_t>(1, ncrit) + 1)), 0);
-    sc.counters.reserve(64);
-    int32_t *err = sc.counters.as<int32_t>(), *summary = err + 8;
-    k_root_record<<<1, 64, 0, s>>>((int32_t)N, tree.X0R0.as<double>(), sc.rec_begin.as<int32_t>(),
-                                   sc.rec_end.as<int32_t>(), sc.rec_parent.as<int32_t>(), sc.rec_rank.as<int32_t>(),
-                                   sc.rec_cx.as<double>(), sc.rec_cy.as<double>(), sc.rec_cz.as<double>(), err);
+    k_keys<<<nblocks(N), BLK, 0, s>>>(x, y, z, N, tree.X0R0.as<double>(), sc.keys0.as<uint64_t>(),
+                                       sc.idx0.as<uint32_t>());
+    k_zero_u32<<<1, BLK, 0, s>>>(TOT_COUNT, tot);
     UVLM_LAUNCH_CHECK();
-    off = {0, 1};
-    bool deeper = false;  // a cell must split below the sorted digits
-    for (int l = 0;; l++) {
-      const int64_t o = off[l], cnt = off[l + 1] - off[l];
-      k_count_children<<<nblocks(cnt), BLK, 0, s>>>(o, cnt, l, ncrit, dlim, sc.rec_begin.as<int32_t>(),
-                                                    sc.rec_end.as<int32_t>(), keys, sc.rec_nchild.as<int32_t>(), err);
-      UVLM_LAUNCH_CHECK();
-      excl_scan_i32(s, sc, sc.rec_nchild.as<int32_t>() + o, sc.rec_scan.as<int32_t>(), cnt);
-      k_level_summary<<<1, 64, 0, s>>>(sc.rec_scan.as<int32_t>() + cnt - 1, sc.rec_nchild.as<int32_t>() + o + cnt - 1,
-                                       err, summary);
-      UVLM_LAUNCH_CHECK();
-      int32_t sm3[3] = {0, 0, 0};
-      to_host(s, sm3, summary, 3);
-      if (sm3[2] & 1) throw Error(UVLM_ERR_DEPTH, "more than ncrit coincident bodies: octree deeper than 21 levels");
-      if (sm3[2] & 2) {
-        deeper = true;
-        break;
-      }
-      const int64_t total = (int64_t)sm3[0] + sm3[1];
-      if (total == 0) break;
-      ensure_rec(off[l + 1] + total + 1, off[l + 1]);
-      k_write_children<<<nblocks(cnt), BLK, 0, s>>>(
-          o, cnt, l, sc.rec_begin.as<int32_t>(), sc.rec_end.as<int32_t>(), keys, sc.rec_nchild.as<int32_t>(),
-          sc.rec_scan.as<int32_t>(), off[l + 1], tree.X0R0.as<double>(), sc.rec_begin.as<int32_t>(),
-          sc.rec_end.as<int32_t>(), sc.rec_parent.as<int32_t>(), sc.rec_rank.as<int32_t>(), sc.rec_cx.as<double>(),
-          sc.rec_cy.as<double>(), sc.rec_cz.as<double>());
-      UVLM_LAUNCH_CHECK();
-      off.push_back(off[l + 1] + total);
-    }
-    if (deeper) {  // sort all digits and build again
-      dlim = KEY_LEVELS;
-      continue;
-    }
-    break;
+    // stable sort of (key, index) on the top dlim digits
+    size_t    bytes = 0;
+    const int b0    = 3 * (KEY_LEVELS - dlim);
+    UVLM_HIP(rocprim::radix_sort_pairs(nullptr, bytes, sc.keys0.as<uint64_t>(), sc.keys1.as<uint64_t>(),
+                                       sc.idx0.as<uint32_t>(), sc.idx1.as<uint32_t>(), (size_t)N, b0, 3 * KEY_LEVELS,
+                                       s));
+    sc.sort_tmp.reserve(bytes);
+    UVLM_HIP(rocprim::radix_sort_pairs(sc.sort_tmp.p, bytes, sc.keys0.as<uint64_t>(), sc.keys1.as<uint64_t>(),
+                                       sc.idx0.as<uint32_t>(), sc.idx1.as<uint32_t>(), (size_t)N, b0, 3 * KEY_LEVELS,
+                                       s));
+    // 4. cells, numbered in pre-order
+    k_cells_count<<<std::min(COUNT_BLOCKS, nblocks(N)), BLK, 0, s>>>(N, ncrit, dlim, keys, info, tot);
+    UVLM_LAUNCH_CHECK();
+    excl_scan(s, sc, rocprim::make_transform_iterator(info, CellCount{}), scan, N);
+    to_host(s, h, tot, TOT_COUNT);
+    if (h[TOT_ERR] & 1) throw Error(UVLM_ERR_DEPTH, "more than ncrit coincident bodies: octree deeper than 21 levels");
+    if (!(h[TOT_ERR] & 2)) break;
+    dlim = KEY_LEVELS;  // a cell splits below the sorted digits: all of them, again from the keys
   }
-  tree.sort_digits = (int)off.size() - 1;  // digits 0 .. nlev-1: this tree's splits plus one spare level
-
+  LevelOffsets         lo{};
+  std::vector<int64_t> off{0};
+  int64_t              nleaf = 0;
+  for (int l = 0; l <= KEY_LEVELS && h[TOT_LEVEL + l]; l++) {
+    lo.off[l]  = (int32_t)off.back();
+    lo.leaf[l] = (int32_t)nleaf;
+    off.push_back(off.back() + h[TOT_LEVEL + l]);
+    nleaf += h[TOT_LEAVES + l];
+  }
   const int64_t C    = off.back();
   const int     nlev = (int)off.size() - 1;
-  if (nlev > KEY_LEVELS + 1) throw Error(UVLM_ERR_INTERNAL, "level count");
-  if (C >= (int64_t(1) << 31)) throw Error(UVLM_ERR_ARG, "too many cells");
+  tree.sort_digits   = nlev;  // digits 0 .. nlev-1: this tree's splits plus one spare level
+  tree.C             = C;
+  tree.nlevels       = nlev;
+  tree.nleaf         = nleaf;
+  tree.lvl_off       = off;
 
   // 5. numbering
-  int32_t *nchild = sc.rec_nchild.as<int32_t>();
-  k_flags<<<nblocks(C), BLK, 0, s>>>(C, nchild, sc.rec_scan.as<int32_t>());
-  // pfx has C+1 entries: exclusive scan of C+1 flags with a zero appended
-  UVLM_HIP(hipMemsetAsync(sc.rec_scan.as<int32_t>() + C, 0, 4, s));
-  excl_scan_i32(s, sc, sc.rec_scan.as<int32_t>(), sc.rec_pfx.as<int32_t>(), C + 1);
-  int32_t n_internal = 0;
-  to_host(s, &n_internal, sc.rec_pfx.as<int32_t>() + C);
-  LevelOffsets lo{};
-  lo.nlev = nlev;
-  for (int l = 0; l <= nlev; l++) lo.off[l] = (int32_t)off[l];
-  int32_t *pre_nchild = sc.rec_pre.as<int32_t>();
-  int32_t *pre_rank   = sc.rec_childoff.as<int32_t>();
-  k_preorder_rank<<<nblocks(C), BLK, 0, s>>>(C, lo, sc.rec_begin.as<int32_t>(), nchild, sc.rec_pfx.as<int32_t>(),
-                                             pre_nchild, pre_rank);
-  UVLM_LAUNCH_CHECK();
-  int32_t *pre_scan = sc.rec_scan.as<int32_t>();
-  if (n_internal > 0) excl_scan_i32(s, sc, pre_nchild, pre_scan, n_internal);
-  k_assign<<<nblocks(C), BLK, 0, s>>>(C, sc.rec_parent.as<int32_t>(), sc.rec_rank.as<int32_t>(), pre_rank, pre_scan,
-                                      sc.rec_gidx.as<int32_t>());
-  UVLM_LAUNCH_CHECK();
-  tree.C       = C;
-  tree.nlevels = nlev;
-  tree.nleaf   = C - n_internal;
-  tree.lvl_off = off;
+  for (DevBuf *b : {&sc.rec_begin, &sc.rec_end, &sc.rec_parent, &sc.rec_level, &sc.rec_scan}) b->reserve(4 * C);
+  sc.rec_mask.reserve(4 * (C + TOT_COUNT));
   for (DevBuf *b : {&tree.nchild, &tree.nbody, &tree.child, &tree.body, &tree.level, &tree.parent, &tree.lvl_cells})
     b->reserve(4 * C);
   for (DevBuf *b : {&tree.cx, &tree.cy, &tree.cz, &tree.R}) b->reserve(8 * C);
   tree.leaves.reserve(4 * tree.nleaf);
-  k_scatter_cells<<<nblocks(C), BLK, 0, s>>>(
-      C, lo, sc.rec_begin.as<int32_t>(), sc.rec_end.as<int32_t>(), nchild, sc.rec_parent.as<int32_t>(), pre_rank,
-      pre_scan, sc.rec_gidx.as<int32_t>(), sc.rec_pfx.as<int32_t>(), sc.rec_cx.as<double>(), sc.rec_cy.as<double>(),
-      sc.rec_cz.as<double>(), tree.X0R0.as<double>(), tree.nchild.as<int32_t>(), tree.nbody.as<int32_t>(),
-      tree.child.as<int32_t>(), tree.body.as<int32_t>(), tree.level.as<int32_t>(), tree.parent.as<int32_t>(),
-      tree.cx.as<double>(), tree.cy.as<double>(), tree.cz.as<double>(), tree.R.as<double>(),
-      tree.lvl_cells.as<int32_t>(), tree.leaves.as<int32_t>());
+  int32_t  *rb = sc.rec_begin.as<int32_t>(), *re = sc.rec_end.as<int32_t>(), *rpar = sc.rec_parent.as<int32_t>();
+  int32_t  *rlvl = sc.rec_level.as<int32_t>(), *cscan = sc.rec_scan.as<int32_t>();
+  uint32_t *mask = sc.rec_mask.as<uint32_t>(), *cursor = mask + C;
+  k_zero_u32<<<nblocks(C + TOT_COUNT), BLK, 0, s>>>(C + TOT_COUNT, mask);
+  k_cells_write<<<nblocks(N), BLK, 0, s>>>(N, ncrit, dlim, keys, info, scan, rb, re, rpar, rlvl, mask);
+  UVLM_LAUNCH_CHECK();
+  excl_scan(s, sc, rocprim::make_transform_iterator(mask, Popcount{}), cscan, C);
+  k_cells_out<<<nblocks(C), BLK, 0, s>>>(
+      C, lo, keys, rb, re, rpar, rlvl, mask, cscan, tree.X0R0.as<double>(), cursor, tree.nchild.as<int32_t>(),
+      tree.nbody.as<int32_t>(), tree.child.as<int32_t>(), tree.body.as<int32_t>(), tree.level.as<int32_t>(),
+      tree.parent.as<int32_t>(), tree.cx.as<double>(), tree.cy.as<double>(), tree.cz.as<double>(),
+      tree.R.as<double>(), tree.lvl_cells.as<int32_t>(), tree.leaves.as<int32_t>());
   UVLM_LAUNCH_CHECK();
 
-  // 6. final permutation: the input indices 0..N-1, stably sorted by their leaf's first body
+  // 6. final permutation
+  if (ncrit <= RANK_MAX) {
+    k_leaf_rank<<<(int)tree.nleaf, 64, 4 * ncrit, s>>>(tree.leaves.as<int32_t>(), tree.body.as<int32_t>(),
+                                                       tree.nbody.as<int32_t>(), idx, (uint32_t *)perm_out);
+    UVLM_LAUNCH_CHECK();
+    return;
+  }
+  // large leaves: the input indices 0..N-1, stably sorted by their leaf's first body
   uint32_t *lb = sc.keys0.as<uint32_t>(), *lb_sorted = sc.keys1.as<uint32_t>(), *iota = sc.idx0.as<uint32_t>();
   k_leaf_begin<<<nblocks(tree.nleaf * 64), BLK, 0, s>>>(tree.nleaf, tree.leaves.as<int32_t>(),
                                                         tree.body.as<int32_t>(), tree.nbody.as<int32_t>(), idx, lb);
@@ -743,9 +737,15 @@ void gather_fields(hipStream_t s, const double *src, double *dst, int64_t src_ca
   UVLM_LAUNCH_CHECK();
 }
 
-void gather_i32(hipStream_t s, const int32_t *src, int32_t *dst, const int32_t *perm, int64_t N)
+void gather_state(hipStream_t s, const double *src, double *dst, int64_t cap, const uint8_t *fields, int nfields,
+                  const int32_t *osrc, int32_t *odst, const int32_t *perm, int64_t N)
 {
-  k_gather_i32<<<nblocks(N), BLK, 0, s>>>(src, dst, perm, N);
+  if (N <= 0) return;
+  FieldList fl{};
+  fl.n = nfields;
+  for (int k = 0; k < nfields; k++) fl.f[k] = fields[k];
+  k_gather_state<<<dim3(nblocks(N), (nfields + GATHER_FIELDS - 1) / GATHER_FIELDS + 1), BLK, 0, s>>>(
+      src, dst, cap, perm, N, fl, osrc, odst);
   UVLM_LAUNCH_CHECK();
 }
 
