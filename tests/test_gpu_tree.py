@@ -59,3 +59,61 @@ def test_too_deep_is_refused():
     g.set_bodies(make_bodies(X, X, np.ones(500)))
     g.build()
     g.close()
+
+
+@pytest.mark.parametrize("n,m,ncrit", [(3000, 1, 1), (20000, 2, 1), (6000, 60, 4)])
+def test_long_rows(orc, n, m, ncrit):
+    """Few targets against many sources: rows past the sizes that are ranked by a wavefront (1,024
+    entries) and sorted in LDS (16,384), through the getList entry point, and their transposes
+    through the probe adjoint's lists (run only)."""
+    from uvlm_amd import _capi
+    import ctypes
+
+    X, Y = points(n, 5, 1.0, 0), points(max(m, 2), 6, 1.0, 0)[:m]
+    g, h = FMMCalculator(P=4, theta=1e-3, ncrit=ncrit), FMMCalculator(P=4, theta=1e-3, ncrit=ncrit)
+    trees = []
+    for c, Z in ((h, Y), (g, X)):
+        c.set_bodies(make_bodies(Z, Z, np.ones(len(Z))))
+        c.build()
+        trees.append(c.cells())
+    (ti, tr), (si, sr) = trees
+    print(f"[tree] long rows {len(ti)} x {len(si)} cells", flush=True)
+
+    def ip(a):
+        return a.ctypes.data_as(ctypes.POINTER(ctypes.c_int64))
+
+    def dp(a):
+        return a.ctypes.data_as(ctypes.POINTER(ctypes.c_double))
+
+    a, b = ctypes.c_int64(), ctypes.c_int64()
+    args = (0, 1e-3, len(ti), ip(ti), dp(tr), len(si), ip(si), dp(sr))
+    _capi.check(g.lib.uvlm_get_list(*args, 0, 0, ctypes.byref(a), ctypes.byref(b), None, None))
+    p2p, m2l = np.zeros((a.value, 2), dtype=np.int64), np.zeros((b.value, 2), dtype=np.int64)
+    _capi.check(g.lib.uvlm_get_list(*args, a.value, b.value, ctypes.byref(a), ctypes.byref(b), ip(p2p), ip(m2l)))
+    # the same walk on the host, with the device's test
+    want_p, want_m, front = [], [], [(0, 0)]
+    if ti[0, 0] == 0 and si[0, 0] == 0:
+        want_p, front = [(0, 0)], []
+    while front:
+        nxt = []
+        for t, s in front:
+            if si[s, 0] == 0 or (tr[t, 3] >= sr[s, 3] and ti[t, 0] != 0):
+                kids = [(ti[t, 2] + c, s) for c in range(ti[t, 0])]
+            else:
+                kids = [(t, si[s, 2] + c) for c in range(si[s, 0])]
+            for x, y in kids:
+                d = tr[x, :3] - sr[y, :3]
+                if (d[0] * d[0] + d[1] * d[1] + d[2] * d[2]) * 1e-3 * 1e-3 < (tr[x, 3] + sr[y, 3]) ** 2:
+                    (want_p if ti[x, 0] == 0 and si[y, 0] == 0 else nxt).append((x, y))
+                else:
+                    want_m.append((x, y))
+        front = nxt
+    assert np.array_equal(p2p, np.array(sorted(want_p)).reshape(-1, 2))
+    assert np.array_equal(m2l, np.array(sorted(want_m)).reshape(-1, 2))
+    assert np.bincount(p2p[:, 0]).max() > (1024 if n < 20000 else 16384)
+    W_ = np.ones((len(Y), 3))
+    ga, gx = g.probe_adjoint(Y + 0.01, W_)
+    ga2, gx2 = g.probe_adjoint(Y + 0.01, W_)
+    assert np.array_equal(ga, ga2) and np.array_equal(gx, gx2) and np.isfinite(ga).all()
+    g.close()
+    h.close()

@@ -187,9 +187,9 @@ void do_build(uvlm_handle h, bool defer_outputs = false)
   h->out_deferred = defer_outputs;
   UVLM_HIP(hipEventRecord(h->ev[EV_TREE], s));
   h->gap = h->near_c > 0.0 ? h->near_c * max_value(s, h->sc, h->F(F_SIG), h->N) : 0.0;
-  traverse(s, h->sc, h->tree, h->tree, h->prm.theta, h->lists, h->gap);
+  traverse(s, h->sc, h->tree, h->tree, h->prm.theta, h->lists, h->gap, h->prm.ncrit);
   UVLM_HIP(hipEventRecord(h->ev[EV_LISTS], s));
-  near_units(s, h->sc, h->tree, h->tree, h->prm.ncrit, h->lists);  // ends with a synchronisation
+  UVLM_HIP(hipStreamSynchronize(s));
   h->tm.tree_ms        = ev_ms(h, EV_B0, EV_TREE);
   h->tm.lists_ms       = ev_ms(h, EV_TREE, EV_LISTS);
   h->tm.n_bodies       = h->N;
@@ -293,8 +293,7 @@ void copy_out_records(const std::vector<double> &rec, int64_t m, void *dst, int6
 void probe_vorticity(uvlm_handle h, int64_t m)
 {
   Region region("Calculation of Vorticity");  // fmmCalculator.hpp:735
-  traverse(h->s, h->sc, h->stree, h->tree, h->prm.theta, h->slists, h->gap);
-  near_units(h->s, h->sc, h->stree, h->tree, h->prm.ncrit, h->slists);
+  traverse(h->s, h->sc, h->stree, h->tree, h->prm.theta, h->slists, h->gap, h->prm.ncrit);
   zero_fields(h->s, h->sst.as<double>(), h->scap, m, F_UOLD, 3);
   gauss_near(h->s, h->sc, h->stree, h->tree, h->slists, h->sst.as<double>(), h->scap, h->st.as<double>(), h->cap,
              h->sst.as<double>(), h->scap, 1, F_UOLD, 0.0);
@@ -326,8 +325,7 @@ void sensor_pass(uvlm_handle h, int64_t m, bool with_j = false)
              h->sperm.as<int32_t>());
   gather_fields(s, h->sst.as<double>(), h->sst2.as<double>(), sc, sc, N_FIELDS, h->sperm.as<int32_t>(), m);
   swap_buf(h->sst, h->sst2);
-  traverse(s, h->sc, h->stree, h->tree, h->prm.theta, h->slists, h->gap);
-  near_units(s, h->sc, h->stree, h->tree, h->prm.ncrit, h->slists);
+  traverse(s, h->sc, h->stree, h->tree, h->prm.theta, h->slists, h->gap, h->prm.ncrit);
   const int P = h->prm.P;
   h->Ls.reserve(sizeof(double2) * h->NT * h->stree.C);
   double2 *Ls = h->Ls.as<double2>();
@@ -423,9 +421,8 @@ void probe_adjoint_core(uvlm_handle h, int64_t m)
   gather_fields(s, h->sst.as<double>(), h->sst2.as<double>(), sc, sc, N_FIELDS, h->sperm.as<int32_t>(), m);
   swap_buf(h->sst, h->sst2);
   // the forward probe lists, transposed: targets = particle cells, sources = probe cells
-  traverse(s, h->sc, h->stree, h->tree, h->prm.theta, h->slists, h->gap);
-  transpose_lists(s, h->sc, h->stree, h->tree, h->slists, h->alists);
-  near_units(s, h->sc, h->tree, h->stree, h->prm.ncrit, h->alists);
+  traverse(s, h->sc, h->stree, h->tree, h->prm.theta, h->slists, h->gap, h->prm.ncrit);
+  transpose_lists(s, h->sc, h->stree, h->tree, h->slists, h->alists, h->prm.ncrit);
   // probe multipoles (root included: a probe cell is a source here)
   h->Ms.reserve(sizeof(double2) * NT * h->stree.C);
   double2 *Ms = h->Ms.as<double2>();
@@ -504,8 +501,7 @@ void vjp_core(uvlm_handle h, double *sbar = nullptr)
   p2p_adj(s, h->sc, t, h->lists, 0, h->prm.precision == UVLM_MIXED, st, aux, cap);
   // source side: adjoint sources up the tree, across the transposed M2L list, down to the bodies
   if (!h->tlists_ok) {
-    transpose_lists(s, h->sc, t, t, h->lists, h->tlists);
-    near_units(s, h->sc, t, t, h->prm.ncrit, h->tlists);
+    transpose_lists(s, h->sc, t, t, h->lists, h->tlists, h->prm.ncrit);
     h->tlists_ok = true;
   }
   double2 *M = h->M.as<double2>(), *L = h->L.as<double2>();
@@ -1055,7 +1051,7 @@ int uvlm_get_list(int device, double theta, int64_t ct, const int64_t *t_ints, c
     };
     upload(tt, ct, t_ints, t_reals);
     upload(st, cs, s_ints, s_reals);
-    traverse(s, sc, tt, st, theta, lists);
+    traverse(s, sc, tt, st, theta, lists, 0.0, -1);
     *n_p2p = lists.np2p;
     *n_m2l = lists.nm2l;
     auto expand = [&](DevBuf &off, DevBuf &src, int64_t n, int64_t cap, int64_t *out) {
@@ -1296,8 +1292,7 @@ int uvlm_rbf_aos(uvlm_handle h, void *points, int64_t m, int64_t stride, int64_t
     if (k == 0) return;
     // tree over the kept points and its self lists (createSensorTree(sensorOnly), 164-201)
     upload_probes(h, keep.data(), k, 296);
-    traverse(s, h->sc, h->stree, h->stree, h->prm.theta, h->slists, h->gap);
-    near_units(s, h->sc, h->stree, h->stree, h->prm.ncrit, h->slists);
+    traverse(s, h->sc, h->stree, h->stree, h->prm.theta, h->slists, h->gap, h->prm.ncrit);
     double       *st = h->sst.as<double>();
     const int64_t sc = h->scap;
     h->sc.partial.reserve(sizeof(double) * 3 * 512);

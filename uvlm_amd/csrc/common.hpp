@@ -109,17 +109,20 @@ struct Lists {
   // near-field units of the P2P list (near_units): runs of entries of one target leaf each, rows of
   // partial sums and leaves cut into several units
   int64_t n_units = 0, n_rows = 0, n_multi = 0;
-  bool    wide = false;  // 256 lanes per unit's workgroup, else 64
+  bool    wide = false;       // 256 lanes per unit's workgroup, else 64
+  bool    long_rows = false;  // a row was too long for LDS: the next build sorts at once
   DevBuf  units, multi;  // int4
 };
 
-// Scratch shared by tree builds and traversals.
+// Scratch shared by tree builds and traversals.  `counters` holds N_COUNTERS 64-bit totals: the build's
+// or the traversal's first, the near-field units' from UNIT_COUNTERS on.
+constexpr int N_COUNTERS = 32, UNIT_COUNTERS = 16;
 struct Scratch {
   DevBuf keys0, keys1, idx0, idx1, sort_tmp, scan_tmp;
   DevBuf rec_begin, rec_end, rec_parent, rec_level, rec_mask, rec_scan;  // cells in pre-order
   DevBuf partial, counters, perm;
-  DevBuf front0, front1, out_p2p, out_m2l;
-  DevBuf unit_work, unit_cnt, p2p_part;  // near-field units: work per leaf, totals, partial sums
+  DevBuf front0, front1, out_p2p, out_m2l, row_cnt, row_off, row_place, row_long;
+  DevBuf unit_work, p2p_part;  // near-field units: work per leaf, totals, partial sums
   DevBuf m2l_seg, m2l_part;  // M2L list segments and their partial sums (few-target case)
 };
 
@@ -129,8 +132,10 @@ struct Scratch {
 void build_tree(hipStream_t s, Scratch &sc, const double *x, const double *y, const double *z, int64_t N, int64_t ncrit,
                 Tree &tree, int32_t *perm_out);
 // gap > 0: pairs whose bodies can come closer than gap are near too (the near-field option)
-void traverse(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &st, double theta, Lists &lists,
-              double gap = 0.0);
+// max_leaf >= 0: an upper bound of the target leaves' body counts (ncrit for a built tree); the lists'
+// near-field units are made too
+void traverse(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &st, double theta, Lists &lists, double gap,
+              int64_t max_leaf);
 double max_value(hipStream_t s, Scratch &sc, const double *x, int64_t n);
 void gather_fields(hipStream_t s, const double *src, double *dst, int64_t src_cap, int64_t dst_cap, int nfields,
                    const int32_t *perm, int64_t N);
@@ -139,7 +144,7 @@ void gather_state(hipStream_t s, const double *src, double *dst, int64_t cap, co
                   const int32_t *osrc, int32_t *odst, const int32_t *perm, int64_t N);
 // Lists of (sources as targets): CSR by the cells of `in_sources`, entries = cells of `in_targets`.
 void transpose_lists(hipStream_t s, Scratch &sc, const Tree &in_targets, const Tree &in_sources, const Lists &in,
-                     Lists &out);
+                     Lists &out, int64_t max_leaf);
 
 // far.hip
 struct M2LSchedule {
@@ -182,8 +187,10 @@ void l2p_stretch(hipStream_t s, int P, const Tree &t, const double2 *L, double *
                  int formulation, int sensor_mode);
 
 // near.hip
-// max_leaf: an upper bound of the target leaves' body counts (ncrit for a built tree)
-void near_units(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &st, int64_t max_leaf, Lists &l);
+// np2p: the list's size, on the device
+void near_units_enqueue(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &st, int64_t max_leaf,
+                        const unsigned long long *np2p, Lists &l);
+void near_units_set(const unsigned long long *counters, Lists &l);
 void p2p(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &stree, const Lists &l, const double *tgt, int64_t tcap,
          const double *src, int64_t scap, double *out, int64_t ocap, int precision, int sensor_mode);
 

@@ -375,7 +375,20 @@ void direct(hipStream_t s, int64_t m, const double *xt, const double *at, const 
 // 4096, 9.9 with 8192, 9.6 with 16384.
 constexpr int                LANE_STEPS_MIN = 64;
 constexpr unsigned long long UNITS_AIM      = 16384;
-enum { NU_INTER = 0, NU_WORK, NU_UNITS, NU_ROWS, NU_MULTI, NU_COUNT };
+enum { NU_INTER = 0, NU_WORK, NU_UNITS, NU_ROWS, NU_MULTI, NU_WIDE, NU_COUNT };
+static_assert(UNIT_COUNTERS + NU_COUNT <= N_COUNTERS, "near-field unit totals");
+
+// Lanes per near-field workgroup.  With 64 lanes a leaf of 33..64 targets leaves up to half of them
+// idle (one split), with 256 a twentieth, and four waves share a staged chunk: 1M cube (leaves of
+// about 32 bodies, mixed) P2P 5.58 -> 4.03 ms, 60k cube with c = 6 1.39 -> 1.18, 8k ring (FP64) 0.110
+// -> 0.075 ms.  64 lanes stay for the lists of a few entries that an adjoint of few probes leaves most
+// leaves with (1M blobs, 4096 probes, 1.6 entries a leaf: 2.96 against 3.08 ms for the whole pass),
+// where 256 lanes have nothing to share.
+constexpr int64_t WIDE_ENTRIES = 8;  // list entries per target leaf from which 256 lanes are used
+__device__ __forceinline__ bool units_wide(int64_t nleaf, int64_t max_leaf, unsigned long long np2p)
+{
+  return max_leaf > 64 || (int64_t)np2p >= WIDE_ENTRIES * nleaf;
+}
 
 __global__ void k_units_clear(unsigned long long *__restrict__ cnt)
 {
@@ -386,14 +399,16 @@ __global__ void k_units_clear(unsigned long long *__restrict__ cnt)
 // wavefront per leaf at a time, lanes over its list; at most UNITS_WORK_BLOCKS blocks keep the
 // same-address atomics few.
 constexpr int UNITS_WORK_BLOCKS = 512;
-template <int BLK>
 __global__ __launch_bounds__(256) void k_units_work(const int32_t *__restrict__ leaves, int64_t nleaf,
+                                                    int64_t max_leaf, const unsigned long long *__restrict__ np2p,
                                                     const int32_t *__restrict__ tnbody,
                                                     const int32_t *__restrict__ off, const int32_t *__restrict__ src,
                                                     const int32_t *__restrict__ snbody, uint32_t *__restrict__ work,
                                                     unsigned long long *__restrict__ cnt)
 {
   __shared__ unsigned long long sum[2][4];
+  const bool                    wide = units_wide(nleaf, max_leaf, *np2p);
+  if (blockIdx.x == 0 && threadIdx.x == 0) cnt[NU_WIDE] = wide;
   const int          lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   unsigned long long inter = 0, all = 0;
   for (int64_t w = blockIdx.x * 4ll + wv; w < nleaf; w += gridDim.x * 4ll) {
@@ -401,7 +416,8 @@ __global__ __launch_bounds__(256) void k_units_work(const int32_t *__restrict__ 
     unsigned  ns = 0;
     for (int q = off[t] + lane; q < q1; q += 64) ns += (unsigned)snbody[src[q]];
     for (int o = 32; o > 0; o >>= 1) ns += __shfl_xor(ns, o, 64);
-    const int ntp = near_targets_per_pass<BLK>(nt), S = near_splits<BLK>(ntp);
+    const int ntp = wide ? near_targets_per_pass<256>(nt) : near_targets_per_pass<64>(nt);
+    const int S   = wide ? near_splits<256>(ntp) : near_splits<64>(ntp);
     const unsigned long long steps = ((unsigned long long)ns * ((nt + ntp - 1) / ntp) + S - 1) / S;
     const uint32_t           wk    = (uint32_t)min(steps, 0xffffffffull);
     if (lane == 0) work[w] = wk;
@@ -430,7 +446,7 @@ __global__ __launch_bounds__(256) void k_units_fill(const int32_t *__restrict__ 
   const int64_t            w    = blockIdx.x * 256ll + threadIdx.x;
   const int                lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const unsigned long long lim = max((unsigned long long)LANE_STEPS_MIN, cnt[NU_WORK] / UNITS_AIM);
-  int                      nu = 0, q0 = 0, len = 0, nt = 0;
+  int                      nu = 0, q0 = 0, len = 0, nt = 0;  // no units past the last leaf
   if (w < nleaf) {
     const int t = leaves[w];
     nt = tnbody[t], q0 = off[t], len = off[t + 1] - q0;
@@ -459,12 +475,25 @@ __global__ __launch_bounds__(256) void k_units_fill(const int32_t *__restrict__ 
     ex[c] += base[c];
     for (int k = 0; k < wv; k++) ex[c] += tot[k][c];
   }
-  if (w >= nleaf) return;
-  for (int j = 0; j < nu; j++) {
-    const int a = q0 + (int)((int64_t)len * j / nu), b = q0 + (int)((int64_t)len * (j + 1) / nu);
-    units[ex[0] + j] = make_int4((int)w, a, b, nu > 1 ? (int)(ex[1] + (unsigned long long)j * nt) : -1);
+  if (nu > 1 && w < nleaf) multi[ex[2]] = make_int4((int)w, (int)ex[1], nu, 0);
+  // the block's units, written by all its lanes (a probe tree's few leaves have hundreds each)
+  __shared__ int first[257], row[256], q0s[256], lens[256], nts[256];
+  first[threadIdx.x] = (int)(ex[0] - base[0]);
+  row[threadIdx.x] = (int)ex[1], q0s[threadIdx.x] = q0, lens[threadIdx.x] = len, nts[threadIdx.x] = nt;
+  if (threadIdx.x == 255) first[256] = first[255] + nu;
+  __syncthreads();
+  for (int u = threadIdx.x; u < first[256]; u += 256) {
+    int lo = 0, hi = 255;  // the last leaf with first <= u (leaves past the end have no units)
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (first[mid] <= u) lo = mid;
+      else hi = mid - 1;
+    }
+    const int     n = first[lo + 1] - first[lo], j = u - first[lo];
+    const int64_t ln = lens[lo];
+    units[base[0] + u] = make_int4((int)(blockIdx.x * 256 + lo), q0s[lo] + (int)(ln * j / n),
+                                   q0s[lo] + (int)(ln * (j + 1) / n), n > 1 ? row[lo] + j * nts[lo] : -1);
   }
-  if (nu > 1) multi[ex[2]] = make_int4((int)w, (int)ex[1], nu, 0);
 }
 
 // Sums of the leaves cut into several units, units in order, stored as k_p2p stores a single one.
@@ -629,43 +658,36 @@ __global__ __launch_bounds__(256) void k_gauss_reduce(const int4 *__restrict__ m
   }
 }
 
-// Lanes per near-field workgroup.  With 64 lanes a leaf of 33..64 targets leaves up to half of them
-// idle (one split), with 256 a twentieth, and four waves share a staged chunk: 1M cube (leaves of
-// about 32 bodies, mixed) P2P 5.58 -> 4.03 ms, 60k cube with c = 6 1.39 -> 1.18, 8k ring (FP64) 0.110
-// -> 0.075 ms.  64 lanes stay for the lists of a few entries that an adjoint of few probes leaves most
-// leaves with (1M blobs, 4096 probes, 1.6 entries a leaf: 2.96 against 3.08 ms for the whole pass),
-// where 256 lanes have nothing to share.
-constexpr int64_t WIDE_ENTRIES = 8;  // list entries per target leaf from which 256 lanes are used
-
-// Units of the P2P list `l` of target tree tt against source tree st (see k_units_work), and the
-// number of near-field interactions.  One read-back of the totals.
-void near_units(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &st, int64_t max_leaf, Lists &l)
+// Units of the P2P list `l` (np2p entries, on the device) of target tree tt against source tree st
+// (see k_units_work), and the number of near-field interactions.
+void near_units_enqueue(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &st, int64_t max_leaf,
+                        const unsigned long long *np2p, Lists &l)
 {
-  l.n_units = l.n_rows = l.n_multi = l.n_interactions = 0;
   if (tt.nleaf == 0) return;
   sc.unit_work.reserve(4 * tt.nleaf);
-  sc.unit_cnt.reserve(8 * NU_COUNT);
-  unsigned long long *cnt = sc.unit_cnt.as<unsigned long long>();
+  unsigned long long *cnt = sc.counters.as<unsigned long long>() + UNIT_COUNTERS;
   // at most UNITS_AIM units beyond one per leaf: sum ceil(work / limit) <= nleaf + work / limit
   l.units.reserve(sizeof(int4) * (tt.nleaf + UNITS_AIM));
   l.multi.reserve(sizeof(int4) * std::min<int64_t>(tt.nleaf, UNITS_AIM));
-  const int32_t *lv = tt.leaves.as<int32_t>(), *tn = tt.nbody.as<int32_t>(), *sn = st.nbody.as<int32_t>();
-  const int32_t *off = l.p2p_off.as<int32_t>(), *src = l.p2p_src.as<int32_t>();
-  const int      gw = (int)std::min<int64_t>(UNITS_WORK_BLOCKS, (tt.nleaf + 3) / 4);
-  l.wide = max_leaf > 64 || l.np2p >= WIDE_ENTRIES * tt.nleaf;
+  const int32_t *lv = tt.leaves.as<int32_t>(), *tn = tt.nbody.as<int32_t>();
+  const int32_t *off = l.p2p_off.as<int32_t>();
   k_units_clear<<<1, 64, 0, s>>>(cnt);
-  if (l.wide) k_units_work<256><<<gw, 256, 0, s>>>(lv, tt.nleaf, tn, off, src, sn, sc.unit_work.as<uint32_t>(), cnt);
-  else k_units_work<64><<<gw, 256, 0, s>>>(lv, tt.nleaf, tn, off, src, sn, sc.unit_work.as<uint32_t>(), cnt);
+  k_units_work<<<(int)std::min<int64_t>(UNITS_WORK_BLOCKS, (tt.nleaf + 3) / 4), 256, 0, s>>>(
+      lv, tt.nleaf, max_leaf, np2p, tn, off, l.p2p_src.as<int32_t>(), st.nbody.as<int32_t>(),
+      sc.unit_work.as<uint32_t>(), cnt);
   k_units_fill<<<(int)((tt.nleaf + 255) / 256), 256, 0, s>>>(lv, tt.nleaf, tn, off, sc.unit_work.as<uint32_t>(), cnt,
                                                              l.units.as<int4>(), l.multi.as<int4>());
   UVLM_LAUNCH_CHECK();
-  unsigned long long h[NU_COUNT];
-  UVLM_HIP(hipMemcpyAsync(h, cnt, sizeof(h), hipMemcpyDeviceToHost, s));
-  UVLM_HIP(hipStreamSynchronize(s));
+}
+
+// Takes over what near_units_enqueue left at counters[UNIT_COUNTERS ..], read back by the caller.
+void near_units_set(const unsigned long long *h, Lists &l)
+{
   l.n_interactions = (int64_t)h[NU_INTER];
   l.n_units        = (int64_t)h[NU_UNITS];
   l.n_rows         = (int64_t)h[NU_ROWS];
   l.n_multi        = (int64_t)h[NU_MULTI];
+  l.wide           = h[NU_WIDE] != 0;
   if (l.n_rows >= (int64_t(1) << 31)) throw Error(UVLM_ERR_INTERNAL, "near-field partial rows");
 }
 

@@ -24,7 +24,7 @@
 //      leaf): each leaf's input indices are ranked among themselves
 // Traversal (semantics of src/traverse.hpp:32-85): breadth-first over (target, source)
 // pairs with the reference's split rule and MAC; outputs are appended with one atomic per
-// wavefront and category, then sorted by (target, source).
+// block and category, then put in CSR rows by target, ascending in the source.
 #include <cstdlib>
 #include <cstring>
 
@@ -147,6 +147,7 @@ __device__ __forceinline__ int common_digits(uint64_t a, uint64_t b, int dlim)
 // Totals of a build (32-bit): cells per level, leaves per level, error bits (0: deeper than the key holds;
 // 1: a split needs a digit below the sorted ones).
 enum { TOT_LEVEL = 0, TOT_LEAVES = 24, TOT_ERR = 47, TOT_COUNT = 48 };
+static_assert(4 * TOT_COUNT <= 8 * N_COUNTERS, "build totals");
 __global__ void k_zero_u32(int64_t n, uint32_t *__restrict__ p)
 {
   const int64_t i = blockIdx.x * (int64_t)BLK + threadIdx.x;
@@ -403,144 +404,300 @@ struct TreeView {
   const double  *cx, *cy, *cz, *R;
 };
 
-__device__ __forceinline__ int wave_excl_scan(int v, int &total)
-{
-  const int lane = threadIdx.x & 63;
-  int       s    = v;
-  for (int o = 1; o < 64; o <<= 1) {
-    const int t = __shfl_up(s, o, 64);
-    if (lane >= o) s += t;
-  }
-  total = __shfl(s, 63, 64);
-  return s - v;
-}
+// Counters of a traversal (64-bit, sc.counters): list sizes so far, flags (1 frontier, 2 P2P, 4 M2L
+// buffer overflowed: the traversal starts again with larger ones; 8 a row longer than ROW_LONG), the
+// largest frontier, the frontier sizes of steps k, k + 1, k + 2 (mod 4), and the rows longer than
+// ROW_RANK.
+enum { TC_P2P = 0, TC_M2L = 1, TC_FLAGS = 2, TC_MAXF = 3, TC_FRONT = 4, TC_LONG = 8, TC_COUNT = 9 };
+static_assert(TC_COUNT <= UNIT_COUNTERS, "traversal counters");
+enum { TF_FRONT = 1, TF_P2P = 2, TF_M2L = 4, TF_LONG = 8 };
 
-// One BFS step.  counters: [0] next frontier, [1] P2P, [2] M2L (64-bit).
+// One breadth-first step over the frontier's pairs.  Lanes are (pair, child of the split side), 32
+// pairs a round.  A block takes up to eight rounds before it reserves its output ranges, one atomic
+// per class: the same-address atomics are the traversal's only serialisation (one reservation per 32
+// pairs made it 3.8 times slower on the 4M tree).  The loads of all rounds are issued together, at
+// clamped indices without branches; small frontiers spread over more blocks with fewer rounds.
 // gap > 0 (near-field option, off in the reference): a pair is also near when its bodies can come
 // closer than gap, |dX| < gap + sqrt(3) (Rt + Rs), tested on squares (rounds as the oracle does).
-__device__ __forceinline__ void traverse_round(const int32_t *__restrict__ ft, int64_t nf, int64_t i, TreeView T,
-                                               TreeView S, double theta, double gap, int32_t *__restrict__ nxt,
-                                               int64_t cap_f,
-                                               uint64_t *__restrict__ p2p, int64_t cap_p, uint64_t *__restrict__ m2l,
-                                               int64_t cap_m, unsigned long long *__restrict__ counters, int sbits,
-                                               unsigned long long (*blk)[BLK / 64][3])
+__global__ __launch_bounds__(BLK) void k_traverse(const int2 *__restrict__ ft, TreeView T, TreeView S, double theta,
+                                                  double gap, int2 *__restrict__ nxt, int64_t cap_f,
+                                                  uint2 *__restrict__ p2p, int64_t cap_p, uint2 *__restrict__ m2l,
+                                                  int64_t cap_m, unsigned long long *__restrict__ cnt, int step)
 {
-  int           cls[8];  // 0 push, 1 P2P, 2 M2L
-  int           ct[8], cs[8];
-  int           nout = 0, npush = 0, np2p = 0, nm2l = 0;
-  if (i < nf) {
-    const int t = ft[2 * i], s = ft[2 * i + 1];
-    const bool split_t = (S.nchild[s] == 0) || (T.R[t] >= S.R[s] && T.nchild[t] != 0);
-    const int  first   = split_t ? T.child[t] : S.child[s];
-    const int  cnt     = split_t ? T.nchild[t] : S.nchild[s];
-    for (int c = 0; c < cnt; c++) {
-      const int    a = split_t ? first + c : t;
-      const int    b = split_t ? s : first + c;
-      const double dx = T.cx[a] - S.cx[b], dy = T.cy[a] - S.cy[b], dz = T.cz[a] - S.cz[b];
-      const double D2 = dx * dx + dy * dy + dz * dz, R2 = D2 * theta * theta;
-      const double Rs = T.R[a] + S.R[b];
-      const double Gs = gap + 1.7320508075688772 * Rs;
-      int          k;
-      if (R2 < Rs * Rs || (gap > 0.0 && D2 < Gs * Gs)) k = (T.nchild[a] == 0 && S.nchild[b] == 0) ? 1 : 0;
-      else k = 2;
-      cls[nout] = k;
-      ct[nout]  = a;
-      cs[nout]  = b;
-      nout++;
-      npush += k == 0;
-      np2p += k == 1;
-      nm2l += k == 2;
-    }
+  constexpr int                 ROUNDS = 8, PAIRS = BLK / 8;
+  __shared__ unsigned           tot[BLK / 64][3];
+  __shared__ unsigned long long base[3];
+  const int                     tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, ch = tid & 7;
+  int64_t                       nf = (int64_t)cnt[TC_FRONT + (step & 3)];
+  if (blockIdx.x == 0 && tid == 0) {
+    cnt[TC_FRONT + ((step + 2) & 3)] = 0;
+    atomicMax(&cnt[TC_MAXF], (unsigned long long)nf);
+    if (nf > cap_f) atomicOr(&cnt[TC_FLAGS], (unsigned long long)TF_FRONT);
   }
-  int tf, tp, tm;
-  int of = wave_excl_scan(npush, tf), op = wave_excl_scan(np2p, tp), om = wave_excl_scan(nm2l, tm);
-  // one atomic per class and block: the wavefronts' totals meet in LDS, three lanes reserve the
-  // block's ranges and hand each wavefront its base (the counters are the traversal's only
-  // serialisation point)
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  if (lane == 0) {
-    blk[0][wv][0] = tf;
-    blk[0][wv][1] = tp;
-    blk[0][wv][2] = tm;
-  }
-  __syncthreads();
-  if (threadIdx.x < 3) {
-    const int          cl  = threadIdx.x;
-    unsigned long long tot = 0;
-    for (int w = 0; w < BLK / 64; w++) tot += blk[0][w][cl];
-    unsigned long long base = tot ? atomicAdd(&counters[cl], tot) : 0;
-    for (int w = 0; w < BLK / 64; w++) {
-      blk[1][w][cl] = base;
-      base += blk[0][w][cl];
-    }
-  }
-  __syncthreads();
-  const unsigned long long bf = blk[1][wv][0], bp = blk[1][wv][1], bm = blk[1][wv][2];
-  for (int c = 0; c < nout; c++) {
-    const uint64_t key = ((uint64_t)(uint32_t)ct[c] << sbits) | (uint64_t)(uint32_t)cs[c];
-    if (cls[c] == 0) {
-      const int64_t q = (int64_t)bf + of++;
-      if (q < cap_f) {
-        nxt[2 * q]     = ct[c];
-        nxt[2 * q + 1] = cs[c];
+  if (nf > cap_f) nf = 0;  // the frontier was not stored whole
+  const int64_t per = PAIRS * min((int64_t)ROUNDS, (nf + (int64_t)PAIRS * gridDim.x - 1) / ((int64_t)PAIRS * gridDim.x));
+  for (int64_t b0 = blockIdx.x * per; b0 < nf; b0 += gridDim.x * per) {
+    const int64_t b1 = min(nf, b0 + per);
+    const int     nr = (int)((b1 - b0 + PAIRS - 1) / PAIRS);
+    int           a[ROUNDS], b[ROUNDS], cls[ROUNDS];  // 0 push, 1 P2P, 2 M2L, 3 none
+    auto          rounds = [&](auto count) {
+      constexpr int R = decltype(count)::value;
+      int           nct[R], ncs[R], fc[R];
+      double        Rt[R], Rsrc[R];
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        const int2 pr = ft[min(b0 + r * PAIRS + (tid >> 3), b1 - 1)];
+        a[r] = pr.x, b[r] = pr.y;
       }
-    } else if (cls[c] == 1) {
-      const int64_t q = (int64_t)bp + op++;
-      if (q < cap_p) p2p[q] = key;
-    } else {
-      const int64_t q = (int64_t)bm + om++;
-      if (q < cap_m) m2l[q] = key;
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        nct[r] = T.nchild[a[r]], ncs[r] = S.nchild[b[r]];
+        Rt[r] = T.R[a[r]], Rsrc[r] = S.R[b[r]];
+        fc[r] = T.child[a[r]];
+      }
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        const bool split_t = ncs[r] == 0 || (Rt[r] >= Rsrc[r] && nct[r] != 0);
+        const int  sc = S.child[b[r]];
+        const bool on = ch < (split_t ? nct[r] : ncs[r]) && b0 + r * PAIRS + (tid >> 3) < b1;
+        if (on && split_t) a[r] = fc[r] + ch;
+        if (on && !split_t) b[r] = sc + ch;
+        cls[r] = on ? 0 : 3;
+      }
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        const double dx = T.cx[a[r]] - S.cx[b[r]], dy = T.cy[a[r]] - S.cy[b[r]], dz = T.cz[a[r]] - S.cz[b[r]];
+        const double D2 = dx * dx + dy * dy + dz * dz, R2 = D2 * theta * theta;
+        const double Rs = T.R[a[r]] + S.R[b[r]];
+        const double Gs = gap + 1.7320508075688772 * Rs;
+        const int    k  = R2 < Rs * Rs || (gap > 0.0 && D2 < Gs * Gs)
+                              ? (T.nchild[a[r]] == 0 && S.nchild[b[r]] == 0 ? 1 : 0)
+                              : 2;
+        if (cls[r] == 0) cls[r] = k;
+      }
+#pragma unroll
+      for (int r = R; r < ROUNDS; r++) a[r] = b[r] = 0, cls[r] = 3;
+    };
+    if (nr <= 1) rounds(std::integral_constant<int, 1>{});
+    else if (nr <= 2) rounds(std::integral_constant<int, 2>{});
+    else if (nr <= 4) rounds(std::integral_constant<int, 4>{});
+    else rounds(std::integral_constant<int, ROUNDS>{});
+    unsigned sum[3] = {0, 0, 0};
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++)
+      for (int k = 0; k < 3; k++) sum[k] += (unsigned)__popcll(__ballot(cls[r] == k));
+    __syncthreads();  // the last pass's bases are read
+    if (lane == 0)
+      for (int k = 0; k < 3; k++) tot[wv][k] = sum[k];
+    __syncthreads();
+    if (tid < 3) {
+      unsigned n = 0;
+      for (int w = 0; w < BLK / 64; w++) n += tot[w][tid];
+      const int slot = tid == 0 ? TC_FRONT + ((step + 1) & 3) : tid == 1 ? TC_P2P : TC_M2L;
+      base[tid]      = n ? atomicAdd(&cnt[slot], (unsigned long long)n) : 0;
     }
+    __syncthreads();
+    int64_t at[3];
+    for (int k = 0; k < 3; k++) {
+      at[k] = (int64_t)base[k];
+      for (int w = 0; w < wv; w++) at[k] += tot[w][k];
+    }
+    const unsigned long long below = (1ull << lane) - 1;
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++)
+      for (int k = 0; k < 3; k++) {
+        const unsigned long long m = __ballot(cls[r] == k);
+        const int64_t            q = at[k] + __popcll(m & below);
+        at[k] += __popcll(m);
+        if (cls[r] != k) continue;
+        if (k == 0) {
+          if (q < cap_f) nxt[q] = make_int2(a[r], b[r]);
+        } else if (k == 1) {
+          if (q < cap_p) p2p[q] = make_uint2((unsigned)b[r], (unsigned)a[r]);
+        } else if (q < cap_m) m2l[q] = make_uint2((unsigned)b[r], (unsigned)a[r]);
+      }
   }
-}
-
-// One breadth-first step.  counters: [0] next frontier size, [1] P2P and [2] M2L list sizes so far,
-// [3] this step's frontier size (read here, so a batch of steps runs without the host).  The
-// blocks stride over the frontier; every lane of a block takes part in each round.
-__global__ void k_traverse(const int32_t *__restrict__ ft, TreeView T, TreeView S, double theta, double gap,
-                           int32_t *__restrict__ nxt, int64_t cap_f, uint64_t *__restrict__ p2p, int64_t cap_p,
-                           uint64_t *__restrict__ m2l, int64_t cap_m, unsigned long long *__restrict__ counters,
-                           int sbits)
-{
-  __shared__ unsigned long long blk[2][BLK / 64][3];  // per wavefront: totals, then bases
-  const int64_t nf = (int64_t)counters[3];
-  for (int64_t base = blockIdx.x * (int64_t)BLK; base < nf; base += (int64_t)gridDim.x * BLK)
-    traverse_round(ft, nf, base + threadIdx.x, T, S, theta, gap, nxt, cap_f, p2p, cap_p, m2l, cap_m, counters,
-                   sbits, blk);
 }
 
 // Start of a traversal: the root pair (0, 0) is the first frontier, or, when both roots are leaves,
 // the single P2P pair (traverse.hpp:41-44); the counters are cleared.
-__global__ void k_traverse_start(TreeView T, TreeView S, int32_t *__restrict__ front, uint64_t *__restrict__ p2p,
+__global__ void k_traverse_start(TreeView T, TreeView S, int2 *__restrict__ front, uint2 *__restrict__ p2p,
                                  unsigned long long *__restrict__ c)
 {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
   const bool leaves = T.nchild[0] == 0 && S.nchild[0] == 0;
-  if (leaves) p2p[0] = 0;
-  front[0] = 0;
-  front[1] = 0;
-  c[0] = 0;
-  c[1] = leaves ? 1 : 0;
-  c[2] = 0;
-  c[3] = leaves ? 0 : 1;
-  c[4] = 0;
-  c[5] = 0;
+  if (leaves) p2p[0] = make_uint2(0, 0);
+  front[0] = make_int2(0, 0);
+  for (int k = 0; k < TC_COUNT; k++) c[k] = 0;
+  c[TC_P2P]   = leaves ? 1 : 0;
+  c[TC_FRONT] = leaves ? 0 : 1;
 }
 
-// End of a step: the next frontier becomes the current one.  counters[4] (sticky) flags a buffer
-// that overflowed (1 frontier, 2 P2P, 4 M2L); the traversal then stops (frontier 0) and the host
-// starts it again with larger buffers.  counters[5] keeps the largest frontier seen.
-__global__ void k_step_end(unsigned long long *__restrict__ c, int64_t cap_f, int64_t cap_p, int64_t cap_m)
+// ---- lists to CSR ---------------------------------------------------------------
+// Pairs are (x = source, y = target), read as 64-bit keys target << 32 | source by the sort below.
+// Rows of the CSR are filled by counting (each pair takes the next place of its row), then every row
+// is put in ascending source order by one wavefront that ranks its entries against each other in
+// LDS, or by a workgroup's bitonic sort from ROW_RANK entries on (ranking is quadratic).  Against two
+// radix sorts of all pairs by (target, source), with their searches for the row starts: a quarter of
+// the launches and half the time for small trees.  Large lists stay with the radix sort: the counting
+// atomics go to the memory side (a row's entries lie on different XCDs), 23 a ns at best, and fall
+// behind it from some million pairs on (100k rings, 0.39M pairs: lists phase 0.39 -> 0.26 ms; 60k cube
+// with c = 6, 4.2M pairs in long rows: 0.55 ms sorted, 1.0 counted; 4M rings, 12.6M: 1.08 and 1.28).
+// The size is that of the last lists built here; rows of more than ROW_LONG entries do not fit in
+// LDS, and such lists are radix-sorted too.
+constexpr int     ROW_RANK = 256, ROW_LONG = 16384;
+constexpr int64_t ROWS_SORTED = 3 << 20;
+
+// place[i] = number of pairs of the same row before pair i, in no fixed order; rows counts them.
+// i < n0 are P2P pairs (rows 0..C), the others M2L pairs (rows C + 1 ..).
+__global__ void k_row_count(int64_t C, unsigned long long *cnt, int64_t cap_p, int64_t cap_m,
+                            const uint2 *__restrict__ p2p, const uint2 *__restrict__ m2l, uint32_t *__restrict__ rows,
+                            uint32_t *__restrict__ place)
 {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  unsigned long long f = c[4];
-  if ((int64_t)c[0] > cap_f) f |= 1;
-  if ((int64_t)c[1] > cap_p) f |= 2;
-  if ((int64_t)c[2] > cap_m) f |= 4;
-  c[5] = c[0] > c[5] ? c[0] : c[5];
-  c[4] = f;
-  c[3] = f ? 0 : c[0];
-  c[0] = 0;
+  const int64_t n0 = min((int64_t)cnt[TC_P2P], cap_p), n1 = min((int64_t)cnt[TC_M2L], cap_m);
+  for (int64_t i = blockIdx.x * (int64_t)BLK + threadIdx.x; i < n0 + n1; i += (int64_t)gridDim.x * BLK) {
+    const unsigned t = i < n0 ? p2p[i].y : m2l[i - n0].y;
+    const uint32_t q = atomicAdd(&rows[(i < n0 ? 0 : C + 1) + t], 1u);
+    place[i]         = q;
+    if (q >= ROW_LONG) atomicOr(&cnt[TC_FLAGS], (unsigned long long)TF_LONG);
+  }
+}
+
+// Row starts of both lists (rowoff: the exclusive scan of the counts, P2P rows then M2L rows) and the
+// pairs' sources at their places.
+__global__ void k_row_fill(int64_t C, const unsigned long long *__restrict__ cnt, int64_t cap_p, int64_t cap_m,
+                           const uint2 *__restrict__ p2p, const uint2 *__restrict__ m2l,
+                           const uint32_t *__restrict__ rowoff, const uint32_t *__restrict__ place,
+                           int32_t *__restrict__ off_p, int32_t *__restrict__ src_p, int32_t *__restrict__ off_m,
+                           int32_t *__restrict__ src_m)
+{
+  const int64_t  n0 = min((int64_t)cnt[TC_P2P], cap_p), n1 = min((int64_t)cnt[TC_M2L], cap_m);
+  const uint32_t m0 = rowoff[C + 1];
+  for (int64_t i = blockIdx.x * (int64_t)BLK + threadIdx.x; i < max(n0 + n1, C + 1); i += (int64_t)gridDim.x * BLK) {
+    if (i <= C) {
+      off_p[i] = (int32_t)rowoff[i];
+      off_m[i] = (int32_t)(rowoff[C + 1 + i] - m0);
+    }
+    if (i < n0) {
+      const uint2 pr                     = p2p[i];
+      src_p[rowoff[pr.y] + place[i]] = (int32_t)pr.x;
+    } else if (i < n0 + n1) {
+      const uint2 pr                              = m2l[i - n0];
+      src_m[rowoff[C + 1 + pr.y] - m0 + place[i]] = (int32_t)pr.x;
+    }
+  }
+}
+
+// Every row of both lists in ascending order, one wavefront per row (rows r < C: P2P).
+__global__ __launch_bounds__(BLK) void k_row_sort(int64_t C, const int32_t *__restrict__ off_p,
+                                                  int32_t *__restrict__ src_p, const int32_t *__restrict__ off_m,
+                                                  int32_t *__restrict__ src_m, unsigned long long *__restrict__ nlong,
+                                                  uint32_t *__restrict__ longs)
+{
+  __shared__ __align__(16) int v[BLK / 64][ROW_RANK + 4];
+  const int      wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int64_t  r  = blockIdx.x * (int64_t)(BLK / 64) + wv;
+  if (r >= 2 * C) return;
+  const int32_t *off = r < C ? off_p + r : off_m + (r - C);
+  int32_t       *src = (r < C ? src_p : src_m) + off[0];
+  const int      n   = off[1] - off[0];
+  if (n <= 1) return;
+  if (n > ROW_RANK) {
+    if (lane == 0) longs[atomicAdd(nlong, 1ull)] = (uint32_t)r;
+    return;
+  }
+  int *w = v[wv];
+  int  m[ROW_RANK / 64], q[ROW_RANK / 64];
+#pragma unroll
+  for (int i = 0; i < ROW_RANK / 64; i++) {
+    const int j = lane + 64 * i;
+    m[i]        = j < n ? src[j] : 0x7fffffff;
+    q[i]        = 0;
+    if (64 * i < n + 4) w[j] = m[i];
+  }
+  __builtin_amdgcn_wave_barrier();
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  auto rank = [&](auto count) {
+    for (int k = 0; k < n; k += 4) {  // entries past the end compare greater
+      const int4 e = *reinterpret_cast<const int4 *>(w + k);
+#pragma unroll
+      for (int i = 0; i < decltype(count)::value; i++)
+        q[i] += (e.x < m[i]) + (e.y < m[i]) + (e.z < m[i]) + (e.w < m[i]);
+    }
+  };
+  if (n <= 64) rank(std::integral_constant<int, 1>{});
+  else if (n <= 128) rank(std::integral_constant<int, 2>{});
+  else rank(std::integral_constant<int, ROW_RANK / 64>{});
+#pragma unroll
+  for (int i = 0; i < ROW_RANK / 64; i++)
+    if (lane + 64 * i < n) src[q[i]] = m[i];
+}
+
+// The rows k_row_sort left, a workgroup each: bitonic sort of the next power of two entries.
+constexpr int LONG_LANES = 512, LONG_BLOCKS = 512;
+__global__ __launch_bounds__(LONG_LANES) void k_row_sort_long(int64_t C, const int32_t *__restrict__ off_p,
+                                                              int32_t *__restrict__ src_p,
+                                                              const int32_t *__restrict__ off_m,
+                                                              int32_t *__restrict__ src_m,
+                                                              const unsigned long long *__restrict__ nlong,
+                                                              const uint32_t *__restrict__ longs)
+{
+  __shared__ int v[ROW_LONG];
+  const int      nl = (int)*nlong;
+  for (int k = blockIdx.x; k < nl; k += gridDim.x) {
+    const int64_t  r   = longs[k];
+    const int32_t *off = r < C ? off_p + r : off_m + (r - C);
+    int32_t       *src = (r < C ? src_p : src_m) + off[0];
+    const int      n   = off[1] - off[0];
+    if (n > ROW_LONG) continue;  // flagged: the radix sort takes the lists
+    int m = 2 * ROW_RANK;
+    while (m < n) m *= 2;
+    for (int j = threadIdx.x; j < m; j += LONG_LANES) v[j] = j < n ? src[j] : 0x7fffffff;
+    for (int w = 2; w <= m; w *= 2)
+      for (int d = w / 2; d > 0; d /= 2) {
+        __syncthreads();
+        for (int j = threadIdx.x; j < m / 2; j += LONG_LANES) {
+          const int  a = 2 * j - (j & (d - 1)), b = a + d;
+          const bool up = (a & w) == 0;
+          const int  x = v[a], y = v[b];
+          if ((x > y) == up) v[a] = y, v[b] = x;
+        }
+      }
+    __syncthreads();
+    for (int j = threadIdx.x; j < n; j += LONG_LANES) src[j] = v[j];
+    __syncthreads();
+  }
+}
+
+// The pairs of the transposed lists (row = the source cell), one wavefront per row of both lists.
+__global__ __launch_bounds__(BLK) void k_transpose_pairs(int64_t Ct, const int32_t *__restrict__ off_p,
+                                                         const int32_t *__restrict__ src_p, int64_t n0,
+                                                         const int32_t *__restrict__ off_m,
+                                                         const int32_t *__restrict__ src_m,
+                                                         uint2 *__restrict__ pairs_p, uint2 *__restrict__ pairs_m,
+                                                         unsigned long long *__restrict__ cnt)
+{
+  const int64_t r = blockIdx.x * (int64_t)(BLK / 64) + (threadIdx.x >> 6);
+  const int     lane = threadIdx.x & 63;
+  if (r == 0 && lane == 0) {
+    cnt[TC_P2P]   = (unsigned long long)n0;
+    cnt[TC_M2L]   = (unsigned long long)off_m[Ct];
+    cnt[TC_FLAGS] = 0;
+    cnt[TC_LONG]  = 0;
+  }
+  if (r >= 2 * Ct) return;
+  const bool     near = r < Ct;
+  const int64_t  t    = near ? r : r - Ct;
+  const int32_t *off  = near ? off_p : off_m, *src = near ? src_p : src_m;
+  uint2         *out  = near ? pairs_p : pairs_m;
+  for (int q = off[t] + lane; q < off[t + 1]; q += 64) out[q] = make_uint2((unsigned)t, (unsigned)src[q]);
+}
+
+// Keys (row << lbits) | entry of the radix sort.
+__global__ void k_pack_keys(int64_t n, const uint2 *__restrict__ pairs, int lbits, uint64_t *__restrict__ keys)
+{
+  const int64_t i = blockIdx.x * (int64_t)BLK + threadIdx.x;
+  if (i < n) keys[i] = (uint64_t)pairs[i].y << lbits | pairs[i].x;
 }
 
 // List keys are (row << lbits) | entry, sorted: off[c] = the first key of row c.
@@ -562,22 +719,6 @@ __global__ void k_low_bits(int64_t n, const uint64_t *__restrict__ keys, int lbi
 {
   const int64_t i = blockIdx.x * (int64_t)BLK + threadIdx.x;
   if (i < n) out[i] = (int32_t)(uint32_t)(keys[i] & ((1ull << lbits) - 1));
-}
-
-// One lane per list entry q: its row t (the last t with off[t] <= q) by binary search, key
-// (source, target) for the transposed CSR.
-__global__ void k_transpose_keys(int64_t C, int64_t n, const int32_t *__restrict__ off,
-                                 const int32_t *__restrict__ src, int tbits, uint64_t *__restrict__ keys)
-{
-  const int64_t q = blockIdx.x * (int64_t)BLK + threadIdx.x;
-  if (q >= n) return;
-  int64_t lo = 0, hi = C - 1;
-  while (lo < hi) {
-    const int64_t mid = (lo + hi + 1) >> 1;
-    if (off[mid] <= q) lo = mid;
-    else hi = mid - 1;
-  }
-  keys[q] = ((uint64_t)(uint32_t)src[q] << tbits) | (uint64_t)(uint32_t)lo;
 }
 
 void h2d(hipStream_t s, void *d, const void *h, size_t bytes)
@@ -639,7 +780,7 @@ void build_tree(hipStream_t s, Scratch &sc, const double *x, const double *y, co
   const uint32_t *idx  = sc.idx1.as<uint32_t>();
   uint32_t       *info = sc.idx0.as<uint32_t>();  // free once sorted
   int32_t        *scan = sc.keys0.as<int32_t>();
-  sc.counters.reserve(4 * TOT_COUNT);
+  sc.counters.reserve(8 * N_COUNTERS);
   uint32_t *tot  = sc.counters.as<uint32_t>();
   int       dlim = std::min(KEY_LEVELS, std::max(1, tree.sort_digits));
   uint32_t  h[TOT_COUNT];
@@ -785,10 +926,65 @@ static TreeView view(const Tree &t)
                   (const double *)t.R.p};
 }
 
-void traverse(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &st, double theta, Lists &lists, double gap)
+// CSR rows by target of the np P2P and nm M2L pairs in sc.out_p2p / out_m2l (their numbers are read
+// on the device; np and nm bound them).  C target cells, entries below Cs.
+static void rows_by_counting(hipStream_t s, Scratch &sc, int64_t C, int64_t np, int64_t nm, Lists &l)
 {
-  TreeView  T = view(tt), S = view(st);
-  const int sbits = bits_for(std::max<int64_t>(st.C, 1));  // list keys: (target << sbits) | source
+  unsigned long long *cnt = sc.counters.as<unsigned long long>();
+  l.p2p_off.reserve(4 * (C + 1));
+  l.m2l_off.reserve(4 * (C + 1));
+  l.p2p_src.reserve(4 * std::max<int64_t>(np, 1));
+  l.m2l_src.reserve(4 * std::max<int64_t>(nm, 1));
+  sc.row_cnt.reserve(4 * 2 * (C + 1));
+  sc.row_off.reserve(4 * 2 * (C + 1));
+  sc.row_place.reserve(4 * std::max<int64_t>(np + nm, 1));
+  sc.row_long.reserve(4 * ((np + nm) / ROW_RANK + 1));
+  uint32_t    *rows = sc.row_cnt.as<uint32_t>(), *ro = sc.row_off.as<uint32_t>(), *pl = sc.row_place.as<uint32_t>();
+  const uint2 *p2p = sc.out_p2p.as<uint2>(), *m2l = sc.out_m2l.as<uint2>();
+  const int    grid = (int)std::min<int64_t>(4096, nblocks(std::max<int64_t>(np + nm, C + 1)));
+  k_zero_u32<<<nblocks(2 * (C + 1)), BLK, 0, s>>>(2 * (C + 1), rows);
+  k_row_count<<<grid, BLK, 0, s>>>(C, cnt, np, nm, p2p, m2l, rows, pl);
+  excl_scan(s, sc, rows, ro, 2 * (C + 1));
+  k_row_fill<<<grid, BLK, 0, s>>>(C, cnt, np, nm, p2p, m2l, ro, pl, l.p2p_off.as<int32_t>(), l.p2p_src.as<int32_t>(),
+                                  l.m2l_off.as<int32_t>(), l.m2l_src.as<int32_t>());
+  k_row_sort<<<nblocks(2 * C, BLK / 64), BLK, 0, s>>>(C, l.p2p_off.as<int32_t>(), l.p2p_src.as<int32_t>(),
+                                                      l.m2l_off.as<int32_t>(), l.m2l_src.as<int32_t>(),
+                                                      cnt + TC_LONG, sc.row_long.as<uint32_t>());
+  if (np + nm > ROW_RANK)
+    k_row_sort_long<<<LONG_BLOCKS, LONG_LANES, 0, s>>>(C, l.p2p_off.as<int32_t>(), l.p2p_src.as<int32_t>(),
+                                                       l.m2l_off.as<int32_t>(), l.m2l_src.as<int32_t>(), cnt + TC_LONG,
+                                                       sc.row_long.as<uint32_t>());
+  UVLM_LAUNCH_CHECK();
+}
+
+// The same by a radix sort of the pairs (rows of any length); the sizes are known here.
+static void rows_by_sorting(hipStream_t s, Scratch &sc, int64_t C, int64_t Cs, Lists &l)
+{
+  const int lbits = bits_for(std::max<int64_t>(Cs, 1)), eb = lbits + bits_for(std::max<int64_t>(C, 1));
+  for (int which = 0; which < 2; which++) {
+    const int64_t n   = which == 0 ? l.np2p : l.nm2l;
+    DevBuf       &raw = which == 0 ? sc.out_p2p : sc.out_m2l;
+    DevBuf       &off = which == 0 ? l.p2p_off : l.m2l_off;
+    DevBuf       &src = which == 0 ? l.p2p_src : l.m2l_src;
+    off.reserve(4 * (C + 1));
+    src.reserve(4 * std::max<int64_t>(n, 1));
+    sc.keys0.reserve(8 * std::max<int64_t>(n, 1));
+    sc.keys1.reserve(8 * std::max<int64_t>(n, 1));
+    if (n > 0) {
+      k_pack_keys<<<nblocks(n), BLK, 0, s>>>(n, raw.as<uint2>(), lbits, sc.keys0.as<uint64_t>());
+      sort_keys_u64(s, sc, sc.keys0.as<uint64_t>(), sc.keys1.as<uint64_t>(), n, eb);
+    }
+    k_csr<<<nblocks(C + 1), BLK, 0, s>>>(C, sc.keys1.as<uint64_t>(), n, lbits, off.as<int32_t>());
+    k_low_bits<<<nblocks(n), BLK, 0, s>>>(n, sc.keys1.as<uint64_t>(), lbits, src.as<int32_t>());
+    UVLM_LAUNCH_CHECK();
+  }
+}
+
+// max_leaf >= 0: also the lists' near-field units (near.hip), read back together with the sizes.
+void traverse(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &st, double theta, Lists &lists, double gap,
+              int64_t max_leaf)
+{
+  TreeView T = view(tt), S = view(st);
   int64_t cap_f = std::max<int64_t>(4096, 8 * (tt.C + st.C));
   int64_t cap_p = std::max<int64_t>(4096, 32 * tt.nleaf);
   int64_t cap_m = std::max<int64_t>(4096, 64 * tt.C);
@@ -800,92 +996,103 @@ void traverse(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &st, double
   sc.front1.reserve(8 * cap_f);
   sc.out_p2p.reserve(8 * cap_p);
   sc.out_m2l.reserve(8 * cap_m);
-  cap_f = std::min(sc.front0.bytes, sc.front1.bytes) / 8;
-  cap_p = sc.out_p2p.bytes / 8;
-  cap_m = sc.out_m2l.bytes / 8;
-  unsigned long long cnt[6] = {0, 0, 0, 0, 0, 0};
-  sc.counters.reserve(64);
-  unsigned long long *dcnt = (unsigned long long *)sc.counters.p;
-  {
-    // steps run in batches of STEPS without the host; a batch ends with one read of the counters
-    constexpr int STEPS = 6;
-    for (;;) {
-      k_traverse_start<<<1, 64, 0, s>>>(T, S, sc.front0.as<int32_t>(), sc.out_p2p.as<uint64_t>(), dcnt);
-      const int grid = nblocks(std::min<int64_t>(cap_f, 2048 * (int64_t)BLK));
-      int       par  = 0;
-      for (;;) {
-        for (int k = 0; k < STEPS; k++, par ^= 1) {
-          DevBuf &fin = par ? sc.front1 : sc.front0, &fout = par ? sc.front0 : sc.front1;
-          k_traverse<<<grid, BLK, 0, s>>>(fin.as<int32_t>(), T, S, theta, gap, fout.as<int32_t>(), cap_f,
-                                          sc.out_p2p.as<uint64_t>(), cap_p, sc.out_m2l.as<uint64_t>(), cap_m, dcnt,
-                                          sbits);
-          k_step_end<<<1, 64, 0, s>>>(dcnt, cap_f, cap_p, cap_m);
-          UVLM_LAUNCH_CHECK();
-        }
-        to_host(s, cnt, dcnt, 6);
-        if (cnt[4] || cnt[3] == 0) break;
+  sc.counters.reserve(8 * N_COUNTERS);
+  unsigned long long *dcnt = sc.counters.as<unsigned long long>();
+  // every step splits one side of each pair, so a frontier of two trees of known depth is empty after
+  // their levels' sum; trees handed in by a caller are walked until it is
+  const int  depth = tt.nlevels > 0 && st.nlevels > 0 ? tt.nlevels + st.nlevels - 2 : -1;
+  constexpr int BATCH = 6;
+  for (;;) {
+    cap_f = std::min(sc.front0.bytes, sc.front1.bytes) / 8;
+    cap_p = sc.out_p2p.bytes / 8;
+    cap_m = sc.out_m2l.bytes / 8;
+    unsigned long long cnt[N_COUNTERS] = {};
+    k_traverse_start<<<1, 64, 0, s>>>(T, S, sc.front0.as<int2>(), sc.out_p2p.as<uint2>(), dcnt);
+    int64_t most = 1;  // pairs a step's frontier can hold
+    for (int k = 0;; k++) {
+      if (depth >= 0 ? k >= depth : k > 0 && k % BATCH == 0) {
+        if (depth >= 0) break;
+        to_host(s, cnt, dcnt, TC_COUNT);
+        if (cnt[TC_FRONT + (k & 3)] == 0 || (cnt[TC_FLAGS] & TF_FRONT)) break;
       }
-      if (!cnt[4]) break;
-      // a buffer overflowed: grow what did (at least doubled) and traverse again
-      if (cnt[4] & 1) {
-        const int64_t want = std::max<int64_t>(2 * cap_f, 2 * (int64_t)cnt[5]);
+      DevBuf &fin = k & 1 ? sc.front1 : sc.front0, &fout = k & 1 ? sc.front0 : sc.front1;
+      k_traverse<<<(int)std::min<int64_t>(2048, nblocks(most, BLK / 8)), BLK, 0, s>>>(
+          fin.as<int2>(), T, S, theta, gap, fout.as<int2>(), cap_f, sc.out_p2p.as<uint2>(), cap_p,
+          sc.out_m2l.as<uint2>(), cap_m, dcnt, k);
+      UVLM_LAUNCH_CHECK();
+      most = std::min<int64_t>(8 * most, cap_f);
+    }
+    // with lists of this kind built before, their size picks the way and the sizes are read back with
+    // the units; without, the sizes are read first
+    const bool ahead = lists.np2p > 0 && !lists.long_rows && lists.np2p + lists.nm2l <= ROWS_SORTED;
+    auto       by_counting = [&](int64_t np, int64_t nm) {
+      rows_by_counting(s, sc, tt.C, np, nm, lists);
+      if (max_leaf >= 0) near_units_enqueue(s, sc, tt, st, max_leaf, dcnt + TC_P2P, lists);
+    };
+    if (ahead) by_counting(cap_p, cap_m);
+    to_host(s, cnt, dcnt, N_COUNTERS);
+    if (depth >= 0 && !(cnt[TC_FLAGS] & TF_FRONT) && cnt[TC_FRONT + (depth & 3)] != 0)
+      throw Error(UVLM_ERR_INTERNAL, "the traversal did not end");
+    int over = (int)(cnt[TC_FLAGS] & TF_FRONT);
+    if ((int64_t)cnt[TC_P2P] > cap_p) over |= TF_P2P;
+    if ((int64_t)cnt[TC_M2L] > cap_m) over |= TF_M2L;
+    if (over) {  // grow what overflowed (at least doubled) and traverse again
+      if (over & TF_FRONT) {
+        const int64_t want = std::max<int64_t>(2 * cap_f, 2 * (int64_t)cnt[TC_MAXF]);
         sc.front0.reserve(8 * want);
         sc.front1.reserve(8 * want);
       }
-      if (cnt[4] & 2) sc.out_p2p.reserve(8 * std::max<int64_t>(2 * cap_p, 2 * (int64_t)cnt[1]));
-      if (cnt[4] & 4) sc.out_m2l.reserve(8 * std::max<int64_t>(2 * cap_m, 2 * (int64_t)cnt[2]));
-      cap_f = std::min(sc.front0.bytes, sc.front1.bytes) / 8;
-      cap_p = sc.out_p2p.bytes / 8;
-      cap_m = sc.out_m2l.bytes / 8;
+      if (over & TF_P2P) sc.out_p2p.reserve(8 * std::max<int64_t>(2 * cap_p, 2 * (int64_t)cnt[TC_P2P]));
+      if (over & TF_M2L) sc.out_m2l.reserve(8 * std::max<int64_t>(2 * cap_m, 2 * (int64_t)cnt[TC_M2L]));
+      continue;
     }
-  }
-  lists.np2p = (int64_t)cnt[1];
-  lists.nm2l = (int64_t)cnt[2];
-  const int64_t C  = tt.C;
-  const int     eb = sbits + bits_for(std::max<int64_t>(tt.C, 1));
-  for (int which = 0; which < 2; which++) {
-    const int64_t n   = which == 0 ? lists.np2p : lists.nm2l;
-    DevBuf       &raw = which == 0 ? sc.out_p2p : sc.out_m2l;
-    DevBuf       &off = which == 0 ? lists.p2p_off : lists.m2l_off;
-    DevBuf       &src = which == 0 ? lists.p2p_src : lists.m2l_src;
-    off.reserve(4 * (C + 1));
-    src.reserve(4 * std::max<int64_t>(n, 1));
-    sc.keys1.reserve(8 * std::max<int64_t>(n, 1));
-    if (n > 0) sort_keys_u64(s, sc, raw.as<uint64_t>(), sc.keys1.as<uint64_t>(), n, eb);
-    k_csr<<<nblocks(C + 1), BLK, 0, s>>>(C, sc.keys1.as<uint64_t>(), n, sbits, off.as<int32_t>());
-    k_low_bits<<<nblocks(n), BLK, 0, s>>>(n, sc.keys1.as<uint64_t>(), sbits, src.as<int32_t>());
-    UVLM_LAUNCH_CHECK();
+    lists.np2p = (int64_t)cnt[TC_P2P];
+    lists.nm2l = (int64_t)cnt[TC_M2L];
+    if (!ahead && !lists.long_rows && lists.np2p + lists.nm2l <= ROWS_SORTED) {
+      by_counting(lists.np2p, lists.nm2l);
+      to_host(s, cnt, dcnt, N_COUNTERS);
+    } else if (!ahead) cnt[TC_FLAGS] |= TF_LONG;
+    if (cnt[TC_FLAGS] & TF_LONG) {
+      lists.long_rows = lists.long_rows || lists.np2p + lists.nm2l <= ROWS_SORTED;
+      rows_by_sorting(s, sc, tt.C, st.C, lists);
+      if (max_leaf >= 0) {
+        near_units_enqueue(s, sc, tt, st, max_leaf, dcnt + TC_P2P, lists);
+        to_host(s, cnt, dcnt, N_COUNTERS);
+      }
+    }
+    if (max_leaf >= 0) near_units_set(cnt + UNIT_COUNTERS, lists);
+    return;
   }
 }
 
 void transpose_lists(hipStream_t s, Scratch &sc, const Tree &in_targets, const Tree &in_sources, const Lists &in,
-                     Lists &out)
+                     Lists &out, int64_t max_leaf)
 {
-  const int64_t Cs    = in_sources.C;
-  const int     tbits = bits_for(std::max<int64_t>(in_targets.C, 1));  // entry (target cell) bits of a key
-  const int     eb    = tbits + bits_for(std::max<int64_t>(Cs, 1));
-  out.np2p         = in.np2p;
-  out.nm2l         = in.nm2l;
-  for (int which = 0; which < 2; which++) {
-    const int64_t n    = which == 0 ? in.np2p : in.nm2l;
-    const DevBuf &ioff = which == 0 ? in.p2p_off : in.m2l_off;
-    const DevBuf &isrc = which == 0 ? in.p2p_src : in.m2l_src;
-    DevBuf       &off  = which == 0 ? out.p2p_off : out.m2l_off;
-    DevBuf       &src  = which == 0 ? out.p2p_src : out.m2l_src;
-    off.reserve(4 * (Cs + 1));
-    src.reserve(4 * std::max<int64_t>(n, 1));
-    sc.keys0.reserve(8 * std::max<int64_t>(n, 1));
-    sc.keys1.reserve(8 * std::max<int64_t>(n, 1));
-    if (n > 0) {
-      k_transpose_keys<<<nblocks(n), BLK, 0, s>>>(in_targets.C, n, ioff.as<int32_t>(), isrc.as<int32_t>(), tbits,
-                                                  sc.keys0.as<uint64_t>());
-      UVLM_LAUNCH_CHECK();
-    }
-    if (n > 0) sort_keys_u64(s, sc, sc.keys0.as<uint64_t>(), sc.keys1.as<uint64_t>(), n, eb);
-    k_csr<<<nblocks(Cs + 1), BLK, 0, s>>>(Cs, sc.keys1.as<uint64_t>(), n, tbits, off.as<int32_t>());
-    k_low_bits<<<nblocks(n), BLK, 0, s>>>(n, sc.keys1.as<uint64_t>(), tbits, src.as<int32_t>());
-    UVLM_LAUNCH_CHECK();
+  const int64_t Ct = in_targets.C, Cs = in_sources.C;
+  out.np2p = in.np2p;
+  out.nm2l = in.nm2l;
+  sc.out_p2p.reserve(8 * std::max<int64_t>(in.np2p, 1));
+  sc.out_m2l.reserve(8 * std::max<int64_t>(in.nm2l, 1));
+  sc.counters.reserve(8 * N_COUNTERS);
+  unsigned long long *dcnt = sc.counters.as<unsigned long long>();
+  k_transpose_pairs<<<nblocks(2 * Ct, BLK / 64), BLK, 0, s>>>(
+      Ct, in.p2p_off.as<int32_t>(), in.p2p_src.as<int32_t>(), in.np2p, in.m2l_off.as<int32_t>(),
+      in.m2l_src.as<int32_t>(), sc.out_p2p.as<uint2>(), sc.out_m2l.as<uint2>(), dcnt);
+  UVLM_LAUNCH_CHECK();
+  unsigned long long cnt[N_COUNTERS] = {};
+  const bool         sorted = out.long_rows || in.np2p + in.nm2l > ROWS_SORTED;
+  if (!sorted) {
+    rows_by_counting(s, sc, Cs, in.np2p, in.nm2l, out);
+    near_units_enqueue(s, sc, in_sources, in_targets, max_leaf, dcnt + TC_P2P, out);
+    to_host(s, cnt, dcnt, N_COUNTERS);
+    out.long_rows = (cnt[TC_FLAGS] & TF_LONG) != 0;
   }
+  if (sorted || out.long_rows) {
+    rows_by_sorting(s, sc, Cs, Ct, out);
+    near_units_enqueue(s, sc, in_sources, in_targets, max_leaf, dcnt + TC_P2P, out);
+    to_host(s, cnt, dcnt, N_COUNTERS);
+  }
+  near_units_set(cnt + UNIT_COUNTERS, out);
 }
 
 }  // namespace uvlm
