@@ -15,20 +15,40 @@ namespace {
 constexpr int BLK = 256;
 inline int    nblocks(int64_t n) { return (int)std::max<int64_t>(1, (n + BLK - 1) / BLK); }
 
-__global__ void k_aos_to_soa(const double *__restrict__ aos, int64_t n, int64_t stride, double *__restrict__ st,
-                             int64_t cap)
+// Records of nf doubles (every `stride` doubles) <-> nf field arrays, TB bodies per workgroup through
+// LDS, so that both sides are read and written in consecutive lanes.  Bound by HBM.  A lane per body
+// walking its record (296 bytes apart) moved the 37 fields of 4M bodies in 1.55 ms (1.6 TB/s).
+// Bodies n .. m - 1 get zero fields.
+constexpr int TB = 64, MAX_RECORD = N_FIELDS;
+__global__ __launch_bounds__(BLK) void k_records_in(const double *__restrict__ aos, int64_t n, int64_t m, int nf,
+                                                    int64_t stride, double *__restrict__ f0, int64_t cap)
 {
-  const int64_t i = blockIdx.x * (int64_t)BLK + threadIdx.x;
-  if (i >= n) return;
-  for (int f = 0; f < N_FIELDS; f++) st[f * cap + i] = aos[i * stride + f];
+  __shared__ double v[TB * MAX_RECORD];
+  const int64_t     i0 = blockIdx.x * (int64_t)TB;
+  const int         nb = (int)min((int64_t)TB, m - i0), nin = (int)max((int64_t)0, min((int64_t)TB, n - i0));
+  if (stride == nf)
+    for (int k = threadIdx.x; k < nin * nf; k += BLK) v[k] = aos[i0 * nf + k];
+  else
+    for (int k = threadIdx.x; k < nin * nf; k += BLK) v[k] = aos[(i0 + k / nf) * stride + k % nf];
+  __syncthreads();
+  const int b = threadIdx.x & (TB - 1);
+  if (b < nb)
+    for (int f = threadIdx.x / TB; f < nf; f += BLK / TB) f0[f * cap + i0 + b] = b < nin ? v[b * nf + f] : 0.0;
 }
 
-__global__ void k_soa_to_aos(const double *__restrict__ st, int64_t cap, double *__restrict__ aos, int64_t n,
-                             int64_t stride)
+__global__ __launch_bounds__(BLK) void k_records_out(const double *__restrict__ f0, int64_t cap, int64_t n, int nf,
+                                                     int64_t stride, double *__restrict__ aos)
 {
-  const int64_t i = blockIdx.x * (int64_t)BLK + threadIdx.x;
-  if (i >= n) return;
-  for (int f = 0; f < N_FIELDS; f++) aos[i * stride + f] = st[f * cap + i];
+  __shared__ double v[TB * MAX_RECORD];
+  const int64_t     i0 = blockIdx.x * (int64_t)TB;
+  const int         nb = (int)min((int64_t)TB, n - i0), b = threadIdx.x & (TB - 1);
+  if (b < nb)
+    for (int f = threadIdx.x / TB; f < nf; f += BLK / TB) v[b * nf + f] = f0[f * cap + i0 + b];
+  __syncthreads();
+  if (stride == nf)
+    for (int k = threadIdx.x; k < nb * nf; k += BLK) aos[i0 * nf + k] = v[k];
+  else
+    for (int k = threadIdx.x; k < nb * nf; k += BLK) aos[(i0 + k / nf) * stride + k % nf] = v[k];
 }
 
 __global__ void k_rk(double *__restrict__ st, int64_t cap, int64_t N, int scheme, int stage, double dt)
@@ -295,18 +315,31 @@ void rbf_vec(hipStream_t s, double *st, int64_t cap, int64_t N, int mode, const 
   UVLM_LAUNCH_CHECK();
 }
 
-void aos_to_soa(hipStream_t s, const void *aos, int64_t n, int64_t stride_doubles, double *st, int64_t cap)
+void records_in(hipStream_t s, const double *aos, int64_t n, int64_t m, int nf, int64_t stride, double *fields,
+                int64_t cap)
+{
+  if (m <= 0) return;
+  if (nf > MAX_RECORD) throw Error(UVLM_ERR_INTERNAL, "record width");
+  k_records_in<<<(int)((m + TB - 1) / TB), BLK, 0, s>>>(aos, n, m, nf, stride, fields, cap);
+  UVLM_LAUNCH_CHECK();
+}
+
+void records_out(hipStream_t s, const double *fields, int64_t cap, int64_t n, int nf, int64_t stride, double *aos)
 {
   if (n <= 0) return;
-  k_aos_to_soa<<<nblocks(n), BLK, 0, s>>>((const double *)aos, n, stride_doubles, st, cap);
+  if (nf > MAX_RECORD) throw Error(UVLM_ERR_INTERNAL, "record width");
+  k_records_out<<<(int)((n + TB - 1) / TB), BLK, 0, s>>>(fields, cap, n, nf, stride, aos);
   UVLM_LAUNCH_CHECK();
+}
+
+void aos_to_soa(hipStream_t s, const void *aos, int64_t n, int64_t stride_doubles, double *st, int64_t cap)
+{
+  records_in(s, (const double *)aos, n, n, N_FIELDS, stride_doubles, st, cap);
 }
 
 void soa_to_aos(hipStream_t s, const double *st, int64_t cap, void *aos, int64_t n, int64_t stride_doubles)
 {
-  if (n <= 0) return;
-  k_soa_to_aos<<<nblocks(n), BLK, 0, s>>>(st, cap, (double *)aos, n, stride_doubles);
-  UVLM_LAUNCH_CHECK();
+  records_out(s, st, cap, n, N_FIELDS, stride_doubles, (double *)aos);
 }
 
 void rk_stage(hipStream_t s, double *st, int64_t cap, int64_t N, int scheme, int stage, double dt, int)

@@ -277,6 +277,10 @@ void probe_velocity_grad_out(hipStream_t s, int64_t m, const int32_t *perm, cons
                              double *Jout);
 
 // body.hip
+// n records of nf doubles (every stride doubles) into nf fields, bodies n .. m - 1 zero; and back
+void records_in(hipStream_t s, const double *aos, int64_t n, int64_t m, int nf, int64_t stride, double *fields,
+                int64_t cap);
+void records_out(hipStream_t s, const double *fields, int64_t cap, int64_t n, int nf, int64_t stride, double *aos);
 void aos_to_soa(hipStream_t s, const void *aos, int64_t n, int64_t stride_doubles, double *st, int64_t cap);
 void soa_to_aos(hipStream_t s, const double *st, int64_t cap, void *aos, int64_t n, int64_t stride_doubles);
 void rk_stage(hipStream_t s, double *st, int64_t cap, int64_t N, int scheme, int stage, double dt, int store_initial);
