@@ -149,9 +149,10 @@ void transpose_lists(hipStream_t s, Scratch &sc, const Tree &in_targets, const T
 // far.hip
 struct M2LSchedule {
   int     budget = 0;  // accumulator slots per lane (0: default)
-  int     waves  = 0;  // wavefronts per M2L workgroup (1 or 2; 0: 1 for P <= 8, else 2)
+  int     waves  = 0;  // wavefronts per M2L workgroup (1 or 2; 0: by P, m2l_waves)
   int     W      = 1;  // the wavefronts per workgroup of the current schedule
   M2LPlan plan;
+  bool    fixed = false;  // the plan is the one k_m2l_fixed is compiled for
   DevBuf  dev;         // slots, lev, out_off, out_src
   int64_t dev_slots = 0, dev_lev = 0, dev_out_off = 0, dev_out_src = 0;
   DevBuf  ytab;        // singular harmonics of the lattice vectors [-K, K]^3 (M2L_TABLE_K)

@@ -22,7 +22,8 @@
 //           cells); 4 groups of 16 lanes take every 4th source of the list; the singular
 //           harmonics and the source multipole sit in LDS; the lanes of a group walk (n, m)
 //           in lock step, each adding the terms of the outputs bound to its accumulator
-//           slots (plan in m2l_plan.hpp).  Partial sums are combined in a fixed order at
+//           slots (plan in m2l_plan.hpp), with the multipole from LDS or from the group's
+//           registers (k_m2l_ns, k_m2l_fixed).  Partial sums are combined in a fixed order at
 //           the end, so results are deterministic and no atomics are used
 //   L2L   : one workgroup per child cell of a level (gather from the parent)
 //   L2P   : one workgroup per leaf, lane <-> body
@@ -929,8 +930,8 @@ __global__ __launch_bounds__(WG) void k_m2l_table(int P, double2 *__restrict__ Y
 // The n-synchronous M2L (plan in m2l_plan.hpp).  One workgroup (W wavefronts) per target
 // cell; the 4 groups of 16 lanes of a wavefront take every 4th source.  All lanes of a group walk the source
 // degrees n and orders m in the same sequence, so M[n,m] is one LDS broadcast per group, and
-// each lane adds the terms of the outputs bound to its S accumulator slots.  Blocks are
-// mapped so that each of the 8 XCDs takes one contiguous range of targets: spatially close
+// each lane adds the terms of the outputs bound to its S accumulator slots (k_m2l_fixed below is
+// the same for the usual orders, its plan compiled in).  Blocks are mapped so that each of the 8 XCDs takes one contiguous range of targets: spatially close
 // targets share most of their sources, and those multipoles then hit the XCD's own L2.
 
 // Order m >= 1 of output (j,k) at degree n: terms m and -m taken together (multipoleKernels.hpp:534-546),
@@ -980,23 +981,205 @@ __device__ __forceinline__ void m2l_terms_run(double2 (&a)[3], const double2 *__
   for (int i = 1; i <= T; i++) m2l_step(a, Ya[i], Yb[i], Mm + 3 * i, sk);
 }
 
+// f(integral_constant<0>), ..., f(integral_constant<N - 1>)
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_seq(F &&f, std::integer_sequence<int, I...>)
+{
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F &&f)
+{
+  static_for_seq(f, std::make_integer_sequence<int, N>{});
+}
+
+// W wavefronts share the staged sources: with W = 2 each takes the source degrees the plan
+// gives it, with its own 16-lane plan for them, and the output loop adds both wavefronts'
+// pieces of each output in a fixed order (W = 2 halves the LDS per wavefront, so up to 5
+// slots run at 4 waves per SIMD).
+template <int W>
+__device__ __forceinline__ void m2l_sync()
+{
+  if (W == 1) wave_lds_sync();
+  else block_lds_sync();
+}
+
+// Slot s of lane sl, decoded once per workgroup into an int4 of the wavefront's table (byte
+// offsets; hi(x) = high word of the double x).  At degree n the slot adds orders
+// m0 .. m0 + c - 1 of output (j, k), J = j + n, from Ya = Yx[J, m0 - k] and
+// Yb = Yx[J, m0 + k] = Ya + 32 k, with M[n, m0] = Mn + 48 m0:
+//  * home slot, output w = 16 s + sl = tri(j) + k, active where w < tri(P - n), m0 = 0,
+//    c = n + 1: {16 (j(j+1) - k), 16 (2j + 1), 32 k, hi((-1)^k)}, Ya = Yx + x + y n + 16 n^2;
+//  * helper slot of degree d (a chunk of c = cn orders):
+//    {16 (J(J+1) - k + m0 - d^2), 48 m0, 32 k, hi((-1)^k)}, Ya = Yx + x + 16 d^2;
+//    its first step's sign is 0 for m0 = 0 (the step is then the order-0 term, see
+//    m2l_terms_run);
+//  * unused helper lane: {0, 0, 0, 0} (a sign word of 0 marks it idle).
+__device__ __forceinline__ int4 m2l_slot(int v)
+{
+  const int j = v & 31, k = (v >> 5) & 31, m0 = (v >> 10) & 31, d = (v >> 15) & 31;
+  const int hk = (k & 1) ? (int)0xBFF00000 : 0x3FF00000;
+  if (v < 0) return make_int4(0, 0, 0, 0);
+  if (d == M2LPlan::HOME) return make_int4(16 * (j * (j + 1) - k), 16 * (2 * j + 1), 32 * k, hk);
+  const int J = j + d;
+  return make_int4(16 * (J * (J + 1) - k + m0 - d * d), 48 * m0, 32 * k, hk);
+}
+
+// What a workgroup needs to stage a source: its target's centre and level and, for the lattice
+// table, R0^-(J+1) in sinv and the row J of each harmonic entry this lane copies,
+// e = min(pl + 16 W i, P*P - 1) (J*J <= e <= J*J + 2J), 4 bits per entry i.  pl numbers the
+// W * 16 lanes of a source's group.
+template <int W>
+struct M2LStage {
+  using JRows = typename std::conditional<W == 1, uint64_t, uint32_t>::type;
+  double  X, Y, Z;
+  int     lt, pl;
+  JRows   jrow;
+  double *sinv;
+
+  __device__ __forceinline__ void init(int P, int tid, int pl_, double *sinv_, const M2LTable &tab, const double *tx,
+                                       const double *ty, const double *tz, int64_t t)
+  {
+    X = tx[t], Y = ty[t], Z = tz[t];
+    lt   = tab.Y ? tab.level[t] : 0;
+    pl   = pl_;
+    sinv = sinv_;
+    jrow = 0;
+    if (tab.Y) {
+      const double inv0 = 1.0 / tab.X0R0[3];
+      if (tid < P) {
+        double q = inv0;
+        for (int i = 0; i < tid; i++) q *= inv0;
+        sinv[tid] = q;
+      }
+      for (int i = 0; i < 2 * (int)sizeof(JRows); i++) {
+        const int e = min(pl + 16 * W * i, P * P - 1);
+        int       J = 0;
+        while ((J + 1) * (J + 1) <= e) J++;
+        jrow |= (JRows)J << (4 * i);
+      }
+      m2l_sync<W>();
+    }
+  }
+
+  // source s: its multipole to Mg, its extended harmonics about the target to Yx
+  __device__ __forceinline__ void source(int P, int NT, int s, const double *__restrict__ sx,
+                                         const double *__restrict__ sy, const double *__restrict__ sz,
+                                         const double2 *__restrict__ M, const M2LTable &tab, double2 *Yx,
+                                         double2 *Mg) const
+  {
+    const double cx = sx[s], cy = sy[s], cz = sz[s];
+    const int    ls = tab.Y ? tab.level[s] : 0;
+    // four loads in flight per lane before the first LDS store: at immediate offsets from the
+    // lane's first entry while every lane's four entries exist, then with indices past the end
+    // clamped to the last entry, whose owner writes the same value (no branches)
+    const double2 *Ms = M + (int64_t)s * NT;
+    // (the scheduling barriers keep the four loads ahead of the stores)
+    int            q0 = 0;
+#pragma unroll 1
+    for (; q0 + 64 * W <= NT; q0 += 64 * W) {
+      double2 v[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) v[i] = Ms[pl + q0 + 16 * W * i];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 4; i++) Mg[pl + q0 + 16 * W * i] = v[i];
+    }
+    if (q0 < NT) {
+      double2 v[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) v[i] = Ms[min(pl + q0 + 16 * W * i, NT - 1)];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 4; i++) Mg[min(pl + q0 + 16 * W * i, NT - 1)] = v[i];
+    }
+    // same tree: X_t - X_s = r k with r = R0 / 2^l the smaller cell's half-width and k an
+    // integer vector, and Y_n(r k) = r^-(n+1) Y_n(k); offsets inside the table's cube are read
+    // from it and scaled per row, the rest (and other trees) are computed here
+    if (tab.Y) {
+      const int    l  = max(lt, ls);
+      const double sc = ldexp(sinv[0], l);  // 1 / r
+      const double qx = (X - cx) * sc, qy = (Y - cy) * sc, qz = (Z - cz) * sc;
+      const double kx = rint(qx), ky = rint(qy), kz = rint(qz);
+      const double dev = fmax(fabs(qx - kx), fmax(fabs(qy - ky), fabs(qz - kz)));
+      const double km  = fmax(fabs(kx), fmax(fabs(ky), fabs(kz)));
+      if (dev < 1e-6 && km <= M2L_TABLE_K && km > 0.0) {
+        const int      w   = 2 * M2L_TABLE_K + 1;  // |k| <= K: 32-bit index arithmetic is exact
+        const int      idx = ((int)kx + M2L_TABLE_K) * w * w + ((int)ky + M2L_TABLE_K) * w + ((int)kz + M2L_TABLE_K);
+        const double2 *Yk  = tab.Y + (int64_t)idx * (P * P);
+        // indices past the end are clamped to the last entry (its row is in jrow too)
+        for (int e0 = 0, b0 = 0; e0 < P * P; e0 += 64 * W, b0 += 16) {
+          double2 y[4];
+#pragma unroll
+          for (int i = 0; i < 4; i++) y[i] = Yk[min(pl + e0 + 16 * W * i, P * P - 1)];
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            const int    e = min(pl + e0 + 16 * W * i, P * P - 1);
+            const int    J = (int)(jrow >> (b0 + 4 * i)) & 15;
+            const double f = ldexp(sinv[J], l * (J + 1));
+            Yx[e]          = make_double2(y[i].x * f, y[i].y * f);
+          }
+        }
+        return;
+      }
+    }
+    if (pl < P) singular_column_ext(P, pl, sph(X - cx, Y - cy, Z - cz), Yx);
+  }
+};
+
+// The end of a workgroup: the 4 source groups (same slot in lanes sl, sl+16, sl+32, sl+48) are
+// combined, and the pieces of each output added in the plan's order.
+template <int S, int W>
+__device__ __forceinline__ void m2l_store(double2 (&acc)[S][3], int ny, int tid, double2 *sm2,
+                                          const int32_t *__restrict__ out_off, const int32_t *__restrict__ out_src,
+                                          double2 *__restrict__ Lu)
+{
+  const int lane = tid & 63, wv = W == 1 ? 0 : tid >> 6;
+  for (int s = 0; s < S; s++)
+    for (int d = 0; d < 3; d++) {
+      double2 &a = acc[s][d];
+      a.x += __shfl_xor(a.x, 16, 64);
+      a.y += __shfl_xor(a.y, 16, 64);
+      a.x += __shfl_xor(a.x, 32, 64);
+      a.y += __shfl_xor(a.y, 32, 64);
+    }
+  double2 *part = sm2;  // [W][16][S][3]: every wavefront's slots, read by the output loop
+  if (W > 1) m2l_sync<W>();
+  if (lane < 16)
+    for (int s = 0; s < S; s++)
+      for (int d = 0; d < 3; d++) part[((wv * 16 + lane) * S + s) * 3 + d] = acc[s][d];
+  __syncthreads();
+  for (int q = tid; q < ny; q += W * WG) {
+    int j = 0;
+    while (tri(j + 1) <= q) j++;
+    double2 r[3] = {make_double2(0, 0), make_double2(0, 0), make_double2(0, 0)};
+    for (int e = out_off[q]; e < out_off[q + 1]; e++) {
+      const int pc = out_src[e];
+      for (int d = 0; d < 3; d++) {
+        r[d].x += part[pc * 3 + d].x;
+        r[d].y += part[pc * 3 + d].y;
+      }
+    }
+    const double sjk = sgn(j + q - tri(j));  // (-1)^j of the M2L rule, (-1)^k of the folded rows
+    for (int d = 0; d < 3; d++) Lu[3 * q + d] = make_double2(sjk * r[d].x, sjk * r[d].y);
+  }
+}
+
 // SPLIT: the unit of work is a list segment (seg[3u] = target, [seg[3u+1], seg[3u+2]) = list
 // entries), ncell counts segments, and the segment's local expansion goes to L + u * NT;
 // k_m2l_reduce adds the segments of each target in order.
 // With two wavefronts, up to 5 slots are held to 128 VGPRs (4 waves per SIMD, a few bytes of
 // spill at 5); more slots keep their registers.
+#define UVLM_M2L_ARGS                                                                                               \
+  int NT, int64_t ncell, int64_t per_xcd, const int32_t *__restrict__ off, const int32_t *__restrict__ src,         \
+      const double *__restrict__ tx, const double *__restrict__ ty, const double *__restrict__ tz,                  \
+      const double *__restrict__ sx, const double *__restrict__ sy, const double *__restrict__ sz,                  \
+      const double2 *__restrict__ M, double2 *__restrict__ L, const int32_t *__restrict__ slots,                    \
+      const int32_t *__restrict__ lev, const int32_t *__restrict__ out_off, const int32_t *__restrict__ out_src,    \
+      const M2LTable tab, const int32_t *__restrict__ seg
 template <int S, bool SPLIT = false, int W = 1>
 __global__ __launch_bounds__(W * WG) __attribute__((amdgpu_waves_per_eu(W == 2 && S <= 5 ? 4 : 1))) void k_m2l_ns(
-                                               int P, int NT, int64_t ncell, int64_t per_xcd,
-                                               const int32_t *__restrict__ off, const int32_t *__restrict__ src,
-                                               const double *__restrict__ tx, const double *__restrict__ ty,
-                                               const double *__restrict__ tz, const double *__restrict__ sx,
-                                               const double *__restrict__ sy, const double *__restrict__ sz,
-                                               const double2 *__restrict__ M, double2 *__restrict__ L,
-                                               const int32_t *__restrict__ slots, const int32_t *__restrict__ lev,
-                                               const int32_t *__restrict__ out_off,
-                                               const int32_t *__restrict__ out_src, const M2LTable tab,
-                                               const int32_t *__restrict__ seg = nullptr)
+                                               int P, UVLM_M2L_ARGS)
 {
   extern __shared__ double2 sm2[];
   __shared__ double sinv[16];  // R0^-(J+1), J = 0..P-1 (lattice table only)
@@ -1004,46 +1187,15 @@ __global__ __launch_bounds__(W * WG) __attribute__((amdgpu_waves_per_eu(W == 2 &
   const int64_t u = (b & 7) * per_xcd + (b >> 3);
   if (u >= ncell) return;
   const int64_t t = SPLIT ? seg[3 * u] : u;  // target cell; the output row is u
-  // W wavefronts share the staged sources: with W = 2 each takes the source degrees the plan
-  // gives it, with its own 16-lane plan for them, and the output loop adds both wavefronts'
-  // pieces of each output in a fixed order (W = 2 halves the LDS per wavefront, so up to 5
-  // slots run at 4 waves per SIMD); pl numbers the W * 16 lanes of a group for the staging
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, sl = lane & 15;
   const int wv = W == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform in the wavefront
-  const int pl = sl + 16 * wv;
   const int ny = tri(P), per = P * P + NT;
-  auto      sync = [] {
-    if (W == 1) wave_lds_sync();
-    else block_lds_sync();
-  };
   double2  *Yx = sm2 + g * per;  // extended singular rows, P*P entries
   double2  *Mg = Yx + P * P;
   // This wavefront's plan: slots [16][S] and per-degree words [P] (0: a degree of the other).
   const int32_t *wslots = slots + wv * 16 * S, *wlev = lev + wv * P;
-  // Slot s of lane sl, decoded once per workgroup into an int4 of this wavefront's table after
-  // the 4 groups' areas (byte offsets; hi(x) = high word of the double x).  At degree n the
-  // slot adds orders m0 .. m0 + c - 1 of output (j, k), J = j + n, from Ya = Yx[J, m0 - k] and
-  // Yb = Yx[J, m0 + k] = Ya + 32 k, with M[n, m0] = Mn + 48 m0:
-  //  * home slot, output w = 16 s + sl = tri(j) + k, active where w < tri(P - n), m0 = 0,
-  //    c = n + 1: {16 (j(j+1) - k), 16 (2j + 1), 32 k, hi((-1)^k)}, Ya = Yx + x + y n + 16 n^2;
-  //  * helper slot of degree d (a chunk of c = cn orders):
-  //    {16 (J(J+1) - k + m0 - d^2), 48 m0, 32 k, hi((-1)^k)}, Ya = Yx + x + 16 d^2;
-  //    its first step's sign is 0 for m0 = 0 (the step is then the order-0 term, see
-  //    m2l_terms_run);
-  //  * unused helper lane: {0, 0, 0, 0} (a sign word of 0 marks it idle).
   int4 *htab = reinterpret_cast<int4 *>(sm2 + 4 * per) + wv * 16 * S;
-  for (int q = lane; q < 16 * S; q += WG) {
-    const int s = q >> 4, l = q & 15, v = wslots[l * S + s];
-    const int j = v & 31, k = (v >> 5) & 31, m0 = (v >> 10) & 31, d = (v >> 15) & 31;
-    const int hk = (k & 1) ? (int)0xBFF00000 : 0x3FF00000;
-    int4      e  = make_int4(0, 0, 0, 0);
-    if (v >= 0 && d == 31) e = make_int4(16 * (j * (j + 1) - k), 16 * (2 * j + 1), 32 * k, hk);
-    else if (v >= 0) {
-      const int J = j + d;
-      e = make_int4(16 * (J * (J + 1) - k + m0 - d * d), 48 * m0, 32 * k, hk);
-    }
-    htab[q] = e;
-  }
+  for (int q = lane; q < 16 * S; q += WG) htab[q] = m2l_slot(wslots[(q & 15) * S + (q >> 4)]);
   double2 acc[S][3];
   for (int s = 0; s < S; s++)
     for (int d = 0; d < 3; d++) acc[s][d] = make_double2(0, 0);
@@ -1051,97 +1203,17 @@ __global__ __launch_bounds__(W * WG) __attribute__((amdgpu_waves_per_eu(W == 2 &
   for (int n = 0; n < P; n++)
     if (wlev[n]) wdeg |= 1 << n;
   const int    s0 = SPLIT ? seg[3 * u + 1] : off[t], nsrc = (SPLIT ? seg[3 * u + 2] : off[t + 1]) - s0;
-  const double X = tx[t], Yc = ty[t], Z = tz[t];
-  const int    lt = tab.Y ? tab.level[t] : 0;
-  // lattice table only: R0^-(J+1) in sinv, and the row J of each harmonic entry this lane copies,
-  // e = min(pl + 16 W i, P*P - 1) (J*J <= e <= J*J + 2J), 4 bits per entry i
-  using JRows = typename std::conditional<W == 1, uint64_t, uint32_t>::type;
-  JRows jrow = 0;
-  if (tab.Y) {
-    const double inv0 = 1.0 / tab.X0R0[3];
-    if (tid < P) {
-      double q = inv0;
-      for (int i = 0; i < tid; i++) q *= inv0;
-      sinv[tid] = q;
-    }
-    for (int i = 0; i < 2 * (int)sizeof(JRows); i++) {
-      const int e = min(pl + 16 * W * i, P * P - 1);
-      int       J = 0;
-      while ((J + 1) * (J + 1) <= e) J++;
-      jrow |= (JRows)J << (4 * i);
-    }
-    sync();
-  }
+  M2LStage<W>  st;
+  st.init(P, tid, sl + 16 * wv, sinv, tab, tx, ty, tz, t);
   // the next batch's source index is loaded a batch ahead, so its latency overlaps the current
   // batch's multiply-adds; the source's centre and level are loaded with its multipole
   int s_cur = g < nsrc ? src[s0 + g] : 0;
   for (int base = 0; base < nsrc; base += 4) {
     const int  si     = base + g;
     const bool active = si < nsrc;
-    if (active) {
-      const double cx_cur = sx[s_cur], cy_cur = sy[s_cur], cz_cur = sz[s_cur];
-      const int    ls_cur = tab.Y ? tab.level[s_cur] : 0;
-      // four loads in flight per lane before the first LDS store: at immediate offsets from the
-      // lane's first entry while every lane's four entries exist, then with indices past the end
-      // clamped to the last entry, whose owner writes the same value (no branches)
-      const double2 *Ms = M + (int64_t)s_cur * NT;
-      // (the scheduling barriers keep the four loads ahead of the stores)
-      int            q0 = 0;
-#pragma unroll 1
-      for (; q0 + 64 * W <= NT; q0 += 64 * W) {
-        double2 v[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) v[i] = Ms[pl + q0 + 16 * W * i];
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int i = 0; i < 4; i++) Mg[pl + q0 + 16 * W * i] = v[i];
-      }
-      if (q0 < NT) {
-        double2 v[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) v[i] = Ms[min(pl + q0 + 16 * W * i, NT - 1)];
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int i = 0; i < 4; i++) Mg[min(pl + q0 + 16 * W * i, NT - 1)] = v[i];
-      }
-      // same tree: X_t - X_s = r k with r = R0 / 2^l the smaller cell's half-width and k an
-      // integer vector, and Y_n(r k) = r^-(n+1) Y_n(k); offsets inside the table's cube are read
-      // from it and scaled per row, the rest (and other trees) are computed here
-      bool from_table = false;
-      if (tab.Y) {
-        const int    l  = max(lt, ls_cur);
-        const double sc = ldexp(sinv[0], l);  // 1 / r
-        const double qx = (X - cx_cur) * sc, qy = (Yc - cy_cur) * sc, qz = (Z - cz_cur) * sc;
-        const double kx = rint(qx), ky = rint(qy), kz = rint(qz);
-        const double dev = fmax(fabs(qx - kx), fmax(fabs(qy - ky), fabs(qz - kz)));
-        const double km  = fmax(fabs(kx), fmax(fabs(ky), fabs(kz)));
-        if (dev < 1e-6 && km <= M2L_TABLE_K && km > 0.0) {
-          const int      w   = 2 * M2L_TABLE_K + 1;  // |k| <= K: 32-bit index arithmetic is exact
-          const int      idx = ((int)kx + M2L_TABLE_K) * w * w + ((int)ky + M2L_TABLE_K) * w + ((int)kz + M2L_TABLE_K);
-          const double2 *Yk  = tab.Y + (int64_t)idx * (P * P);
-          // indices past the end are clamped to the last entry (its row is in jrow too)
-          for (int e0 = 0, b0 = 0; e0 < P * P; e0 += 64 * W, b0 += 16) {
-            double2 y[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) y[i] = Yk[min(pl + e0 + 16 * W * i, P * P - 1)];
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-              const int    e = min(pl + e0 + 16 * W * i, P * P - 1);
-              const int    J = (int)(jrow >> (b0 + 4 * i)) & 15;
-              const double f = ldexp(sinv[J], l * (J + 1));
-              Yx[e]          = make_double2(y[i].x * f, y[i].y * f);
-            }
-          }
-          from_table = true;
-        }
-      }
-      if (!from_table && pl < P) {
-        const Sph sp = sph(X - cx_cur, Yc - cy_cur, Z - cz_cur);
-        singular_column_ext(P, pl, sp, Yx);
-      }
-    }
+    if (active) st.source(P, NT, s_cur, sx, sy, sz, M, tab, Yx, Mg);
     const int s_next = si + 4 < nsrc ? src[s0 + si + 4] : 0;
-    sync();
+    m2l_sync<W>();
     if (active) {
       for (int dm = wdeg; dm; dm &= dm - 1) {
         const int      n = __builtin_ctz(dm), lv = wlev[n];
@@ -1174,38 +1246,181 @@ __global__ __launch_bounds__(W * WG) __attribute__((amdgpu_waves_per_eu(W == 2 &
         }
       }
     }
-    sync();
+    m2l_sync<W>();
     s_cur = s_next;
   }
-  // combine the 4 source groups (same slot in lanes sl, sl+16, sl+32, sl+48)
-  for (int s = 0; s < S; s++)
-    for (int d = 0; d < 3; d++) {
-      double2 &a = acc[s][d];
-      a.x += __shfl_xor(a.x, 16, 64);
-      a.y += __shfl_xor(a.y, 16, 64);
-      a.x += __shfl_xor(a.x, 32, 64);
-      a.y += __shfl_xor(a.y, 32, 64);
-    }
-  double2 *part = sm2;  // [W][16][S][3]: every wavefront's slots, read by the output loop
-  if (W > 1) sync();
-  if (g == 0)
-    for (int s = 0; s < S; s++)
-      for (int d = 0; d < 3; d++) part[((wv * 16 + sl) * S + s) * 3 + d] = acc[s][d];
-  __syncthreads();
-  for (int q = tid; q < ny; q += W * WG) {
-    int j = 0;
-    while (tri(j + 1) <= q) j++;
-    double2 r[3] = {make_double2(0, 0), make_double2(0, 0), make_double2(0, 0)};
-    for (int e = out_off[q]; e < out_off[q + 1]; e++) {
-      const int pc = out_src[e];
-      for (int d = 0; d < 3; d++) {
-        r[d].x += part[pc * 3 + d].x;
-        r[d].y += part[pc * 3 + d].y;
-      }
-    }
-    const double sjk = sgn(j + q - tri(j));  // (-1)^j of the M2L rule, (-1)^k of the folded rows
-    for (int d = 0; d < 3; d++) L[u * NT + 3 * q + d] = make_double2(sjk * r[d].x, sjk * r[d].y);
+  m2l_store<S, W>(acc, ny, tid, sm2, out_off, out_src, L + u * NT);
+}
+
+// Orders 0..n of a home slot with M[n, K] taken from lane K of the group (v_fmac_f64 with
+// row_newbcast; a group is one row of 16 lanes): the multipole then costs neither an LDS read
+// nor an instruction.  Every lane K <= n of the row has to be active.  The sums are those of
+// m2l_step, per component in the same order.  s_nop 1: the two wait states between a VALU write
+// of a register and its DPP read, should the compiler copy m right before (it does not look
+// into the asm).
+template <int K>
+__device__ __forceinline__ void m2l_fma_row(double2 (&a)[3], const double2 (&m)[3], double2 Sv, double2 Dv)
+{
+#define UVLM_ROW "row_newbcast:%16 row_mask:0xf bank_mask:0xf\n\t"
+  asm("s_nop 1\n\t"
+      "v_fmac_f64_dpp %0, %6, %12 " UVLM_ROW
+      "v_fmac_f64_dpp %1, %6, %13 " UVLM_ROW
+      "v_fmac_f64_dpp %2, %8, %12 " UVLM_ROW
+      "v_fmac_f64_dpp %3, %8, %13 " UVLM_ROW
+      "v_fmac_f64_dpp %4, %10, %12 " UVLM_ROW
+      "v_fmac_f64_dpp %5, %10, %13 " UVLM_ROW
+      "v_fmac_f64_dpp %0, -%7, %15 " UVLM_ROW
+      "v_fmac_f64_dpp %1, %7, %14 " UVLM_ROW
+      "v_fmac_f64_dpp %2, -%9, %15 " UVLM_ROW
+      "v_fmac_f64_dpp %3, %9, %14 " UVLM_ROW
+      "v_fmac_f64_dpp %4, -%11, %15 " UVLM_ROW
+      "v_fmac_f64_dpp %5, %11, %14 " UVLM_ROW
+      : "+&v"(a[0].x), "+&v"(a[0].y), "+&v"(a[1].x), "+&v"(a[1].y), "+&v"(a[2].x), "+&v"(a[2].y)
+      : "v"(m[0].x), "v"(m[0].y), "v"(m[1].x), "v"(m[1].y), "v"(m[2].x), "v"(m[2].y), "v"(Sv.x), "v"(Sv.y),
+        "v"(Dv.x), "v"(Dv.y), "n"(K));
+#undef UVLM_ROW
+}
+
+// Order 0: M[n, 0] is real (M[n, -m] = (-1)^m conj(M[n, m]), the symmetry that folds m and -m).
+__device__ __forceinline__ void m2l_fma_row0(double2 (&a)[3], const double2 (&m)[3], double2 y)
+{
+#define UVLM_ROW "row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
+  asm("s_nop 1\n\t"
+      "v_fmac_f64_dpp %0, %6, %9 " UVLM_ROW
+      "v_fmac_f64_dpp %1, %6, %10 " UVLM_ROW
+      "v_fmac_f64_dpp %2, %7, %9 " UVLM_ROW
+      "v_fmac_f64_dpp %3, %7, %10 " UVLM_ROW
+      "v_fmac_f64_dpp %4, %8, %9 " UVLM_ROW
+      "v_fmac_f64_dpp %5, %8, %10 " UVLM_ROW
+      : "+&v"(a[0].x), "+&v"(a[0].y), "+&v"(a[1].x), "+&v"(a[1].y), "+&v"(a[2].x), "+&v"(a[2].y)
+      : "v"(m[0].x), "v"(m[1].x), "v"(m[2].x), "v"(y.x), "v"(y.y));
+#undef UVLM_ROW
+}
+
+// The batch loop of wavefront WV with the plan's degrees, rounds and chunks as constants: one
+// straight run of code, the LDS offsets of a run immediate.
+template <int P, int WV, int S, int W>
+__device__ __forceinline__ void m2l_fixed_loop(double2 (&acc)[S][3], const M2LStage<W> &st, int s0, int nsrc, int g,
+                                               int sl, const int4 *htab, double2 *Yx, double2 *Mg,
+                                               const int32_t *__restrict__ src, const double *__restrict__ sx,
+                                               const double *__restrict__ sy, const double *__restrict__ sz,
+                                               const double2 *__restrict__ M, const M2LTable &tab)
+{
+  constexpr M2LFixed F = m2l_fixed(P);
+  constexpr int NT = 3 * (P * (P + 1) / 2), H = F.home(WV);
+  // the home slots' addresses (of degree 0) and their steps stay in registers
+  int ya[H], yj[H], yk[H], hk[H];
+  for (int s = 0; s < H; s++) {
+    const int4 e = htab[16 * s + sl];
+    ya[s] = e.x, yj[s] = e.y, yk[s] = e.z, hk[s] = e.w;
   }
+  int s_cur = g < nsrc ? src[s0 + g] : 0;
+  for (int base = 0; base < nsrc; base += 4) {
+    const int  si     = base + g;
+    const bool active = si < nsrc;
+    if (active) st.source(P, NT, s_cur, sx, sy, sz, M, tab, Yx, Mg);
+    const int s_next = si + 4 < nsrc ? src[s0 + si + 4] : 0;
+    m2l_sync<W>();
+    if (active) {
+      // the empty asms make a batch's addresses its own: hoisted out of the loop they would take
+      // some 40 registers
+      int tq = 0, row = sl;
+      asm volatile("" : "+s"(tq), "+v"(row));
+      for (int s = 0; s < H; s++) asm volatile("" : "+v"(ya[s]), "+v"(yj[s]), "+v"(yk[s]), "+v"(hk[s]));
+      const int4 *hl = htab + tq + sl;
+      static_for<P>([&](auto degree) {
+        constexpr int n = decltype(degree)::value, lv = F.lev[WV * P + n];
+        constexpr int cn = lv & 255, hr = (lv >> 8) & 255, used = lv >> 16;
+        constexpr int A = (P - n) * (P - n + 1) / 2, Mo = 3 * (n * (n + 1) / 2);
+        const double2 *Mn = Mg + Mo;
+        double2        mrow[3];  // M[n, sl], sl <= n
+        if constexpr (hr > 0 && m2l_row(A, 0, n)) {
+          const double2 *Mr = Mn + 3 * min(row, n);
+          for (int d = 0; d < 3; d++) mrow[d] = Mr[d];
+        }
+        static_for<S>([&](auto slot) {
+          constexpr int s = decltype(slot)::value;
+          if constexpr (lv != 0 && ((used >> s) & 1) && s < hr) {
+            auto run = [&] {
+              const char    *Y0 = reinterpret_cast<const char *>(Yx) + ya[s] + __umul24(yj[s], n);
+              const double2 *Ya = reinterpret_cast<const double2 *>(Y0) + n * n;
+              const double2 *Yb = reinterpret_cast<const double2 *>(Y0 + yk[s]) + n * n;
+              const double   sk = __hiloint2double(hk[s], 0);
+              if constexpr (m2l_row(A, s, n)) {
+                // one order ahead: more would cost the registers of a wavefront a SIMD
+                double2 va = Ya[0], vb = va;
+                static_for<n + 1>([&](auto order) {
+                  constexpr int m  = decltype(order)::value;
+                  const double2 ca = va, cb = vb;
+                  if constexpr (m < n) va = Ya[m + 1], vb = Yb[m + 1];
+                  __builtin_amdgcn_sched_barrier(0);
+                  if constexpr (m == 0) m2l_fma_row0(acc[s], mrow, ca);
+                  else
+                    m2l_fma_row<m>(acc[s], mrow, make_double2(fma(sk, cb.x, ca.x), fma(-sk, cb.y, ca.y)),
+                                   make_double2(fma(-sk, cb.x, ca.x), fma(sk, cb.y, ca.y)));
+                });
+              } else m2l_terms_run(acc[s], Ya, Yb, Mn, sk, true, sk, n);
+            };
+            if constexpr (A - 16 * s >= 16) run();
+            else if (16 * s + sl < A) run();
+          } else if constexpr (lv != 0 && ((used >> s) & 1)) {
+            const int4 e = hl[16 * s];
+            if (e.w != 0) {
+              const char    *Y0 = reinterpret_cast<const char *>(Yx) + e.x;
+              const double2 *Ya = reinterpret_cast<const double2 *>(Y0) + n * n;
+              const double2 *Yb = reinterpret_cast<const double2 *>(Y0 + e.z) + n * n;
+              const double2 *Mm = reinterpret_cast<const double2 *>(reinterpret_cast<const char *>(Mn) + e.y);
+              m2l_terms_run(acc[s], Ya, Yb, Mm, __hiloint2double(e.w, 0), false, __hiloint2double(e.y ? e.w : 0, 0),
+                            cn - 1);
+            }
+          }
+        });
+      });
+    }
+    m2l_sync<W>();
+    s_cur = s_next;
+  }
+}
+
+// k_m2l_ns for the orders of m2l_fixed under their default plan, as straight code.  k_m2l_ns is
+// bound by LDS reads (83% of its cycles at P = 10: five 16-byte reads an order for 16 FP64
+// instructions) and spends a third of its instructions around the orders.  Here a home slot
+// reads two, and its set-up at a degree is a few instructions; what bounds it is the FP64 rate
+// (about 1150 instructions of a SIMD's four sources, 900 of them the orders).  M2L phase, k_m2l_ns
+// and this: 1M-body cube (P = 10) 5.77 -> 4.12 ms, 1M leapfrog 4.02 -> 3.04, 60001-body cube
+// (P = 14) 5.82 -> 3.56, 260003 bodies (P = 8) 1.68 -> 1.09, 8192-body ring (P = 8) 152 -> 73 us,
+// 100002 bodies (P = 6) 208 -> 124.  Three wavefronts a SIMD: with four (128 registers) P = 10
+// spills in the batch loop, 7.5 ms.  The other orders (odd ones, 2, 16) and other slot budgets
+// take k_m2l_ns.
+template <int P, bool SPLIT>
+__global__ __launch_bounds__(m2l_fixed(P).W * WG) __attribute__((amdgpu_waves_per_eu(m2l_fixed(P).eu))) void k_m2l_fixed(
+    UVLM_M2L_ARGS)
+{
+  constexpr M2LFixed F = m2l_fixed(P);
+  constexpr int      W = F.W, S = F.S, per = P * P + 3 * (P * (P + 1) / 2);
+  extern __shared__ double2 sm2[];
+  __shared__ double sinv[16];  // R0^-(J+1), J = 0..P-1 (lattice table only)
+  const int64_t b = blockIdx.x;
+  const int64_t u = (b & 7) * per_xcd + (b >> 3);
+  if (u >= ncell) return;
+  const int64_t t = SPLIT ? seg[3 * u] : u;  // target cell; the output row is u
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, sl = lane & 15;
+  const int wv = W == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform in the wavefront
+  double2  *Yx = sm2 + g * per, *Mg = Yx + P * P;
+  const int32_t *wslots = slots + wv * 16 * S;
+  int4 *htab = reinterpret_cast<int4 *>(sm2 + 4 * per) + wv * 16 * S;
+  for (int q = lane; q < 16 * S; q += WG) htab[q] = m2l_slot(wslots[(q & 15) * S + (q >> 4)]);
+  wave_lds_sync();
+  const int   s0 = SPLIT ? seg[3 * u + 1] : off[t], nsrc = (SPLIT ? seg[3 * u + 2] : off[t + 1]) - s0;
+  M2LStage<W> st;
+  st.init(P, tid, sl + 16 * wv, sinv, tab, tx, ty, tz, t);
+  double2 acc[S][3];
+  for (int s = 0; s < S; s++)
+    for (int d = 0; d < 3; d++) acc[s][d] = make_double2(0, 0);
+  // (the wavefronts meet at the same number of barriers)
+  if (W == 1 || wv == 0) m2l_fixed_loop<P, 0, S, W>(acc, st, s0, nsrc, g, sl, htab, Yx, Mg, src, sx, sy, sz, M, tab);
+  else m2l_fixed_loop<P, W - 1, S, W>(acc, st, s0, nsrc, g, sl, htab, Yx, Mg, src, sx, sy, sz, M, tab);
+  m2l_store<S, W>(acc, P * (P + 1) / 2, tid, sm2, out_off, out_src, L + u * NT);
 }
 
 // L of each target = the sum of its segments' expansions, in segment order.
@@ -1408,9 +1623,12 @@ __global__ void k_zero(double *p, int64_t n)
 // M2L schedule: the work plan of k_m2l_ns (m2l_plan.hpp) for the handle's slot budget, copied
 // to the device, and the lattice and octant harmonic tables for P.
 // Two wavefronts per workgroup when one wavefront's LDS (16 (P^2 + NT) bytes per staged source,
-// 4 sources) would cap the occupancy below what its registers allow: from P = 9 on (measured:
-// P = 8 is 12% faster with one, P = 10 10% faster with two, P = 12 and 14 a third).
-int m2l_waves(int P, int waves) { return waves == 1 || waves == 2 ? waves : (P <= 8 ? 1 : 2); }
+// 4 sources) would cap the occupancy below what its registers allow: from P = 9 on (k_m2l_ns:
+// P = 8 is 12% faster with one, P = 10 10% faster with two, P = 12 and 14 a third).  k_m2l_fixed
+// runs P = 6 and 8 with two as well: 5 slots there hold what one wavefront needs 6 for, and a
+// target's list is worked off in half the time where targets are few (8192-body ring, P = 8:
+// 73 against 93 us; 260003-body pass 1.09 against 1.13 ms; 100002 at P = 6 124 against 141 us).
+int m2l_waves(int P, int waves) { return waves == 1 || waves == 2 ? waves : (P <= 8 && P != 6 && P != 8 ? 1 : 2); }
 
 // Term table of k_m2m_tab for P <= M2M_TAB_MAXP: per lane (output q = (j,k) = lane, tri(P) <= 64)
 // the counts of its plain and conjugated terms, then RP rows of plain terms and RC rows of
@@ -1504,6 +1722,7 @@ void make_m2l_schedule(int P, M2LSchedule &s)
   const int budget = s.budget > 0 ? s.budget : (s.W == 2 ? 5 : 0);
   if (!make_m2l_plan(P, budget, s.plan, 16, s.W)) throw Error(UVLM_ERR_INTERNAL, "no M2L plan");
   const M2LPlan &pl = s.plan;
+  s.fixed           = m2l_plan_fixed(pl);
   s.dev_slots       = 0;
   s.dev_lev         = pl.slots.size();
   s.dev_out_off     = s.dev_lev + pl.lev.size();
@@ -1697,17 +1916,30 @@ void m2l(hipStream_t s, int P, const Tree &tt, const Tree &st, const Lists &l, c
     M2LTable tab{};
     if (&tt == &st && sch.ytab_P == P)
       tab = M2LTable{sch.ytab.as<double2>(), tt.level.as<int32_t>(), tt.X0R0.as<double>()};
-#define UVLM_M2L_LAUNCH(SS, WW)                                                                              \
-  if (split)                                                                                               \
-    k_m2l_ns<SS, true, WW><<<grid, WW * WG, lds_ns, s>>>(                                                  \
-        P, NT, units, per_xcd, l.m2l_off.as<int32_t>(), l.m2l_src.as<int32_t>(), tt.cx.as<double>(),       \
-        tt.cy.as<double>(), tt.cz.as<double>(), st.cx.as<double>(), st.cy.as<double>(), st.cz.as<double>(), M, \
-        out, d + sch.dev_slots, d + sch.dev_lev, d + sch.dev_out_off, d + sch.dev_out_src, tab, dseg);    \
-  else                                                                                                     \
-    k_m2l_ns<SS, false, WW><<<grid, WW * WG, lds_ns, s>>>(                                                 \
-        P, NT, tt.C, per_xcd, l.m2l_off.as<int32_t>(), l.m2l_src.as<int32_t>(), tt.cx.as<double>(),        \
-        tt.cy.as<double>(), tt.cz.as<double>(), st.cx.as<double>(), st.cy.as<double>(), st.cz.as<double>(), M, \
-        L, d + sch.dev_slots, d + sch.dev_lev, d + sch.dev_out_off, d + sch.dev_out_src, tab);
+#define UVLM_M2L_CALL_ARGS                                                                                     \
+  NT, units, per_xcd, l.m2l_off.as<int32_t>(), l.m2l_src.as<int32_t>(), tt.cx.as<double>(), tt.cy.as<double>(),  \
+      tt.cz.as<double>(), st.cx.as<double>(), st.cy.as<double>(), st.cz.as<double>(), M, out, d + sch.dev_slots, \
+      d + sch.dev_lev, d + sch.dev_out_off, d + sch.dev_out_src, tab, dseg
+#define UVLM_M2L_LAUNCH(SS, WW)                                                                                  \
+  if (split) k_m2l_ns<SS, true, WW><<<grid, WW * WG, lds_ns, s>>>(P, UVLM_M2L_CALL_ARGS);                         \
+  else k_m2l_ns<SS, false, WW><<<grid, WW * WG, lds_ns, s>>>(P, UVLM_M2L_CALL_ARGS);
+#define UVLM_M2L_FIXED(PP)                                                                                       \
+  if (sch.fixed && P == PP) {                                                                                    \
+    if (split) k_m2l_fixed<PP, true><<<grid, m2l_fixed(PP).W * WG, lds_ns, s>>>(UVLM_M2L_CALL_ARGS);              \
+    else k_m2l_fixed<PP, false><<<grid, m2l_fixed(PP).W * WG, lds_ns, s>>>(UVLM_M2L_CALL_ARGS);                   \
+    UVLM_LAUNCH_CHECK();                                                                                         \
+    if (split) {                                                                                                 \
+      k_m2l_reduce<<<(int)tt.C, WG, 0, s>>>(NT, tt.C, dsegoff, out, L);                                          \
+      UVLM_LAUNCH_CHECK();                                                                                       \
+    }                                                                                                            \
+    return;                                                                                                      \
+  }
+    UVLM_M2L_FIXED(4)
+    UVLM_M2L_FIXED(6)
+    UVLM_M2L_FIXED(8)
+    UVLM_M2L_FIXED(10)
+    UVLM_M2L_FIXED(12)
+    UVLM_M2L_FIXED(14)
 #define UVLM_M2L_NS(SS)                                                                                    \
   if (S == SS) {                                                                                           \
     if (W == 2) {                                                                                          \
@@ -1729,6 +1961,9 @@ void m2l(hipStream_t s, int P, const Tree &tt, const Tree &st, const Lists &l, c
     UVLM_M2L_NS(12)
     UVLM_M2L_NS(16)
 #undef UVLM_M2L_NS
+#undef UVLM_M2L_FIXED
+#undef UVLM_M2L_LAUNCH
+#undef UVLM_M2L_CALL_ARGS
 #undef UVLM_M2L_LAUNCH
     throw Error(UVLM_ERR_INTERNAL, "unsupported M2L plan size");
   }

@@ -178,4 +178,50 @@ inline bool make_m2l_plan(int P, int budget, M2LPlan &pl, int G = 16, int W = 1)
   return true;
 }
 
+// The words `lev` of the plans that k_m2l_fixed is compiled for: those that make_m2l_plan gives
+// for an order's default budget and wavefronts (tests/cpp/m2l_fixed_check.cpp compares them);
+// S = 0 for the other orders.  eu: wavefronts per SIMD that the registers are held to.
+struct M2LFixed {
+  int P = 0, S = 0, W = 1, eu = 1;
+  int lev[32] = {};
+  // home slots of wavefront w
+  constexpr int home(int w) const
+  {
+    int h = 1;
+    for (int n = 0; n < P; n++)
+      if (((lev[w * P + n] >> 8) & 255) > h) h = (lev[w * P + n] >> 8) & 255;
+    return h;
+  }
+};
+constexpr M2LFixed m2l_fixed(int P)
+{
+  switch (P) {
+  case 4: return {4, 6, 1, 3, {0x10101, 0x20001, 0x40001, 0x80001}};
+  case 6: return {6, 5, 2, 3, {0x30201, 0x10102, 0, 0, 0x40001, 0,
+                               0, 0, 0x10103, 0x20002, 0, 0x40001}};
+  case 8: return {8, 5, 2, 3, {0x70301, 0x30202, 0, 0, 0x10105, 0x80003, 0, 0,
+                               0, 0, 0x50101, 0x10104, 0, 0, 0x10107, 0x80001}};
+  case 10: return {10, 5, 2, 3, {0xf0401, 0x70302, 0x130201, 0, 0x30205, 0, 0, 0, 0, 0,
+                                 0, 0, 0, 0x30204, 0, 0x10106, 0x10107, 0x40004, 0x80003, 0x100001}};
+  case 12: return {12, 5, 2, 3, {0x1f0501, 0x1f0502, 0xf0403, 0x70304, 0x70305, 0, 0, 0, 0, 0, 0, 0,
+                                 0, 0, 0, 0, 0, 0x30206, 0x30207, 0x10108, 0x10109, 0x40005, 0x1010b, 0x80001}};
+  case 14: return {14, 8, 2, 2, {0x7f0701, 0x3f0602, 0x1f0503, 0x1f0504, 0, 0, 0x70307, 0, 0, 0, 0, 0, 0x1010d, 0,
+                                 0, 0, 0, 0, 0xf0405, 0x70306, 0, 0x30208, 0x110103, 0x1010a, 0x1010b, 0x200006,
+                                 0, 0x400001}};
+  default: return {};
+  }
+}
+// Home slot s at degree n (A = tri(P - n) active outputs) can take M[n, m] from the registers of
+// its lanes m = 0..n: all of them are active in the slot.
+constexpr bool m2l_row(int A, int s, int n) { return A - 16 * s > n; }
+// whether a plan is that one
+inline bool m2l_plan_fixed(const M2LPlan &pl)
+{
+  const M2LFixed f = m2l_fixed(pl.P);
+  if (!f.S || pl.S != f.S || pl.W != f.W || pl.G != 16) return false;
+  for (int i = 0; i < pl.W * pl.P; i++)
+    if (pl.lev[i] != f.lev[i]) return false;
+  return true;
+}
+
 }  // namespace uvlm
