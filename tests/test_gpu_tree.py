@@ -117,3 +117,17 @@ def test_long_rows(orc, n, m, ncrit):
     assert np.array_equal(ga, ga2) and np.array_equal(gx, gx2) and np.isfinite(ga).all()
     g.close()
     h.close()
+
+
+@pytest.mark.parametrize("n,ncrit", [(1, 1), (2, 1), (9, 1), (9, 8), (70, 1), (600, 3), (600, 40)])
+@pytest.mark.parametrize("capacity", [None, "1"])
+def test_first_steps(orc, monkeypatch, n, ncrit, capacity):
+    """Traversals that end within, at and after the steps that one workgroup takes, and with
+    buffers that overflow in them."""
+    if capacity:
+        monkeypatch.setenv("UVLM_LIST_CAPACITY", capacity)
+    print(f"[first] n={n} ncrit={ncrit} capacity={capacity}", flush=True)
+    g = FMMCalculator(P=4, theta=0.5, ncrit=ncrit)
+    for seed in (n, n + 1):
+        check(g, orc, points(n, seed, 0.5, 0), ncrit)
+    g.close()

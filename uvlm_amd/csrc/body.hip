@@ -18,14 +18,16 @@ inline int    nblocks(int64_t n) { return (int)std::max<int64_t>(1, (n + BLK - 1
 // Records of nf doubles (every `stride` doubles) <-> nf field arrays, TB bodies per workgroup through
 // LDS, so that both sides are read and written in consecutive lanes.  Bound by HBM.  A lane per body
 // walking its record (296 bytes apart) moved the 37 fields of 4M bodies in 1.55 ms (1.6 TB/s).
-// Bodies n .. m - 1 get zero fields.
+// Bodies n .. m - 1 get zero fields.  index (or null) gets the bodies' numbers 0 .. m - 1.
 constexpr int TB = 64, MAX_RECORD = N_FIELDS;
 __global__ __launch_bounds__(BLK) void k_records_in(const double *__restrict__ aos, int64_t n, int64_t m, int nf,
-                                                    int64_t stride, double *__restrict__ f0, int64_t cap)
+                                                    int64_t stride, double *__restrict__ f0, int64_t cap,
+                                                    int32_t *__restrict__ index)
 {
   __shared__ double v[TB * MAX_RECORD];
   const int64_t     i0 = blockIdx.x * (int64_t)TB;
   const int         nb = (int)min((int64_t)TB, m - i0), nin = (int)max((int64_t)0, min((int64_t)TB, n - i0));
+  if (index && (int)threadIdx.x < nb) index[i0 + threadIdx.x] = (int32_t)(i0 + threadIdx.x);
   if (stride == nf)
     for (int k = threadIdx.x; k < nin * nf; k += BLK) v[k] = aos[i0 * nf + k];
   else
@@ -316,11 +318,11 @@ void rbf_vec(hipStream_t s, double *st, int64_t cap, int64_t N, int mode, const 
 }
 
 void records_in(hipStream_t s, const double *aos, int64_t n, int64_t m, int nf, int64_t stride, double *fields,
-                int64_t cap)
+                int64_t cap, int32_t *index)
 {
   if (m <= 0) return;
   if (nf > MAX_RECORD) throw Error(UVLM_ERR_INTERNAL, "record width");
-  k_records_in<<<(int)((m + TB - 1) / TB), BLK, 0, s>>>(aos, n, m, nf, stride, fields, cap);
+  k_records_in<<<(int)((m + TB - 1) / TB), BLK, 0, s>>>(aos, n, m, nf, stride, fields, cap, index);
   UVLM_LAUNCH_CHECK();
 }
 
@@ -332,9 +334,10 @@ void records_out(hipStream_t s, const double *fields, int64_t cap, int64_t n, in
   UVLM_LAUNCH_CHECK();
 }
 
-void aos_to_soa(hipStream_t s, const void *aos, int64_t n, int64_t stride_doubles, double *st, int64_t cap)
+void aos_to_soa(hipStream_t s, const void *aos, int64_t n, int64_t stride_doubles, double *st, int64_t cap,
+                int32_t *index)
 {
-  records_in(s, (const double *)aos, n, n, N_FIELDS, stride_doubles, st, cap);
+  records_in(s, (const double *)aos, n, n, N_FIELDS, stride_doubles, st, cap, index);
 }
 
 void soa_to_aos(hipStream_t s, const double *st, int64_t cap, void *aos, int64_t n, int64_t stride_doubles)

@@ -807,8 +807,7 @@ int uvlm_set_bodies_aos(uvlm_handle h, const void *bodies, int64_t n, int64_t st
     h->ensure_cap(n);
     h->staging.reserve((size_t)n * stride);
     UVLM_HIP(hipMemcpyAsync(h->staging.p, bodies, (size_t)n * stride, hipMemcpyHostToDevice, h->s));
-    aos_to_soa(h->s, h->staging.p, n, stride / 8, h->st.as<double>(), h->cap);
-    iota(h->s, h->orig.as<int32_t>(), n);
+    aos_to_soa(h->s, h->staging.p, n, stride / 8, h->st.as<double>(), h->cap, h->orig.as<int32_t>());
     UVLM_HIP(hipStreamSynchronize(h->s));
     h->built = h->evaluated = false;
   });

@@ -190,7 +190,7 @@ void l2p_stretch(hipStream_t s, int P, const Tree &t, const double2 *L, double *
 // near.hip
 // np2p: the list's size, on the device
 void near_units_enqueue(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &st, int64_t max_leaf,
-                        const unsigned long long *np2p, Lists &l);
+                        const unsigned long long *np2p, bool cleared, Lists &l);
 void near_units_set(const unsigned long long *counters, Lists &l);
 void p2p(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &stree, const Lists &l, const double *tgt, int64_t tcap,
          const double *src, int64_t scap, double *out, int64_t ocap, int precision, int sensor_mode);
@@ -280,9 +280,10 @@ void probe_velocity_grad_out(hipStream_t s, int64_t m, const int32_t *perm, cons
 // body.hip
 // n records of nf doubles (every stride doubles) into nf fields, bodies n .. m - 1 zero; and back
 void records_in(hipStream_t s, const double *aos, int64_t n, int64_t m, int nf, int64_t stride, double *fields,
-                int64_t cap);
+                int64_t cap, int32_t *index = nullptr);
 void records_out(hipStream_t s, const double *fields, int64_t cap, int64_t n, int nf, int64_t stride, double *aos);
-void aos_to_soa(hipStream_t s, const void *aos, int64_t n, int64_t stride_doubles, double *st, int64_t cap);
+void aos_to_soa(hipStream_t s, const void *aos, int64_t n, int64_t stride_doubles, double *st, int64_t cap,
+                int32_t *index = nullptr);
 void soa_to_aos(hipStream_t s, const double *st, int64_t cap, void *aos, int64_t n, int64_t stride_doubles);
 void rk_stage(hipStream_t s, double *st, int64_t cap, int64_t N, int scheme, int stage, double dt, int store_initial);
 void reset_sensor_rates(hipStream_t s, double *st, int64_t cap, int64_t N);

@@ -659,9 +659,9 @@ __global__ __launch_bounds__(256) void k_gauss_reduce(const int4 *__restrict__ m
 }
 
 // Units of the P2P list `l` (np2p entries, on the device) of target tree tt against source tree st
-// (see k_units_work), and the number of near-field interactions.
+// (see k_units_work), and the number of near-field interactions.  cleared: the units' counters are zero.
 void near_units_enqueue(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &st, int64_t max_leaf,
-                        const unsigned long long *np2p, Lists &l)
+                        const unsigned long long *np2p, bool cleared, Lists &l)
 {
   if (tt.nleaf == 0) return;
   sc.unit_work.reserve(4 * tt.nleaf);
@@ -671,7 +671,7 @@ void near_units_enqueue(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &
   l.multi.reserve(sizeof(int4) * std::min<int64_t>(tt.nleaf, UNITS_AIM));
   const int32_t *lv = tt.leaves.as<int32_t>(), *tn = tt.nbody.as<int32_t>();
   const int32_t *off = l.p2p_off.as<int32_t>();
-  k_units_clear<<<1, 64, 0, s>>>(cnt);
+  if (!cleared) k_units_clear<<<1, 64, 0, s>>>(cnt);
   k_units_work<<<(int)std::min<int64_t>(UNITS_WORK_BLOCKS, (tt.nleaf + 3) / 4), 256, 0, s>>>(
       lv, tt.nleaf, max_leaf, np2p, tn, off, l.p2p_src.as<int32_t>(), st.nbody.as<int32_t>(),
       sc.unit_work.as<uint32_t>(), cnt);

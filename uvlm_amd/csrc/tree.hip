@@ -73,9 +73,15 @@ __global__ void k_bounds_partial(const double *__restrict__ x, const double *__r
 
 // X0 and R0 exactly as tree.hpp:19-25 computes them from Xmin/Xmax (one workgroup of BLK;
 // min and max are exact in any order, so the parallel reduction gives the serial result).
-__global__ __launch_bounds__(BLK) void k_bounds_final(const double *part, int nb, double *X0R0)
+// Totals of a build (32-bit): cells per level, leaves per level, error bits (0: deeper than the key holds;
+// 1: a split needs a digit below the sorted ones).
+enum { TOT_LEVEL = 0, TOT_LEAVES = 24, TOT_ERR = 47, TOT_COUNT = 48 };
+static_assert(4 * TOT_COUNT <= 8 * N_COUNTERS, "build totals");
+
+__global__ __launch_bounds__(BLK) void k_bounds_final(const double *part, int nb, double *X0R0, uint32_t *tot)
 {
   __shared__ double s[6][BLK];
+  if (threadIdx.x < TOT_COUNT) tot[threadIdx.x] = 0;  // the build's totals
   double mn[3] = {INFINITY, INFINITY, INFINITY}, mx[3] = {-INFINITY, -INFINITY, -INFINITY};
   for (int b = threadIdx.x; b < nb; b += BLK)
     for (int d = 0; d < 3; d++) {
@@ -144,10 +150,6 @@ __device__ __forceinline__ int common_digits(uint64_t a, uint64_t b, int dlim)
   return min(dlim, x ? (__clzll((long long)x) - 1) / 3 : KEY_LEVELS);
 }
 
-// Totals of a build (32-bit): cells per level, leaves per level, error bits (0: deeper than the key holds;
-// 1: a split needs a digit below the sorted ones).
-enum { TOT_LEVEL = 0, TOT_LEAVES = 24, TOT_ERR = 47, TOT_COUNT = 48 };
-static_assert(4 * TOT_COUNT <= 8 * N_COUNTERS, "build totals");
 __global__ void k_zero_u32(int64_t n, uint32_t *__restrict__ p)
 {
   const int64_t i = blockIdx.x * (int64_t)BLK + threadIdx.x;
@@ -519,18 +521,91 @@ __global__ __launch_bounds__(BLK) void k_traverse(const int2 *__restrict__ ft, T
   }
 }
 
-// Start of a traversal: the root pair (0, 0) is the first frontier, or, when both roots are leaves,
-// the single P2P pair (traverse.hpp:41-44); the counters are cleared.
-__global__ void k_traverse_start(TreeView T, TreeView S, int2 *__restrict__ front, uint2 *__restrict__ p2p,
-                                 unsigned long long *__restrict__ c)
+// The first `steps` (at most FIRST_STEPS) steps of a traversal in block 0, the frontier in LDS: the
+// root pair (0, 0) is the first one, or, when both roots are leaves, the single P2P pair
+// (traverse.hpp:41-44).  They hold 1, 8, 64 and 512 pairs at most, a launch each that cost 10 us
+// mostly of launch and atomics (8192-body ring: 5 launches, 47 us with the gaps; here 15).  Clears the
+// counters, the near-field units' too; the other blocks clear the nrows row counts.
+constexpr int FIRST_STEPS = 4, FIRST_PAIRS = 512, FIRST_LANES = 1024;
+static_assert(FIRST_PAIRS == 1 << 3 * (FIRST_STEPS - 1), "frontier of the last first step");
+__global__ __launch_bounds__(FIRST_LANES) void k_traverse_first(TreeView T, TreeView S, double theta, double gap,
+                                                                int steps, int2 *__restrict__ nxt, int64_t cap_f,
+                                                                uint2 *__restrict__ p2p, int64_t cap_p,
+                                                                uint2 *__restrict__ m2l, int64_t cap_m,
+                                                                unsigned long long *__restrict__ cnt,
+                                                                uint32_t *__restrict__ rows, int64_t nrows)
 {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  const bool leaves = T.nchild[0] == 0 && S.nchild[0] == 0;
-  if (leaves) p2p[0] = make_uint2(0, 0);
-  front[0] = make_int2(0, 0);
-  for (int k = 0; k < TC_COUNT; k++) c[k] = 0;
-  c[TC_P2P]   = leaves ? 1 : 0;
-  c[TC_FRONT] = leaves ? 0 : 1;
+  const int tid = threadIdx.x;
+  if (blockIdx.x > 0) {
+    for (int64_t i = (blockIdx.x - 1) * (int64_t)FIRST_LANES + tid; i < nrows; i += (gridDim.x - 1) * (int64_t)FIRST_LANES)
+      rows[i] = 0;
+    return;
+  }
+  constexpr int       WAVES = FIRST_LANES / 64;
+  __shared__ int2     fr[2][FIRST_PAIRS];
+  __shared__ unsigned tot[WAVES][3];
+  const int           lane = tid & 63, wv = tid >> 6, ch = tid & 7;
+  const bool          leaves = T.nchild[0] == 0 && S.nchild[0] == 0;
+  if (leaves && tid == 0) p2p[0] = make_uint2(0, 0);
+  if (tid == 0) fr[0][0] = make_int2(0, 0);
+  unsigned n = leaves ? 0 : 1, most = n;
+  unsigned base[3] = {0, leaves ? 1u : 0u, 0};  // pushed, P2P, M2L so far
+  __syncthreads();
+  for (int st = 0; st < steps; st++) {
+    const bool last = st == steps - 1;
+    base[0]         = 0;
+    for (unsigned b0 = 0; b0 < n; b0 += FIRST_LANES / 8) {
+      const unsigned i = b0 + (tid >> 3);
+      const int2     pr = fr[st & 1][min(i, n - 1)];
+      int            a = pr.x, b = pr.y;
+      const int      nct = T.nchild[a], ncs = S.nchild[b];
+      const bool     split_t = ncs == 0 || (T.R[a] >= S.R[b] && nct != 0);
+      const bool     on = ch < (split_t ? nct : ncs) && i < n;
+      if (on && split_t) a = T.child[a] + ch;
+      if (on && !split_t) b = S.child[b] + ch;
+      int cls = 3;  // 0 push, 1 P2P, 2 M2L, 3 none (k_traverse)
+      if (on) {
+        const double dx = T.cx[a] - S.cx[b], dy = T.cy[a] - S.cy[b], dz = T.cz[a] - S.cz[b];
+        const double D2 = dx * dx + dy * dy + dz * dz, R2 = D2 * theta * theta;
+        const double Rs = T.R[a] + S.R[b];
+        const double Gs = gap + 1.7320508075688772 * Rs;
+        cls = R2 < Rs * Rs || (gap > 0.0 && D2 < Gs * Gs) ? (T.nchild[a] == 0 && S.nchild[b] == 0 ? 1 : 0) : 2;
+      }
+      unsigned long long m[3];
+      for (int k = 0; k < 3; k++) m[k] = __ballot(cls == k);
+      if (lane == 0)
+        for (int k = 0; k < 3; k++) tot[wv][k] = (unsigned)__popcll(m[k]);
+      __syncthreads();
+      unsigned at[3];
+      for (int k = 0; k < 3; k++) {
+        at[k] = base[k] + (unsigned)__popcll(m[k] & ((1ull << lane) - 1));
+        for (int w = 0; w < WAVES; w++) {
+          if (w < wv) at[k] += tot[w][k];
+          base[k] += tot[w][k];
+        }
+      }
+      if (cls == 0) {
+        if (!last) fr[(st + 1) & 1][at[0]] = make_int2(a, b);
+        else if (at[0] < cap_f) nxt[at[0]] = make_int2(a, b);
+      } else if (cls == 1) {
+        if (at[1] < cap_p) p2p[at[1]] = make_uint2((unsigned)b, (unsigned)a);
+      } else if (cls == 2 && at[2] < cap_m) m2l[at[2]] = make_uint2((unsigned)b, (unsigned)a);
+      __syncthreads();
+    }
+    n    = base[0];
+    most = max(most, n);
+  }
+  if (tid >= N_COUNTERS) return;
+  unsigned long long v = 0;
+  if (tid == TC_P2P) v = base[1];
+  if (tid == TC_M2L) v = base[2];
+  if (tid == TC_MAXF) v = most;
+  if (tid == TC_FRONT + (steps & 3)) v = n;
+  if (steps == 0 && tid == TC_FRONT && !leaves) {  // no step here: the root pair is the frontier
+    nxt[0] = make_int2(0, 0);
+    v      = 1;
+  }
+  cnt[tid] = v;
 }
 
 // ---- lists to CSR ---------------------------------------------------------------
@@ -560,6 +635,48 @@ __global__ void k_row_count(int64_t C, unsigned long long *cnt, int64_t cap_p, i
     const uint32_t q = atomicAdd(&rows[(i < n0 ? 0 : C + 1) + t], 1u);
     place[i]         = q;
     if (q >= ROW_LONG) atomicOr(&cnt[TC_FLAGS], (unsigned long long)TF_LONG);
+  }
+}
+
+// The same for few rows: a block counts its pairs in LDS and reserves each row's places at once.  The
+// atomics on memory are then one a block and row, where every pair's atomic on a few hundred rows is
+// serialised there (200003 bodies, 4096 probes: k_row_count 121 us, here 7; 8192-body ring, some
+// thousand rows less contended: 11.4 and 7.1).  ROWS_LDS rows clear and flush in 8 steps a lane for
+// the ROW_ITEMS pairs it counts; more rows would cost more than the pairs.
+constexpr int ROWS_LDS = 2048, ROW_ITEMS = 8, ROW_CHUNK = BLK * ROW_ITEMS;
+__global__ __launch_bounds__(BLK) void k_row_count_lds(int64_t C, unsigned long long *cnt, int64_t cap_p,
+                                                       int64_t cap_m, const uint2 *__restrict__ p2p,
+                                                       const uint2 *__restrict__ m2l, uint32_t *__restrict__ rows,
+                                                       uint32_t *__restrict__ place)
+{
+  __shared__ uint32_t h[ROWS_LDS];
+  const int64_t       n0 = min((int64_t)cnt[TC_P2P], cap_p), n1 = min((int64_t)cnt[TC_M2L], cap_m);
+  const int           nr = (int)(2 * (C + 1));
+  for (int64_t c0 = blockIdx.x * (int64_t)ROW_CHUNK; c0 < n0 + n1; c0 += gridDim.x * (int64_t)ROW_CHUNK) {
+    for (int r = threadIdx.x; r < nr; r += BLK) h[r] = 0;
+    __syncthreads();
+    int      row[ROW_ITEMS];
+    uint32_t q[ROW_ITEMS];
+#pragma unroll
+    for (int k = 0; k < ROW_ITEMS; k++) {
+      const int64_t i = c0 + k * BLK + threadIdx.x;
+      row[k]          = i < n0 ? (int)p2p[i].y : i < n0 + n1 ? (int)(C + 1 + m2l[i - n0].y) : -1;
+    }
+#pragma unroll
+    for (int k = 0; k < ROW_ITEMS; k++) q[k] = row[k] >= 0 ? atomicAdd(&h[row[k]], 1u) : 0;
+    __syncthreads();
+    for (int r = threadIdx.x; r < nr; r += BLK) {
+      const uint32_t n = h[r];
+      if (n == 0) continue;
+      const uint32_t at = atomicAdd(&rows[r], n);
+      h[r]              = at;
+      if (at + n > (uint32_t)ROW_LONG) atomicOr(&cnt[TC_FLAGS], (unsigned long long)TF_LONG);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < ROW_ITEMS; k++)
+      if (row[k] >= 0) place[c0 + k * BLK + threadIdx.x] = h[row[k]] + q[k];
+    __syncthreads();
   }
 }
 
@@ -675,16 +792,14 @@ __global__ __launch_bounds__(BLK) void k_transpose_pairs(int64_t Ct, const int32
                                                          const int32_t *__restrict__ off_m,
                                                          const int32_t *__restrict__ src_m,
                                                          uint2 *__restrict__ pairs_p, uint2 *__restrict__ pairs_m,
-                                                         unsigned long long *__restrict__ cnt)
+                                                         unsigned long long *__restrict__ cnt,
+                                                         uint32_t *__restrict__ rows, int64_t nrows)
 {
+  for (int64_t i = blockIdx.x * (int64_t)BLK + threadIdx.x; i < nrows; i += gridDim.x * (int64_t)BLK) rows[i] = 0;
   const int64_t r = blockIdx.x * (int64_t)(BLK / 64) + (threadIdx.x >> 6);
   const int     lane = threadIdx.x & 63;
-  if (r == 0 && lane == 0) {
-    cnt[TC_P2P]   = (unsigned long long)n0;
-    cnt[TC_M2L]   = (unsigned long long)off_m[Ct];
-    cnt[TC_FLAGS] = 0;
-    cnt[TC_LONG]  = 0;
-  }
+  if (r == 0 && lane < N_COUNTERS)
+    cnt[lane] = lane == TC_P2P ? (unsigned long long)n0 : lane == TC_M2L ? (unsigned long long)off_m[Ct] : 0;
   if (r >= 2 * Ct) return;
   const bool     near = r < Ct;
   const int64_t  t    = near ? r : r - Ct;
@@ -769,7 +884,9 @@ void build_tree(hipStream_t s, Scratch &sc, const double *x, const double *y, co
   sc.partial.reserve(sizeof(double) * 6 * nb);
   tree.X0R0.reserve(sizeof(double) * 4);
   k_bounds_partial<<<nb, BLK, 0, s>>>(x, y, z, N, sc.partial.as<double>());
-  k_bounds_final<<<1, BLK, 0, s>>>(sc.partial.as<double>(), nb, tree.X0R0.as<double>());
+  sc.counters.reserve(8 * N_COUNTERS);
+  uint32_t *tot = sc.counters.as<uint32_t>();
+  k_bounds_final<<<1, BLK, 0, s>>>(sc.partial.as<double>(), nb, tree.X0R0.as<double>(), tot);
   UVLM_LAUNCH_CHECK();
   // 2-3. keys and stable sort
   sc.keys0.reserve(8 * N);
@@ -780,14 +897,11 @@ void build_tree(hipStream_t s, Scratch &sc, const double *x, const double *y, co
   const uint32_t *idx  = sc.idx1.as<uint32_t>();
   uint32_t       *info = sc.idx0.as<uint32_t>();  // free once sorted
   int32_t        *scan = sc.keys0.as<int32_t>();
-  sc.counters.reserve(8 * N_COUNTERS);
-  uint32_t *tot  = sc.counters.as<uint32_t>();
-  int       dlim = std::min(KEY_LEVELS, std::max(1, tree.sort_digits));
+  int            dlim = std::min(KEY_LEVELS, std::max(1, tree.sort_digits));
   uint32_t  h[TOT_COUNT];
   for (;;) {
     k_keys<<<nblocks(N), BLK, 0, s>>>(x, y, z, N, tree.X0R0.as<double>(), sc.keys0.as<uint64_t>(),
                                        sc.idx0.as<uint32_t>());
-    k_zero_u32<<<1, BLK, 0, s>>>(TOT_COUNT, tot);
     UVLM_LAUNCH_CHECK();
     // stable sort of (key, index) on the top dlim digits
     size_t    bytes = 0;
@@ -807,6 +921,7 @@ void build_tree(hipStream_t s, Scratch &sc, const double *x, const double *y, co
     if (h[TOT_ERR] & 1) throw Error(UVLM_ERR_DEPTH, "more than ncrit coincident bodies: octree deeper than 21 levels");
     if (!(h[TOT_ERR] & 2)) break;
     dlim = KEY_LEVELS;  // a cell splits below the sorted digits: all of them, again from the keys
+    k_zero_u32<<<1, BLK, 0, s>>>(TOT_COUNT, tot);
   }
   LevelOffsets         lo{};
   std::vector<int64_t> off{0};
@@ -928,7 +1043,9 @@ static TreeView view(const Tree &t)
 
 // CSR rows by target of the np P2P and nm M2L pairs in sc.out_p2p / out_m2l (their numbers are read
 // on the device; np and nm bound them).  C target cells, entries below Cs.
-static void rows_by_counting(hipStream_t s, Scratch &sc, int64_t C, int64_t np, int64_t nm, Lists &l)
+// C target cells, Cs source cells; zeroed: the caller has cleared the row counts.
+static void rows_by_counting(hipStream_t s, Scratch &sc, int64_t C, int64_t Cs, int64_t np, int64_t nm, bool zeroed,
+                             Lists &l)
 {
   unsigned long long *cnt = sc.counters.as<unsigned long long>();
   l.p2p_off.reserve(4 * (C + 1));
@@ -942,15 +1059,18 @@ static void rows_by_counting(hipStream_t s, Scratch &sc, int64_t C, int64_t np, 
   uint32_t    *rows = sc.row_cnt.as<uint32_t>(), *ro = sc.row_off.as<uint32_t>(), *pl = sc.row_place.as<uint32_t>();
   const uint2 *p2p = sc.out_p2p.as<uint2>(), *m2l = sc.out_m2l.as<uint2>();
   const int    grid = (int)std::min<int64_t>(4096, nblocks(std::max<int64_t>(np + nm, C + 1)));
-  k_zero_u32<<<nblocks(2 * (C + 1)), BLK, 0, s>>>(2 * (C + 1), rows);
-  k_row_count<<<grid, BLK, 0, s>>>(C, cnt, np, nm, p2p, m2l, rows, pl);
+  if (!zeroed) k_zero_u32<<<nblocks(2 * (C + 1)), BLK, 0, s>>>(2 * (C + 1), rows);
+  if (2 * (C + 1) <= ROWS_LDS)
+    k_row_count_lds<<<(int)std::min<int64_t>(4096, (np + nm) / ROW_CHUNK + 1), BLK, 0, s>>>(
+        C, cnt, np, nm, p2p, m2l, rows, pl);
+  else k_row_count<<<grid, BLK, 0, s>>>(C, cnt, np, nm, p2p, m2l, rows, pl);
   excl_scan(s, sc, rows, ro, 2 * (C + 1));
   k_row_fill<<<grid, BLK, 0, s>>>(C, cnt, np, nm, p2p, m2l, ro, pl, l.p2p_off.as<int32_t>(), l.p2p_src.as<int32_t>(),
                                   l.m2l_off.as<int32_t>(), l.m2l_src.as<int32_t>());
   k_row_sort<<<nblocks(2 * C, BLK / 64), BLK, 0, s>>>(C, l.p2p_off.as<int32_t>(), l.p2p_src.as<int32_t>(),
                                                       l.m2l_off.as<int32_t>(), l.m2l_src.as<int32_t>(),
                                                       cnt + TC_LONG, sc.row_long.as<uint32_t>());
-  if (np + nm > ROW_RANK)
+  if (np + nm > ROW_RANK && Cs > ROW_RANK)  // a row holds a source cell once
     k_row_sort_long<<<LONG_BLOCKS, LONG_LANES, 0, s>>>(C, l.p2p_off.as<int32_t>(), l.p2p_src.as<int32_t>(),
                                                        l.m2l_off.as<int32_t>(), l.m2l_src.as<int32_t>(), cnt + TC_LONG,
                                                        sc.row_long.as<uint32_t>());
@@ -1007,10 +1127,20 @@ void traverse(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &st, double
     cap_p = sc.out_p2p.bytes / 8;
     cap_m = sc.out_m2l.bytes / 8;
     unsigned long long cnt[N_COUNTERS] = {};
-    k_traverse_start<<<1, 64, 0, s>>>(T, S, sc.front0.as<int2>(), sc.out_p2p.as<uint2>(), dcnt);
-    int64_t most = 1;  // pairs a step's frontier can hold
-    for (int k = 0;; k++) {
-      if (depth >= 0 ? k >= depth : k > 0 && k % BATCH == 0) {
+    // with lists of this kind built before, their size picks the way and the sizes are read back with
+    // the units; without, the sizes are read first
+    const bool    ahead = lists.np2p > 0 && !lists.long_rows && lists.np2p + lists.nm2l <= ROWS_SORTED;
+    const int     first = depth >= 0 ? std::min(depth, FIRST_STEPS) : FIRST_STEPS;
+    const int64_t nrows = ahead || lists.np2p == 0 ? 2 * (tt.C + 1) : 0;  // counts that may be needed
+    if (nrows) sc.row_cnt.reserve(4 * nrows);
+    k_traverse_first<<<1 + (int)std::min<int64_t>(256, (nrows + 4 * FIRST_LANES - 1) / (4 * FIRST_LANES)), FIRST_LANES, 0,
+                       s>>>(T, S, theta, gap, first, (first & 1 ? sc.front1 : sc.front0).as<int2>(), cap_f,
+                            sc.out_p2p.as<uint2>(), cap_p, sc.out_m2l.as<uint2>(), cap_m, dcnt,
+                            sc.row_cnt.as<uint32_t>(), nrows);
+    UVLM_LAUNCH_CHECK();
+    int64_t most = std::min<int64_t>((int64_t)1 << 3 * first, cap_f);  // pairs a step's frontier can hold
+    for (int k = first;; k++) {
+      if (depth >= 0 ? k >= depth : k > first && (k - first) % BATCH == 0) {
         if (depth >= 0) break;
         to_host(s, cnt, dcnt, TC_COUNT);
         if (cnt[TC_FRONT + (k & 3)] == 0 || (cnt[TC_FLAGS] & TF_FRONT)) break;
@@ -1022,12 +1152,14 @@ void traverse(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &st, double
       UVLM_LAUNCH_CHECK();
       most = std::min<int64_t>(8 * most, cap_f);
     }
-    // with lists of this kind built before, their size picks the way and the sizes are read back with
-    // the units; without, the sizes are read first
-    const bool ahead = lists.np2p > 0 && !lists.long_rows && lists.np2p + lists.nm2l <= ROWS_SORTED;
-    auto       by_counting = [&](int64_t np, int64_t nm) {
-      rows_by_counting(s, sc, tt.C, np, nm, lists);
-      if (max_leaf >= 0) near_units_enqueue(s, sc, tt, st, max_leaf, dcnt + TC_P2P, lists);
+    bool units_clear = true;  // the units' counters (k_traverse_first)
+    auto units       = [&] {
+      if (max_leaf >= 0) near_units_enqueue(s, sc, tt, st, max_leaf, dcnt + TC_P2P, units_clear, lists);
+      units_clear = false;
+    };
+    auto by_counting = [&](int64_t np, int64_t nm) {
+      rows_by_counting(s, sc, tt.C, st.C, np, nm, nrows > 0, lists);
+      units();
     };
     if (ahead) by_counting(cap_p, cap_m);
     to_host(s, cnt, dcnt, N_COUNTERS);
@@ -1055,10 +1187,8 @@ void traverse(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &st, double
     if (cnt[TC_FLAGS] & TF_LONG) {
       lists.long_rows = lists.long_rows || lists.np2p + lists.nm2l <= ROWS_SORTED;
       rows_by_sorting(s, sc, tt.C, st.C, lists);
-      if (max_leaf >= 0) {
-        near_units_enqueue(s, sc, tt, st, max_leaf, dcnt + TC_P2P, lists);
-        to_host(s, cnt, dcnt, N_COUNTERS);
-      }
+      units();
+      if (max_leaf >= 0) to_host(s, cnt, dcnt, N_COUNTERS);
     }
     if (max_leaf >= 0) near_units_set(cnt + UNIT_COUNTERS, lists);
     return;
@@ -1074,22 +1204,24 @@ void transpose_lists(hipStream_t s, Scratch &sc, const Tree &in_targets, const T
   sc.out_p2p.reserve(8 * std::max<int64_t>(in.np2p, 1));
   sc.out_m2l.reserve(8 * std::max<int64_t>(in.nm2l, 1));
   sc.counters.reserve(8 * N_COUNTERS);
-  unsigned long long *dcnt = sc.counters.as<unsigned long long>();
+  unsigned long long *dcnt   = sc.counters.as<unsigned long long>();
+  const bool          sorted = out.long_rows || in.np2p + in.nm2l > ROWS_SORTED;
+  const int64_t       nrows  = sorted ? 0 : 2 * (Cs + 1);
+  if (nrows) sc.row_cnt.reserve(4 * nrows);
   k_transpose_pairs<<<nblocks(2 * Ct, BLK / 64), BLK, 0, s>>>(
       Ct, in.p2p_off.as<int32_t>(), in.p2p_src.as<int32_t>(), in.np2p, in.m2l_off.as<int32_t>(),
-      in.m2l_src.as<int32_t>(), sc.out_p2p.as<uint2>(), sc.out_m2l.as<uint2>(), dcnt);
+      in.m2l_src.as<int32_t>(), sc.out_p2p.as<uint2>(), sc.out_m2l.as<uint2>(), dcnt, sc.row_cnt.as<uint32_t>(), nrows);
   UVLM_LAUNCH_CHECK();
   unsigned long long cnt[N_COUNTERS] = {};
-  const bool         sorted = out.long_rows || in.np2p + in.nm2l > ROWS_SORTED;
   if (!sorted) {
-    rows_by_counting(s, sc, Cs, in.np2p, in.nm2l, out);
-    near_units_enqueue(s, sc, in_sources, in_targets, max_leaf, dcnt + TC_P2P, out);
+    rows_by_counting(s, sc, Cs, Ct, in.np2p, in.nm2l, true, out);
+    near_units_enqueue(s, sc, in_sources, in_targets, max_leaf, dcnt + TC_P2P, true, out);
     to_host(s, cnt, dcnt, N_COUNTERS);
     out.long_rows = (cnt[TC_FLAGS] & TF_LONG) != 0;
   }
   if (sorted || out.long_rows) {
     rows_by_sorting(s, sc, Cs, Ct, out);
-    near_units_enqueue(s, sc, in_sources, in_targets, max_leaf, dcnt + TC_P2P, out);
+    near_units_enqueue(s, sc, in_sources, in_targets, max_leaf, dcnt + TC_P2P, sorted, out);
     to_host(s, cnt, dcnt, N_COUNTERS);
   }
   near_units_set(cnt + UNIT_COUNTERS, out);
