@@ -131,3 +131,44 @@ def test_first_steps(orc, monkeypatch, n, ncrit, capacity):
     for seed in (n, n + 1):
         check(g, orc, points(n, seed, 0.5, 0), ncrit)
     g.close()
+
+
+def test_get_list_of_cells_that_share_children(orc):
+    """A caller's tree may hand the same children to two cells: their pairs are listed twice."""
+    from uvlm_amd import _capi
+    import ctypes
+
+    # root 0 with cells 1 and 2, both with the children 3 .. 5
+    ints = np.array([[2, 6, 1, 0, 0], [3, 3, 3, 0, 1], [3, 3, 3, 3, 1], [0, 1, 0, 0, 2], [0, 1, 0, 1, 2], [0, 1, 0, 2, 2]],
+                    dtype=np.int64)
+    reals = np.array([[0, 0, 0, 1], [0.1, 0, 0, 0.5], [-0.1, 0, 0, 0.5], [0.2, 0, 0, 0.1], [0, 0.2, 0, 0.1],
+                      [0, 0, 0.2, 0.1]])
+    ip = lambda a: a.ctypes.data_as(ctypes.POINTER(ctypes.c_int64))  # noqa: E731
+    dp = lambda a: a.ctypes.data_as(ctypes.POINTER(ctypes.c_double))  # noqa: E731
+    g = FMMCalculator(P=4, theta=0.5, ncrit=4)
+    a, b = ctypes.c_int64(), ctypes.c_int64()
+    p2p, m2l = np.zeros((200, 2), dtype=np.int64), np.zeros((200, 2), dtype=np.int64)
+    print("[tree] shared children", flush=True)
+    _capi.check(g.lib.uvlm_get_list(0, 0.5, 6, ip(ints), dp(reals), 6, ip(ints), dp(reals), 200, 200, ctypes.byref(a),
+                                    ctypes.byref(b), ip(p2p), ip(m2l)))
+    want, front = [[], []], [(0, 0)]
+    while front:
+        nxt = []
+        for t, s in front:
+            if ints[s, 0] == 0 or (reals[t, 3] >= reals[s, 3] and ints[t, 0] != 0):
+                kids = [(ints[t, 2] + c, s) for c in range(ints[t, 0])]
+            else:
+                kids = [(t, ints[s, 2] + c) for c in range(ints[s, 0])]
+            for x, y in kids:
+                d2 = ((reals[x, :3] - reals[y, :3]) ** 2).sum()
+                if d2 * 0.25 < (reals[x, 3] + reals[y, 3]) ** 2:
+                    if ints[x, 0] == 0 and ints[y, 0] == 0:
+                        want[0].append((x, y))
+                    else:
+                        nxt.append((x, y))
+                else:
+                    want[1].append((x, y))
+        front = nxt
+    assert len(set(want[0])) < len(want[0])
+    assert np.array_equal(p2p[: a.value], np.array(sorted(want[0])))
+    assert np.array_equal(m2l[: b.value], np.array(sorted(want[1])).reshape(-1, 2))

@@ -1129,9 +1129,12 @@ void traverse(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &st, double
     unsigned long long cnt[N_COUNTERS] = {};
     // with lists of this kind built before, their size picks the way and the sizes are read back with
     // the units; without, the sizes are read first
-    const bool    ahead = lists.np2p > 0 && !lists.long_rows && lists.np2p + lists.nm2l <= ROWS_SORTED;
-    const int     first = depth >= 0 ? std::min(depth, FIRST_STEPS) : FIRST_STEPS;
-    const int64_t nrows = ahead || lists.np2p == 0 ? 2 * (tt.C + 1) : 0;  // counts that may be needed
+    // trees handed in by a caller are always sorted: cells there may share children, and ranking a
+    // row takes its sources to be distinct
+    const bool    own   = depth >= 0;
+    const bool    ahead = own && lists.np2p > 0 && !lists.long_rows && lists.np2p + lists.nm2l <= ROWS_SORTED;
+    const int     first = own ? std::min(depth, FIRST_STEPS) : FIRST_STEPS;
+    const int64_t nrows = ahead || (own && lists.np2p == 0) ? 2 * (tt.C + 1) : 0;  // counts that may be needed
     if (nrows) sc.row_cnt.reserve(4 * nrows);
     k_traverse_first<<<1 + (int)std::min<int64_t>(256, (nrows + 4 * FIRST_LANES - 1) / (4 * FIRST_LANES)), FIRST_LANES, 0,
                        s>>>(T, S, theta, gap, first, (first & 1 ? sc.front1 : sc.front0).as<int2>(), cap_f,
@@ -1180,7 +1183,7 @@ void traverse(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &st, double
     }
     lists.np2p = (int64_t)cnt[TC_P2P];
     lists.nm2l = (int64_t)cnt[TC_M2L];
-    if (!ahead && !lists.long_rows && lists.np2p + lists.nm2l <= ROWS_SORTED) {
+    if (own && !ahead && !lists.long_rows && lists.np2p + lists.nm2l <= ROWS_SORTED) {
       by_counting(lists.np2p, lists.nm2l);
       to_host(s, cnt, dcnt, N_COUNTERS);
     } else if (!ahead) cnt[TC_FLAGS] |= TF_LONG;
