@@ -128,3 +128,27 @@ def test_gaussian_sums(orc, n, ncrit):
     assert np.array_equal(s[:, 9:12], sb[:, 9:12])
     assert rel(s[:, 21:24], sb[:, 21:24]) < 1e-10
     g.close()
+
+
+@pytest.mark.parametrize("m,ncrit,theta", [(2, 2, 0.05), (40, 2, 0.05), (300, 8, 0.2)])
+def test_probes_with_long_rows(orc, m, ncrit, theta):
+    """Probe lists of thousands of sources a row: rows sorted by a workgroup, M2L lists in segments."""
+    X, A, S = cluster(6000, 5, 0.02)
+    pts = X[:: 6000 // m][:m] + 0.003
+    ref_b = orc.make_bodies(X, A, S)
+    ref = orc.Calculator(P=6, theta=theta, ncrit=ncrit)
+    ref.init(ref_b)
+    ref.calculate()
+    sb = orc.make_bodies(pts, np.zeros((m, 3)), np.ones(m))
+    ref.sensor_data(sb)
+    print(f"[near] long rows m={m} ncrit={ncrit}", flush=True)
+    g = FMMCalculator(P=6, theta=theta, ncrit=ncrit)
+    g.set_bodies(make_bodies(X, A, S))
+    g.build()
+    g.calculate()
+    for _ in range(2):  # the second pass counts the rows ahead
+        s = make_bodies(pts, np.zeros((m, 3)), np.ones(m))
+        g.getSensorData(s)
+        assert np.array_equal(s[:, 9:12], sb[:, 9:12])
+        assert rel(s[:, 15:18], sb[:, 15:18]) < 1e-10
+    g.close()

@@ -1187,6 +1187,7 @@ __global__ __launch_bounds__(W * WG) __attribute__((amdgpu_waves_per_eu(W == 2 &
   const int64_t u = (b & 7) * per_xcd + (b >> 3);
   if (u >= ncell) return;
   const int64_t t = SPLIT ? seg[3 * u] : u;  // target cell; the output row is u
+  if (SPLIT && seg[3 * u + 2] < 0) return;   // past the last segment
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, sl = lane & 15;
   const int wv = W == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform in the wavefront
   const int ny = tri(P), per = P * P + NT;
@@ -1404,6 +1405,7 @@ __global__ __launch_bounds__(m2l_fixed(P).W * WG) __attribute__((amdgpu_waves_pe
   const int64_t u = (b & 7) * per_xcd + (b >> 3);
   if (u >= ncell) return;
   const int64_t t = SPLIT ? seg[3 * u] : u;  // target cell; the output row is u
+  if (SPLIT && seg[3 * u + 2] < 0) return;   // past the last segment
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, sl = lane & 15;
   const int wv = W == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform in the wavefront
   double2  *Yx = sm2 + g * per, *Mg = Yx + P * P;
@@ -1423,19 +1425,85 @@ __global__ __launch_bounds__(m2l_fixed(P).W * WG) __attribute__((amdgpu_waves_pe
   m2l_store<S, W>(acc, P * (P + 1) / 2, tid, sm2, out_off, out_src, L + u * NT);
 }
 
-// L of each target = the sum of its segments' expansions, in segment order.
-__global__ __launch_bounds__(WG) void k_m2l_reduce(int NT, int64_t ncell, const int32_t *__restrict__ segoff,
-                                                   const double2 *__restrict__ part, double2 *__restrict__ L)
+// Below this many target cells (probe trees), long lists are cut into segments that run as
+// separate workgroups (see the P2P launcher for the same rule).
+constexpr int64_t M2L_SPLIT_TARGETS = 4096, M2L_SPLIT_SEGMENTS = 8192;
+
+// Segments of few targets' lists: target t's list in pieces of E entries, at least one (empty) piece;
+// seg[u] = {target, first, end} in target order, segoff[t] target t's first, and the rest of the U
+// units (a bound on the segments, known to the host) {0, 0, -1}.  One workgroup (11 us; the
+// table was made on the host, two synchronisations and three copies, 180 us of the same pass).
+constexpr int SEG_LANES = 1024;
+__global__ __launch_bounds__(SEG_LANES) void k_m2l_segments(int C, int E, int U, const int32_t *__restrict__ off,
+                                                            int32_t *__restrict__ seg, int32_t *__restrict__ segoff)
 {
-  const int64_t t = blockIdx.x;
-  if (t >= ncell) return;
-  for (int q = threadIdx.x; q < NT; q += WG) {
-    double2 r = make_double2(0, 0);
-    for (int u = segoff[t]; u < segoff[t + 1]; u++) {
-      r.x += part[(int64_t)u * NT + q].x;
-      r.y += part[(int64_t)u * NT + q].y;
+  constexpr int  PER = M2L_SPLIT_TARGETS / SEG_LANES;
+  __shared__ int so[M2L_SPLIT_TARGETS + 1], ws[SEG_LANES / 64];
+  const int      tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  int            n[PER], sum = 0;
+  for (int i = 0; i < PER; i++) {
+    const int t = tid * PER + i;
+    n[i]        = t < C ? max(1, (off[t + 1] - off[t] + E - 1) / E) : 0;
+    sum += n[i];
+  }
+  int inc = sum;
+  for (int d = 1; d < 64; d *= 2) {
+    const int v = __shfl_up(inc, d, 64);
+    if (lane >= d) inc += v;
+  }
+  if (lane == 63) ws[wv] = inc;
+  __syncthreads();
+  int at = inc - sum;
+  for (int w = 0; w < wv; w++) at += ws[w];
+  for (int i = 0; i < PER; i++) {
+    const int t = tid * PER + i;
+    if (t <= C) so[t] = at, segoff[t] = at;
+    at += n[i];
+    if (t == C - 1) so[C] = at, segoff[C] = at;
+  }
+  __syncthreads();
+  const int total = so[C];
+  for (int u = tid; u < U; u += SEG_LANES) {
+    int lo = 0, hi = C - 1;
+    while (lo < hi) {  // the last target whose segments start at or before u
+      const int mid = (lo + hi + 1) >> 1;
+      if (so[mid] <= u) lo = mid;
+      else hi = mid - 1;
     }
-    L[t * NT + q] = r;
+    const int64_t e0 = off[lo] + (int64_t)E * (u - so[lo]);
+    seg[3 * u]     = u < total ? lo : 0;
+    seg[3 * u + 1] = u < total ? (int)e0 : 0;
+    seg[3 * u + 2] = u < total ? (int)min((int64_t)off[lo + 1], e0 + E) : -1;
+  }
+}
+
+// L of each target = the sum of its segments' expansions: four runs of consecutive segments, one a
+// wavefront, each in segment order, added in run order.  Bound by the latency of the partial sums
+// (one wavefront walking all segments of its target: 41 us for 4096 probes of 200003 bodies; 5).
+__global__ __launch_bounds__(4 * WG) void k_m2l_reduce(int NT, int64_t ncell, const int32_t *__restrict__ segoff,
+                                                       const double2 *__restrict__ part, double2 *__restrict__ L)
+{
+  __shared__ double2 v[4][WG];
+  const int64_t      t = blockIdx.x;
+  const int          lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int          u0 = segoff[t], n = segoff[t + 1] - u0, run = (n + 3) / 4;
+  const int          b = u0 + min(n, wv * run), e = u0 + min(n, (wv + 1) * run);
+  for (int q0 = blockIdx.y * WG; q0 < NT; q0 += gridDim.y * WG) {
+    const int q = min(q0 + lane, NT - 1);
+    double2   r = make_double2(0, 0);
+#pragma unroll 4
+    for (int u = b; u < e; u++) {
+      const double2 p = part[(int64_t)u * NT + q];
+      r.x += p.x;
+      r.y += p.y;
+    }
+    __syncthreads();
+    v[wv][lane] = r;
+    __syncthreads();
+    if (wv == 0 && q0 + lane < NT) {
+      for (int w = 1; w < 4; w++) r.x += v[w][lane].x, r.y += v[w][lane].y;
+      L[t * NT + q] = r;
+    }
   }
 }
 
@@ -1864,10 +1932,6 @@ void l2l_level(hipStream_t s, int P, const Tree &t, int level, double2 *L, const
   UVLM_LAUNCH_CHECK();
 }
 
-// Below this many target cells (probe trees), long lists are cut into segments that run as
-// separate workgroups (see the P2P launcher for the same rule).
-constexpr int64_t M2L_SPLIT_TARGETS = 4096, M2L_SPLIT_SEGMENTS = 8192;
-
 void m2l(hipStream_t s, int P, const Tree &tt, const Tree &st, const Lists &l, const M2LSchedule &sch, const double2 *M,
          double2 *L, Scratch *sc)
 {
@@ -1885,28 +1949,14 @@ void m2l(hipStream_t s, int P, const Tree &tt, const Tree &st, const Lists &l, c
     double2       *out  = L;
     if (split) {
       const int64_t        E = std::max<int64_t>(2, (l.nm2l + M2L_SPLIT_SEGMENTS - 1) / M2L_SPLIT_SEGMENTS);
-      std::vector<int32_t> off(tt.C + 1), seg, segoff(tt.C + 1, 0);
-      UVLM_HIP(hipMemcpyAsync(off.data(), l.m2l_off.p, 4 * off.size(), hipMemcpyDeviceToHost, s));
-      UVLM_HIP(hipStreamSynchronize(s));
-      for (int64_t t = 0; t < tt.C; t++) {
-        int32_t e0 = off[t];
-        do {
-          const int32_t e1 = (int32_t)std::min<int64_t>(off[t + 1], e0 + E);
-          seg.push_back((int32_t)t);
-          seg.push_back(e0);
-          seg.push_back(e1);
-          e0 = e1;
-        } while (e0 < off[t + 1]);
-        segoff[t + 1] = (int32_t)(seg.size() / 3);
-      }
-      units = segoff[tt.C];
-      sc->m2l_seg.reserve(4 * (seg.size() + segoff.size()));
+      // sum max(1, ceil(n / E)) <= C + nm2l / E; the units past the last segment return at once
+      units = tt.C + l.nm2l / E;
+      sc->m2l_seg.reserve(4 * (3 * units + tt.C + 1));
       int32_t *ds = sc->m2l_seg.as<int32_t>();
-      UVLM_HIP(hipMemcpyAsync(ds, seg.data(), 4 * seg.size(), hipMemcpyHostToDevice, s));
-      UVLM_HIP(hipMemcpyAsync(ds + seg.size(), segoff.data(), 4 * segoff.size(), hipMemcpyHostToDevice, s));
-      UVLM_HIP(hipStreamSynchronize(s));
-      dseg    = ds;
-      dsegoff = ds + seg.size();
+      dseg        = ds;
+      dsegoff     = ds + 3 * units;
+      k_m2l_segments<<<1, SEG_LANES, 0, s>>>((int)tt.C, (int)E, (int)units, l.m2l_off.as<int32_t>(), ds, ds + 3 * units);
+      UVLM_LAUNCH_CHECK();
       sc->m2l_part.reserve(sizeof(double2) * units * NT);
       out = sc->m2l_part.as<double2>();
     }
@@ -1929,7 +1979,7 @@ void m2l(hipStream_t s, int P, const Tree &tt, const Tree &st, const Lists &l, c
     else k_m2l_fixed<PP, false><<<grid, m2l_fixed(PP).W * WG, lds_ns, s>>>(UVLM_M2L_CALL_ARGS);                   \
     UVLM_LAUNCH_CHECK();                                                                                         \
     if (split) {                                                                                                 \
-      k_m2l_reduce<<<(int)tt.C, WG, 0, s>>>(NT, tt.C, dsegoff, out, L);                                          \
+      k_m2l_reduce<<<dim3((unsigned)tt.C, (unsigned)((NT + WG - 1) / WG)), 4 * WG, 0, s>>>(NT, tt.C, dsegoff, out, L);                                          \
       UVLM_LAUNCH_CHECK();                                                                                       \
     }                                                                                                            \
     return;                                                                                                      \
@@ -1949,7 +1999,7 @@ void m2l(hipStream_t s, int P, const Tree &tt, const Tree &st, const Lists &l, c
     }                                                                                                      \
     UVLM_LAUNCH_CHECK();                                                                                   \
     if (split) {                                                                                           \
-      k_m2l_reduce<<<(int)tt.C, WG, 0, s>>>(NT, tt.C, dsegoff, out, L);                                    \
+      k_m2l_reduce<<<dim3((unsigned)tt.C, (unsigned)((NT + WG - 1) / WG)), 4 * WG, 0, s>>>(NT, tt.C, dsegoff, out, L);                                    \
       UVLM_LAUNCH_CHECK();                                                                                 \
     }                                                                                                      \
     return;                                                                                                \

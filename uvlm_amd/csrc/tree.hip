@@ -750,7 +750,63 @@ __global__ __launch_bounds__(BLK) void k_row_sort(int64_t C, const int32_t *__re
     if (lane + 64 * i < n) src[q[i]] = m[i];
 }
 
-// The rows k_row_sort left, a workgroup each: bitonic sort of the next power of two entries.
+// The rows k_row_sort left, a workgroup each.  A row holds a source cell once, so its order is a bit
+// map of the Cs <= ROW_BITS source cells: set the entries' bits, count the bits below each word, write
+// the set bits out.  Linear in the entries and in Cs / 32, where the bitonic sort takes log^2 steps with
+// a barrier each (200003 bodies, 4096 probes, rows of thousands of entries: 80 us, here
+// 7.3).
+constexpr int BITS_LANES = 512, BITS_BLOCKS = 512, ROW_WORDS = 7168, ROW_BITS = 32 * ROW_WORDS;
+__global__ __launch_bounds__(BITS_LANES) void k_row_sort_bits(int64_t C, int64_t Cs, const int32_t *__restrict__ off_p,
+                                                              int32_t *__restrict__ src_p,
+                                                              const int32_t *__restrict__ off_m,
+                                                              int32_t *__restrict__ src_m,
+                                                              const unsigned long long *__restrict__ nlong,
+                                                              const uint32_t *__restrict__ longs)
+{
+  __shared__ unsigned bits[ROW_WORDS];
+  __shared__ int      below[ROW_WORDS], ws[BITS_LANES / 64];
+  const int           nl = (int)*nlong, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int           W = (int)((Cs + 31) / 32), per = (W + BITS_LANES - 1) / BITS_LANES;
+  const int           w0 = min(W, tid * per), w1 = min(W, w0 + per);
+  for (int k = blockIdx.x; k < nl; k += gridDim.x) {
+    const int64_t  r   = longs[k];
+    const int32_t *off = r < C ? off_p + r : off_m + (r - C);
+    int32_t       *src = (r < C ? src_p : src_m) + off[0];
+    const int      n   = off[1] - off[0];
+    for (int w = tid; w < W; w += BITS_LANES) bits[w] = 0;
+    __syncthreads();
+    for (int j = tid; j < n; j += BITS_LANES) {
+      const unsigned c = (unsigned)src[j];
+      if (c < (unsigned)Cs) atomicOr(&bits[c >> 5], 1u << (c & 31));
+    }
+    __syncthreads();
+    int sum = 0;
+    for (int w = w0; w < w1; w++) {
+      below[w] = sum;
+      sum += __popc(bits[w]);
+    }
+    int inc = sum;
+    for (int d = 1; d < 64; d *= 2) {
+      const int v = __shfl_up(inc, d, 64);
+      if (lane >= d) inc += v;
+    }
+    if (lane == 63) ws[wv] = inc;
+    __syncthreads();
+    int at = inc - sum;
+    for (int v = 0; v < wv; v++) at += ws[v];
+    for (int w = w0; w < w1; w++) below[w] += at;
+    __syncthreads();
+    for (int w = tid; w < W; w += BITS_LANES) {
+      int q = below[w];
+      for (unsigned b = bits[w]; b; b &= b - 1, q++)
+        if (q < n) src[q] = 32 * w + __builtin_ctz(b);
+    }
+    __syncthreads();
+  }
+}
+
+// The rows k_row_sort left, a workgroup each: bitonic sort of the next power of two entries, for
+// source trees beyond k_row_sort_bits.
 constexpr int LONG_LANES = 512, LONG_BLOCKS = 512;
 __global__ __launch_bounds__(LONG_LANES) void k_row_sort_long(int64_t C, const int32_t *__restrict__ off_p,
                                                               int32_t *__restrict__ src_p,
@@ -1070,7 +1126,12 @@ static void rows_by_counting(hipStream_t s, Scratch &sc, int64_t C, int64_t Cs, 
   k_row_sort<<<nblocks(2 * C, BLK / 64), BLK, 0, s>>>(C, l.p2p_off.as<int32_t>(), l.p2p_src.as<int32_t>(),
                                                       l.m2l_off.as<int32_t>(), l.m2l_src.as<int32_t>(),
                                                       cnt + TC_LONG, sc.row_long.as<uint32_t>());
-  if (np + nm > ROW_RANK && Cs > ROW_RANK)  // a row holds a source cell once
+  const bool may_long = np + nm > ROW_RANK && Cs > ROW_RANK;  // a row holds a source cell once
+  if (may_long && Cs <= ROW_BITS)
+    k_row_sort_bits<<<BITS_BLOCKS, BITS_LANES, 0, s>>>(C, Cs, l.p2p_off.as<int32_t>(), l.p2p_src.as<int32_t>(),
+                                                       l.m2l_off.as<int32_t>(), l.m2l_src.as<int32_t>(), cnt + TC_LONG,
+                                                       sc.row_long.as<uint32_t>());
+  else if (may_long)
     k_row_sort_long<<<LONG_BLOCKS, LONG_LANES, 0, s>>>(C, l.p2p_off.as<int32_t>(), l.p2p_src.as<int32_t>(),
                                                        l.m2l_off.as<int32_t>(), l.m2l_src.as<int32_t>(), cnt + TC_LONG,
                                                        sc.row_long.as<uint32_t>());
