@@ -188,14 +188,22 @@ __global__ __launch_bounds__(256) void k_lu_inverse(int n, const double *__restr
   }
 }
 
-// out_i = sum_c Xc[c * n + i] b_c (= A^{-1} b), one lane per row, columns in order.
-__global__ void k_matvec_inv(int n, const double *__restrict__ Xc, const double *__restrict__ b,
-                             double *__restrict__ out)
+// out_i = sum_c Xc[c * n + i] b_c (= A^{-1} b): 64 rows a workgroup, lanes over rows, wavefront w the
+// columns w, w + 16, ..; the wavefronts' sums are added in order.  Bound by the latency of the loads
+// (one lane per row over all columns: 98 us at n = 400, here 8.4).
+constexpr int MV_WAVES = 16;
+__global__ __launch_bounds__(64 * MV_WAVES) void k_matvec_inv(int n, const double *__restrict__ Xc,
+                                                              const double *__restrict__ b, double *__restrict__ out)
 {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  double r = 0.0;
-  for (int c = 0; c < n; c++) r += Xc[(int64_t)c * n + i] * b[c];
+  __shared__ double v[MV_WAVES][64];
+  const int         lane = threadIdx.x & 63, w = threadIdx.x >> 6, i = blockIdx.x * 64 + lane, ic = min(i, n - 1);
+  double            r = 0.0;
+#pragma unroll 8
+  for (int c = w; c < n; c += MV_WAVES) r += Xc[(int64_t)c * n + ic] * b[c];
+  v[w][lane] = r;
+  __syncthreads();
+  if (w != 0 || i >= n) return;
+  for (int k = 1; k < MV_WAVES; k++) r += v[k][lane];
   out[i] = r;
 }
 
@@ -724,7 +732,7 @@ void lu_inverse(hipStream_t s, int n, const double *LU, const int *piv, double *
 
 void matvec_inv(hipStream_t s, int n, const double *Xc, const double *b, double *out)
 {
-  k_matvec_inv<<<nb256(n), 256, 0, s>>>(n, Xc, b, out);
+  k_matvec_inv<<<(n + 63) / 64, 64 * MV_WAVES, 0, s>>>(n, Xc, b, out);
   UVLM_LAUNCH_CHECK();
 }
 
