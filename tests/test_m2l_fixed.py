@@ -50,3 +50,29 @@ def test_fixed_against_general(monkeypatch, P, n, ncrit, theta):
     assert out[0][0] in (5, 6, 8) and out[1][0] == 12 and out[0][1] == out[1][1] > 0
     for a, c in zip(out[0][2:], out[1][2:]):
         assert np.isfinite(a).all() and np.abs(a - c).max() <= 1e-12 * np.abs(c).max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("P", [4, 14])
+@pytest.mark.parametrize("n,ncrit", [(40, 1), (900, 70)])
+def test_unrolled_orders_against_the_oracle(orc, P, n, ncrit):
+    """P2M and L2P with these orders as constants: the parity bar of the other orders, 1e-10."""
+    rng = W.SplitMix64(n)
+    X = rng.uniform(3 * n).reshape(n, 3) * 2.0 - 1.0
+    A, S = rng.normal(3 * n).reshape(n, 3), np.full(n, 0.05)
+    ref_b = orc.make_bodies(X, A, S)
+    ref = orc.Calculator(P=P, theta=0.4, ncrit=ncrit)
+    ref.init(ref_b)
+    ref.calculate()
+    want = ref.bodies(n)
+    print(f"[orders] P={P} n={n}", flush=True)
+    g = FMMCalculator(P=P, theta=0.4, ncrit=ncrit)
+    g.set_bodies(make_bodies(X, A, S))
+    g.build()
+    g.calculate()
+    got = g.copyBodies2Host()
+    assert np.array_equal(got[:, 9:12], want[:, 9:12])
+    for sl in (slice(0, 9), slice(15, 21)):
+        ok = np.isfinite(want[:, sl])  # a body at its leaf's centre: the reference's L2P is NaN there
+        assert np.linalg.norm((got[:, sl] - want[:, sl])[ok]) < 1e-10 * np.linalg.norm(want[:, sl][ok])
+    g.close()
