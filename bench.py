@@ -647,7 +647,7 @@ def main():
     wl = {"particles": N, "P": args.P, "theta": args.theta, "ncrit": ncrit_used, "precision": args.precision}
     p2p_peak = PEAK["fp32"] if args.precision == "mixed" else PEAK["fp64"]
     roofs = {
-        "M2L": ("k_m2l_ns", tm["n_m2l_pairs"] * m2l_flop_per_pair(args.P), ph["m2l_ms"], PEAK["fp64"],
+        "M2L": ("k_m2l_", tm["n_m2l_pairs"] * m2l_flop_per_pair(args.P), ph["m2l_ms"], PEAK["fp64"],
                 "FP64 vector ALU: no dense contraction and no MFMA (FP64 vector and matrix peaks coincide on "
                 "MI355X); not HBM-bound (profiles/)"),
         "P2P": ("k_p2p", tm["n_interactions"] * P2P_FLOP, ph["p2p_ms"], p2p_peak,

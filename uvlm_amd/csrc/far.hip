@@ -1386,8 +1386,9 @@ __device__ __forceinline__ void m2l_fixed_loop(double2 (&acc)[S][3], const M2LSt
 // k_m2l_ns for the orders of m2l_fixed under their default plan, as straight code.  k_m2l_ns is
 // bound by LDS reads (83% of its cycles at P = 10: five 16-byte reads an order for 16 FP64
 // instructions) and spends a third of its instructions around the orders.  Here a home slot
-// reads two, and its set-up at a degree is a few instructions; what bounds it is the FP64 rate
-// (about 1150 instructions of a SIMD's four sources, 900 of them the orders).  M2L phase, k_m2l_ns
+// reads two, and its set-up at a degree is a few instructions (some 1050 for four sources against
+// 1505, 900 of them the orders).  Bound by latency at three wavefronts a SIMD: VALU issues in 63% of
+// the cycles, LDS is active in 82%; cutting its bank conflicts by a quarter gained nothing.  M2L phase, k_m2l_ns
 // and this: 1M-body cube (P = 10) 5.77 -> 4.12 ms, 1M leapfrog 4.02 -> 3.04, 60001-body cube
 // (P = 14) 5.82 -> 3.56, 260003 bodies (P = 8) 1.68 -> 1.09, 8192-body ring (P = 8) 152 -> 73 us,
 // 100002 bodies (P = 6) 208 -> 124.  Three wavefronts a SIMD: with four (128 registers) P = 10
