@@ -765,6 +765,7 @@ int uvlm_create(const uvlm_params *p, uvlm_handle *out)
     set_device(h);
     scratch_setup(p->device);
     UVLM_HIP(hipStreamCreateWithFlags(&h->s, hipStreamNonBlocking));
+    h->sc.back.create();
     for (auto &e : h->ev) UVLM_HIP(hipEventCreate(&e));
     for (auto &e : h->aev) UVLM_HIP(hipEventCreate(&e));
     // UVLM_M2L_SLOTS overrides the M2L plan's accumulator-slot budget (uvlm_autotune also sets

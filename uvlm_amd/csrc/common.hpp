@@ -82,6 +82,29 @@ struct DevBuf {
   }
   template <class T> T *as() const { return (T *)p; }
 };
+// A few words of page-locked memory that kernels write for the host.  Without it (it could not be
+// allocated, or the object lives for one call) the reader copies instead.
+struct HostWords {
+  static constexpr size_t BYTES = 512;
+  uint32_t *h = nullptr, *d = nullptr;  // the host's and the device's address
+  HostWords() = default;
+  HostWords(const HostWords &) = delete;
+  HostWords &operator=(const HostWords &) = delete;
+  ~HostWords()
+  {
+    if (h) (void)hipHostFree(h);
+  }
+  void create()
+  {
+    if (h) return;
+    if (hipHostMalloc((void **)&h, BYTES, hipHostMallocMapped) != hipSuccess) h = nullptr;
+    if (h && hipHostGetDevicePointer((void **)&d, h, 0) != hipSuccess) {
+      (void)hipHostFree(h);
+      h = d = nullptr;
+    }
+    (void)hipGetLastError();
+  }
+};
 inline void swap_buf(DevBuf &a, DevBuf &b)
 {
   std::swap(a.p, b.p);
@@ -122,6 +145,7 @@ struct Scratch {
   DevBuf rec_begin, rec_end, rec_parent, rec_level, rec_mask, rec_scan;  // cells in pre-order
   DevBuf partial, counters, perm;
   DevBuf front0, front1, out_p2p, out_m2l, row_cnt, row_off, row_place, row_long;
+  HostWords back;              // totals that the host waits for
   DevBuf unit_work, p2p_part;  // near-field units: work per leaf, totals, partial sums
   DevBuf m2l_seg, m2l_part;  // M2L list segments and their partial sums (few-target case)
 };
