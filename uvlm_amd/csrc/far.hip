@@ -1697,7 +1697,13 @@ __global__ void k_zero(double *p, int64_t n)
 // runs P = 6 and 8 with two as well: 5 slots there hold what one wavefront needs 6 for, and a
 // target's list is worked off in half the time where targets are few (8192-body ring, P = 8:
 // 73 against 93 us; 260003-body pass 1.09 against 1.13 ms; 100002 at P = 6 124 against 141 us).
-int m2l_waves(int P, int waves) { return waves == 1 || waves == 2 ? waves : (P <= 8 && P != 6 && P != 8 ? 1 : 2); }
+// That is the plan of 5 slots, the default; other budgets at these orders keep one.
+int m2l_waves(int P, int waves, int budget)
+{
+  if (waves == 1 || waves == 2) return waves;
+  if (P == 6 || P == 8) return budget <= 0 || budget == 5 ? 2 : 1;
+  return P <= 8 ? 1 : 2;
+}
 
 // Term table of k_m2m_tab for P <= M2M_TAB_MAXP: per lane (output q = (j,k) = lane, tri(P) <= 64)
 // the counts of its plain and conjugated terms, then RP rows of plain terms and RC rows of
@@ -1787,7 +1793,7 @@ static bool make_l2l_table(int P, std::vector<uint16_t> &tab)
 void make_m2l_schedule(int P, M2LSchedule &s)
 {
   // Default budget: with two wavefronts, 5 slots run at 4 waves per SIMD at P = 10.
-  s.W              = m2l_waves(P, s.waves);
+  s.W              = m2l_waves(P, s.waves, s.budget);
   const int budget = s.budget > 0 ? s.budget : (s.W == 2 ? 5 : 0);
   if (!make_m2l_plan(P, budget, s.plan, 16, s.W)) throw Error(UVLM_ERR_INTERNAL, "no M2L plan");
   const M2LPlan &pl = s.plan;
