@@ -414,6 +414,7 @@ __global__ __launch_bounds__(256) void k_units_work(const int32_t *__restrict__ 
   for (int64_t w = blockIdx.x * 4ll + wv; w < nleaf; w += gridDim.x * 4ll) {
     const int t = leaves[w], nt = tnbody[t], q1 = off[t + 1];
     unsigned  ns = 0;
+#pragma unroll 4  // four gathers in flight: 29 -> 13 us for lists of thousands (4096 probes of 200003 bodies)
     for (int q = off[t] + lane; q < q1; q += 64) ns += (unsigned)snbody[src[q]];
     for (int o = 32; o > 0; o >>= 1) ns += __shfl_xor(ns, o, 64);
     const int ntp = wide ? near_targets_per_pass<256>(nt) : near_targets_per_pass<64>(nt);
@@ -510,7 +511,7 @@ __global__ __launch_bounds__(256) void k_p2p_reduce(const int4 *__restrict__ mul
   for (int o = threadIdx.x; o < (WITH_J ? 12 : 3) * nt; o += 256) {
     const int k = o / nt;
     double    v = 0.0;
-#pragma unroll 4
+#pragma unroll 16  // 16 rows in flight (4: 22 us for the same probes, 16: 13)
     for (int u = 0; u < m.z; u++) v += p[(int64_t)u * 12 * nt + o];
     out[(k < 3 ? F_U + k : F_J + k - 3) * ocap + tb + (o - k * nt)] = -v;
   }
