@@ -30,8 +30,6 @@ namespace uvlm {
 
 namespace {
 
-constexpr int WG = 64;
-
 // acc[0..2] += f1 c, acc[3..10] += f2 c (x) dX with c = dX x a, and acc[12..14] += f1 a: the
 // f1 eps_{abk} a_k part of J is antisymmetric, so its sum is kept as one vector and folded
 // into J once per chunk (fold_antisym) instead of six multiply-adds per pair.  c is
