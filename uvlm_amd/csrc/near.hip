@@ -20,6 +20,7 @@
 // trip count for all lanes), per-chunk FP32 partial sums added into FP64 per-target
 // accumulators; G = g/s^3 and its derivative from pair_kernel.hpp.
 #include "common.hpp"
+#include "near_units.hpp"
 #include "pair_kernel.hpp"
 
 #include <vector>
@@ -363,16 +364,7 @@ void direct(hipStream_t s, int64_t m, const double *xt, const double *at, const 
   UVLM_LAUNCH_CHECK();
 }
 
-// Units of the near field: each target leaf's list in one or more runs of entries of about equal
-// work, so that a wave never walks a list far longer than the others' (a leaf next to much smaller
-// ones, a probe tree with few leaves) while the chip is idle.  A leaf's work is its lane steps: the
-// bodies of its list times its passes over its splits.  It is cut into ceil(work / limit) units,
-// limit = the larger of LANE_STEPS_MIN and 1/UNITS_AIM of all leaves' work: below LANE_STEPS_MIN the
-// staging and the prefix sums cost more than the pairs they serve (32 and 64 steps: 8k ring 72 and
-// 77 us; 128: 100 us).  More units shorten the last wave: 4M two rings (86k leaves) 10.0 ms with
-// 4096, 9.9 with 8192, 9.6 with 16384.
-constexpr int                LANE_STEPS_MIN = 64;
-constexpr unsigned long long UNITS_AIM      = 16384;
+// Totals of the near-field units (near_units.hpp).
 enum { NU_INTER = 0, NU_WORK, NU_UNITS, NU_ROWS, NU_MULTI, NU_WIDE, NU_COUNT };
 static_assert(UNIT_COUNTERS + NU_COUNT <= N_COUNTERS, "near-field unit totals");
 
@@ -444,13 +436,12 @@ __global__ __launch_bounds__(256) void k_units_fill(const int32_t *__restrict__ 
   __shared__ unsigned long long tot[4][3], base[3];
   const int64_t            w    = blockIdx.x * 256ll + threadIdx.x;
   const int                lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const unsigned long long lim = max((unsigned long long)LANE_STEPS_MIN, cnt[NU_WORK] / UNITS_AIM);
+  const uint64_t           lim = units_limit(cnt[NU_WORK]);
   int                      nu = 0, q0 = 0, len = 0, nt = 0;  // no units past the last leaf
   if (w < nleaf) {
     const int t = leaves[w];
     nt = tnbody[t], q0 = off[t], len = off[t + 1] - q0;
-    nu = (int)min((unsigned long long)max(len, 1), (work[w] + lim - 1) / lim);
-    nu = max(nu, 1);
+    nu = units_of_leaf(work[w], len, lim);
   }
   // exclusive prefix sums over the block of units, rows and cut leaves
   unsigned long long v[3] = {(unsigned long long)nu, nu > 1 ? (unsigned long long)nu * nt : 0, nu > 1 ? 1ull : 0}, ex[3];
@@ -488,10 +479,9 @@ __global__ __launch_bounds__(256) void k_units_fill(const int32_t *__restrict__ 
       if (first[mid] <= u) lo = mid;
       else hi = mid - 1;
     }
-    const int     n = first[lo + 1] - first[lo], j = u - first[lo];
-    const int64_t ln = lens[lo];
-    units[base[0] + u] = make_int4((int)(blockIdx.x * 256 + lo), q0s[lo] + (int)(ln * j / n),
-                                   q0s[lo] + (int)(ln * (j + 1) / n), n > 1 ? row[lo] + j * nts[lo] : -1);
+    const int n = first[lo + 1] - first[lo], j = u - first[lo], ln = lens[lo];
+    units[base[0] + u] = make_int4((int)(blockIdx.x * 256 + lo), q0s[lo] + units_first(ln, j, n),
+                                   q0s[lo] + units_first(ln, j + 1, n), n > 1 ? row[lo] + j * nts[lo] : -1);
   }
 }
 
@@ -665,9 +655,8 @@ void near_units_enqueue(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &
   if (tt.nleaf == 0) return;
   sc.unit_work.reserve(4 * tt.nleaf);
   unsigned long long *cnt = sc.counters.as<unsigned long long>() + UNIT_COUNTERS;
-  // at most UNITS_AIM units beyond one per leaf: sum ceil(work / limit) <= nleaf + work / limit
-  l.units.reserve(sizeof(int4) * (tt.nleaf + UNITS_AIM));
-  l.multi.reserve(sizeof(int4) * std::min<int64_t>(tt.nleaf, UNITS_AIM));
+  l.units.reserve(sizeof(int4) * units_bound(tt.nleaf));
+  l.multi.reserve(sizeof(int4) * units_multi_bound(tt.nleaf));
   const int32_t *lv = tt.leaves.as<int32_t>(), *tn = tt.nbody.as<int32_t>();
   const int32_t *off = l.p2p_off.as<int32_t>();
   if (!cleared) k_units_clear<<<1, 64, 0, s>>>(cnt);
