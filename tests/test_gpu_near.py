@@ -152,3 +152,31 @@ def test_probes_with_long_rows(orc, m, ncrit, theta):
         assert np.array_equal(s[:, 9:12], sb[:, 9:12])
         assert rel(s[:, 15:18], sb[:, 15:18]) < 1e-10
     g.close()
+
+
+@pytest.mark.parametrize("n,m,ncrit", [(40, 5, 64), (900, 37, 7)])
+def test_nan_coordinates_show_in_the_vorticity(n, m, ncrit):
+    """exp(NaN) is NaN: a body with a NaN coordinate shows at every probe whose list holds its leaf (with
+    theta 1e-3 all of them), a NaN probe at itself alone."""
+    X, A, S = cluster(n, n, 0.3)
+    pts = X[:m] + 0.01
+
+    def vorticity(X, pts):
+        g = FMMCalculator(P=4, theta=1e-3, ncrit=ncrit)
+        g.set_bodies(make_bodies(X, A, S))
+        g.build()
+        s = make_bodies(pts, np.arange(3.0 * m).reshape(m, 3), np.ones(m))
+        g.vorticity(s)
+        g.close()
+        return s[np.argsort(s[:, 12])][:, 21:24]  # in the probes' order
+
+    print(f"[near] NaN n={n} m={m}", flush=True)
+    want = vorticity(X, pts)
+    assert np.isfinite(want).all()
+    bad = X.copy()
+    bad[n // 2, 1] = np.nan
+    assert np.isnan(vorticity(bad, pts)).all()
+    badp = pts.copy()
+    badp[m // 2, 0] = np.nan
+    got = vorticity(X, badp)
+    assert np.isnan(got[m // 2]).all() and np.isfinite(np.delete(got, m // 2, 0)).all()

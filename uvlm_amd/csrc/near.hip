@@ -546,20 +546,33 @@ __global__ __launch_bounds__(BLK) void k_gauss(const int4 *__restrict__ units, c
       for (int d = 0; d < 3; d++) ai[d] = tst[(F_A + d) * tcap + bi];
     }
     double acc[3] = {0.0, 0.0, 0.0};
-    auto   pair = [&](const double4 &A, const double4 &B) {
-      const double dx = xi - A.x, dy = yi - A.y, dz = zi - A.z, R2 = dx * dx + dy * dy + dz * dz;
+    auto   sep  = [&](const double4 &A) {
+      const double dx = xi - A.x, dy = yi - A.y, dz = zi - A.z;
+      return dx * dx + dy * dy + dz * dz;
+    };
+    auto add = [&](const double4 &A, const double4 &B, double R2, double r, double x) {
       if (MODE == GAUSS_PSE) {
-        const double r = rsqrt64(s2i + A.w), o2 = r * r;
-        const double e = R2 == 0.0 ? 0.0 : exp64_neg(0.5 * R2 * o2, c_exp64) * (o2 * o2 * r);
+        const double o2 = r * r, e = R2 == 0.0 ? 0.0 : exp64_neg(x, c_exp64) * (o2 * o2 * r);
         acc[0] = fma(voli * B.x - B.w * ai[0], e, acc[0]);
         acc[1] = fma(voli * B.y - B.w * ai[1], e, acc[1]);
         acc[2] = fma(voli * B.z - B.w * ai[2], e, acc[2]);
       } else {
-        const double e = exp64_neg(R2 * A.w, c_exp64);
+        const double e = exp64_neg(x, c_exp64);
         acc[0] = fma(B.x, e, acc[0]);
         acc[1] = fma(B.y, e, acc[1]);
         acc[2] = fma(B.z, e, acc[2]);
       }
+    };
+    auto pairs = [&](const double4 &A0, const double4 &B0, const double4 &A1, const double4 &B1) {
+      const double R0 = sep(A0), R1 = sep(A1);
+      double       r0 = 0.0, r1 = 0.0, x0, x1;  // PSE: 1 / s_ij
+      if (MODE == GAUSS_PSE) {
+        r0 = rsqrt64(s2i + A0.w), r1 = rsqrt64(s2i + A1.w);
+        x0 = 0.5 * R0 * (r0 * r0), x1 = 0.5 * R1 * (r1 * r1);
+      } else x0 = R0 * A0.w, x1 = R1 * A1.w;
+      x0 = exp64_arg(x0), x1 = exp64_arg(x1);
+      add(A0, B0, R0, r0, x0);
+      add(A1, B1, R1, r1, x1);
     };
     for (int g0 = q0; g0 < q1; g0 += SEG) {
       const int nseg = min(SEG, q1 - g0);
@@ -604,10 +617,7 @@ __global__ __launch_bounds__(BLK) void k_gauss(const int4 *__restrict__ units, c
         for (int e = cnt + lane; e < T2 * S; e += BLK) sv[2 * e] = pad, sv[2 * e + 1] = none;
         __syncthreads();
         const double4 *ps = sv + 2 * (lane_on ? si : 0);
-        for (int k = 0; k < T2; k += 2, ps += 4 * S) {
-          pair(ps[0], ps[1]);
-          pair(ps[2 * S], ps[2 * S + 1]);
-        }
+        for (int k = 0; k < T2; k += 2, ps += 4 * S) pairs(ps[0], ps[1], ps[2 * S], ps[2 * S + 1]);
         __syncthreads();
       }
     }

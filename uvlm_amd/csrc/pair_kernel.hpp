@@ -206,12 +206,15 @@ __device__ __forceinline__ double fma_sc(double a, double b, double c)
   return d;
 }
 
-// e^{-x} for x >= 0 (0 from x = 745 on).  c: c_exp64, or here(c_exp64) where the call is rare.
+// An exponent of exp64_neg: what lies beyond 800 is 800 there.  NaN stays NaN, as it does in exp (fmin
+// would make 800 of it, and a body with a NaN coordinate would add 0).
+__device__ __forceinline__ double exp64_arg(double x) { return x > 800.0 ? 800.0 : x; }
+
+// e^{-x} for 0 <= x <= 800 (0 from x = 745 on).  c: c_exp64, or here(c_exp64) where the call is rare.
 template <class C> __device__ __forceinline__ double exp64_neg(double x, C c)
 {
-  const double xe = fmin(x, 800.0);
-  const double k  = rint(xe * -1.4426950408889634);
-  const double r  = fma(k, -2.3190468138462996e-17, fma(k, -0.6931471805599453, -xe))  /* ln 2 in two parts */;
+  const double k  = rint(x * -1.4426950408889634);
+  const double r  = fma(k, -2.3190468138462996e-17, fma(k, -0.6931471805599453, -x))  /* ln 2 in two parts */;
   double       p  = c[NEXP64 - 1];
 #pragma unroll
   for (int i = NEXP64 - 2; i >= 0; i--) p = fma_sc(p, r, c[i]);
