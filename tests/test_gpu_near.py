@@ -180,3 +180,76 @@ def test_nan_coordinates_show_in_the_vorticity(n, m, ncrit):
     badp[m // 2, 0] = np.nan
     got = vorticity(X, badp)
     assert np.isnan(got[m // 2]).all() and np.isfinite(np.delete(got, m // 2, 0)).all()
+
+
+@pytest.mark.parametrize("sigma", [1e-30, 1e-40, 1e-62, 1e-104, 1e-120, 1e-150])
+def test_tiny_cores(orc, sigma):
+    """FP64 with cores so small that powers of 1 / sigma leave the range of a double: the singular
+    kernel, as the reference's formula gives it (f1 and f2 there have R alone in them).  Same bars as
+    for ordinary cores."""
+    n, m = 200, 40
+    X, A, _ = cluster(n, 11, 1.0)
+    S = np.full(n, sigma)
+    ref_b = orc.make_bodies(X, A, S)
+    ref = orc.Calculator(P=6, theta=0.5, ncrit=64)
+    ref.init(ref_b)
+    ref.calculate()
+    want = ref.bodies(n)
+    print(f"[near] sigma={sigma}", flush=True)
+    g = FMMCalculator(P=6, theta=0.5, ncrit=64)
+    g.set_bodies(make_bodies(X, A, S))
+    g.build()
+    g.calculate()
+    got = g.copyBodies2Host()
+    for sl in (slice(0, 9), slice(15, 18), slice(18, 21)):
+        assert rel(got[:, sl], want[:, sl]) < 1e-10
+    xt = np.concatenate([X[:m], X[:m] + 0.01])
+    at = A[: 2 * m]
+    u, J, D = g.direct(xt, at)
+    wu, wJ = orc.direct(xt, X, A, S)
+    assert rel(u, wu) < 1e-12 and rel(J, wJ.reshape(-1, 9)) < 1e-11
+    s, w = make_bodies(X[:m] + 0.01, A[:m], np.ones(m)), orc.make_bodies(X[:m] + 0.01, A[:m], np.ones(m))
+    g.vorticity(s)
+    ref.vorticity(w)
+    assert np.array_equal(s[:, 21:24], w[:, 21:24])  # e^{-R^2 / 2 sigma^2} = 0
+    g.close()
+    # both sides of the adjoint's near pairs, one leaf
+    g = FMMCalculator(P=6, theta=0.5, ncrit=1024)
+    g.set_arrays(X, A, S)
+    g.build()
+    ub, ab = A[::-1].copy(), X[::-1].copy()
+    xb, alb = g.eval_vjp(ub, ab)
+    arr = g.arrays()
+    exb, ealb = orc.direct_vjp(arr["X"], arr["alpha"], arr["sigma"], ub, ab, "transposed")
+    assert rel(xb, exb) < 1e-10 and rel(alb, ealb) < 1e-10
+    g.close()
+
+
+def test_bodies_without_a_core(orc):
+    """sigma = 0 or NaN leaves a body without a near kernel; it still skips itself.  Two such bodies in
+    leaves apart see each other through the far field alone and stay finite, in the rates, the direct
+    sum and both sides of the adjoint; any other near pair is neither finite."""
+    X = np.array([[0.0, 0.0, 0.0], [1.0, 1.1, 0.9]])
+    A = np.array([[1.0, -0.5, 0.3], [0.2, 0.7, -0.4]])
+    for S in (np.zeros(2), np.array([0.1, np.nan])):
+        ref_b = orc.make_bodies(X, A, S)
+        ref = orc.Calculator(P=4, theta=0.9, ncrit=1)
+        ref.init(ref_b)
+        ref.calculate()
+        want = ref.bodies(2)
+        print(f"[near] sigma={S}", flush=True)
+        g = FMMCalculator(P=4, theta=0.9, ncrit=1)
+        g.set_bodies(make_bodies(X, A, S))
+        g.build()
+        assert g.timings()["n_m2l_pairs"] > 0
+        g.calculate()
+        got = g.copyBodies2Host()
+        assert np.isfinite(want[:, :9]).all() and np.isfinite(want[:, 15:21]).all()
+        for sl in (slice(0, 9), slice(15, 18), slice(18, 21)):
+            assert rel(got[:, sl], want[:, sl]) < 1e-10
+        xb, ab = g.eval_vjp(A, X)
+        assert np.isfinite(xb).all() and np.isfinite(ab).all()
+        g.set_bodies(make_bodies(X[1:], A[1:], S[1:]))
+        u, J, _ = g.direct(np.concatenate([X[1:], X[:1]]))
+        assert np.all(u[0] == 0) and np.all(J[0] == 0) and not np.isfinite(u[1]).any() and not np.isfinite(J[1]).any()
+        g.close()

@@ -54,7 +54,7 @@ __device__ __forceinline__ void pair_g(float r2, float q, float &G, float &Gp, f
 __device__ __forceinline__ void pair_g(double r2, double q, double &G, double &Gp, double &Gpp)
 {
   const double x = r2 * q;
-  if ((unsigned)__double2hiint(x) < X64_HI) {
+  if (__double2hiint(x) < (int)X64_HI) {  // (x <= -0, of a core without a kernel, too: see core_q64)
     const double t = x - 0.5 * X64;
     double       g = c_g64[NG64 - 1], p = c_gp64[NG64 - 1], d = c_gpp64[NGPP64 - 1];
 #pragma unroll
@@ -124,7 +124,7 @@ __global__ __launch_bounds__(BLK) void k_p2p_adj(const int4 *__restrict__ units,
       for (int d = 0; d < 3; d++) al[d] = (T)st[(F_A + d) * cap + bi];
       sgd = st[F_SIG * cap + bi];
     }
-    const double oqd = 0.5 / (sgd * sgd), oc1 = oqd * sqrt(oqd) * INV_4PI;
+    const double oqd = MIXED ? 0.5 / (sgd * sgd) : core_q64(sgd), oc1 = pow32(oqd) * INV_4PI;
     const T      o_q = (T)oqd, o_c1 = (T)oc1, o_c2 = (T)(2.0 * oqd * oc1), o_c3 = (T)(4.0 * oqd * oqd * oc1);
     double       ax[3] = {0, 0, 0}, aa[3] = {0, 0, 0};
     for (int g0 = q0; g0 < q1; g0 += SEG) {
@@ -148,10 +148,10 @@ __global__ __launch_bounds__(BLK) void k_p2p_adj(const int4 *__restrict__ units,
           v[1] = (T)(st[(F_X + 1) * cap + bj] - cyt);
           v[2] = (T)(st[(F_X + 2) * cap + bj] - czt);
           if (SIDE == 0) {
-            const double sg = st[F_SIG * cap + bj], qq = 0.5 / (sg * sg);
+            const double sg = st[F_SIG * cap + bj], qq = MIXED ? 0.5 / (sg * sg) : core_q64(sg);
             v[3] = (T)qq;
             for (int d = 0; d < 3; d++) v[4 + d] = (T)st[(F_A + d) * cap + bj];
-            const double c1 = qq * sqrt(qq) * INV_4PI;
+            const double c1 = pow32(qq) * INV_4PI;
             v[7] = (T)c1, v[8] = (T)(2.0 * qq * c1), v[9] = (T)(4.0 * qq * qq * c1);
           } else {
             double Jd[9];

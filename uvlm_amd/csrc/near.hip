@@ -128,7 +128,7 @@ __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(MIXED ? 5 :
             rzi = (T)(tst[(F_X + 2) * tcap + bi] - czt);
     // target-sigma constants (TSIG only)
     const double tsg = TSIG ? tst[F_SIG * tcap + bi] : 1.0;
-    const double tqq = 0.5 / (tsg * tsg), tc1 = tqq * sqrt(tqq) * INV_4PI;
+    const double tqq = MIXED ? 0.5 / (tsg * tsg) : core_q64(tsg), tc1 = pow32(tqq) * INV_4PI;
     const T      t_q = (T)tqq, t_c1 = (T)tc1, t_c2 = (T)(2.0 * tqq * tc1);
     double       acc[MIXED ? 12 : 15];
     for (int k = 0; k < (MIXED ? 12 : 15); k++) acc[k] = 0.0;
@@ -171,7 +171,7 @@ __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(MIXED ? 5 :
           if (e < cnt) {
             // (offset, q) and (alpha c1, 2 q) with q = 1 / (2 sigma^2), c1 = q^{3/2} / (4 pi): then
             // f1 = G(x) and f2 = 2 q G'(x) for the scaled strength.  TSIG keeps alpha as is.
-            const double qq = 0.5 / (sg[p] * sg[p]), c1 = TSIG ? 1.0 : qq * sqrt(qq) * INV_4PI;
+            const double qq = MIXED ? 0.5 / (sg[p] * sg[p]) : core_q64(sg[p]), c1 = TSIG ? 1.0 : pow32(qq) * INV_4PI;
             T4           A, B;
             A.x = (T)(x[p] - cxt), A.y = (T)(y[p] - cyt), A.z = (T)(z[p] - czt), A.w = (T)qq;
             B.x = (T)(ax[p] * c1), B.y = (T)(ay[p] * c1), B.z = (T)(az[p] * c1), B.w = (T)(2.0 * qq);
@@ -294,9 +294,9 @@ __global__ __launch_bounds__(DIRECT_LANES) void k_direct(int NT, int64_t m, cons
     const int T2  = 2 * ((cnt + 2 * S - 1) / (2 * S));  // entries per lane; T2 * S <= DIRECT_LANES as NT is even
     double4   A, B;
     if (tid < cnt) {
-      const double qq = 0.5 / (v[6] * v[6]);
+      const double qq = core_q64(v[6]);
       A.x = v[0], A.y = v[1], A.z = v[2], A.w = qq;
-      B.x = v[3], B.y = v[4], B.z = v[5], B.w = qq * sqrt(qq) * INV_4PI;
+      B.x = v[3], B.y = v[4], B.z = v[5], B.w = pow32(qq) * INV_4PI;
     } else {  // no strength, x near 1 for targets within some hundred units (see k_p2p)
       A.x = v[0] + 1024.0, A.y = v[1], A.z = v[2], A.w = 0x1p-20;
       B.x = B.y = B.z = B.w = 0.0;
@@ -601,7 +601,8 @@ __global__ __launch_bounds__(BLK) void k_gauss(const int4 *__restrict__ units, c
           const int e = lane + p * BLK;
           if (e < cnt) {
             const double sg = v[p][6], S2 = 2.0 * sg * sg;
-            const double c  = MODE == GAUSS_PSE ? 1.0 : (INV_PI * INV_SQRTPI * 0.70710678118654752440) / S2 / sg;
+            double       c  = MODE == GAUSS_PSE ? 1.0 : (INV_PI * INV_SQRTPI * 0.70710678118654752440) / S2 / sg;
+            if (MODE == GAUSS_VORT && S2 > 0.0) c = fmax(fmin(c, 1e290), -1e290);  // no infinity times e = 0
             double4      A, B;
             A.x = v[p][0], A.y = v[p][1], A.z = v[p][2], A.w = MODE == GAUSS_PSE ? sg * sg : 1.0 / S2;
             B.x = v[p][3] * c, B.y = v[p][4] * c, B.z = v[p][5] * c;

@@ -243,21 +243,35 @@ __device__ __forceinline__ void g64_far(double x, double &G, double &Gp, double 
   if (D2) Gpp = w2 * fma(-2.5, Gp, -ce);
 }
 
+// q = 1 / (2 sigma^2) of the FP64 factors.  The powers of q that scale G, G' and G'' (to q^{7/2}) stay in
+// range with G itself (from x^{-3/2} down) for q <= Q64_MAX; a smaller core (sigma < 7e-36) acts as
+// that one, with the same factors from R = 7e-35 on, where g = 1 either way.  A core without a kernel
+// (sigma = 0 or NaN, so q infinite or NaN) is marked by a negative q: a coincident pair is still skipped,
+// and any other takes a polynomial far outside its range, to infinity or NaN.
+constexpr double Q64_MAX = 1e70;
+__device__ __forceinline__ double core_q64(double sg)
+{
+  const double q = 0.5 / (sg * sg);
+  return q < INFINITY ? fmin(q, Q64_MAX) : -Q64_MAX;
+}
+// |q|^{3/2}
+__device__ __forceinline__ double pow32(double q) { return fabs(q) * sqrt(fabs(q)); }
+
 // G and G' of two pairs at x = R^2 q.  A coincident pair (R^2 = 0) is skipped
 // (multipoleKernels.hpp:242): only the f1 alpha terms survive a zero separation, so G = 0 is enough.
 // The common path is taken where both x lie in (0, X64), one unsigned test of each high word (x
-// below 2^-1022 counts as 0 there and is looked at again).
+// below 2^-1022 counts as 0 there and is looked at again, and so is x <= -0, of a negative q).
 __device__ __forceinline__ void g64_pair2(double r20, double r21, double q0, double q1, double &G0, double &Gp0,
                                           double &G1, double &Gp1)
 {
-  const double   x0 = r20 * q0, x1 = r21 * q1;
-  const unsigned h0 = (unsigned)__double2hiint(x0), h1 = (unsigned)__double2hiint(x1);
+  const double x0 = r20 * q0, x1 = r21 * q1;
+  const int    h0 = __double2hiint(x0), h1 = __double2hiint(x1), far = (int)X64_HI;
   G0 = G1 = Gp0 = Gp1 = 0.0;
-  if (min(h0, h1) < X64_HI) g64_near(x0 - 0.5 * X64, x1 - 0.5 * X64, G0, Gp0, G1, Gp1);
-  if (max(h0 - 1u, h1 - 1u) >= X64_HI - 1u) {
+  if (min(h0, h1) < far) g64_near(x0 - 0.5 * X64, x1 - 0.5 * X64, G0, Gp0, G1, Gp1);
+  if (max((unsigned)h0 - 1u, (unsigned)h1 - 1u) >= X64_HI - 1u) {
     double d2;
-    if (h0 >= X64_HI) g64_far<false>(x0, G0, Gp0, d2);
-    if (h1 >= X64_HI) g64_far<false>(x1, G1, Gp1, d2);
+    if (h0 >= far) g64_far<false>(x0, G0, Gp0, d2);
+    if (h1 >= far) g64_far<false>(x1, G1, Gp1, d2);
     if (r20 == 0.0) G0 = 0.0;
     if (r21 == 0.0) G1 = 0.0;
   }
