@@ -253,3 +253,39 @@ def test_bodies_without_a_core(orc):
         u, J, _ = g.direct(np.concatenate([X[1:], X[:1]]))
         assert np.all(u[0] == 0) and np.all(J[0] == 0) and not np.isfinite(u[1]).any() and not np.isfinite(J[1]).any()
         g.close()
+
+
+@pytest.mark.parametrize("rows", ["0", "40", "3000"])
+def test_units_without_room_for_their_partial_sums(monkeypatch, rows):
+    """Lists cut again with fewer rows of partial sums, down to one unit a leaf: the same pairs in another
+    order, so 1e-12 bounds the rounding of the FP64 sums with two orders to spare."""
+    n, m = 6000, 300
+    X, A, S = cluster(n, 8, 0.05)
+    pts, w = X[:: n // m][:m] + 0.003, A[:m]
+
+    def values():
+        g = FMMCalculator(P=4, theta=0.5, ncrit=64)
+        g.set_bodies(make_bodies(X, A, S))
+        out = []
+        for _ in range(2):  # the second build makes its units ahead
+            g.build()
+            g.calculate()
+        g.set_viscosity("pse", 0.3)
+        g.viscosity(0.01)
+        out += [g.copyBodies2Host()[:, k] for k in (slice(0, 9), slice(15, 18), slice(18, 21))]
+        s = make_bodies(pts, w, np.ones(m))
+        g.getSensorData(s)
+        out.append(s[:, 15:18])
+        s = make_bodies(pts, w, np.ones(m))
+        g.vorticity(s)
+        out.append(s[:, 21:24])
+        g.set_viscosity("inviscid", 0.0)
+        out += list(g.probe_adjoint(pts, w)) + list(g.eval_vjp(A, X))
+        g.close()
+        return out
+
+    want = values()
+    monkeypatch.setenv("UVLM_NEAR_ROWS", rows)
+    print(f"[near] rows {rows}", flush=True)
+    for got, ref in zip(values(), want):
+        assert rel(got, ref) < 1e-12

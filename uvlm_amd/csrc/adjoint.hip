@@ -532,7 +532,6 @@ void p2p_adj(hipStream_t s, Scratch &sc, const Tree &t, const Lists &l, int side
 {
   if (t.nleaf == 0) return;
   if (l.n_units < t.nleaf) throw Error(UVLM_ERR_INTERNAL, "near-field adjoint without its units");
-  sc.p2p_part.reserve(sizeof(double) * 12 * l.n_rows);
   double        *part = sc.p2p_part.as<double>();
   const int32_t *lv = t.leaves.as<int32_t>(), *cb = t.body.as<int32_t>(), *cn = t.nbody.as<int32_t>();
   auto           launch = [&](auto kern, int blk) {

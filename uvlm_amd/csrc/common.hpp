@@ -22,6 +22,7 @@
 #include "../../include/uvlm_fmm.h"
 
 #include "m2l_plan.hpp"
+#include "near_units.hpp"
 
 namespace uvlm {
 
@@ -146,7 +147,8 @@ struct Scratch {
   DevBuf partial, counters, perm;
   DevBuf front0, front1, out_p2p, out_m2l, row_cnt, row_off, row_place, row_long;
   HostWords back;              // totals that the host waits for
-  DevBuf unit_work, p2p_part;  // near-field units: work per leaf, totals, partial sums
+  DevBuf unit_work, p2p_part;  // near-field units: work per leaf, partial sums
+  int64_t near_rows = INT64_MAX;  // rows of partial sums from which their room counts as refused (tests)
   DevBuf m2l_seg, m2l_part;  // M2L list segments and their partial sums (few-target case)
 };
 
@@ -215,8 +217,8 @@ void l2p_stretch(hipStream_t s, int P, const Tree &t, const double2 *L, double *
 // near.hip
 // np2p: the list's size, on the device
 void near_units_enqueue(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &st, int64_t max_leaf,
-                        const unsigned long long *np2p, bool cleared, Lists &l);
-void near_units_set(const unsigned long long *counters, Lists &l);
+                        const unsigned long long *np2p, bool cleared, Lists &l, uint64_t rows = UNITS_ROWS_MAX);
+bool near_units_set(Scratch &sc, const unsigned long long *counters, Lists &l);
 void p2p(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &stree, const Lists &l, const double *tgt, int64_t tcap,
          const double *src, int64_t scap, double *out, int64_t ocap, int precision, int sensor_mode);
 

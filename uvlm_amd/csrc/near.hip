@@ -20,7 +20,6 @@
 // trip count for all lanes), per-chunk FP32 partial sums added into FP64 per-target
 // accumulators; G = g/s^3 and its derivative from pair_kernel.hpp.
 #include "common.hpp"
-#include "near_units.hpp"
 #include "pair_kernel.hpp"
 
 #include <vector>
@@ -365,7 +364,7 @@ void direct(hipStream_t s, int64_t m, const double *xt, const double *at, const 
 }
 
 // Totals of the near-field units (near_units.hpp).
-enum { NU_INTER = 0, NU_WORK, NU_UNITS, NU_ROWS, NU_MULTI, NU_WIDE, NU_COUNT };
+enum { NU_INTER = 0, NU_WORK, NU_ROWWORK, NU_UNITS, NU_ROWS, NU_MULTI, NU_WIDE, NU_COUNT };
 static_assert(UNIT_COUNTERS + NU_COUNT <= N_COUNTERS, "near-field unit totals");
 
 // Lanes per near-field workgroup.  With 64 lanes a leaf of 33..64 targets leaves up to half of them
@@ -385,7 +384,7 @@ __global__ void k_units_clear(unsigned long long *__restrict__ cnt)
   if (threadIdx.x < NU_COUNT) cnt[threadIdx.x] = 0;
 }
 
-// work[w] (lane steps) of each target leaf and the sums over all: interactions, work.  One
+// work[w] (lane steps) of each target leaf and the sums over all: interactions, work, targets times work.  One
 // wavefront per leaf at a time, lanes over its list; at most UNITS_WORK_BLOCKS blocks keep the
 // same-address atomics few.
 constexpr int UNITS_WORK_BLOCKS = 512;
@@ -396,11 +395,11 @@ __global__ __launch_bounds__(256) void k_units_work(const int32_t *__restrict__ 
                                                     const int32_t *__restrict__ snbody, uint32_t *__restrict__ work,
                                                     unsigned long long *__restrict__ cnt)
 {
-  __shared__ unsigned long long sum[2][4];
+  __shared__ unsigned long long sum[3][4];
   const bool                    wide = units_wide(nleaf, max_leaf, *np2p);
   if (blockIdx.x == 0 && threadIdx.x == 0) cnt[NU_WIDE] = wide;
   const int          lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  unsigned long long inter = 0, all = 0;
+  unsigned long long inter = 0, all = 0, rows = 0;
   for (int64_t w = blockIdx.x * 4ll + wv; w < nleaf; w += gridDim.x * 4ll) {
     const int t = leaves[w], nt = tnbody[t], q1 = off[t + 1];
     unsigned  ns = 0;
@@ -414,10 +413,11 @@ __global__ __launch_bounds__(256) void k_units_work(const int32_t *__restrict__ 
     if (lane == 0) work[w] = wk;
     inter += (unsigned long long)nt * ns;
     all += wk;
+    rows += (unsigned long long)nt * wk;
   }
-  if (lane == 0) sum[0][wv] = inter, sum[1][wv] = all;
+  if (lane == 0) sum[0][wv] = inter, sum[1][wv] = all, sum[2][wv] = rows;
   __syncthreads();
-  if (threadIdx.x < 2) {
+  if (threadIdx.x < 3) {
     unsigned long long v = 0;
     for (int k = 0; k < 4; k++) v += sum[threadIdx.x][k];
     if (v) atomicAdd(&cnt[threadIdx.x], v);
@@ -429,14 +429,14 @@ __global__ __launch_bounds__(256) void k_units_work(const int32_t *__restrict__ 
 __global__ __launch_bounds__(256) void k_units_fill(const int32_t *__restrict__ leaves, int64_t nleaf,
                                                     const int32_t *__restrict__ tnbody,
                                                     const int32_t *__restrict__ off,
-                                                    const uint32_t *__restrict__ work,
+                                                    const uint32_t *__restrict__ work, uint64_t rows,
                                                     unsigned long long *__restrict__ cnt, int4 *__restrict__ units,
                                                     int4 *__restrict__ multi)
 {
   __shared__ unsigned long long tot[4][3], base[3];
   const int64_t            w    = blockIdx.x * 256ll + threadIdx.x;
   const int                lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const uint64_t           lim = units_limit(cnt[NU_WORK]);
+  const uint64_t           lim = units_limit(cnt[NU_WORK], cnt[NU_ROWWORK], rows);
   int                      nu = 0, q0 = 0, len = 0, nt = 0;  // no units past the last leaf
   if (w < nleaf) {
     const int t = leaves[w];
@@ -659,9 +659,10 @@ __global__ __launch_bounds__(256) void k_gauss_reduce(const int4 *__restrict__ m
 }
 
 // Units of the P2P list `l` (np2p entries, on the device) of target tree tt against source tree st
-// (see k_units_work), and the number of near-field interactions.  cleared: the units' counters are zero.
+// (see k_units_work), and the number of near-field interactions.  cleared: the units' counters are
+// zero.  rows: the rows of partial sums they may have.
 void near_units_enqueue(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &st, int64_t max_leaf,
-                        const unsigned long long *np2p, bool cleared, Lists &l)
+                        const unsigned long long *np2p, bool cleared, Lists &l, uint64_t rows)
 {
   if (tt.nleaf == 0) return;
   sc.unit_work.reserve(4 * tt.nleaf);
@@ -674,20 +675,30 @@ void near_units_enqueue(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &
   k_units_work<<<(int)std::min<int64_t>(UNITS_WORK_BLOCKS, (tt.nleaf + 3) / 4), 256, 0, s>>>(
       lv, tt.nleaf, max_leaf, np2p, tn, off, l.p2p_src.as<int32_t>(), st.nbody.as<int32_t>(),
       sc.unit_work.as<uint32_t>(), cnt);
-  k_units_fill<<<(int)((tt.nleaf + 255) / 256), 256, 0, s>>>(lv, tt.nleaf, tn, off, sc.unit_work.as<uint32_t>(), cnt,
-                                                             l.units.as<int4>(), l.multi.as<int4>());
+  k_units_fill<<<(int)((tt.nleaf + 255) / 256), 256, 0, s>>>(lv, tt.nleaf, tn, off, sc.unit_work.as<uint32_t>(), rows,
+                                                             cnt, l.units.as<int4>(), l.multi.as<int4>());
   UVLM_LAUNCH_CHECK();
 }
 
-// Takes over what near_units_enqueue left at counters[UNIT_COUNTERS ..], read back by the caller.
-void near_units_set(const unsigned long long *h, Lists &l)
+// Takes over what near_units_enqueue left at counters[UNIT_COUNTERS ..], read back by the caller, and
+// reserves the partial sums.  False where the device has no room for them: the caller makes the units
+// again with fewer rows (none at last), so that no call fails for the sake of its units.
+bool near_units_set(Scratch &sc, const unsigned long long *h, Lists &l)
 {
   l.n_interactions = (int64_t)h[NU_INTER];
   l.n_units        = (int64_t)h[NU_UNITS];
   l.n_rows         = (int64_t)h[NU_ROWS];
   l.n_multi        = (int64_t)h[NU_MULTI];
   l.wide           = h[NU_WIDE] != 0;
-  if (l.n_rows >= (int64_t(1) << 31)) throw Error(UVLM_ERR_INTERNAL, "near-field partial rows");
+  if (l.n_rows > sc.near_rows) return false;
+  try {
+    sc.p2p_part.reserve(sizeof(double) * 12 * l.n_rows);
+  } catch (const Error &e) {
+    if (e.code != UVLM_ERR_NOMEM) throw;
+    (void)hipGetLastError();
+    return false;
+  }
+  return true;
 }
 
 // sensor_mode: 0 particles (u and J), 1 probes (u only), 2 adjoint (u and J, target sigma).
@@ -696,7 +707,6 @@ void p2p(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &stree, const Li
 {
   if (tt.nleaf == 0) return;
   if (l.n_units < tt.nleaf) throw Error(UVLM_ERR_INTERNAL, "P2P without its units");
-  sc.p2p_part.reserve(sizeof(double) * 12 * l.n_rows);
   double    *part  = sc.p2p_part.as<double>();
   const bool mixed = precision == UVLM_MIXED;
   auto       launch = [&](auto kern, int blk) {
@@ -737,7 +747,6 @@ void gauss_near(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &stree, c
 {
   if (tt.nleaf == 0) return;
   if (l.n_units < tt.nleaf) throw Error(UVLM_ERR_INTERNAL, "Gaussian near field without its units");
-  sc.p2p_part.reserve(sizeof(double) * 12 * l.n_rows);
   double        *part = sc.p2p_part.as<double>();
   const int32_t *lv = tt.leaves.as<int32_t>(), *tb = tt.body.as<int32_t>(), *tn = tt.nbody.as<int32_t>();
   auto           launch = [&](auto kern, int blk) {

@@ -1177,6 +1177,18 @@ static void rows_by_sorting(hipStream_t s, Scratch &sc, int64_t C, int64_t Cs, L
   }
 }
 
+// The near-field units as read back into cnt, made again with fewer rows of partial sums while there is no
+// room for them.
+static void take_units(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &st, int64_t max_leaf,
+                       unsigned long long *cnt, Lists &l)
+{
+  unsigned long long *dcnt = sc.counters.as<unsigned long long>();
+  while (!near_units_set(sc, cnt + UNIT_COUNTERS, l)) {
+    near_units_enqueue(s, sc, tt, st, max_leaf, dcnt + TC_P2P, false, l, (uint64_t)l.n_rows / 8);
+    to_host(s, sc, cnt, dcnt, N_COUNTERS);
+  }
+}
+
 // max_leaf >= 0: also the lists' near-field units (near.hip), read back together with the sizes.
 void traverse(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &st, double theta, Lists &lists, double gap,
               int64_t max_leaf)
@@ -1270,7 +1282,7 @@ void traverse(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &st, double
       units();
       if (max_leaf >= 0) to_host(s, sc, cnt, dcnt, N_COUNTERS);
     }
-    if (max_leaf >= 0) near_units_set(cnt + UNIT_COUNTERS, lists);
+    if (max_leaf >= 0) take_units(s, sc, tt, st, max_leaf, cnt, lists);
     return;
   }
 }
@@ -1304,7 +1316,7 @@ void transpose_lists(hipStream_t s, Scratch &sc, const Tree &in_targets, const T
     near_units_enqueue(s, sc, in_sources, in_targets, max_leaf, dcnt + TC_P2P, sorted, out);
     to_host(s, sc, cnt, dcnt, N_COUNTERS);
   }
-  near_units_set(cnt + UNIT_COUNTERS, out);
+  take_units(s, sc, in_sources, in_targets, max_leaf, cnt, out);
 }
 
 }  // namespace uvlm
