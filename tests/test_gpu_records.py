@@ -48,3 +48,47 @@ def test_arrays_round_trip(n):
     g.update_arrays(X=X[::-1])
     assert np.array_equal(g.arrays()["X"], X[::-1]) and np.array_equal(g.arrays()["alpha"], a["alpha"])
     g.close()
+
+
+def test_arrays_in_several_pieces():
+    """Sets whose arrays pass the staging buffer (2^23 doubles) in more than one piece, the last of them
+    ragged: every value back in its place."""
+    n = 2 ** 23 // 3 + 1001
+    X, A, S = (np.arange(k * n, dtype=np.float64).reshape(n, -1) + 0.25 * k for k in (3, 3, 1))
+    print(f"[records] arrays in pieces n={n}", flush=True)
+    g = FMMCalculator(P=4, theta=0.5, ncrit=64)
+    g.set_arrays(X, A[::-1], S[:, 0])
+    a = g.arrays()
+    assert np.array_equal(a["X"], X) and np.array_equal(a["alpha"], A[::-1]) and np.array_equal(a["sigma"], S[:, 0])
+    assert not a["J"].any() and not a["velocity"].any()
+    g.update_arrays(X=A, alpha=X)
+    a = g.arrays()
+    assert np.array_equal(a["X"], A) and np.array_equal(a["alpha"], X)
+    n = 2 ** 23 // 9 + 77
+    b = np.arange(37.0 * n).reshape(n, 37)
+    g.set_bodies(b)
+    a = g.arrays()
+    assert np.array_equal(a["J"], b[:, :9]) and np.array_equal(a["velocity"], b[:, 15:18])
+    g.close()
+
+
+def test_one_array_takes_room_for_itself_alone():
+    """The positions alone take no room for the other arrays on the device."""
+    n = 1 << 20
+    g = FMMCalculator(P=4, theta=0.5, ncrit=64)
+    X, out = np.zeros((n, 3)), np.zeros((n, 3))
+    X[:, 1] = np.arange(n)
+    g.set_arrays(X, X, np.ones(n))
+
+    def free():
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert g.lib.hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0  # of the runtime the library is linked to
+        return a.value
+
+    before = free()
+    print("[records] one array", flush=True)
+    none = ctypes.POINTER(ctypes.c_double)()
+    _capi.check(g.lib.uvlm_get_bodies_soa(g._h, n, dp(out), none, none, none, none, none, none))
+    assert np.array_equal(out, X)
+    assert before - free() < 24 * n * 1.25 + (4 << 20)
+    g.close()

@@ -635,37 +635,47 @@ void load_state_orig(uvlm_handle h, const double *src)
 // Caller's arrays [n][nf] <-> nf fields of `cap` doubles, bodies n .. m - 1 of the fields zero (m >= n;
 // `in` null: all zero).  The arrays cross as they are and are turned on the device: turned on one host
 // core, the cotangents of 260k bodies took 6 of the VJP's 14 ms and the gradients of 1M bodies 5 ms.
-// `room` doubles into the staging buffer, which the caller has reserved; the copy is stream-ordered.
-void put_array(uvlm_handle h, const double *in, int64_t n, int64_t m, int nf, double *fields, int64_t cap,
-               int64_t room = 0)
+// They pass the staging buffer in pieces of at most STAGE_DOUBLES (64 MB), one after another on the
+// stream, so a call needs no room that grows with the bodies.
+constexpr int64_t STAGE_DOUBLES = 1 << 23;
+void put_array(uvlm_handle h, const double *in, int64_t n, int64_t m, int nf, double *fields, int64_t cap)
 {
-  double *st = h->staging.as<double>() + room;
-  if (in && n > 0) UVLM_HIP(hipMemcpyAsync(st, in, 8 * (size_t)nf * n, hipMemcpyHostToDevice, h->s));
-  records_in(h->s, st, in ? n : 0, m, nf, nf, fields, cap);
+  const int64_t rows = STAGE_DOUBLES / nf;
+  if (!in) n = 0;
+  h->staging.reserve(8 * nf * (size_t)std::min(n, rows));
+  double *st = h->staging.as<double>();
+  for (int64_t i = 0; i < m; i += rows) {
+    const int64_t k = std::min(rows, m - i), kin = std::max<int64_t>(0, std::min(k, n - i));
+    if (kin > 0) UVLM_HIP(hipMemcpyAsync(st, in + i * nf, 8 * (size_t)nf * kin, hipMemcpyHostToDevice, h->s));
+    records_in(h->s, st, kin, k, nf, nf, fields + i, cap);
+  }
 }
-void get_array(uvlm_handle h, const double *fields, int64_t cap, int64_t n, int nf, double *out, int64_t room = 0)
+void get_array(uvlm_handle h, const double *fields, int64_t cap, int64_t n, int nf, double *out)
 {
   if (!out || n <= 0) return;
-  double *st = h->staging.as<double>() + room;
-  records_out(h->s, fields, cap, n, nf, nf, st);
-  UVLM_HIP(hipMemcpyAsync(out, st, 8 * (size_t)nf * n, hipMemcpyDeviceToHost, h->s));
+  const int64_t rows = STAGE_DOUBLES / nf;
+  h->staging.reserve(8 * nf * (size_t)std::min(n, rows));
+  double *st = h->staging.as<double>();
+  for (int64_t i = 0; i < n; i += rows) {
+    const int64_t k = std::min(rows, n - i);
+    records_out(h->s, fields + i, cap, k, nf, nf, st);
+    UVLM_HIP(hipMemcpyAsync(out + i * nf, st, 8 * (size_t)nf * k, hipMemcpyDeviceToHost, h->s));
+  }
 }
 
 // Host AoS (n x 3) pairs <-> 6 SoA fields of `cap` doubles on the device.
 void upload_cot(uvlm_handle h, const double *xb, const double *ab, double *dev)
 {
   const int64_t n = h->N, cap = h->cap;
-  h->staging.reserve(8 * 6 * n);
   put_array(h, xb, n, cap, 3, dev, cap);
-  put_array(h, ab, n, cap, 3, dev + 3 * cap, cap, 3 * n);
+  put_array(h, ab, n, cap, 3, dev + 3 * cap, cap);
   UVLM_HIP(hipStreamSynchronize(h->s));
 }
 void download_cot(uvlm_handle h, const double *dev, double *xb, double *ab)
 {
   const int64_t n = h->N, cap = h->cap;
-  h->staging.reserve(8 * 6 * n);
   get_array(h, dev, cap, n, 3, xb);
-  get_array(h, dev + 3 * cap, cap, n, 3, ab, 3 * n);
+  get_array(h, dev + 3 * cap, cap, n, 3, ab);
   UVLM_HIP(hipStreamSynchronize(h->s));
 }
 
@@ -840,11 +850,10 @@ int uvlm_set_bodies_soa(uvlm_handle h, int64_t n, const double *X, const double 
     set_device(h);
     h->N = n;
     h->ensure_cap(n);
-    h->staging.reserve(8 * 7 * (size_t)n);
     zero_fields(h->s, h->st.as<double>(), h->cap, n, 0, N_FIELDS);
     put_array(h, X, n, n, 3, h->F(F_X), h->cap);
-    put_array(h, alpha, n, n, 3, h->F(F_A), h->cap, 3 * n);
-    put_array(h, sigma, n, n, 1, h->F(F_SIG), h->cap, 6 * n);
+    put_array(h, alpha, n, n, 3, h->F(F_A), h->cap);
+    put_array(h, sigma, n, n, 1, h->F(F_SIG), h->cap);
     iota(h->s, h->orig.as<int32_t>(), n);
     UVLM_HIP(hipStreamSynchronize(h->s));
     h->built = h->evaluated = false;
@@ -858,12 +867,9 @@ int uvlm_get_bodies_soa(uvlm_handle h, int64_t n, double *X, double *alpha, doub
     check_handle(h);
     if (n != h->N) throw Error(UVLM_ERR_ARG, "size mismatch");
     set_device(h);
-    h->staging.reserve(8 * 23 * (size_t)n);
-    int64_t room  = 0;
-    auto    fetch = [&](int f0, int nf, double *out) {
-      get_array(h, h->F(f0), h->cap, n, nf, out, room);
-      room += nf * n;
-    };
+    // room for the widest first: no copy is under way when the reservation fails
+    h->staging.reserve(8 * (size_t)std::min(STAGE_DOUBLES, (J ? 9 : 3) * n));
+    auto fetch = [&](int f0, int nf, double *out) { get_array(h, h->F(f0), h->cap, n, nf, out); };
     fetch(F_X, 3, X);
     fetch(F_A, 3, alpha);
     fetch(F_SIG, 1, sigma);
@@ -1130,7 +1136,7 @@ int uvlm_probe_adjoint(uvlm_handle h, int64_t m, const double *probes, const dou
     reserve_probes(h, m);
     const int64_t sc = h->scap;
     // probes as sources: X = probe, alpha = weight, sigma = 1 (the kernel takes the target's)
-    h->staging.reserve(8 * 6 * (size_t)std::max<int64_t>(m, h->N));
+    h->staging.reserve(8 * 6 * (size_t)m);
     double *pts = h->staging.as<double>(), *wts = pts + 3 * m;
     UVLM_HIP(hipMemcpyAsync(pts, probes, 24 * m, hipMemcpyHostToDevice, s));
     UVLM_HIP(hipMemcpyAsync(wts, weights, 24 * m, hipMemcpyHostToDevice, s));
@@ -1141,7 +1147,7 @@ int uvlm_probe_adjoint(uvlm_handle h, int64_t m, const double *probes, const dou
     const int64_t cap = h->cap, N = h->N;
     double       *a   = h->ast.as<double>();
     get_array(h, a + F_U * cap, cap, N, 3, dJ_dalpha);
-    get_array(h, a + F_DADT * cap, cap, N, 3, dJ_dx, 3 * N);
+    get_array(h, a + F_DADT * cap, cap, N, 3, dJ_dx);
     UVLM_HIP(hipStreamSynchronize(s));
     h->tm.adjoint_ms = ev_ms2(h, 0, 1);
   });
@@ -1954,9 +1960,8 @@ int uvlm_update_bodies_soa(uvlm_handle h, int64_t n, const double *X, const doub
     check_handle(h);
     if (n != h->N) throw Error(UVLM_ERR_ARG, "size mismatch");
     set_device(h);
-    h->staging.reserve(8 * 6 * (size_t)n);
     if (X) put_array(h, X, n, n, 3, h->F(F_X), h->cap);
-    if (alpha) put_array(h, alpha, n, n, 3, h->F(F_A), h->cap, 3 * n);
+    if (alpha) put_array(h, alpha, n, n, 3, h->F(F_A), h->cap);
     UVLM_HIP(hipStreamSynchronize(h->s));
     h->evaluated = false;
   });
@@ -1968,8 +1973,10 @@ int uvlm_direct(uvlm_handle h, int64_t m, const double *xt, const double *at, do
     check_direct_args(h, m, xt, at, u, dadt);
     set_device(h);
     const int64_t nin = 3 * m + (at ? 3 * m : 0), nout = 3 * m + (J ? 9 * m : 0) + (dadt ? 3 * m : 0);
-    h->staging.reserve(sizeof(double) * (nin + nout));
-    direct_staged(h, m, xt, at, u, J, dadt, h->staging.as<double>());
+    DevBuf  large;  // what the handle does not keep
+    DevBuf &buf = nin + nout <= STAGE_DOUBLES ? h->staging : large;
+    buf.reserve(sizeof(double) * (nin + nout));
+    direct_staged(h, m, xt, at, u, J, dadt, buf.as<double>());
   });
 }
 
