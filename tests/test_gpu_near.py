@@ -289,3 +289,134 @@ def test_units_without_room_for_their_partial_sums(monkeypatch, rows):
     print(f"[near] rows {rows}", flush=True)
     for got, ref in zip(values(), want):
         assert rel(got, ref) < 1e-12
+
+
+def groups(k, size, seed):
+    """k groups of `size` bodies in different octants: k leaves at ncrit = size."""
+    rng = W.SplitMix64(seed)
+    c = np.array([[-1.0 if i >> d & 1 else 1.0 for d in range(3)] for i in (0, 7, 1, 6, 2, 5, 3)[:k]])
+    X = np.repeat(c, size, 0) * 0.5 + 0.2 * (rng.uniform(3 * k * size).reshape(-1, 3) - 0.5)
+    return X, rng.normal(3 * k * size).reshape(-1, 3), np.full(k * size, 0.1) * (0.5 + rng.uniform(k * size))
+
+
+def pair_factors(r2, sigma):
+    """f1, f2 = 2 df1/dR^2 and f3 = 2 df2/dR^2: the power series of G below x = 2, where the closed form
+    loses x^-3 of its digits to cancellation, and that form above."""
+    from scipy.special import erf
+
+    q = 0.5 / (sigma * sigma)
+    x = r2 * q
+    G = np.zeros((3,) + x.shape)
+    near = x < 2.0
+    k, c, power = 2.0 / np.sqrt(np.pi), 1.0, [np.zeros(near.sum()), np.zeros(near.sum()), np.ones(near.sum())]
+    for i in range(50):  # sum (-1)^i 2 / ((2 i + 3) i!) x^i and its derivatives
+        c = -c / i if i else 1.0  # (-1)^i / i!
+        a = k * c * 2.0 / (2 * i + 3)
+        for d, f in enumerate((1, i, i * (i - 1))):
+            G[d][near] += a * f * power[2 - d]
+        power = [power[1], power[2], power[2] * x[near]]
+    xf = x[~near]
+    e = k * np.exp(-xf)
+    G[0][~near] = (erf(np.sqrt(xf)) - e * np.sqrt(xf)) * xf ** -1.5
+    G[1][~near] = (e - 1.5 * G[0][~near]) / xf
+    G[2][~near] = (-e - 2.5 * G[1][~near]) / xf
+    c1 = q * np.sqrt(q) / (4.0 * np.pi)
+    return [np.where(r2 == 0.0, 0.0, f)[..., None] for f in (G[0] * c1, 2 * G[1] * q * c1, 4 * G[2] * q * q * c1)]
+
+
+def direct_vjp(X, A, S, ub, ab):
+    """xbar and alphabar of sum ub.u + ab.(J^T alpha) over all pairs, in plain numpy: with r = x_i - x_j and
+    Jbar_i = alpha_i (x) ab_i, e its axial vector, pair ij adds -alpha_j . (f1 (ub_i x r + e_i) + f2 (Jbar_i
+    r) x r) to it."""
+    n = len(X)
+    xb, alb = np.zeros((n, 3)), np.zeros((n, 3))
+    Jb = A[:, :, None] * ab[:, None, :]
+    e = np.stack([Jb[:, 1, 2] - Jb[:, 2, 1], Jb[:, 2, 0] - Jb[:, 0, 2], Jb[:, 0, 1] - Jb[:, 1, 0]], 1)
+    for c in range(0, n, 200):
+        i = slice(c, c + 200)
+        r = X[i, None] - X[None]
+        f1, f2, f3 = pair_factors((r * r).sum(-1), np.broadcast_to(S, r.shape[:2]))
+        Jr, rxa = np.einsum("iab,ijb->ija", Jb[i], r), np.cross(r, A[None])
+        w, v = np.cross(ub[i, None], r) + e[i, None], np.cross(Jr, r)
+        c1, c3 = (A * w).sum(-1, keepdims=True), (A * v).sum(-1, keepdims=True)
+        dS = -((f2 * c1 + f3 * c3) * r + f1 * np.cross(A[None], ub[i, None]) +
+               f2 * (np.einsum("iba,ijb->ija", Jb[i], rxa) + np.cross(A[None], Jr)))
+        xb[i] += dS.sum(1)
+        xb -= dS.sum(0)
+        alb -= (f1 * w + f2 * v).sum(0)
+        J, F = -np.einsum("ija,ijb->iab", f2 * rxa, r), (f1 * A).sum(1)
+        for a, b, k, sign in ((0, 1, 2, 1), (1, 2, 0, 1), (2, 0, 1, 1), (1, 0, 2, -1), (2, 1, 0, -1), (0, 2, 1, -1)):
+            J[:, a, b] -= sign * F[:, k]
+        alb[i] += np.einsum("iab,ib->ia", J, ab[i])
+    return xb, alb
+
+
+@pytest.mark.parametrize("kind,n,ncrit", [("groups", 4, 40), ("groups", 7, 64), ("groups", 6, 1), ("cluster", 900, 7),
+                                          ("cluster", 3000, 20), ("cluster", 3000, 100), ("cluster", 2000, 600)])
+def test_adjoint_pairs(kind, n, ncrit):
+    """Both sides of the adjoint's near pairs over many leaves, with lists of a few entries (64 lanes a
+    unit: the groups) and of hundreds, cut into units.  With theta 1e-3 every pair is near, so the
+    direct sum's VJP is the answer: 1e-10, mixed 1e-5, the bars of the one-leaf case.  (The oracle's
+    direct VJP is itself off by 1.3e-10 in the dense half of the 900: its factors cancel there.)"""
+    X, A, S = groups(n, ncrit, n) if kind == "groups" else cluster(n, n, 0.1)
+    rng = W.SplitMix64(n + ncrit)
+    ub, ab = (rng.normal(3 * len(X)).reshape(-1, 3) for _ in range(2))
+    for precision, bar in (("fp64", 1e-10), ("mixed", 1e-5)):
+        print(f"[near] adjoint {kind} n={n} ncrit={ncrit} {precision}", flush=True)
+        g = FMMCalculator(P=4, theta=1e-3, ncrit=ncrit, precision=precision)
+        g.set_arrays(X, A, S)
+        g.build()
+        t = g.timings()
+        assert t["n_m2l_pairs"] == 0 and t["n_leaves"] > 1
+        assert (t["n_p2p_pairs"] < 8 * t["n_leaves"]) == (kind == "groups")
+        xb, alb = g.eval_vjp(ub, ab)
+        arr = g.arrays()
+        exb, ealb = direct_vjp(arr["X"], arr["alpha"], arr["sigma"], ub, ab)
+        assert rel(xb, exb) < bar and rel(alb, ealb) < bar
+        g.close()
+
+
+@pytest.mark.parametrize("k,size", [(2, 1), (4, 40), (7, 64)])
+def test_short_lists(orc, k, size):
+    """Lists of fewer than 8 entries a leaf of at most 64 bodies: the near field, the Gaussian sums and the
+    probes with 64 lanes a unit."""
+    X, A, S = groups(k, size, k + size)
+    n = len(X)
+    ref = orc.Calculator(P=4, theta=1e-3, ncrit=size)
+    ref.init(orc.make_bodies(X, A, S))
+    ref.calculate()
+    want = ref.bodies(n)
+    ref.set_viscosity("pse", 0.3)
+    ref.viscosity(0.01)
+    pse = ref.bodies(n)
+    sb = orc.make_bodies(X + 0.003, np.zeros((n, 3)), np.ones(n))
+    sv = sb.copy()
+    ref.sensor_data(sb)
+    ref.vorticity(sv)
+    print(f"[near] short lists {k} x {size}", flush=True)
+    g = FMMCalculator(P=4, theta=1e-3, ncrit=size)
+    g.set_bodies(make_bodies(X, A, S))
+    g.build()
+    assert g.timings()["n_p2p_pairs"] < 8 * g.timings()["n_leaves"]
+    g.calculate()
+    got = g.copyBodies2Host()
+    for sl in (slice(0, 9), slice(15, 18), slice(18, 21)):
+        assert rel(got[:, sl], want[:, sl]) < 1e-10
+    g.set_viscosity("pse", 0.3)
+    g.viscosity(0.01)
+    assert rel(g.copyBodies2Host()[:, 18:21], pse[:, 18:21]) < 1e-10
+    s = make_bodies(X + 0.003, np.zeros((n, 3)), np.ones(n))
+    v = s.copy()
+    g.getSensorData(s)
+    g.vorticity(v)
+    assert rel(s[:, 15:18], sb[:, 15:18]) < 1e-10 and rel(v[:, 21:24], sv[:, 21:24]) < 1e-10
+    g.close()
+    # mixed: FP32 pair arithmetic, the bar of test_particles
+    g = FMMCalculator(P=4, theta=1e-3, ncrit=size, precision="mixed")
+    g.set_bodies(make_bodies(X, A, S))
+    g.build()
+    g.calculate()
+    mixed = g.copyBodies2Host()
+    for sl in (slice(0, 9), slice(15, 18), slice(18, 21)):
+        assert rel(mixed[:, sl], want[:, sl]) < 1e-6
+    g.close()
