@@ -292,7 +292,7 @@ def test_units_without_room_for_their_partial_sums(monkeypatch, rows):
 
 
 def groups(k, size, seed):
-    """k groups of `size` bodies in different octants: k leaves at ncrit = size."""
+    """k groups of `size` bodies in different octants: k leaves at ncrit = size, lists of k entries."""
     rng = W.SplitMix64(seed)
     c = np.array([[-1.0 if i >> d & 1 else 1.0 for d in range(3)] for i in (0, 7, 1, 6, 2, 5, 3)[:k]])
     X = np.repeat(c, size, 0) * 0.5 + 0.2 * (rng.uniform(3 * k * size).reshape(-1, 3) - 0.5)
@@ -353,11 +353,13 @@ def direct_vjp(X, A, S, ub, ab):
 
 @pytest.mark.parametrize("kind,n,ncrit", [("groups", 4, 40), ("groups", 7, 64), ("groups", 6, 1), ("cluster", 900, 7),
                                           ("cluster", 3000, 20), ("cluster", 3000, 100), ("cluster", 2000, 600)])
-def test_adjoint_pairs(kind, n, ncrit):
-    """Both sides of the adjoint's near pairs over many leaves, with lists of a few entries (64 lanes a
-    unit: the groups) and of hundreds, cut into units.  With theta 1e-3 every pair is near, so the
+@pytest.mark.parametrize("lanes", ["64", "256"])
+def test_adjoint_pairs(monkeypatch, lanes, kind, n, ncrit):
+    """Both sides of the adjoint's near pairs over many leaves, with lists of a few entries (the groups) and
+    of hundreds, cut into units, by workgroups of either width (256 alone above 64 bodies a leaf).  With theta 1e-3 every pair is near, so the
     direct sum's VJP is the answer: 1e-10, mixed 1e-5, the bars of the one-leaf case.  (The oracle's
     direct VJP is itself off by 1.3e-10 in the dense half of the 900: its factors cancel there.)"""
+    monkeypatch.setenv("UVLM_NEAR_LANES", lanes)
     X, A, S = groups(n, ncrit, n) if kind == "groups" else cluster(n, n, 0.1)
     rng = W.SplitMix64(n + ncrit)
     ub, ab = (rng.normal(3 * len(X)).reshape(-1, 3) for _ in range(2))
@@ -368,7 +370,6 @@ def test_adjoint_pairs(kind, n, ncrit):
         g.build()
         t = g.timings()
         assert t["n_m2l_pairs"] == 0 and t["n_leaves"] > 1
-        assert (t["n_p2p_pairs"] < 8 * t["n_leaves"]) == (kind == "groups")
         xb, alb = g.eval_vjp(ub, ab)
         arr = g.arrays()
         exb, ealb = direct_vjp(arr["X"], arr["alpha"], arr["sigma"], ub, ab)
@@ -376,28 +377,41 @@ def test_adjoint_pairs(kind, n, ncrit):
         g.close()
 
 
-@pytest.mark.parametrize("k,size", [(2, 1), (4, 40), (7, 64)])
-def test_short_lists(orc, k, size):
-    """Lists of fewer than 8 entries a leaf of at most 64 bodies: the near field, the Gaussian sums and the
-    probes with 64 lanes a unit."""
-    X, A, S = groups(k, size, k + size)
-    n = len(X)
-    ref = orc.Calculator(P=4, theta=1e-3, ncrit=size)
+def tube(n):
+    """n bodies along a helix: leaves of a few bodies with short lists."""
+    t = np.arange(n) / n
+    rng = W.SplitMix64(n)
+    X = np.stack([np.cos(6 * t) + 0.004 * np.cos(5000 * t), np.sin(6 * t) + 0.004 * np.sin(5000 * t), t], 1)
+    return X, rng.normal(3 * n).reshape(-1, 3), np.full(n, 1e-3)
+
+
+@pytest.mark.parametrize("lanes", ["64", "256", None])
+@pytest.mark.parametrize("kind,n,ncrit", [("groups", 2, 1), ("groups", 4, 40), ("groups", 7, 64), ("tube", 9000, 8),
+                                          ("cluster", 4000, 33)])
+def test_lanes_of_a_unit(orc, monkeypatch, lanes, kind, n, ncrit):
+    """The near field, the Gaussian sums and the probes with workgroups of 64 and of 256 lanes, and with
+    those the lists choose (64 for the tube), on lists of 2 to hundreds of entries."""
+    if lanes:
+        monkeypatch.setenv("UVLM_NEAR_LANES", lanes)
+    X, A, S = groups(n, ncrit, n + ncrit) if kind == "groups" else tube(n) if kind == "tube" else cluster(n, n, 0.02)
+    n, theta = len(X), 1e-3 if kind == "groups" else 0.5
+    pts = X[:: max(1, n // 200)] + 0.003
+    m = len(pts)
+    ref = orc.Calculator(P=4, theta=theta, ncrit=ncrit)
     ref.init(orc.make_bodies(X, A, S))
     ref.calculate()
     want = ref.bodies(n)
     ref.set_viscosity("pse", 0.3)
     ref.viscosity(0.01)
     pse = ref.bodies(n)
-    sb = orc.make_bodies(X + 0.003, np.zeros((n, 3)), np.ones(n))
+    sb = orc.make_bodies(pts, np.zeros((m, 3)), np.ones(m))
     sv = sb.copy()
     ref.sensor_data(sb)
     ref.vorticity(sv)
-    print(f"[near] short lists {k} x {size}", flush=True)
-    g = FMMCalculator(P=4, theta=1e-3, ncrit=size)
+    print(f"[near] lanes {lanes} {kind} n={n}", flush=True)
+    g = FMMCalculator(P=4, theta=theta, ncrit=ncrit)
     g.set_bodies(make_bodies(X, A, S))
     g.build()
-    assert g.timings()["n_p2p_pairs"] < 8 * g.timings()["n_leaves"]
     g.calculate()
     got = g.copyBodies2Host()
     for sl in (slice(0, 9), slice(15, 18), slice(18, 21)):
@@ -405,14 +419,14 @@ def test_short_lists(orc, k, size):
     g.set_viscosity("pse", 0.3)
     g.viscosity(0.01)
     assert rel(g.copyBodies2Host()[:, 18:21], pse[:, 18:21]) < 1e-10
-    s = make_bodies(X + 0.003, np.zeros((n, 3)), np.ones(n))
+    s = make_bodies(pts, np.zeros((m, 3)), np.ones(m))
     v = s.copy()
     g.getSensorData(s)
     g.vorticity(v)
     assert rel(s[:, 15:18], sb[:, 15:18]) < 1e-10 and rel(v[:, 21:24], sv[:, 21:24]) < 1e-10
     g.close()
     # mixed: FP32 pair arithmetic, the bar of test_particles
-    g = FMMCalculator(P=4, theta=1e-3, ncrit=size, precision="mixed")
+    g = FMMCalculator(P=4, theta=theta, ncrit=ncrit, precision="mixed")
     g.set_bodies(make_bodies(X, A, S))
     g.build()
     g.calculate()

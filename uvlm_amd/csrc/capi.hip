@@ -782,6 +782,10 @@ int uvlm_create(const uvlm_params *p, uvlm_handle *out)
     // it); UVLM_M2L_WAVES (1 or 2) the wavefronts per M2L workgroup, chosen by P otherwise
     if (const char *sb = std::getenv("UVLM_M2L_SLOTS")) h->sched.budget = std::atoi(sb);
     if (const char *sw = std::getenv("UVLM_M2L_WAVES")) h->sched.waves = std::atoi(sw);
+    // UVLM_NEAR_LANES (64 or 256) sets the lanes of a near-field workgroup over leaves of at most 64
+    // bodies, chosen by the lists otherwise
+    if (p->precision == UVLM_MIXED) h->sc.near_narrow = NARROW_MIXED;
+    if (const char *nl = std::getenv("UVLM_NEAR_LANES")) h->sc.near_lanes = std::atoi(nl);
     // UVLM_NEAR_ROWS: more rows of near-field partial sums than this count as not allocatable
     if (const char *nr = std::getenv("UVLM_NEAR_ROWS")) h->sc.near_rows = std::max<int64_t>(0, std::atoll(nr));
     make_m2l_schedule(p->P, h->sched);

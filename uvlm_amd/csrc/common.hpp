@@ -148,7 +148,9 @@ struct Scratch {
   DevBuf front0, front1, out_p2p, out_m2l, row_cnt, row_off, row_place, row_long;
   HostWords back;              // totals that the host waits for
   DevBuf unit_work, p2p_part;  // near-field units: work per leaf, partial sums
-  int64_t near_rows = INT64_MAX;  // rows of partial sums from which their room counts as refused (tests)
+  double  near_narrow = NARROW_FP64;  // units_wide: pairs a leaf below which 64 lanes are used
+  int     near_lanes  = 0;            // 64 or 256: lanes asked for
+  int64_t near_rows   = INT64_MAX;    // rows of partial sums from which their room counts as refused (tests)
   DevBuf m2l_seg, m2l_part;  // M2L list segments and their partial sums (few-target case)
 };
 

@@ -367,18 +367,6 @@ void direct(hipStream_t s, int64_t m, const double *xt, const double *at, const 
 enum { NU_INTER = 0, NU_WORK, NU_ROWWORK, NU_UNITS, NU_ROWS, NU_MULTI, NU_WIDE, NU_COUNT };
 static_assert(UNIT_COUNTERS + NU_COUNT <= N_COUNTERS, "near-field unit totals");
 
-// Lanes per near-field workgroup.  With 64 lanes a leaf of 33..64 targets leaves up to half of them
-// idle (one split), with 256 a twentieth, and four waves share a staged chunk: 1M cube (leaves of
-// about 32 bodies, mixed) P2P 5.58 -> 4.03 ms, 60k cube with c = 6 1.39 -> 1.18, 8k ring (FP64) 0.110
-// -> 0.075 ms.  64 lanes stay for the lists of a few entries that an adjoint of few probes leaves most
-// leaves with (1M blobs, 4096 probes, 1.6 entries a leaf: 2.96 against 3.08 ms for the whole pass),
-// where 256 lanes have nothing to share.
-constexpr int64_t WIDE_ENTRIES = 8;  // list entries per target leaf from which 256 lanes are used
-__device__ __forceinline__ bool units_wide(int64_t nleaf, int64_t max_leaf, unsigned long long np2p)
-{
-  return max_leaf > 64 || (int64_t)np2p >= WIDE_ENTRIES * nleaf;
-}
-
 __global__ void k_units_clear(unsigned long long *__restrict__ cnt)
 {
   if (threadIdx.x < NU_COUNT) cnt[threadIdx.x] = 0;
@@ -389,14 +377,17 @@ __global__ void k_units_clear(unsigned long long *__restrict__ cnt)
 // same-address atomics few.
 constexpr int UNITS_WORK_BLOCKS = 512;
 __global__ __launch_bounds__(256) void k_units_work(const int32_t *__restrict__ leaves, int64_t nleaf,
-                                                    int64_t max_leaf, const unsigned long long *__restrict__ np2p,
+                                                    int64_t max_leaf, int64_t nsleaf, double narrow, int lanes,
+                                                    const unsigned long long *__restrict__ np2p,
                                                     const int32_t *__restrict__ tnbody,
                                                     const int32_t *__restrict__ off, const int32_t *__restrict__ src,
                                                     const int32_t *__restrict__ snbody, uint32_t *__restrict__ work,
                                                     unsigned long long *__restrict__ cnt)
 {
   __shared__ unsigned long long sum[3][4];
-  const bool                    wide = units_wide(nleaf, max_leaf, *np2p);
+  // mean pairs a leaf (cell 0 is the root: all bodies)
+  const double pairs = (double)*np2p / nleaf * ((double)tnbody[0] / nleaf) * ((double)snbody[0] / nsleaf);
+  const bool   wide  = units_wide(nleaf, max_leaf, pairs, narrow, lanes);
   if (blockIdx.x == 0 && threadIdx.x == 0) cnt[NU_WIDE] = wide;
   const int          lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   unsigned long long inter = 0, all = 0, rows = 0;
@@ -673,7 +664,7 @@ void near_units_enqueue(hipStream_t s, Scratch &sc, const Tree &tt, const Tree &
   const int32_t *off = l.p2p_off.as<int32_t>();
   if (!cleared) k_units_clear<<<1, 64, 0, s>>>(cnt);
   k_units_work<<<(int)std::min<int64_t>(UNITS_WORK_BLOCKS, (tt.nleaf + 3) / 4), 256, 0, s>>>(
-      lv, tt.nleaf, max_leaf, np2p, tn, off, l.p2p_src.as<int32_t>(), st.nbody.as<int32_t>(),
+      lv, tt.nleaf, max_leaf, st.nleaf, sc.near_narrow, sc.near_lanes, np2p, tn, off, l.p2p_src.as<int32_t>(), st.nbody.as<int32_t>(),
       sc.unit_work.as<uint32_t>(), cnt);
   k_units_fill<<<(int)((tt.nleaf + 255) / 256), 256, 0, s>>>(lv, tt.nleaf, tn, off, sc.unit_work.as<uint32_t>(), rows,
                                                              cnt, l.units.as<int4>(), l.multi.as<int4>());

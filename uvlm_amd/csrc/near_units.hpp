@@ -51,4 +51,29 @@ constexpr int units_first(int len, int j, int n) { return (int)((int64_t)len * j
 constexpr int64_t units_bound(int64_t nleaf) { return nleaf + (int64_t)UNITS_AIM; }
 constexpr int64_t units_multi_bound(int64_t nleaf) { return nleaf < (int64_t)UNITS_AIM ? nleaf : (int64_t)UNITS_AIM; }
 
+// Lanes of a near-field workgroup: 64 for short lists of many small leaves, else 256.  256 lanes share a
+// staged chunk between four waves and leave fewer of them idle on a leaf of 33..64 targets (one
+// split of 64), but a list of a few hundred pairs does not fill them, and with few leaves a wavefront
+// each leaves the chip idle.  `pairs` is the mean number of pairs a leaf: list entries times the mean
+// leaf sizes of both trees.  P2P with 64 against 256 lanes (524,288 bodies, theta 0.5; us):
+//   pairs       40    133    560   1053   2034   3992   4864   7091  10445  16685
+//   mixed      400    474    436    307    515    365    372    519    390   1147
+//             1408   1541    957    573    719    436    432    544    401   1032
+//   FP64       673    800    756    659    831    772    778    755    973   1669
+//             1871   2039   1343    945   1030    773    777    761    785   1453
+// Mixed: 64 below NARROW_MIXED (two rings at 6482 pairs: 902 against 880).  FP64 holds twice the LDS a
+// lane and gains less from the shorter chunk: 64 below NARROW_FP64 (two rings of 60,000 at 2047 pairs
+// are level, a thin helix at 3337 loses 22%).  Below 8192 leaves 64 lanes leave the chip idle unless
+// lists are shorter still: 64 below nleaf / 8 pairs (FP64: 2482 leaves of 264 pairs 29 against 34 us,
+// 4630 of 560 pairs 29 against 47; 1951 of 468 pairs 46 against 35, 390 of 480 pairs 21 against 16).
+constexpr double  NARROW_MIXED = 6000.0, NARROW_FP64 = 1500.0;
+constexpr int64_t NARROW_LEAVES = 8192;
+// lanes: 64 or 256 where the caller asks for them (64 lanes hold leaves of up to 64 targets), else 0
+constexpr bool units_wide(int64_t nleaf, int64_t max_leaf, double pairs, double narrow, int lanes)
+{
+  if (max_leaf > 64) return true;
+  if (lanes) return lanes != 64;
+  return pairs >= (nleaf < NARROW_LEAVES ? (double)(nleaf / 8) : narrow);
+}
+
 }  // namespace uvlm
