@@ -130,7 +130,7 @@ struct Tree {
 struct Lists {
   int64_t np2p = 0, nm2l = 0, n_interactions = 0;
   DevBuf  p2p_off, p2p_src, m2l_off, m2l_src;  // int32
-  // near-field units of the P2P list (near_units): runs of entries of one target leaf each, rows of
+  // near-field units of the P2P list (near_units.hpp): runs of entries of one target leaf each, rows of
   // partial sums and leaves cut into several units
   int64_t n_units = 0, n_rows = 0, n_multi = 0;
   bool    wide = false;       // 256 lanes per unit's workgroup, else 64

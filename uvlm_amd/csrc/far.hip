@@ -1427,7 +1427,7 @@ __global__ __launch_bounds__(m2l_fixed(P).W * WG) __attribute__((amdgpu_waves_pe
 }
 
 // Below this many target cells (probe trees), long lists are cut into segments that run as
-// separate workgroups (see the P2P launcher for the same rule).
+// separate workgroups.
 constexpr int64_t M2L_SPLIT_TARGETS = 4096, M2L_SPLIT_SEGMENTS = 8192;
 
 // Segments of few targets' lists: target t's list in pieces of E entries, at least one (empty) piece;
@@ -2023,7 +2023,6 @@ void m2l(hipStream_t s, int P, const Tree &tt, const Tree &st, const Lists &l, c
 #undef UVLM_M2L_FIXED
 #undef UVLM_M2L_LAUNCH
 #undef UVLM_M2L_CALL_ARGS
-#undef UVLM_M2L_LAUNCH
     throw Error(UVLM_ERR_INTERNAL, "unsupported M2L plan size");
   }
 }

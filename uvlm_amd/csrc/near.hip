@@ -7,12 +7,12 @@
 //   u -= f1 (dX x a_j),   J[a][b] -= f2 (dX x a_j)_a dX_b + f1 eps_{abk} a_j,k.
 // Only the source core size sigma_j enters (multipoleKernels.hpp:243).
 //
-// Layout: one workgroup of BLK lanes (64 or 256) per unit of a target leaf's list (near_units).  Lanes = (target t) x (source split s): a pass takes ntp
-// of the leaf's targets (near_targets_per_pass) and S = BLK / ntp splits, each taking every S-th
-// source, and the partial sums are combined in a fixed order (LDS, no atomics).  The bodies of all
-// source leaves in the unit's list entries are streamed through LDS in full chunks across leaf
-// boundaries (prefix sums of the leaf sizes in LDS, binary search per slot), so small leaves do
-// not pay a barrier per leaf.
+// Layout: one workgroup of BLK lanes (64 or 256) per unit of a target leaf's list (near_units.hpp).
+// Lanes = (target t) x (source split s): a pass takes ntp of the leaf's targets
+// (near_targets_per_pass) and S = BLK / ntp splits, each taking every S-th source, and the partial
+// sums are combined in a fixed order (LDS, no atomics).  The bodies of all source leaves in the
+// unit's list entries are streamed through LDS in full chunks across leaf boundaries (prefix sums
+// of the leaf sizes in LDS, binary search per slot), so small leaves do not pay a barrier per leaf.
 //
 // FP64 path: G = g/s^3 and its derivative in double (pair_kernel.hpp), two sources per step.
 // Mixed path: FP32 arithmetic on coordinates relative to the target leaf centre (the source
@@ -21,8 +21,6 @@
 // accumulators; G = g/s^3 and its derivative from pair_kernel.hpp.
 #include "common.hpp"
 #include "pair_kernel.hpp"
-
-#include <vector>
 
 #include <algorithm>
 
@@ -76,7 +74,7 @@ template <class T> __device__ __forceinline__ void fold_antisym(T *acc)
 // transposed near-field kernel used by the adjoint (a particle's own sigma, with the
 // particle now on the target side).
 //
-// One workgroup per unit (near_units): the list entries [q0, q1) of target leaf w.  A leaf whose
+// One workgroup per unit (near_units.hpp): the list entries [q0, q1) of target leaf w.  A leaf whose
 // list is one unit is stored directly; a leaf cut into several units leaves each unit's sums
 // (12 rows of nt doubles) at part + 12 * row, and k_p2p_reduce adds them in unit order, so the
 // result does not depend on which unit runs when.
@@ -372,9 +370,9 @@ __global__ void k_units_clear(unsigned long long *__restrict__ cnt)
   if (threadIdx.x < NU_COUNT) cnt[threadIdx.x] = 0;
 }
 
-// work[w] (lane steps) of each target leaf and the sums over all: interactions, work, targets times work.  One
-// wavefront per leaf at a time, lanes over its list; at most UNITS_WORK_BLOCKS blocks keep the
-// same-address atomics few.
+// work[w] (lane steps) of each target leaf and the sums over all: interactions, work, targets times
+// work.  One wavefront per leaf at a time, lanes over its list; at most UNITS_WORK_BLOCKS blocks keep
+// the same-address atomics few.
 constexpr int UNITS_WORK_BLOCKS = 512;
 __global__ __launch_bounds__(256) void k_units_work(const int32_t *__restrict__ leaves, int64_t nleaf,
                                                     int64_t max_leaf, int64_t nsleaf, double narrow, int lanes,

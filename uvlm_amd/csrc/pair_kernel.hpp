@@ -129,7 +129,8 @@ __device__ __forceinline__ void g_far(float xq, float &G, float &Gp)
 //    small x (the formula loses a factor 1/x on f1 and 1/x^2 on f2).  3 rather than 2 (degree 14)
 //    costs 4 multiply-adds a pair and keeps more waves off the far form; 4 needs degree 18.
 //  * x >= 3: g = 1 - e^{-x} (erfcx(s) + (2/sqrt(pi)) s) as in FP32, with rsq refined by one cubic
-//    step, a degree-11 e^r on |r| <= ln 2 / 2 and erfcx as a degree-11 minimax polynomial in
+//    step, e^r on |r| <= ln 2 / 2 by its degree-11 interpolant at the Chebyshev nodes there (c_exp64,
+//    computed in 60 digits as the others), and erfcx as a degree-11 minimax polynomial in
 //    w = 1/s whose error weighted by e^{-x} is 1.2e-17.  From x = FAR64 = 44 on, e^{-x} no longer
 //    shows in G or G' and a wave all of whose lanes are there skips it.
 constexpr double X64 = 3.0, FAR64 = 44.0;

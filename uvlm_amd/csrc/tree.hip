@@ -71,13 +71,13 @@ __global__ void k_bounds_partial(const double *__restrict__ x, const double *__r
     for (int d = 0; d < 6; d++) part[blockIdx.x * 6 + d] = s[d][0];
 }
 
-// X0 and R0 exactly as tree.hpp:19-25 computes them from Xmin/Xmax (one workgroup of BLK;
-// min and max are exact in any order, so the parallel reduction gives the serial result).
 // Totals of a build (32-bit): cells per level, leaves per level, error bits (0: deeper than the key holds;
 // 1: a split needs a digit below the sorted ones).
 enum { TOT_LEVEL = 0, TOT_LEAVES = 24, TOT_ERR = 47, TOT_COUNT = 48 };
 static_assert(4 * TOT_COUNT <= 8 * N_COUNTERS, "build totals");
 
+// X0 and R0 exactly as tree.hpp:19-25 computes them from Xmin/Xmax (one workgroup of BLK;
+// min and max are exact in any order, so the parallel reduction gives the serial result).
 __global__ __launch_bounds__(BLK) void k_bounds_final(const double *part, int nb, double *X0R0, uint32_t *tot)
 {
   __shared__ double s[6][BLK];
@@ -406,10 +406,10 @@ struct TreeView {
   const double  *cx, *cy, *cz, *R;
 };
 
-// Counters of a traversal (64-bit, sc.counters): list sizes so far, flags (1 frontier, 2 P2P, 4 M2L
-// buffer overflowed: the traversal starts again with larger ones; 8 a row longer than ROW_LONG), the
-// largest frontier, the frontier sizes of steps k, k + 1, k + 2 (mod 4), and the rows longer than
-// ROW_RANK.
+// Counters of a traversal (64-bit, sc.counters): list sizes so far, flags (TF_FRONT: the frontier's
+// buffer overflowed; TF_LONG: a row longer than ROW_LONG), the largest frontier, the frontier sizes of
+// steps k, k + 1, k + 2 (mod 4), and the rows longer than ROW_RANK.  The host adds TF_P2P and TF_M2L
+// where a list's size passes its buffer; after an overflow the traversal starts again with larger ones.
 enum { TC_P2P = 0, TC_M2L = 1, TC_FLAGS = 2, TC_MAXF = 3, TC_FRONT = 4, TC_LONG = 8, TC_COUNT = 9 };
 static_assert(TC_COUNT <= UNIT_COUNTERS, "traversal counters");
 enum { TF_FRONT = 1, TF_P2P = 2, TF_M2L = 4, TF_LONG = 8 };
@@ -1114,8 +1114,8 @@ static TreeView view(const Tree &t)
 }
 
 // CSR rows by target of the np P2P and nm M2L pairs in sc.out_p2p / out_m2l (their numbers are read
-// on the device; np and nm bound them).  C target cells, entries below Cs.
-// C target cells, Cs source cells; zeroed: the caller has cleared the row counts.
+// on the device; np and nm bound them).  C target cells, Cs source cells; zeroed: the caller has
+// cleared the row counts.
 static void rows_by_counting(hipStream_t s, Scratch &sc, int64_t C, int64_t Cs, int64_t np, int64_t nm, bool zeroed,
                              Lists &l)
 {
