@@ -172,3 +172,23 @@ def test_get_list_of_cells_that_share_children(orc):
     assert len(set(want[0])) < len(want[0])
     assert np.array_equal(p2p[: a.value], np.array(sorted(want[0])))
     assert np.array_equal(m2l[: b.value], np.array(sorted(want[1])).reshape(-1, 2))
+
+
+def test_a_refused_tree_leaves_the_last_one():
+    """A build that is refused as too deep leaves the last tree and its lists in use."""
+    X = points(900, 3, 1e-2, 1)
+    g = FMMCalculator(P=4, theta=0.5, ncrit=8)
+    g.set_bodies(make_bodies(X, X, np.full(900, 0.1)))
+    g.build()
+    g.calculate()
+    want = g.arrays()
+    g.update_arrays(X=np.repeat(want["X"][:1], 900, 0))
+    print("[tree] refused rebuild", flush=True)
+    with pytest.raises(UVLMError):
+        g.build()
+    g.update_arrays(X=want["X"])
+    g.calculate()
+    got = g.arrays()
+    assert np.array_equal(got["X"], want["X"]) and np.isfinite(got["velocity"]).all()
+    assert np.linalg.norm(got["velocity"] - want["velocity"]) < 1e-12 * np.linalg.norm(want["velocity"])
+    g.close()

@@ -172,7 +172,14 @@ void do_build(uvlm_handle h, bool defer_outputs = false)
   hipStream_t s = h->s;
   UVLM_HIP(hipEventRecord(h->ev[EV_B0], s));
   resolve_outputs(h);
-  build_tree(s, h->sc, h->F(F_X), h->F(F_X + 1), h->F(F_X + 2), h->N, h->prm.ncrit, h->tree, h->perm.as<int32_t>());
+  try {
+    build_tree(s, h->sc, h->F(F_X), h->F(F_X + 1), h->F(F_X + 2), h->N, h->prm.ncrit, h->tree, h->perm.as<int32_t>());
+  } catch (const Error &e) {
+    if (e.code != UVLM_ERR_DEPTH) h->built = false;  // (a tree that is too deep leaves the last one as it was)
+    throw;
+  }
+  // the last lists and their units are not of this tree: nothing runs over them if what follows fails
+  h->built = h->evaluated = false;
   uint8_t fields[N_FIELDS];
   int     nf = 0;
   for (int f = 0; f < N_FIELDS; f++) {
